@@ -1129,11 +1129,12 @@ int pca_nearest_binned(const void *x, const void *y, const int64_t *ptr_x,
 size_t pca_fps_workspace_bytes(int64_t n, int64_t d, int64_t num_segments,
                                int64_t max_segment_rows, int dtype) {
   if (n < 0 || n > kMaxRows || d < 1 || d > (1 << 20) || num_segments < 1 ||
-      !nearest_dtype_ok(dtype))
+      num_segments > kMaxRows || !nearest_dtype_ok(dtype))
     return 0;
-  if (pca::fps_in_registers(dtype, (int)d, max_segment_rows))
-    return 256;
-  return align256(pca::fps_dist_bytes(n)) + 256;
+  return align256(pca::fps_scratch_bytes(dtype, (int)n, (int)d,
+                                         (int)num_segments,
+                                         max_segment_rows)) +
+         256;
 }
 
 int pca_fps(const void *src, const int64_t *ptr, const int64_t *out_ptr,
@@ -1164,9 +1165,10 @@ int pca_fps(const void *src, const int64_t *ptr, const int64_t *out_ptr,
       workspace_bytes < need)
     return fail(PCA_ERR_WORKSPACE, "workspace needs %zu bytes, 256-aligned",
                 need);
-  return check_launch(pca::launch_fps(dtype, src, ptr, out_ptr, start, (int)d,
-                                      (int)num_segments, max_segment_rows,
-                                      workspace, out, stream),
+  return check_launch(pca::launch_fps(dtype, src, ptr, out_ptr, start, (int)n,
+                                      (int)d, (int)num_segments,
+                                      max_segment_rows, workspace,
+                                      being_captured(stream), out, stream),
                       "fps kernel");
 }
 

@@ -303,6 +303,22 @@ __device__ __forceinline__ int find_segment(const int *__restrict__ start,
   return lo;
 }
 
+// The same over int64 pointers (NULL: one segment).
+__device__ __forceinline__ int find_segment64(const int64_t *__restrict__ ptr,
+                                              int num_segments, int64_t v) {
+  if (ptr == nullptr)
+    return 0;
+  int lo = 0, hi = num_segments;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (ptr[mid] <= v)
+      lo = mid;
+    else
+      hi = mid;
+  }
+  return lo;
+}
+
 // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  This
 // maps the hardware block id to a logical one such that blocks with
 // neighbouring logical ids (which scan the same segment of x) land on the same

@@ -17,19 +17,20 @@
 //   * `best` starts at -1 and `best_idx` at 0: when no row has a value above
 //     -1 (every distance NaN) the sample is row 0.
 //
-// The sampling is a chain of dependent steps, each a pass over the example's
-// rows plus a workgroup-wide arg-max, so the time per sample is what counts.
-// fps_reg_kernel keeps the rows and their running minima in REGISTERS (up to
-// 16 rows per thread: examples of up to 16,384 rows of up to 4 dimensions),
-// and needs one barrier per sample: every wave finds its best row with two
-// reductions of 32-bit keys by data-parallel lane shifts (value, then tie),
-// the lane that holds it writes value, tie and coordinates to LDS, and after
-// the barrier every row of 16 lanes picks the winner among the 16 wave
-// results the same way and reads its coordinates.  fps_any_kernel (any size,
-// dimension and element type) streams the rows and a `dist` array from memory
-// instead.
+// The sampling is a chain of dependent steps, each an arg-max over the
+// example's rows, so the time per sample is what counts, and an example is one
+// workgroup's (a step that several workgroups share costs two trips through
+// the L2).  Up to 1,024 rows of up to 4 dimensions fps_reg_kernel looks at
+// every row in every step, from registers.  Beyond that most rows are left
+// alone (see "rows in buckets" below): fps_lds_kernel keeps up to 8,192 rows in
+// LDS, fps_bucket_kernel up to 16,384 in registers, fps_stream_kernel any
+// number in memory (up to 3 dimensions).  fps_any_kernel (any size, dimension
+// and element type) streams the rows and a `dist` array from memory.
 #include "device_utils.hpp"
 #include "launchers.hpp"
+
+#include <algorithm>
+#include <type_traits>
 
 #include <hip/hip_fp16.h>
 
@@ -81,6 +82,21 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
   PCA_DPP_UMAX(v, 0x142, 0xa); // row_bcast:15 into rows 1 and 3
   PCA_DPP_UMAX(v, 0x143, 0xc); // row_bcast:31 into rows 2 and 3
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+// U waves' worth of values at once: their steps fill each other's wait states.
+template <int U> __device__ __forceinline__ void wave_umax_of(uint32_t (&v)[U]) {
+#define PCA_DPP_EACH(ctrl, rows)                                               \
+  _Pragma("unroll") for (int u = 0; u < U; ++u) PCA_DPP_UMAX(v[u], ctrl, rows)
+  PCA_DPP_EACH(0x111, 0xf);
+  PCA_DPP_EACH(0x112, 0xf);
+  PCA_DPP_EACH(0x114, 0xf);
+  PCA_DPP_EACH(0x118, 0xf);
+  PCA_DPP_EACH(0x142, 0xa);
+  PCA_DPP_EACH(0x143, 0xc);
+#undef PCA_DPP_EACH
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    v[u] = (uint32_t)__builtin_amdgcn_readlane((int)v[u], 63);
 }
 #undef PCA_DPP_UMAX
 
@@ -220,7 +236,7 @@ __global__ __launch_bounds__(kFpsThreads) void fps_any_kernel(
   }
 }
 
-// ---- fp32, up to 4 dimensions, up to T * P rows per example -------------------
+// ---- fp32, up to 4 dimensions, up to 1,024 rows per example -------------------
 
 // T threads hold P rows each.  With T = 256 S, thread t has the rows
 // t / S + 256 * ((t % S) * P + i), i < P, of its example; a single wave
@@ -433,30 +449,903 @@ __global__ __launch_bounds__(T) void fps_reg_kernel(
   }
 }
 
+// ---- fp32, up to 4 dimensions: rows in buckets, most of them left alone -------
+//
+// A new sample lowers the running minimum only of rows nearer to it than the
+// samples before it, so most rows of an example need no distance at all.  The
+// rows are ordered along a space-filling curve and cut into buckets of 64
+// (one row per lane); the wave that owns a bucket keeps, in one lane of its
+// registers, the bucket's box, its largest running minimum and the row that
+// has it.  Per sample a lane tests its bucket: if the distance from the sample
+// to the box -- formed with the operations of the exact chain on per-axis gaps
+// no larger than any row's difference, hence, rounding being monotone, not
+// above the COMPUTED distance of any of its rows -- is not below the bucket's
+// largest minimum, no minimum of the bucket changes and it is skipped;
+// otherwise the whole wave goes through its 64 rows.  Same values, and so the
+// same samples, as looking at every row.
+//
+// What bounds it: the chain of one step (arg-max over the buckets, box test,
+// one bucket, hand-over through LDS, one barrier), not the rows.  Buckets go
+// round-robin to the waves, so that the few neighbouring ones a sample
+// touches are looked at side by side.
+
+constexpr uint32_t kFpsNoRow = 0xffffffffu; // its tie is the largest one
+
+// What a wave hands over: the largest running minimum (bits of a float that
+// is not negative), the row that has it, and that row's coordinates.
+template <int DIM> struct FpsBest {
+  uint32_t val, rel;
+  float x[DIM];
+};
+
+// Of the lanes in `who` (equal values) the one whose row comes first in the
+// reference's order; the lanes of `who` hold it in `rel`.
+__device__ __forceinline__ int fps_first(uint64_t who, uint32_t rel) {
+  if (__builtin_expect((who & (who - 1)) != 0, 0)) {
+    const int lane = threadIdx.x & (kWave - 1);
+    // (formed here: outside the loop it would take a register per bucket)
+    asm volatile("" : "+v"(rel));
+    // (umax of the complement: the smallest tie; lanes outside take 0)
+    const uint32_t t = (who >> lane) & 1 ? ~fps_tie(rel) : 0u;
+    const uint32_t top = wave_umax(t);
+    who &= __ballot(t == top);
+  }
+  return (int)__builtin_ctzll(who);
+}
+
+// A lane's value, uniform.  (In a scalar register right here: moved into a
+// branch that only some lanes take, the read would see the registers as those
+// lanes left them.)
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) {
+  int s = __builtin_amdgcn_readlane((int)v, lane);
+  asm volatile("" : "+s"(s));
+  return (uint32_t)s;
+}
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __uint_as_float(lane_value(__float_as_uint(v), lane));
+}
+
+// Lower bound of the chain's distance from a sample to any row of a box.
 template <int DIM>
-hipError_t launch_fps_reg(const float *src, const int64_t *ptr,
-                          const int64_t *out_ptr, const int64_t *start, int d,
-                          int num_segments, int64_t max_rows, int64_t *out,
-                          hipStream_t stream) {
-#define PCA_FPS_REG(P_, T_)                                                    \
-  hipLaunchKernelGGL((fps_reg_kernel<DIM, P_, T_>), dim3(num_segments),        \
-                     dim3(T_), 0, stream, src, ptr, out_ptr, start, d, out)
-  // (shapes by measurement: 16 examples of each size on one device)
+__device__ __forceinline__ float fps_box_distance(const float (&q)[DIM],
+                                                  const float (&lo)[DIM],
+                                                  const float (&hi)[DIM]) {
+  float dd = 0.0f;
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) {
+    // (a NaN in the sample leaves a gap of 0: the bucket is looked at)
+    const float gap = __builtin_fmaxf(
+        __builtin_fmaxf(lo[c] - q[c], q[c] - hi[c]), 0.0f);
+    dd = c == 0 ? gap * gap : __builtin_fmaf(gap, gap, dd);
+  }
+  return dd;
+}
+
+// Distance of a row to the sample, and the row's running minimum with it.
+template <int DIM>
+__device__ __forceinline__ float fps_lower(const float (&q)[DIM],
+                                           const float (&x)[DIM], float m) {
+  float dd = 0.0f;
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) {
+    // (zero components beyond d add fma(0, 0, acc) = acc)
+    const float t = q[c] - x[c];
+    dd = c == 0 ? t * t : __builtin_fmaf(t, t, dd);
+  }
+  // a NaN loses to a number, as in fminf; `m` is never a NaN
+  asm("v_min_f32 %0, %1, %2" : "=v"(dd) : "v"(m), "v"(dd));
+  return dd;
+}
+
+// 10 bits spread to every third position
+__device__ __forceinline__ uint32_t fps_spread3(uint32_t v) {
+  v &= 0x3ffu;
+  v = (v | (v << 16)) & 0x030000ffu;
+  v = (v | (v << 8)) & 0x0300f00fu;
+  v = (v | (v << 4)) & 0x030c30c3u;
+  v = (v | (v << 2)) & 0x09249249u;
+  return v;
+}
+
+// Waits for this workgroup's LDS traffic and meets its other waves (global
+// stores stay in flight: what a wave stores only it reads again).
+__device__ __forceinline__ void fps_meet() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// The rows of an example in curve order, by one workgroup: afterwards keys[i],
+// i < count, holds the i-th row's number (relative to the example) in its
+// REL_BITS low bits, above them its cell of the example's box.  `part`: 6 W
+// floats of LDS.
+template <int W, int DIM, int REL_BITS>
+__device__ __forceinline__ void
+fps_curve_order(const float *__restrict__ rows, int count, int d,
+                uint32_t *keys, float (*part)[W]) {
+  constexpr int T = W * kWave;
+  constexpr int AXIS_BITS = (32 - REL_BITS) / 3;
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = tid / kWave;
+  float lo[3], hi[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    lo[c] = __builtin_inff();
+    hi[c] = -__builtin_inff();
+  }
+  for (int i = tid; i < count; i += T) {
+#pragma unroll
+    for (int c = 0; c < (DIM < 3 ? DIM : 3); ++c)
+      if (c < d) {
+        const float v = rows[(size_t)i * d + c];
+        if (__builtin_fabsf(v) < __builtin_inff()) {
+          lo[c] = __builtin_fminf(lo[c], v);
+          hi[c] = __builtin_fmaxf(hi[c], v);
+        }
+      }
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+#pragma unroll
+    for (int sh = 1; sh < kWave; sh <<= 1) {
+      lo[c] = __builtin_fminf(lo[c], __shfl_xor(lo[c], sh));
+      hi[c] = __builtin_fmaxf(hi[c], __shfl_xor(hi[c], sh));
+    }
+    if (lane == 0) {
+      part[c][wave] = lo[c];
+      part[3 + c][wave] = hi[c];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      lo[c] = __builtin_fminf(lo[c], part[c][w]);
+      hi[c] = __builtin_fmaxf(hi[c], part[3 + c][w]);
+    }
+  }
+  int n2 = kWave;
+  while (n2 < count)
+    n2 <<= 1;
+  for (int i = tid; i < n2; i += T) {
+    uint32_t key = 0xffffffffu;
+    if (i < count) {
+      uint32_t code = 0;
+#pragma unroll
+      for (int c = 0; c < (DIM < 3 ? DIM : 3); ++c) {
+        uint32_t cell = 0;
+        if (c < d) {
+          const float cells = (float)(1 << AXIS_BITS);
+          const float t =
+              (rows[(size_t)i * d + c] - lo[c]) / (hi[c] - lo[c]) * cells;
+          // (NaN, also from a flat box, fails the comparison)
+          cell = t >= 0.0f ? (uint32_t)__builtin_fminf(t, cells - 1.0f) : 0u;
+        }
+        code |= fps_spread3(cell) << c;
+      }
+      key = (code << REL_BITS) | (uint32_t)i;
+    }
+    keys[i] = key;
+  }
+  __syncthreads();
+  // bitonic sort; exchanges over fewer than 64 places inside the waves
+  for (int k = kWave; k <= n2; k <<= 1) {
+    for (int j = k >> 1; j >= kWave; j >>= 1) {
+      for (int i = tid; i < n2 / 2; i += T) {
+        const int a = ((i & ~(j - 1)) << 1) | (i & (j - 1));
+        const uint32_t u = keys[a], v = keys[a | j];
+        if ((u > v) == ((a & k) == 0)) {
+          keys[a] = v;
+          keys[a | j] = u;
+        }
+      }
+      __syncthreads();
+    }
+    for (int i = tid; i < n2; i += T) {
+      uint32_t u = keys[i];
+      auto exchange = [&](int j, bool up) {
+        const uint32_t v = (uint32_t)__shfl_xor((int)u, j);
+        u = ((lane & j) == 0) == up ? min(u, v) : max(u, v);
+      };
+      if (k == kWave) {
+#pragma unroll
+        for (int kk = 2; kk < kWave; kk <<= 1)
+#pragma unroll
+          for (int j = kk >> 1; j > 0; j >>= 1)
+            exchange(j, (lane & kk) == 0);
+      }
+#pragma unroll
+      for (int j = kWave / 2; j > 0; j >>= 1)
+        exchange(j, (i & k) == 0);
+      keys[i] = u;
+    }
+    __syncthreads();
+  }
+}
+
+// Examples of up to 4,096 R rows: everything a step needs of a bucket -- its
+// box and its best row -- is in one lane of EVERY wave's registers (64 buckets
+// of 64 R rows), the rows and their running minima are in LDS.  All waves see
+// the same buckets pass, so they share them out without asking each other,
+// whichever wave is free of work taking part; the new best of a bucket
+// reaches the other waves through LDS, one barrier per step.
+//
+// 16 uniform clouds, a quarter sampled, per step (before: every row of a cloud
+// from the registers of 8 waves): 2,048 rows 0.60 -> 0.57 us, 4,096 0.68 ->
+// 0.58, 8,192 0.84 -> 0.65.  About 0.55 us of that is the chain of a step with a
+// single bucket, ~100 dependent instructions and three LDS round trips; at
+// 1,024 rows fps_reg_kernel's chain is as short.  16 waves measured faster
+// than 8 (0.62 us at 4,096 rows) and 4 (0.83): a wave rarely meets two of the
+// 9 buckets that pass.
+template <int DIM, int W, int R>
+__global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
+    const float *__restrict__ src, const int64_t *__restrict__ ptr,
+    const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
+    int d, int64_t *__restrict__ out) {
+  constexpr int T = W * kWave;
+  constexpr int CAP = 64 * kWave * R;
+  constexpr int REL_BITS = R == 1 ? 12 : 13;
+  static_assert(R == 1 || R == 2, "row numbers of 13 bits");
+  constexpr int PER = CAP / T;
+  constexpr int STRIDE = DIM <= 3 ? 4 : 5; // words of a row
+  constexpr int AT_M = STRIDE - 1;
+  __shared__ __align__(16) float rows_lds[CAP * STRIDE];
+  __shared__ uint16_t perm[CAP + 2];
+  __shared__ float part[2 * 3][W];
+  __shared__ __align__(16) float table[2][kWave][8]; // value, place, x ...
+  __shared__ uint16_t sampled[kWave];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int b = blockIdx.x;
+  const int64_t start_idx = ptr[b];
+  // (CAP: the caller's bound on the rows of an example)
+  const int count = (int)min(ptr[b + 1] - start_idx, (int64_t)CAP);
+  const int64_t o_begin = out_ptr[b];
+  const int64_t o_end = out_ptr[b + 1];
+  if (o_begin >= o_end)
+    return;
+  const float *rows = src + (size_t)start_idx * d;
+  const int buckets = (count + kWave * R - 1) / (kWave * R);
+
+  uint32_t *keys = reinterpret_cast<uint32_t *>(rows_lds);
+  fps_curve_order<W, DIM, REL_BITS>(rows, count, d, keys, part);
+  // (the keys give way to the rows)
+  uint16_t rel[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int at = i * T + tid;
+    rel[i] = at < count ? (uint16_t)(keys[at] & ((1u << REL_BITS) - 1))
+                        : (uint16_t)0xffffu;
+  }
+  __syncthreads();
+#pragma unroll 4
+  for (int i = 0; i < PER; ++i) {
+    const int at = i * T + tid;
+    if (at >= buckets * kWave * R)
+      break;
+    const bool ok = rel[i] != 0xffffu;
+    perm[at] = rel[i];
+#pragma unroll
+    for (int c = 0; c < (DIM <= 3 ? 3 : DIM); ++c)
+      rows_lds[at * STRIDE + c] =
+          ok && c < d ? rows[(size_t)rel[i] * d + c] : 0.0f;
+    // (places without a row: minimum 0 and the last of all ties)
+    rows_lds[at * STRIDE + AT_M] = ok ? 5e4f : 0.0f;
+  }
+  if (tid == 0)
+    perm[CAP] = 0xffffu;
+  __syncthreads();
+
+  // lane = bucket: its box, and the best of its rows.  (Every minimum is 5e4
+  // before the first sample; the first test lets every bucket through.)
+  float blo[DIM], bhi[DIM], bx[DIM];
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) {
+    blo[c] = __builtin_inff();
+    bhi[c] = -__builtin_inff();
+    bx[c] = 0.0f;
+  }
+  {
+    // (a wave goes through its share of the buckets, a row per lane; the
+    // boxes then travel through the table)
+    for (int i = wave; i < buckets; i += W) {
+      float l[DIM], h[DIM];
+#pragma unroll
+      for (int c = 0; c < DIM; ++c) {
+        l[c] = __builtin_inff();
+        h[c] = -__builtin_inff();
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int at = (i * R + r) * kWave + lane;
+        const bool ok = at < count;
+#pragma unroll
+        for (int c = 0; c < DIM; ++c) {
+          // (fminf / fmaxf drop a NaN; such a row's minimum never changes)
+          const float v = rows_lds[at * STRIDE + c];
+          l[c] = __builtin_fminf(l[c], ok ? v : __builtin_inff());
+          h[c] = __builtin_fmaxf(h[c], ok ? v : -__builtin_inff());
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < DIM; ++c) {
+#pragma unroll
+        for (int sh = 1; sh < kWave; sh <<= 1) {
+          l[c] = __builtin_fminf(l[c], __shfl_xor(l[c], sh));
+          h[c] = __builtin_fmaxf(h[c], __shfl_xor(h[c], sh));
+        }
+        if (lane == 0) {
+          table[0][i][c] = l[c];
+          table[1][i][c] = h[c];
+        }
+      }
+    }
+    __syncthreads();
+    if (lane < buckets) {
+#pragma unroll
+      for (int c = 0; c < DIM; ++c) {
+        blo[c] = table[0][lane][c];
+        bhi[c] = table[1][lane][c];
+      }
+    }
+    __syncthreads();
+  }
+  uint32_t val = lane < buckets ? __float_as_uint(__builtin_inff()) : 0u;
+  int place = CAP; // (of no row)
+
+  float cur[DIM];
+  {
+    const int64_t first = start_idx + (start ? start[b] : 0);
+    if (tid == 0)
+      out[o_begin] = first;
+#pragma unroll
+    for (int c = 0; c < DIM; ++c)
+      cur[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
+  }
+
+  // of the lanes `who` of equal value the one whose place holds the row that
+  // comes first in the reference's order
+  auto first_of = [&](uint64_t who, int at_place) -> int {
+    if (__builtin_expect((who & (who - 1)) != 0, 0))
+      return fps_first(who, perm[at_place]);
+    return (int)__builtin_ctzll(who);
+  };
+  const int steps = (int)(o_end - o_begin);
+  for (int m = 1; m < steps; ++m) {
+    const int par = m & 1;
+    const bool passes =
+        !(fps_box_distance<DIM>(cur, blo, bhi) >= __uint_as_float(val));
+    const uint64_t pass = __ballot(passes);
+    const int passing = __builtin_popcountll(pass);
+    // (how many passing buckets come before this lane's)
+    const int before = __builtin_amdgcn_mbcnt_hi(
+        (uint32_t)(pass >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)pass, 0u));
+    const int rank = passes ? before : -1;
+    for (int j = wave; j < passing; j += W) {
+      const int bucket = (int)__builtin_ctzll(__ballot(rank == j));
+      float x[R][DIM], low[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const float *row = rows_lds + ((bucket * R + r) * kWave + lane) * STRIDE;
+        if (DIM <= 3) {
+          const float4 v = *reinterpret_cast<const float4 *>(row);
+          x[r][0] = v.x;
+          if (DIM > 1)
+            x[r][DIM > 1 ? 1 : 0] = v.y;
+          if (DIM > 2)
+            x[r][DIM > 2 ? 2 : 0] = v.z;
+          low[r] = v.w;
+        } else {
+#pragma unroll
+          for (int c = 0; c < DIM; ++c)
+            x[r][c] = row[c];
+          low[r] = row[AT_M];
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        low[r] = fps_lower<DIM>(cur, x[r], low[r]);
+        rows_lds[((bucket * R + r) * kWave + lane) * STRIDE + AT_M] = low[r];
+      }
+      uint32_t most = __float_as_uint(low[0]);
+      if (R == 2)
+        most = max(most, __float_as_uint(low[R - 1]));
+      const uint32_t top = wave_umax(most);
+      // which of a lane's two rows has the value; both: the earlier one
+      int at_place = bucket * R * kWave + lane;
+      int r = 0;
+      if (R == 2) {
+        r = __float_as_uint(low[0]) == top ? 0 : 1;
+        const bool both = r == 0 && __float_as_uint(low[R - 1]) == top;
+        if (__builtin_expect(__ballot(both) != 0, 0)) {
+          if (both && fps_tie(perm[at_place + kWave]) < fps_tie(perm[at_place]))
+            r = 1;
+        }
+        at_place += r * kWave;
+      }
+      const int at = first_of(__ballot(most == top), at_place);
+      if (lane == at) {
+        float *e = table[par][bucket];
+        float4 head;
+        head.x = __uint_as_float(top);
+        head.y = __int_as_float(at_place);
+        head.z = r ? x[R - 1][0] : x[0][0];
+        head.w = r ? x[R - 1][DIM > 1 ? 1 : 0] : x[0][DIM > 1 ? 1 : 0];
+        *reinterpret_cast<float4 *>(e) = head;
+#pragma unroll
+        for (int c = 2; c < DIM; ++c)
+          e[2 + c] = r ? x[R - 1][c] : x[0][c];
+      }
+    }
+    fps_meet();
+    if (passes) {
+      const float *e = table[par][lane];
+      const float4 head = *reinterpret_cast<const float4 *>(e);
+      val = __float_as_uint(head.x);
+      place = __float_as_int(head.y);
+      bx[0] = head.z;
+      if (DIM > 1)
+        bx[DIM > 1 ? 1 : 0] = head.w;
+#pragma unroll
+      for (int c = 2; c < DIM; ++c)
+        bx[c] = e[2 + c];
+    }
+    const uint32_t top = wave_umax(val);
+    const int at = first_of(__ballot(val == top), place);
+#pragma unroll
+    for (int c = 0; c < DIM; ++c)
+      cur[c] = lane_value(bx[c], at);
+    if (wave == 0) {
+      // (64 samples are written out at a time: the store's way to memory is
+      // then no part of a step)
+      const int chosen = (int)lane_value((uint32_t)place, at);
+      if (lane == 0)
+        sampled[m & (kWave - 1)] = (uint16_t)chosen;
+      if ((m & (kWave - 1)) == kWave - 1 || m == steps - 1) {
+        const int from = m & ~(kWave - 1);
+        if (from + lane <= m && from + lane > 0)
+          out[o_begin + from + lane] = start_idx + perm[sampled[lane]];
+      }
+    }
+  }
+}
+
+// Examples of up to 64 W P rows: bucket i of wave w is in the registers of
+// that wave (row of a lane in px[.][i], pm[i]), its box and best in lane i.
+// The buckets of 16,384 rows (and those of 4 dimensions beyond 4,096) do not
+// fit the LDS.  8 x 16,384 uniform rows, a quarter sampled: 1.27 -> 0.86 us
+// per step (before: every row, from the same registers).
+template <int DIM, int W, int P>
+__global__ __launch_bounds__(W *kWave) void fps_bucket_kernel(
+    const float *__restrict__ src, const int64_t *__restrict__ ptr,
+    const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
+    int d, int64_t *__restrict__ out) {
+  constexpr int T = W * kWave;
+  constexpr int CAP = T * P;
+  constexpr int REL_BITS = 14;
+  static_assert(CAP <= 16384 && P <= 16 && W <= 16, "row numbers in the keys");
+  __shared__ uint32_t keys[CAP];
+  __shared__ float part[2 * 3][W];
+  __shared__ FpsBest<DIM> table[2][W];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int b = blockIdx.x;
+  const int64_t start_idx = ptr[b];
+  // (CAP: the caller's bound on the rows of an example)
+  const int count = (int)min(ptr[b + 1] - start_idx, (int64_t)CAP);
+  const int64_t o_begin = out_ptr[b];
+  const int64_t o_end = out_ptr[b + 1];
+  if (o_begin >= o_end)
+    return;
+  const float *rows = src + (size_t)start_idx * d;
+
+  fps_curve_order<W, DIM, REL_BITS>(rows, count, d, keys, part);
+
+  // -- the buckets of this wave -----------------------------------------------
+  float px[DIM][P];
+  float pm[P];
+  uint32_t pr[P];
+  float blo[DIM], bhi[DIM];
+  FpsBest<DIM> best; // of the bucket of this lane
+  best.val = 0u;
+  best.rel = kFpsNoRow;
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) {
+    blo[c] = 0.0f;
+    bhi[c] = 0.0f;
+    best.x[c] = 0.0f;
+  }
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    const int pos = (i * W + wave) * kWave + lane;
+    const bool ok = pos < count;
+    const int rel = ok ? (int)(keys[pos] & (CAP - 1)) : 0;
+    pr[i] = ok ? (uint32_t)rel : kFpsNoRow;
+    // (lanes without a row: minimum 0 and the last of all ties)
+    pm[i] = ok ? 5e4f : 0.0f;
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) {
+      const float v = ok && c < d ? rows[(size_t)rel * d + c] : 0.0f;
+      px[c][i] = v;
+      asm volatile("" : "+v"(px[c][i]));
+      // (fminf / fmaxf drop a NaN; such a row's minimum never changes)
+      float l = ok ? v : __builtin_inff(), h = ok ? v : -__builtin_inff();
+#pragma unroll
+      for (int sh = 1; sh < kWave; sh <<= 1) {
+        l = __builtin_fminf(l, __shfl_xor(l, sh));
+        h = __builtin_fmaxf(h, __shfl_xor(h, sh));
+      }
+      if (lane == i) {
+        blo[c] = l;
+        bhi[c] = h;
+      }
+    }
+    // (before the first sample every minimum is 5e4: any value will do, the
+    // first test must let every bucket with rows through)
+    if (lane == i && (i * W + wave) * kWave < count)
+      best.val = __float_as_uint(__builtin_inff());
+    // (one bucket after the other: all loads and reductions at once would
+    // take several times the registers the loop below needs)
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  const int64_t first = start_idx + (start ? start[b] : 0);
+  if (tid == 0)
+    out[o_begin] = first;
+  float cur[DIM];
+#pragma unroll
+  for (int c = 0; c < DIM; ++c)
+    cur[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
+
+  for (int64_t m = o_begin + 1; m < o_end; ++m) {
+    const int par = (int)(m & 1);
+    uint32_t pass = (uint32_t)__ballot(
+        !(fps_box_distance<DIM>(cur, blo, bhi) >= __uint_as_float(best.val)));
+    // (every bucket's code with its own registers: a uniform branch each,
+    // four at a time where none passes)
+#pragma unroll
+    for (int g = 0; g < P; g += 4) {
+      if ((pass & (0xfu << g)) == 0)
+        continue;
+#pragma unroll
+      for (int i = g; i < (g + 4 < P ? g + 4 : P); ++i) {
+        if ((pass & (1u << i)) == 0)
+          continue;
+        float x[DIM];
+#pragma unroll
+        for (int c = 0; c < DIM; ++c)
+          x[c] = px[c][i];
+        pm[i] = fps_lower<DIM>(cur, x, pm[i]);
+        const uint32_t bits = __float_as_uint(pm[i]);
+        const uint32_t top = wave_umax(bits);
+        const int at = fps_first(__ballot(bits == top), pr[i]);
+        const uint32_t row = lane_value(pr[i], at);
+        float at_x[DIM];
+#pragma unroll
+        for (int c = 0; c < DIM; ++c)
+          at_x[c] = lane_value(x[c], at);
+        const bool mine = lane == i;
+        best.val = mine ? top : best.val;
+        best.rel = mine ? row : best.rel;
+#pragma unroll
+        for (int c = 0; c < DIM; ++c)
+          best.x[c] = mine ? at_x[c] : best.x[c];
+      }
+    }
+    {
+      const uint32_t top =
+          (uint32_t)__builtin_amdgcn_readlane((int)row16_umax(best.val), 15);
+      const int at =
+          fps_first(__ballot(best.val == top) & ((1ull << P) - 1), best.rel);
+      if (lane == at)
+        table[par][wave] = best;
+    }
+    fps_meet();
+    const FpsBest<DIM> e = table[par][lane & (W - 1)];
+    static_assert(W == 16, "one row of 16 lanes looks at the waves' bests");
+    const uint32_t top =
+        (uint32_t)__builtin_amdgcn_readlane((int)row16_umax(e.val), 15);
+    const int at = fps_first(__ballot(e.val == top) & 0xffffull, e.rel);
+    const uint32_t row = lane_value(e.rel, at);
+    if (tid == 0)
+      out[m] = start_idx + (int64_t)row;
+#pragma unroll
+    for (int c = 0; c < DIM; ++c)
+      cur[c] = lane_value(e.x[c], at);
+  }
+}
+
+// ---- fp32, up to 3 dimensions, larger examples ---------------------------------
+
+// Rows in curve order: (x, y, z, row of the example), their running minima,
+// and the box of every piece of 64 rows.  Piece i of example b has the number
+// ptr[b] / 64 + b + i (no two examples meet).  A wave per piece.
+struct FpsPieces {
+  float4 *rows;   // [n]
+  float *minima;  // [n]
+  float *boxes;   // [pieces][8]: lower corner, -, upper corner, -
+};
+__device__ __forceinline__ int64_t fps_first_piece(int64_t begin, int b) {
+  return begin / kWave + b;
+}
+__global__ __launch_bounds__(kBlock) void fps_gather_kernel(
+    const float *__restrict__ src, const int64_t *__restrict__ ptr, int d,
+    int first_segment, const uint32_t *__restrict__ perm, FpsPieces out) {
+  const int b = first_segment + blockIdx.y;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t piece = (int64_t)blockIdx.x * (kBlock / kWave) +
+                        threadIdx.x / kWave;
+  const int64_t begin = ptr[b], end = ptr[b + 1];
+  if (begin + piece * kWave >= end)
+    return;
+  const int64_t at = begin + piece * kWave + lane;
+  const bool ok = at < end;
+  const int64_t id = ok ? (int64_t)perm[at] : begin;
+  float v[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    v[c] = c < d ? src[(size_t)id * d + c] : 0.0f;
+  if (ok) {
+    out.rows[at] =
+        make_float4(v[0], v[1], v[2], __uint_as_float((uint32_t)(id - begin)));
+    out.minima[at] = 5e4f;
+  }
+  float *box = out.boxes + (size_t)(fps_first_piece(begin, b) + piece) * 8;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    // (fminf / fmaxf drop a NaN; such a row's minimum never changes)
+    float lo = ok ? v[c] : __builtin_inff();
+    float hi = ok ? v[c] : -__builtin_inff();
+#pragma unroll
+    for (int sh = 1; sh < kWave; sh <<= 1) {
+      lo = __builtin_fminf(lo, __shfl_xor(lo, sh));
+      hi = __builtin_fmaxf(hi, __shfl_xor(hi, sh));
+    }
+    if (lane == 0) {
+      box[c] = lo;
+      box[4 + c] = hi;
+    }
+  }
+}
+
+// Bucket k of an example belongs to wave k % W: its box and its best row are in
+// lane (k / W) % 64, slot k / W / 64, of that wave; the rows and their running
+// minima stay in memory, that is in the L2 of the workgroup's XCD.  S slots
+// hold buckets of one piece for up to 65,536 S rows; MANY: more than that,
+// several pieces to a bucket.
+//
+// Eight ragged LiDAR-like scans of 60,000 - 200,000 rows, 2 % sampled: 419.6 ->
+// 6.9 ms per call, 1.7 instead of 157 us per step of the longest scan (before:
+// fps_any_kernel, the whole scan through one compute unit in every step).
+// Bound by the chain of a step: the trip to the L2 is a third of it.
+template <int W, int S, bool MANY>
+__global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
+    const float *__restrict__ src, const int64_t *__restrict__ ptr,
+    const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
+    int d, FpsPieces p, int64_t *__restrict__ out) {
+  constexpr int DIM = 3;
+  __shared__ FpsBest<DIM> table[2][W];
+  __shared__ uint32_t sampled[kWave];
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int b = blockIdx.x;
+  const int64_t start_idx = ptr[b];
+  const int count = (int)(ptr[b + 1] - start_idx);
+  const int64_t o_begin = out_ptr[b];
+  const int64_t o_end = out_ptr[b + 1];
+  if (o_begin >= o_end)
+    return;
+  float4 *rows = p.rows + start_idx;
+  float *minima = p.minima + start_idx;
+  // (MANY: examples of more than 64 W S pieces, several of them to a bucket)
+  const int pieces = (count + kWave - 1) / kWave;
+  const int chunks =
+      MANY ? max(1, (pieces + kWave * W * S - 1) / (kWave * W * S)) : 1;
+  const int buckets = (pieces + chunks - 1) / chunks;
+
+  float blo[S][DIM], bhi[S][DIM];
+  FpsBest<DIM> best[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int k = (s * kWave + lane) * W + wave;
+    const bool any = k < buckets;
+    best[s].val = any ? __float_as_uint(__builtin_inff()) : 0u;
+    best[s].rel = kFpsNoRow;
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) {
+      blo[s][c] = __builtin_inff();
+      bhi[s][c] = -__builtin_inff();
+      best[s].x[c] = 0.0f;
+    }
+    const float *box =
+        p.boxes + (size_t)(fps_first_piece(start_idx, b) + k * chunks) * 8;
+    for (int i = 0; any && i < chunks && k * chunks + i < pieces; ++i) {
+#pragma unroll
+      for (int c = 0; c < DIM; ++c) {
+        blo[s][c] = __builtin_fminf(blo[s][c], box[i * 8 + c]);
+        bhi[s][c] = __builtin_fmaxf(bhi[s][c], box[i * 8 + 4 + c]);
+      }
+    }
+  }
+
+  float cur[DIM];
+  {
+    const int64_t first = start_idx + (start ? start[b] : 0);
+    if (tid == 0)
+      out[o_begin] = first;
+#pragma unroll
+    for (int c = 0; c < DIM; ++c)
+      cur[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
+  }
+
+  int own = 0; // lane of the wave's best
+  FpsBest<DIM> mine = best[0];
+  const int64_t steps = o_end - o_begin;
+  for (int64_t m = 1; m < steps; ++m) {
+    const int par = (int)(m & 1);
+    uint64_t pass[S], any = 0;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      pass[s] = __ballot(!(fps_box_distance<DIM>(cur, blo[s], bhi[s]) >=
+                           __uint_as_float(best[s].val)));
+      any |= pass[s];
+    }
+    if (any != 0) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        // U buckets at a time, so that their rows are on the way together
+        auto look = [&](auto many, const int (&at_lane)[decltype(many)::value]) {
+          constexpr int U = decltype(many)::value;
+          FpsBest<DIM> found[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            found[u].val = 0u;
+            found[u].rel = kFpsNoRow;
+#pragma unroll
+            for (int c = 0; c < DIM; ++c)
+              found[u].x[c] = 0.0f;
+          }
+          for (int i = 0; i < chunks; ++i) {
+            float4 v[U];
+            float low[U];
+            int at[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              const int k = (s * kWave + at_lane[u]) * W + wave;
+              at[u] = (k * chunks + i) * kWave + lane;
+              const int in = min(at[u], count - 1);
+              v[u] = rows[in];
+              low[u] = minima[in];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              const float x[DIM] = {v[u].x, v[u].y, v[u].z};
+              low[u] = fps_lower<DIM>(cur, x, low[u]);
+              const bool ok = at[u] < count;
+              if (ok)
+                minima[at[u]] = low[u];
+              const uint32_t bits = ok ? __float_as_uint(low[u]) : 0u;
+              const uint32_t rel = ok ? __float_as_uint(v[u].w) : kFpsNoRow;
+              // (a lane's rows of a bucket of several pieces)
+              const bool take =
+                  !MANY || i == 0 || bits > found[u].val ||
+                  (bits == found[u].val && fps_tie(rel) < fps_tie(found[u].rel));
+              found[u].val = take ? bits : found[u].val;
+              found[u].rel = take ? rel : found[u].rel;
+#pragma unroll
+              for (int c = 0; c < DIM; ++c)
+                found[u].x[c] = take ? x[c] : found[u].x[c];
+            }
+          }
+          uint32_t top[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            top[u] = found[u].val;
+          wave_umax_of<U>(top);
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int at =
+                fps_first(__ballot(found[u].val == top[u]), found[u].rel);
+            const uint32_t row = lane_value(found[u].rel, at);
+            float at_x[DIM];
+#pragma unroll
+            for (int c = 0; c < DIM; ++c)
+              at_x[c] = lane_value(found[u].x[c], at);
+            const bool here = lane == at_lane[u];
+            best[s].val = here ? top[u] : best[s].val;
+            best[s].rel = here ? row : best[s].rel;
+#pragma unroll
+            for (int c = 0; c < DIM; ++c)
+              best[s].x[c] = here ? at_x[c] : best[s].x[c];
+          }
+        };
+        uint64_t left = pass[s];
+        while (left != 0) {
+          int id[4];
+          id[0] = (int)__builtin_ctzll(left);
+          left &= left - 1;
+          if (left == 0) {
+            const int one[1] = {id[0]};
+            look(std::integral_constant<int, 1>{}, one);
+            break;
+          }
+          // (fewer than four: the first one again, which changes nothing)
+#pragma unroll
+          for (int u = 1; u < 4; ++u) {
+            id[u] = left != 0 ? (int)__builtin_ctzll(left) : id[0];
+            left &= left - 1;
+          }
+          look(std::integral_constant<int, 4>{}, id);
+        }
+      }
+      mine = best[0];
+#pragma unroll
+      for (int s = 1; s < S; ++s) {
+        const bool take = best[s].val > mine.val ||
+                          (best[s].val == mine.val &&
+                           fps_tie(best[s].rel) < fps_tie(mine.rel));
+        mine.val = take ? best[s].val : mine.val;
+        mine.rel = take ? best[s].rel : mine.rel;
+#pragma unroll
+        for (int c = 0; c < DIM; ++c)
+          mine.x[c] = take ? best[s].x[c] : mine.x[c];
+      }
+      const uint32_t top = wave_umax(mine.val);
+      own = fps_first(__ballot(mine.val == top), mine.rel);
+    }
+    if (lane == own)
+      table[par][wave] = mine;
+    fps_meet();
+    FpsBest<DIM> e = table[par][lane & (W - 1)];
+    static_assert(W == 16, "one row of 16 lanes looks at the waves' bests");
+    const uint32_t top =
+        (uint32_t)__builtin_amdgcn_readlane((int)row16_umax(e.val), 15);
+    const int at = fps_first(__ballot(e.val == top) & 0xffffull, e.rel);
+#pragma unroll
+    for (int c = 0; c < DIM; ++c)
+      cur[c] = lane_value(e.x[c], at);
+    if (wave == 0) {
+      // (64 samples are written out at a time)
+      const uint32_t chosen = lane_value(e.rel, at);
+      if (lane == 0)
+        sampled[m & (kWave - 1)] = chosen;
+      if ((m & (kWave - 1)) == kWave - 1 || m == steps - 1) {
+        const int64_t to = (m & ~(int64_t)(kWave - 1)) + lane;
+        if (to <= m && to > 0)
+          out[o_begin + to] = start_idx + (int64_t)sampled[lane];
+      }
+    }
+  }
+}
+
+template <int DIM>
+hipError_t launch_fps_on_chip(const float *src, const int64_t *ptr,
+                              const int64_t *out_ptr, const int64_t *start,
+                              int d, int num_segments, int64_t max_rows,
+                              int64_t *out, hipStream_t stream) {
+#define PCA_FPS_LAUNCH(kernel_, threads_)                                      \
+  hipLaunchKernelGGL((kernel_), dim3(num_segments), dim3(threads_), 0, stream, \
+                     src, ptr, out_ptr, start, d, out)
+  // (shapes by measurement: 16 examples of each size on one device; the
+  // kernels' comments give the times on both sides of a limit)
   if (max_rows <= 256)
-    PCA_FPS_REG(4, 64);
+    PCA_FPS_LAUNCH((fps_reg_kernel<DIM, 4, 64>), 64);
   else if (max_rows <= 512)
-    PCA_FPS_REG(8, 64);
+    PCA_FPS_LAUNCH((fps_reg_kernel<DIM, 8, 64>), 64);
   else if (max_rows <= 1024)
-    PCA_FPS_REG(2, 512);
-  else if (max_rows <= 2048)
-    PCA_FPS_REG(4, 512);
+    PCA_FPS_LAUNCH((fps_reg_kernel<DIM, 2, 512>), 512);
   else if (max_rows <= 4096)
-    PCA_FPS_REG(8, 512);
-  else if (max_rows <= 8192)
-    PCA_FPS_REG(16, 512);
+    PCA_FPS_LAUNCH((fps_lds_kernel<DIM, 16, 1>), 1024);
+  else if (DIM <= 3 && max_rows <= 8192)
+    PCA_FPS_LAUNCH((fps_lds_kernel<DIM <= 3 ? DIM : 3, 16, 2>), 1024);
   else
-    PCA_FPS_REG(16, 1024);
-#undef PCA_FPS_REG
+    PCA_FPS_LAUNCH((fps_bucket_kernel<DIM, 16, 16>), 1024);
+#undef PCA_FPS_LAUNCH
   return hipGetLastError();
 }
 
@@ -475,38 +1364,111 @@ hipError_t launch_fps_any(const void *src, const int64_t *ptr,
 
 } // namespace
 
-bool fps_in_registers(int dtype, int d, int64_t max_rows) {
+// Examples of up to 16,384 rows of up to 4 dimensions.
+static bool fps_on_chip(int dtype, int d, int64_t max_rows) {
   return dtype == 0 && d >= 1 && d <= 4 && max_rows >= 1 &&
          max_rows <= 16 * kFpsThreads;
 }
 
-size_t fps_dist_bytes(int64_t n) { return sizeof(double) * (size_t)n; }
+// Larger examples of up to three dimensions: rows in curve order in memory.
+static bool fps_streams(int dtype, int d, int64_t max_rows) {
+  return dtype == 0 && d >= 1 && d <= 3 && max_rows > 16 * kFpsThreads;
+}
+
+static size_t fps_align(size_t v) { return (v + 255) & ~(size_t)255; }
+
+size_t fps_scratch_bytes(int dtype, int n, int d, int num_segments,
+                         int64_t max_rows) {
+  if (fps_on_chip(dtype, d, max_rows))
+    return 0;
+  const size_t dist = fps_align(sizeof(double) * (size_t)n);
+  if (!fps_streams(dtype, d, max_rows))
+    return dist;
+  const size_t pieces = (size_t)n / kWave + (size_t)num_segments + 1;
+  // (a stream that is being captured takes fps_any_kernel and its `dist`)
+  return std::max(dist, fps_align(sizeof(float4) * (size_t)n) +
+                            fps_align(sizeof(float) * (size_t)n) +
+                            fps_align(sizeof(float) * 8 * pieces) +
+                            curve_order_bytes(n, num_segments));
+}
+
+namespace {
+hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
+                             const int64_t *out_ptr, const int64_t *start,
+                             int n, int d, int num_segments, int64_t max_rows,
+                             void *scratch, int64_t *out, hipStream_t stream) {
+  char *cursor = static_cast<char *>(scratch);
+  auto take = [&cursor](size_t bytes) {
+    char *piece = cursor;
+    cursor += fps_align(bytes);
+    return static_cast<void *>(piece);
+  };
+  FpsPieces p;
+  p.rows = static_cast<float4 *>(take(sizeof(float4) * (size_t)n));
+  p.minima = static_cast<float *>(take(sizeof(float) * (size_t)n));
+  p.boxes = static_cast<float *>(
+      take(sizeof(float) * 8 *
+           ((size_t)n / kWave + (size_t)num_segments + 1)));
+  const uint32_t *perm = nullptr;
+  hipError_t err = launch_curve_order(src, ptr, n, d, num_segments, cursor,
+                                      &perm, stream);
+  if (err != hipSuccess)
+    return err;
+  const int per_block = kWave * (kBlock / kWave);
+  const int64_t rows = std::min(max_rows, (int64_t)n);
+  for (int b0 = 0; b0 < num_segments; b0 += 65535) {
+    const int some = std::min(65535, num_segments - b0);
+    hipLaunchKernelGGL(fps_gather_kernel,
+                       dim3((unsigned)((rows + per_block - 1) / per_block),
+                            some),
+                       dim3(kBlock), 0, stream, src, ptr, d, b0, perm, p);
+  }
+#define PCA_FPS_STREAM(S_, MANY_)                                              \
+  hipLaunchKernelGGL((fps_stream_kernel<kFpsWaves, S_, MANY_>),                \
+                     dim3(num_segments), dim3(kFpsThreads), 0, stream, src,    \
+                     ptr, out_ptr, start, d, p, out)
+  if (rows <= 1 * kWave * kFpsThreads)
+    PCA_FPS_STREAM(1, false);
+  else if (rows <= 2 * kWave * kFpsThreads)
+    PCA_FPS_STREAM(2, false);
+  else if (rows <= 4 * kWave * kFpsThreads)
+    PCA_FPS_STREAM(4, false);
+  else
+    PCA_FPS_STREAM(4, true);
+#undef PCA_FPS_STREAM
+  return hipGetLastError();
+}
+} // namespace
 
 hipError_t launch_fps(int dtype, const void *src, const int64_t *ptr,
-                      const int64_t *out_ptr, const int64_t *start, int d,
-                      int num_segments, int64_t max_rows, void *dist,
-                      int64_t *out, hipStream_t stream) {
-  if (fps_in_registers(dtype, d, max_rows)) {
+                      const int64_t *out_ptr, const int64_t *start, int n,
+                      int d, int num_segments, int64_t max_rows, void *scratch,
+                      bool captured, int64_t *out, hipStream_t stream) {
+  if (fps_on_chip(dtype, d, max_rows)) {
     const float *s = static_cast<const float *>(src);
     if (d <= 2)
-      return launch_fps_reg<2>(s, ptr, out_ptr, start, d, num_segments,
-                               max_rows, out, stream);
+      return launch_fps_on_chip<2>(s, ptr, out_ptr, start, d, num_segments,
+                                   max_rows, out, stream);
     if (d == 3)
-      return launch_fps_reg<3>(s, ptr, out_ptr, start, d, num_segments,
-                               max_rows, out, stream);
-    return launch_fps_reg<4>(s, ptr, out_ptr, start, d, num_segments, max_rows,
-                             out, stream);
+      return launch_fps_on_chip<3>(s, ptr, out_ptr, start, d, num_segments,
+                                   max_rows, out, stream);
+    return launch_fps_on_chip<4>(s, ptr, out_ptr, start, d, num_segments,
+                                 max_rows, out, stream);
   }
+  if (fps_streams(dtype, d, max_rows) && !captured)
+    return launch_fps_stream(static_cast<const float *>(src), ptr, out_ptr,
+                             start, n, d, num_segments, max_rows, scratch, out,
+                             stream);
   switch (dtype) {
   case 0:
     return launch_fps_any<FpsF32>(src, ptr, out_ptr, start, d, num_segments,
-                                  dist, out, stream);
+                                  scratch, out, stream);
   case 1:
     return launch_fps_any<FpsF64>(src, ptr, out_ptr, start, d, num_segments,
-                                  dist, out, stream);
+                                  scratch, out, stream);
   case 2:
     return launch_fps_any<FpsF16>(src, ptr, out_ptr, start, d, num_segments,
-                                  dist, out, stream);
+                                  scratch, out, stream);
   default:
     return hipErrorInvalidValue;
   }

@@ -69,21 +69,6 @@ __device__ __forceinline__ float from_ordered_int(int i) {
   return __int_as_float(i >= 0 ? i : i ^ 0x7fffffff);
 }
 
-__device__ __forceinline__ int find_segment64(const int64_t *__restrict__ ptr,
-                                              int num_segments, int64_t v) {
-  if (ptr == nullptr)
-    return 0;
-  int lo = 0, hi = num_segments;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (ptr[mid] <= v)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  return lo;
-}
-
 // The first launch of a binned search (a call starts with kernels so short
 // that the host's launch rate sets the pace: one launch instead of five):
 // workgroups 0-3 count the work items of the segments - tiles and groups of
@@ -210,6 +195,13 @@ __global__ __launch_bounds__(kBlock) void morton_keys_kernel(
   // csrc/cuda/utils.cuh:11-19): they sort behind every segment's rows
   if (searched_side && ptr != nullptr && (int64_t)i >= ptr[num_segments]) {
     keys[i] = 0xffffffffu;
+    vals[i] = (uint32_t)i;
+    return;
+  }
+  // rows in front of the first pointer sort in front (the sort is stable and
+  // their numbers are the lowest)
+  if (searched_side && ptr != nullptr && (int64_t)i < ptr[0]) {
+    keys[i] = 0u;
     vals[i] = (uint32_t)i;
     return;
   }
@@ -1025,6 +1017,15 @@ hipError_t order_tasks(const SearchInput &in, Bins &bins, uint32_t *task_keys,
   return hipGetLastError();
 }
 
+// Workgroups per segment of seg_box_kernel: enough to fill the device when
+// segments are few (more of them were no quicker: their atomic updates of the
+// same few words take turns).
+int seg_box_parts(int n, int num_segments) {
+  return std::max(1, std::min((n / num_segments + 16 * kBlock - 1) /
+                                  (16 * kBlock),
+                              std::max(1, 1024 / num_segments)));
+}
+
 // Orders rows and queries along the curve, copies the rows, builds the boxes;
 // with `with_tasks` also the tasks of 32 queries and their starting order.
 hipError_t prepare_bins(const SearchInput &in, void *scratch, bool with_tasks,
@@ -1109,13 +1110,8 @@ hipError_t prepare_bins(const SearchInput &in, void *scratch, bool with_tasks,
                        dim3(kPlanThreads), 0, stream, setup);
   }
   {
-    // enough workgroups per segment to fill the device when segments are few
-    // (more of them were no quicker: their atomic updates of the same few
-    // words take turns)
-    const int parts = std::max(
-        1, std::min((in.n / nseg + 16 * kBlock - 1) / (16 * kBlock),
-                    std::max(1, 1024 / nseg)));
-    hipLaunchKernelGGL(seg_box_kernel, dim3(parts, std::min(nseg, 65535)),
+    hipLaunchKernelGGL(seg_box_kernel,
+                       dim3(seg_box_parts(in.n, nseg), std::min(nseg, 65535)),
                        dim3(kBlock), 0, stream, x, in.ptr_x, in.n, in.d, nseg,
                        seg_box);
   }
@@ -1251,6 +1247,75 @@ void fill_params(BinnedParams &p, const SearchInput &in, const Bins &bins,
 }
 
 } // namespace
+
+// The rows of every segment in curve order, for kernels that look at them in
+// that order only (fps): boxes, keys and the sort of prepare_bins.
+namespace {
+struct CurveLayout {
+  size_t seg_box, keys, keys_out, vals, perm, temp;
+  size_t total() const {
+    return seg_box + keys + keys_out + vals + perm + temp;
+  }
+};
+CurveLayout curve_layout(int n, int num_segments) {
+  CurveLayout w;
+  w.seg_box = align256(sizeof(int) * 6 * (size_t)num_segments);
+  w.keys = w.keys_out = w.vals = w.perm =
+      align256(sizeof(uint32_t) * (size_t)n);
+  size_t temp = 0;
+  const hipError_t err = sort_pairs(nullptr, temp, nullptr, nullptr, nullptr,
+                                    nullptr, n, num_segments, nullptr);
+  // (a failed size query leaves a size no workspace can meet)
+  w.temp = err == hipSuccess ? align256(temp) : ~(size_t)0 / 2;
+  return w;
+}
+__global__ __launch_bounds__(kBlock) void seg_box_reset_kernel(
+    int num_segments, int *__restrict__ seg_box) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < 6 * num_segments)
+    seg_box[i] = (i % 6) < 3 ? INT_MAX : INT_MIN;
+}
+} // namespace
+
+size_t curve_order_bytes(int n, int num_segments) {
+  return curve_layout(n, num_segments).total();
+}
+
+hipError_t launch_curve_order(const float *x, const int64_t *ptr, int n, int d,
+                              int num_segments, void *scratch,
+                              const uint32_t **perm, hipStream_t stream) {
+  const CurveLayout lay = curve_layout(n, num_segments);
+  char *cursor = static_cast<char *>(scratch);
+  auto take = [&cursor](size_t bytes) {
+    char *piece = cursor;
+    cursor += bytes;
+    return static_cast<void *>(piece);
+  };
+  int *seg_box = static_cast<int *>(take(lay.seg_box));
+  uint32_t *keys = static_cast<uint32_t *>(take(lay.keys));
+  uint32_t *keys_out = static_cast<uint32_t *>(take(lay.keys_out));
+  uint32_t *vals = static_cast<uint32_t *>(take(lay.vals));
+  uint32_t *order = static_cast<uint32_t *>(take(lay.perm));
+  void *temp = take(lay.temp);
+  hipLaunchKernelGGL(seg_box_reset_kernel,
+                     dim3((6 * num_segments + kBlock - 1) / kBlock),
+                     dim3(kBlock), 0, stream, num_segments, seg_box);
+  hipLaunchKernelGGL(seg_box_kernel,
+                     dim3(seg_box_parts(n, num_segments),
+                          std::min(num_segments, 65535)),
+                     dim3(kBlock), 0, stream, x, ptr, n, d, num_segments,
+                     seg_box);
+  hipLaunchKernelGGL(morton_keys_kernel, dim3((n + kBlock - 1) / kBlock),
+                     dim3(kBlock), 0, stream, x, ptr, n, d, num_segments,
+                     seg_box, axis_bits(num_segments), keys, vals, true);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess)
+    return err;
+  size_t bytes = lay.temp;
+  *perm = order;
+  return sort_pairs(temp, bytes, keys, keys_out, vals, order, n, num_segments,
+                    stream);
+}
 
 bool knn_binned_supported(int d, int k, bool cosine) {
   return !cosine && d >= 1 && d <= 3 && k >= 1 && k <= 64;

@@ -264,18 +264,30 @@ hipError_t launch_nearest_any(int dtype, const SearchInput &in,
                               const int *work_start, int grid_bound,
                               int64_t *out, hipStream_t stream);
 
+// --- knn_binned.hip: rows in curve order ------------------------------------
+
+// perm: the rows of every segment along a space-filling curve inside the
+// segment's box (the segments one after the other, ptr required), in scratch.
+// fp32, up to 3 dimensions.  Not for a stream that is being captured.
+size_t curve_order_bytes(int n, int num_segments);
+hipError_t launch_curve_order(const float *x, const int64_t *ptr, int n, int d,
+                              int num_segments, void *scratch,
+                              const uint32_t **perm, hipStream_t stream);
+
 // --- fps.hip ---------------------------------------------------------------
 
-// fp32 rows of up to 4 dimensions in examples of up to 16,384 rows are sampled
-// from registers; everything else streams `dist` ([n], fps_dist_bytes) and
-// the rows from memory.
-bool fps_in_registers(int dtype, int d, int64_t max_rows);
-size_t fps_dist_bytes(int64_t n);
+// Scratch of launch_fps: none for fp32 rows of up to 4 dimensions in examples
+// of up to 16,384 rows, the rows in curve order for larger examples of up to 3
+// dimensions, a running minimum per row for everything else (and for an
+// unknown bound, max_rows = 0).
+size_t fps_scratch_bytes(int dtype, int n, int d, int num_segments,
+                         int64_t max_rows);
 // One workgroup per example.  start: NULL = first row of every example.
+// captured: the stream is being captured into a graph (no sort then).
 hipError_t launch_fps(int dtype, const void *src, const int64_t *ptr,
-                      const int64_t *out_ptr, const int64_t *start, int d,
-                      int num_segments, int64_t max_rows, void *dist,
-                      int64_t *out, hipStream_t stream);
+                      const int64_t *out_ptr, const int64_t *start, int n,
+                      int d, int num_segments, int64_t max_rows, void *scratch,
+                      bool captured, int64_t *out, hipStream_t stream);
 
 // --- radius_mc.hip ---------------------------------------------------------
 

@@ -88,6 +88,57 @@ def test_register_and_streaming_kernels_agree(oracle):
         assert (gpu_fps(oracle, x, ptr, ratio, max_rows=0) == want).all()
 
 
+# 1,025 / 4,097 / 8,193: where the kernels that skip rows change; 16,385: from
+# memory on; 65,537 and 131,073: two and four slots per lane; 262,145: several
+# pieces of 64 rows to a bucket
+@pytest.mark.parametrize("kind", ["grid", "far", "odd"])
+@pytest.mark.parametrize("rows,d", [(1025, 3), (4097, 3), (4097, 4), (8193, 2),
+                                    (16385, 3), (65537, 1), (131073, 2),
+                                    (262145, 3)])
+def test_skipped_rows_change_nothing(oracle, rows, d, kind):
+    """Rows in buckets, whole buckets left alone: ties (a coarse grid, and
+    distances beyond the 5e4 cap), rows with NaN and infinite coordinates,
+    examples of very different sizes, rows in front of the first example."""
+    rng = np.random.default_rng(rows + d)
+    ptr = np.cumsum([5, 70, rows, 1, 300]).astype(np.int64)
+    n = ptr[-1] + 3
+    x = (rng.integers(0, 9, (n, d)) if kind == "grid" else
+         rng.standard_normal((n, d)) * (300 if kind == "far" else 1))
+    x = x.astype(np.float32)
+    if kind == "odd":
+        x[100] = np.nan
+        x[rows // 2, 0] = np.inf
+    share = np.array([0.5, 60.0 / rows, 1.0, 0.1])
+    start = np.array([3, rows - 1, 0, 12], dtype=np.int64)
+    got = gpu_fps(oracle, x, ptr, share, start)
+    want = oracle.fps_op(x, ptr, share, start)
+    assert (got == want).all()
+
+
+def test_captured_into_a_graph(oracle):
+    """While its stream is being captured the search does without the sort of
+    the large examples; every replay samples the same rows."""
+    rng = np.random.default_rng(8)
+    x = rng.standard_normal((18000, 3)).astype(np.float32)
+    ptr = np.array([0, 18000], dtype=np.int64)
+    want = oracle.fps_op(x, ptr, 40.0 / 18000)
+    out_ptr = oracle.fps_out_ptr(ptr, 40.0 / 18000, np.float32)
+    args = (dev(x), dev(ptr, torch.long), dev(out_ptr, torch.long),
+            int(out_ptr[-1]), None, 18000)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, _ws = capi.fps_launch(*args)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (out.cpu().numpy() == want).all()
+        eager, _ws2 = capi.fps_launch(*args)
+        torch.cuda.synchronize()
+        assert (eager.cpu().numpy() == want).all()
+
+
 def test_start_offsets_nan_rows_and_oversampling(oracle):
     rng = np.random.default_rng(6)
     x = rng.standard_normal((700, 3)).astype(np.float32)
