@@ -87,6 +87,12 @@ bool sizes_ok(int64_t n, int64_t m, int64_t d, int64_t num_segments) {
 }
 
 // two arrays of num_segments + 1 pointers (PCA_SEGMENTS_BY_ID)
+// Up to this many examples the launch that plans the work derives their
+// pointers itself, by the waves of one workgroup; more get a launch of their
+// own, one wave per pointer.  (A round of 16 searches takes ~1.3 us, the extra
+// launch ~5 us.)
+constexpr int64_t kPlanDerivesExamples = 32;
+
 size_t segment_pointer_bytes(int64_t num_segments) {
   return 2 * align256(sizeof(int64_t) * (size_t)(num_segments + 1));
 }
@@ -523,8 +529,16 @@ int knn_call(const void *x, const void *y, const int64_t *ptr_x,
     dense.dist = nullptr;
   pca::SegmentSource src;
   const bool by_id = (edge_flags & PCA_SEGMENTS_BY_ID) != 0 && ptr_x != nullptr;
+  int rc = PCA_OK;
   if (by_id)
     src = segments_by_id(ptr_x, ptr_y, n, m, num_segments, take(lay.ptrs));
+  const bool plan_derives = by_id && num_segments <= kPlanDerivesExamples;
+  if (by_id && !plan_derives)
+    rc = check_launch(
+        pca::launch_segment_pointers(src, (int)num_segments, stream),
+        "segment_pointers_kernel");
+  if (rc != PCA_OK)
+    return rc;
   pca::KnnLowdConfig cfg = pca::knn_lowd_config(
       (int)d, (int)k, (int)n, (int)m, (int)num_segments, cosine != 0);
   // (the matrix-core kernels count the edges while they write their lists)
@@ -552,12 +566,11 @@ int knn_call(const void *x, const void *y, const int64_t *ptr_x,
     cfg.tile_queries = pca::kMfmaTileQueries;
   else if (!low_d)
     cfg.tile_queries = pca::kBlock; // any-dimension kernel: one query per lane
-  int rc = PCA_OK;
   // (the low-dimensional path plans its work inside its own first launch)
   if (!low_d)
     rc = check_launch(pca::launch_plan(ptr_y, (int)m, (int)num_segments,
                                        cfg.tile_queries, work_start, stream,
-                                       by_id ? &src : nullptr),
+                                       plan_derives ? &src : nullptr),
                       "plan_kernel");
   if (rc != PCA_OK)
     return rc;
@@ -569,7 +582,8 @@ int knn_call(const void *x, const void *y, const int64_t *ptr_x,
     rc = check_launch(pca::launch_knn_lowd(in, (int)k, cosine != 0, cfg,
                                            work_start, lowd_scratch, dense,
                                            timer.start, timer.stop, stream,
-                                           nullptr, by_id ? &src : nullptr),
+                                           nullptr,
+                                           plan_derives ? &src : nullptr),
                       "knn_lowd_kernel");
     timer.stop = nullptr;
   } else if (feat) {
@@ -807,9 +821,17 @@ int pca_radius(const void *x, const void *y, const int64_t *ptr_x,
   void *compact_ws = ws.take<char>(pca::compact_workspace_bytes((int)m));
   pca::SegmentSource src;
   const bool by_id = (edge_flags & PCA_SEGMENTS_BY_ID) != 0 && ptr_x != nullptr;
+  int rc = PCA_OK;
   if (by_id)
     src = segments_by_id(ptr_x, ptr_y, n, m, num_segments,
                          ws.take<char>(segment_pointer_bytes(num_segments)));
+  const bool plan_derives = by_id && num_segments <= kPlanDerivesExamples;
+  if (by_id && !plan_derives)
+    rc = check_launch(
+        pca::launch_segment_pointers(src, (int)num_segments, stream),
+        "segment_pointers_kernel");
+  if (rc != PCA_OK)
+    return rc;
 
   // r * r in double, narrowed to the element type at the launch
   // (csrc/cuda/radius_cuda.cu:90)
@@ -820,12 +842,11 @@ int pca_radius(const void *x, const void *y, const int64_t *ptr_x,
   const int per_item = matrix_cores    ? pca::kRadiusMcTileQueries
                        : feature_space ? pca::kMfmaTileQueries
                                        : pca::kRadiusQueriesPerWave;
-  int rc = PCA_OK;
   // (the matrix-core path plans its work in the launch that packs the rows)
   if (!matrix_cores)
     rc = check_launch(pca::launch_plan(ptr_y, (int)m, (int)num_segments,
                                        per_item, work_start, stream,
-                                       by_id ? &src : nullptr),
+                                       plan_derives ? &src : nullptr),
                       "plan_kernel");
   if (rc != PCA_OK)
     return rc;
@@ -848,7 +869,7 @@ int pca_radius(const void *x, const void *y, const int64_t *ptr_x,
     rc = check_launch(pca::launch_radius_mc(in, r2, ignore_same_index != 0,
                                             work_start, bound, packed_rows,
                                             dense, timer.start, stream,
-                                            by_id ? &src : nullptr),
+                                            plan_derives ? &src : nullptr),
                       "radius_mc_kernel");
   else if (dtype == PCA_F32)
     rc = check_launch(pca::launch_radius(in, r2, ignore_same_index != 0,

@@ -369,21 +369,26 @@ plan_segments(const int64_t *__restrict__ ptr, int m, int num_segments,
     work_start[num_segments] = partial[tid];
 }
 
-// Pointers of both sides from sorted example ids, by all waves of one
-// workgroup: ptr[b] = number of rows whose id is below b.  A wave takes one
-// (side, b) at a time and narrows the range 65-fold per step -- its 64 lanes
-// probe evenly spaced rows at once, so a million rows take four dependent
-// reads instead of twenty.  Src is launchers.hpp's SegmentSource.
+// Pointers of both sides from sorted example ids, by all waves of `blocks`
+// workgroups (this one is number `block`): ptr[b] = number of rows whose id is
+// below b.  A wave takes one (side, b) at a time and narrows the range 65-fold
+// per step -- its 64 lanes probe evenly spaced rows at once, so a million rows
+// take four dependent reads instead of twenty.  Both sides the same vector (a
+// graph's): searched once.  Src is launchers.hpp's SegmentSource.
 template <typename Src>
 __device__ __forceinline__ void pointers_from_ids(const Src &src,
-                                                  int num_segments) {
+                                                  int num_segments,
+                                                  int block = 0,
+                                                  int blocks = 1) {
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int waves = blockDim.x >> 6;
-  const int searches = 2 * (num_segments + 1);
+  const int per_block = blockDim.x >> 6;
+  const int wave = block * per_block + (threadIdx.x >> 6);
+  const int waves = blocks * per_block;
+  const bool same = src.ids_x == src.ids_y && src.n == src.m;
+  const int searches = (same ? 1 : 2) * (num_segments + 1);
   // for a caller that guessed num_segments: the examples the ids speak of
   // (sorted ids: the last ones are the largest)
-  if (src.examples_out != nullptr && threadIdx.x == 0) {
+  if (src.examples_out != nullptr && block == 0 && threadIdx.x == 0) {
     int64_t last = -1;
     if (src.n > 0)
       last = src.ids_x[src.n - 1];
@@ -392,8 +397,8 @@ __device__ __forceinline__ void pointers_from_ids(const Src &src,
     *src.examples_out = last + 1;
   }
   for (int s = wave; s < searches; s += waves) {
-    const int side = s & 1;
-    const int b = s >> 1;
+    const int side = same ? 0 : s & 1;
+    const int b = same ? s : s >> 1;
     const int64_t *ids = side ? src.ids_y : src.ids_x;
     const int count = side ? src.m : src.n;
     // invariant: ids[i] < b for i < lo, ids[i] >= b for i >= hi
@@ -414,15 +419,17 @@ __device__ __forceinline__ void pointers_from_ids(const Src &src,
       hi = new_hi;
     }
     const bool is_below = lo + lane < hi && ids[lo + lane] < (int64_t)b;
-    int result = lo + __builtin_popcountll(__ballot(is_below));
+    const int result = lo + __builtin_popcountll(__ballot(is_below));
     // Rows whose id is num_segments or more (a caller's batch_size below the
     // largest id + 1): the reference's lookup hands such a query to the LAST
     // example (csrc/cuda/utils.cuh:11-19 returns num_examples - 1 when no
     // pointer lies above the row), and never searches such a row of x.
-    if (side == 1 && b == num_segments)
-      result = count;
-    if (lane == 0)
-      (side ? src.ptr_y : src.ptr_x)[b] = result;
+    if (lane == 0) {
+      if (side == 0)
+        src.ptr_x[b] = result;
+      if (side == 1 || same)
+        src.ptr_y[b] = b == num_segments ? count : result;
+    }
   }
 }
 

