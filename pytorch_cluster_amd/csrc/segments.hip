@@ -204,77 +204,120 @@ __global__ __launch_bounds__(kBlock) void count_block_kernel(
     block_sums[blockIdx.x] = total;
 }
 
+// Inclusive prefix sum over the lanes of a wave.
+__device__ __forceinline__ int wave_inclusive_scan(int v, int lane) {
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const int t = __shfl_up(v, off);
+    v += lane >= off ? t : 0;
+  }
+  return v;
+}
+
 // count: slots to write per query (without the self slot when self_pos is
 // given).  x_first: the x row goes to the first half of `edges`.
 // inline_scan: block_offsets holds the blocks' SUMS; this block adds up the
 // ones before it and all of them (block 0 also stores the total).
+//
+// Bound by the latency of its reads -- counts and sums, then slots -- as long
+// as the device is not full: 1 << parts_log2 workgroups share a block of
+// queries (every one scans the block's counts and writes its part of the
+// rows), and the scans stay inside the waves, with one barrier for everything.
 __global__ __launch_bounds__(kBlock) void scatter_kernel(
     const int *__restrict__ idx, const float *__restrict__ dist,
     const int *__restrict__ count, const int *__restrict__ self_pos, int m,
-    int slots, uint32_t magic, int x_first,
+    int slots, uint32_t magic, int x_first, int parts_log2, int num_blocks,
     const int64_t *__restrict__ block_offsets,
     int64_t *__restrict__ num_edges, int64_t *__restrict__ edges,
     float *__restrict__ dist_out, int inline_scan) {
-  __shared__ int lds[kBlock];
-  __shared__ int64_t s_before[kBlock], s_all[kBlock];
+  constexpr int W = kBlock / kWave;
+  __shared__ int64_t s_before[W], s_all[W];
+  __shared__ int s_sum[W];
   __shared__ int s_count[kCompactQueries];
-  __shared__ int s_offset[kCompactQueries];
+  __shared__ int s_offset[kCompactQueries]; // within the wave's queries
   __shared__ int s_self[kCompactQueries];
+  static_assert(kBlock == kCompactQueries, "one thread per query");
   const int tid = threadIdx.x;
-  const int q0 = blockIdx.x * kCompactQueries;
+  const int lane = tid & (kWave - 1);
+  const int wave = tid / kWave;
+  const int block = blockIdx.x >> parts_log2;
+  const int part = blockIdx.x - (block << parts_log2);
+  const int q0 = block * kCompactQueries;
   const int q = q0 + tid;
   const int c = q < m ? count[q] : 0;
-  int total;
-  const int off = block_exclusive_scan(c, lds, &total);
-  s_count[tid] = c;
-  s_offset[tid] = off;
-  // (a position no slot has when nothing is left out)
-  s_self[tid] = (self_pos && q < m && self_pos[q] >= 0) ? self_pos[q] : slots;
-  __syncthreads();
-  int64_t E, base;
-  if (inline_scan) {
-    int64_t before = 0, all = 0;
-    for (int b = tid; b < (int)gridDim.x; b += kBlock) {
+  const int self = self_pos && q < m ? self_pos[q] : -1;
+  int64_t before = 0, all = 0;
+  if (inline_scan)
+    for (int b = tid; b < num_blocks; b += kBlock) {
       const int64_t v = block_offsets[b];
       all += v;
-      before += b < (int)blockIdx.x ? v : 0;
+      before += b < block ? v : 0;
     }
-    s_before[tid] = before;
-    s_all[tid] = all;
-    __syncthreads();
-    for (int off = kBlock / 2; off >= 1; off >>= 1) {
-      if (tid < off) {
-        s_before[tid] += s_before[tid + off];
-        s_all[tid] += s_all[tid + off];
-      }
-      __syncthreads();
+  const int inclusive = wave_inclusive_scan(c, lane);
+  s_count[tid] = c;
+  s_offset[tid] = inclusive - c;
+  // (a position no slot has when nothing is left out)
+  s_self[tid] = self >= 0 ? self : slots;
+  if (lane == kWave - 1)
+    s_sum[wave] = inclusive;
+  if (inline_scan) {
+#pragma unroll
+    for (int sh = 1; sh < kWave; sh <<= 1) {
+      before += __shfl_xor(before, sh);
+      all += __shfl_xor(all, sh);
     }
-    E = s_all[0];
-    base = s_before[0];
+    if (lane == 0) {
+      s_before[wave] = before;
+      s_all[wave] = all;
+    }
+  }
+  __syncthreads();
+  int wave_base[W];
+  int64_t E = 0, base = 0;
+  {
+    int run = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      wave_base[w] = run;
+      run += s_sum[w];
+    }
+  }
+  if (inline_scan) {
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      E += s_all[w];
+      base += s_before[w];
+    }
     if (blockIdx.x == 0 && tid == 0)
       *num_edges = E;
   } else {
-    E = block_offsets[gridDim.x];
-    base = block_offsets[blockIdx.x];
+    E = block_offsets[num_blocks];
+    base = block_offsets[block];
   }
-  if (total == 0)
-    return;
 
-  const int nq = min(kCompactQueries, m - q0);
+  const int per_part = kCompactQueries >> parts_log2;
+  const int first_q = part * per_part;
+  const int nq = min(per_part, m - q0 - first_q);
   int64_t *first = x_first ? edges + E : edges;  // receives the query rows
   int64_t *second = x_first ? edges : edges + E; // receives the x rows
-  const int *rows = idx + (size_t)q0 * slots;
-  const float *row_dist = dist ? dist + (size_t)q0 * slots : nullptr;
-  const int span = nq * slots;
+  const size_t row0 = (size_t)(q0 + first_q) * slots;
+  const int *rows = idx + row0;
+  const float *row_dist = dist ? dist + row0 : nullptr;
+  const int span = nq * slots; // (nothing to do for nq <= 0)
 #pragma unroll 4
   for (int e = tid; e < span; e += kBlock) {
-    const int ql = quotient_by_slots(e, slots, magic);
-    const int sl = e - ql * slots;
+    const int el = quotient_by_slots(e, slots, magic);
+    const int ql = first_q + el;
+    const int sl = e - el * slots;
     const int skip = s_self[ql];
     // slot sl goes to position sl, or sl - 1 behind the left-out slot
     const int pos = sl - (sl > skip ? 1 : 0);
     if (sl != skip && pos < s_count[ql]) {
-      const int64_t o = base + s_offset[ql] + pos;
+      int in_block = s_offset[ql] + pos;
+#pragma unroll
+      for (int w = 1; w < W; ++w)
+        in_block += ql / kWave == w ? wave_base[w] : 0;
+      const int64_t o = base + in_block;
       first[o] = q0 + ql;
       second[o] = rows[e];
       if (dist_out)
@@ -282,6 +325,9 @@ __global__ __launch_bounds__(kBlock) void scatter_kernel(
     }
   }
 }
+
+// workgroups of 4 waves that fill 256 CUs
+constexpr int kScatterGroups = 2048;
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
@@ -338,13 +384,19 @@ hipError_t launch_compact(const DenseResult &dense, int m, int64_t *edges,
   int *kept = reinterpret_cast<int *>(ws + align256(sizeof(int) * (size_t)m));
   const int *count = dense.count;
   const uint32_t magic = slots_magic(dense.slots);
+  // as many workgroups as bring the device to eight waves per SIMD, at least
+  // 32 queries each
+  int parts_log2 = 0;
+  while (parts_log2 < 3 && (blocks << (parts_log2 + 1)) <= kScatterGroups)
+    ++parts_log2;
+  const dim3 scatter_grid((unsigned)blocks << parts_log2);
   if (dense.edge_sums != nullptr && blocks <= kInlineScanBlocks &&
       (!drop_self || dense.self_pos != nullptr)) {
     // the search left the block sums (and the self slots) behind
-    hipLaunchKernelGGL(scatter_kernel, dim3(blocks), dim3(kBlock), 0, stream,
+    hipLaunchKernelGGL(scatter_kernel, scatter_grid, dim3(kBlock), 0, stream,
                        dense.idx, dense.dist, drop_self ? dense.kept : count,
                        drop_self ? dense.self_pos : (const int *)nullptr, m,
-                       dense.slots, magic, x_first ? 1 : 0,
+                       dense.slots, magic, x_first ? 1 : 0, parts_log2, blocks,
                        reinterpret_cast<const int64_t *>(dense.edge_sums),
                        num_edges, edges, dist_out, 1);
     return hipGetLastError();
@@ -354,10 +406,10 @@ hipError_t launch_compact(const DenseResult &dense, int m, int64_t *edges,
                        stream, dense.idx, dense.count, m, dense.slots, magic,
                        drop_self ? self_pos : (int *)nullptr, kept,
                        block_sums);
-    hipLaunchKernelGGL(scatter_kernel, dim3(blocks), dim3(kBlock), 0, stream,
+    hipLaunchKernelGGL(scatter_kernel, scatter_grid, dim3(kBlock), 0, stream,
                        dense.idx, dense.dist, drop_self ? kept : count,
                        drop_self ? self_pos : (const int *)nullptr, m,
-                       dense.slots, magic, x_first ? 1 : 0, block_sums,
+                       dense.slots, magic, x_first ? 1 : 0, parts_log2, blocks, block_sums,
                        num_edges, edges, dist_out, 1);
     return hipGetLastError();
   }
@@ -371,10 +423,10 @@ hipError_t launch_compact(const DenseResult &dense, int m, int64_t *edges,
                      count, m, block_sums);
   hipLaunchKernelGGL(scan_block_sums_kernel, dim3(1), dim3(kPlanThreads), 0,
                      stream, block_sums, blocks, num_edges);
-  hipLaunchKernelGGL(scatter_kernel, dim3(blocks), dim3(kBlock), 0, stream,
+  hipLaunchKernelGGL(scatter_kernel, scatter_grid, dim3(kBlock), 0, stream,
                      dense.idx, dense.dist, count,
                      drop_self ? self_pos : (const int *)nullptr, m,
-                     dense.slots, magic, x_first ? 1 : 0, block_sums, num_edges,
+                     dense.slots, magic, x_first ? 1 : 0, parts_log2, blocks, block_sums, num_edges,
                      edges, dist_out, 0);
   return hipGetLastError();
 }

@@ -625,3 +625,23 @@ def test_operators_refuse_graph_capture():
         torch.cuda.synchronize()
     # and work as before afterwards
     assert pca.knn(x, x, 3).shape == (2, 1500)
+
+
+@pytest.mark.parametrize("n", [2, 31, 33, 255, 257, 2049, 65537, 262145,
+                               524289])
+def test_compaction_at_the_edges_of_its_parts(oracle, n):
+    # rows of a block are written by 8, 4, 2 or 1 workgroups, by the number of
+    # blocks; beyond 2,048 blocks the sums are scanned by a launch of their own
+    rng = np.random.default_rng(n)
+    x = rng.random((n, 2)).astype(np.float32)
+    ptr = np.append(np.arange(0, n, 61), n).astype(np.int64)
+    row, col, dist = oracle.knn_dense(x, x, ptr, ptr, 5, False, fma_mode=1)
+    col, dist = col.reshape(n, 5), dist.reshape(n, 5)
+    keep = (col != -1) & (col != np.arange(n)[:, None])
+    rows = np.broadcast_to(np.arange(n)[:, None], (n, 5))[keep]
+    e, d = capi.knn_edges(dev(x), dev(x), dev(ptr), dev(ptr), 5, False, True,
+                          drop_self=True, x_first=True)
+    torch.cuda.synchronize()
+    assert (e[0].cpu().numpy() == col[keep]).all()
+    assert (e[1].cpu().numpy() == rows).all()
+    assert (d.cpu().numpy() == dist[keep]).all()
