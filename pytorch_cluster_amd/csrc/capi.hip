@@ -253,10 +253,19 @@ bool nearest_mfma(int64_t d, int dtype) {
          pca::knn_mfma_supported((int)d, 1, false);
 }
 
+// (the searched rows are y here, m of them)
+bool nearest_feat(int64_t n, int64_t m, int64_t d, int64_t num_segments,
+                  int dtype) {
+  return dtype == PCA_F32 && pca::nearest_feat_supported((int)m, (int)n, (int)d,
+                                                         (int)num_segments);
+}
+
 size_t nearest_workspace(int64_t n, int64_t m, int64_t d,
                          int64_t num_segments, int dtype) {
   size_t bytes = align256(sizeof(int) * (size_t)(num_segments + 1));
-  if (nearest_mfma(d, dtype))
+  if (nearest_feat(n, m, d, num_segments, dtype))
+    bytes += pca::nearest_feat_scratch_bytes((int)m, (int)d);
+  else if (nearest_mfma(d, dtype))
     bytes += pca::knn_mfma_scratch_bytes((int)m, (int)n, (int)d,
                                          (int)num_segments, 1);
   if (nearest_low_d(d, dtype)) {
@@ -1038,6 +1047,16 @@ int pca_nearest(const void *x, const void *y, const int64_t *ptr_x,
   Carver ws(workspace);
   int *work_start = ws.take<int>((size_t)num_segments + 1);
   const bool low_d = nearest_low_d(d, dtype);
+  if (nearest_feat(n, m, d, num_segments, dtype)) {
+    void *scratch =
+        ws.take<char>(pca::nearest_feat_scratch_bytes((int)m, (int)d));
+    const int rc = check_launch(
+        pca::launch_nearest_feat(in, work_start, scratch, out, timer.start,
+                                 timer.stop, stream),
+        "nearest_feat_kernel");
+    timer.stop = nullptr;
+    return rc;
+  }
   const bool mfma = nearest_mfma(d, dtype);
   pca::KnnLowdConfig cfg;
   int per_item = mfma ? pca::kMfmaTileQueries : pca::kBlock;

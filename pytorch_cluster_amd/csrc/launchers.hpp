@@ -173,6 +173,19 @@ hipError_t launch_knn_mfma(const SearchInput &in, int k, bool cosine,
                            int64_t *nearest_out = nullptr,
                            const MfmaSecondPass *second = nullptr);
 
+// --- nearest_feat*.hip -------------------------------------------------------
+
+// The `nearest` search over fp32 rows of 9 .. 128 components by one fp16
+// product per pair (nearest_feat_impl.hpp): in.x are the candidates, in.y the
+// rows that search.  Plans the work itself (work_start: num_segments + 1
+// entries).  PCA_NEAREST_FEAT=0: never, 1: whenever the dimension fits.
+bool nearest_feat_supported(int n, int m, int d, int num_segments);
+size_t nearest_feat_scratch_bytes(int n, int d);
+hipError_t launch_nearest_feat(const SearchInput &in, int *work_start,
+                               void *scratch, int64_t *out,
+                               hipEvent_t time_start, hipEvent_t time_stop,
+                               hipStream_t stream);
+
 // --- knn_feat*.hip ---------------------------------------------------------
 
 // Feature-space kNN with the fp16 matrix-core filter and the exact second

@@ -1,0 +1,624 @@
+// `nearest` in feature space (fp32, 8 < d <= 128): every row of y gets the
+// nearest row of x, the entries of a code book as a rule, with the results of
+// the reference's loop (csrc/cuda/nearest_cuda.cu:10-66) bit for bit.
+//
+// ONE fp16 product per pair and component on the matrix cores ranks a query's
+// candidates, and a few of them are evaluated exactly afterwards.  With
+// a = s_c x, b = s_q y (s_c, s_q powers of two, of the call and of the
+// workgroup's queries, that bring the largest component into [2^10, 2^11)) and
+// r = s_q / s_c, a chain of v_mfma_f32_32x32x16_f16 that starts from
+// kappa |a|^2 gives
+//     s = kappa |a|^2 + sum_c h(a_c) h(-2 b_c),    h: fp16, |h| < 2^-14 flushed,
+// and  s + |b|^2 / r - C  is a LOWER bound of s_c s_q |x - y|^2 for
+//   * |a_c b_c' - h(a_c) h(b_c')| summed over the components (b' = 2 b): at
+//     most (2^-10 + 2^-22) |a| |b'| + 2^-14 (1 + 2^-11) sqrt(d) (|a| + |b'|)
+//     + d 2^-28;
+//   * the accumulation: d + 16 terms, each within 2^-22 of a running magnitude
+//     below |kappa| |a|^2 + 1.01 |a| |b'|;
+//   * |a| |b'| <= l |a|^2 + |b|^2 / l with l = B / A, B the largest |b| of the
+//     workgroup and A the root mean square |a|, and |a| <= (|a|^2 / A + A) / 2,
+// so that  kappa = r (1 - delta) - eps l - 2^-15 sqrt(d) / A  and
+//     C = eps |b|^2 / l + 2^-15 sqrt(d) A + 2^-13 sqrt(d) |b| + d 2^-27
+// (each sqrt term times 1.01), eps = 2^-10 + (d + 20) 2^-21,
+// delta = (d + 20) 2^-21.
+//
+// A scan keeps, per query and half of the rows (lanes l and l + 32 share a
+// query and see rows 8 v + 4 (l / 32) + 0..3 of 32), the three smallest
+// MINIMA OF FOUR consecutive rows, the number of the four in the low nine bits
+// of the value (2^-14 of it, which the cut allows for).  That is 24 vector
+// instructions for 16 values; the matrix cores need 32 cycles per 16
+// components for them, and the vector ALU 4 cycles each: neither waits for
+// long from 48 components on.  After 4,096 rows the four rows of a query's
+// smallest minimum are evaluated exactly; their distance D gives the cut
+// below which s has to lie for a row to come before them; of the other
+// minima kept, those below the cut are evaluated too.  Only if even the third
+// lies below it (four fours of rows within the rounding margin of the nearest
+// one: duplicates, rows much larger than the others) there may be candidates
+// that were not kept: the workgroup then goes through these 4,096 rows again
+// and evaluates whatever lies below the cut.
+//
+// Rows of x with a component that is not finite never qualify (their distance
+// is not below 1e38); finite ones of |x|^2 > 1e30 enter with s = -1e37, always
+// looked at.  Queries likewise: not finite, no candidate; too large, every
+// candidate is evaluated.
+//
+// Mapping: a workgroup owns 4 waves x S x 32 queries of one segment; the query
+// operands stay in registers, packed rows of x (2 NB units of 16 bytes, an odd
+// stride against bank conflicts) go through two LDS tiles of 128 rows filled
+// by LDS-direct loads.  S sets of queries per wave share the reads of a row:
+// with one set the LDS would have to deliver 128 bytes per cycle and CU, all
+// it can.
+//
+// Measured figures: nearest_feat.hip.
+#pragma once
+
+#include "device_utils.hpp"
+#include "knn_lowd_impl.hpp"
+#include "launchers.hpp"
+
+namespace pca {
+
+typedef _Float16 nf_f16x8_t __attribute__((ext_vector_type(8)));
+typedef float nf_acc_t __attribute__((ext_vector_type(16)));
+// four floats at any float's address
+typedef float nf_float4 __attribute__((ext_vector_type(4), aligned(4)));
+
+constexpr int kNfTileRows = 128;
+constexpr int kNfEpochRows = 4096; // nine bits: 128 steps of 32 rows, 8 fours
+constexpr uint32_t kNfIndexMask = 511u;
+constexpr float kNfNothing = 1.7e38f;  // s of a row that is none
+constexpr float kNfAlways = -1e37f;    // s of a row that is always looked at
+constexpr float kNfCutLimit = 1e38f;
+
+struct NearestFeatGlobals {
+  unsigned max_bits; // largest |component| of the moderate rows of x
+  unsigned rows;     // moderate rows of x
+  double sum_sq;     // of their squared norms
+};
+
+struct NearestFeatParams {
+  const float *x; // [n, d] candidates
+  const float *y; // [m, d] rows that search
+  const int64_t *ptr_x;
+  const int64_t *ptr_y;
+  int n, m, d, num_segments;
+  const int *work_start;
+  const uint4 *pack;   // [n + kNfTileRows][2 NB + 1] fp16 rows
+  const float *weight; // [n] |x|^2, -1: always looked at, -2: never
+  const NearestFeatGlobals *globals;
+  int64_t *out;
+};
+
+// The power of two that brings a largest component into [2^10, 2^11).
+__device__ __forceinline__ float nf_scale(unsigned max_bits) {
+  if (max_bits == 0)
+    return 1.0f;
+  int e = 137 - (int)((max_bits >> 23) & 0xffu);
+  e = e > 100 ? 100 : (e < -100 ? -100 : e);
+  return __uint_as_float((uint32_t)(e + 127) << 23);
+}
+
+__device__ __forceinline__ uint32_t nf_half(float v) {
+  if (!(__builtin_fabsf(v) >= 6.103515625e-05f)) // 2^-14
+    return 0u;
+  return (uint32_t)__builtin_bit_cast(unsigned short, (_Float16)v);
+}
+
+__device__ __forceinline__ uint4 nf_pack8(const float (&v)[8]) {
+  uint32_t h[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    h[e] = nf_half(v[e]);
+  return make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16),
+                    h[4] | (h[5] << 16), h[6] | (h[7] << 16));
+}
+
+// Components c0 .. c0 + 7 of a row (zeros from d on).
+__device__ __forceinline__ void nf_load8(const float *row, int c0, int d,
+                                         float (&v)[8]) {
+  if (c0 + 8 <= d) {
+    const nf_float4 a = *reinterpret_cast<const nf_float4 *>(row + c0);
+    const nf_float4 b = *reinterpret_cast<const nf_float4 *>(row + c0 + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = a[e];
+      v[4 + e] = b[e];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      v[e] = c0 + e < d ? row[c0 + e] : 0.0f;
+  }
+}
+
+// The reference's distance: direct differences, one fused multiply-add per
+// component in ascending order.  R rows at a time.
+template <int R>
+__device__ __forceinline__ void nf_exact(const float *y, const float *x,
+                                         const int (&row)[R], int d,
+                                         float (&dist)[R]) {
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+    dist[i] = 0.0f;
+  int c = 0;
+#pragma unroll 2
+  for (; c + 4 <= d; c += 4) {
+    const nf_float4 q = *reinterpret_cast<const nf_float4 *>(y + c);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const nf_float4 p = *reinterpret_cast<const nf_float4 *>(
+          x + (size_t)row[i] * d + c);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float t = p[e] - q[e];
+        dist[i] = __builtin_fmaf(t, t, dist[i]);
+      }
+    }
+  }
+#pragma unroll 1
+  for (; c < d; ++c) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const float t = x[(size_t)row[i] * d + c] - y[c];
+      dist[i] = __builtin_fmaf(t, t, dist[i]);
+    }
+  }
+}
+
+// (distance, order among equal ones) as one number; kNfNoKey: none below 1e38
+constexpr unsigned long long kNfNoKey = ~0ull;
+__device__ __forceinline__ unsigned long long nf_key(float dist, int rel) {
+  return dist < kNearestLimit
+             ? ((unsigned long long)__float_as_uint(dist) << 32) |
+                   nearest_tie((uint32_t)rel)
+             : kNfNoKey;
+}
+
+// NB blocks of 16 components (16 (NB - 1) < d <= 16 NB), S sets of 32 queries
+// per wave.
+template <int NB, int S>
+__global__ __launch_bounds__(kBlock, 2) void
+nearest_feat_kernel(NearestFeatParams p) {
+  constexpr int RSU = 2 * NB + 1;
+  constexpr int TR = kNfTileRows;
+  constexpr int UNITS = TR * RSU;
+  constexpr int PIECES = (UNITS + kWave - 1) / kWave;
+  constexpr int WAVES = kBlock / kWave;
+  constexpr int WAVE_PIECES = (PIECES + WAVES - 1) / WAVES;
+  constexpr int TQ = WAVES * S * 32;
+  static_assert(UNITS % kWave == 0, "whole pieces");
+  __shared__ __attribute__((aligned(16))) uint4 tile_rows[2][UNITS];
+  __shared__ __attribute__((aligned(16))) float tile_weight[2][TR];
+  __shared__ unsigned wave_bits[WAVES];
+  __shared__ float wave_norm[WAVES];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int half = lane >> 5;
+  const int col = lane & 31;
+
+  const int tile = blockIdx.x;
+  if (tile >= p.work_start[p.num_segments])
+    return;
+  const int seg = find_segment(p.work_start, p.num_segments, tile);
+  const int x_begin = p.ptr_x ? (int)p.ptr_x[seg] : 0;
+  const int x_end = p.ptr_x ? (int)p.ptr_x[seg + 1] : p.n;
+  const int y_begin = p.ptr_y ? (int)p.ptr_y[seg] : 0;
+  const int y_end = p.ptr_y ? (int)p.ptr_y[seg + 1] : p.m;
+  const int q0 = y_begin + (tile - p.work_start[seg]) * TQ + wave * (S * 32) +
+                 col;
+  const int d = p.d;
+
+  // ---- queries ------------------------------------------------------------
+  // 0: no query, or one no candidate is close enough to; 1: through the
+  // filter; 2: every candidate is evaluated
+  int kind[S];
+  unsigned bits = 0;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int q = q0 + s * 32;
+    kind[s] = 0;
+    if (q < y_end) {
+      const float *row = p.y + (size_t)q * d;
+      float sq = 0.0f;
+      unsigned top = 0;
+#pragma unroll 1
+      for (int b = 0; b < NB; ++b) {
+        float v[8];
+        nf_load8(row, 16 * b + 8 * half, d, v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          sq = __builtin_fmaf(v[e], v[e], sq);
+          top = max(top, __float_as_uint(v[e]) & 0x7fffffffu);
+        }
+      }
+      sq += __shfl_xor(sq, 32);
+      top = max(top, (unsigned)__shfl_xor((int)top, 32));
+      kind[s] = top >= 0x7f800000u ? 0 : sq <= kFilterNormLimit ? 1 : 2;
+      if (kind[s] == 1)
+        bits = max(bits, top);
+    }
+  }
+#pragma unroll
+  for (int sh = 1; sh < 32; sh <<= 1)
+    bits = max(bits, (unsigned)__shfl_xor((int)bits, sh));
+  if (lane == 0)
+    wave_bits[wave] = bits;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w)
+    bits = max(bits, wave_bits[w]);
+  const float s_q = nf_scale(bits);
+
+  nf_f16x8_t yb[S][NB];
+  float ysq[S]; // |b|^2
+  float top_sq = 0.0f;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int q = q0 + s * 32;
+    ysq[s] = 0.0f;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      float v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      if (kind[s] == 1)
+        nf_load8(p.y + (size_t)q * d, 16 * b + 8 * half, d, v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        v[e] *= s_q;
+        ysq[s] = __builtin_fmaf(v[e], v[e], ysq[s]);
+        v[e] *= -2.0f;
+      }
+      yb[s][b] = __builtin_bit_cast(nf_f16x8_t, nf_pack8(v));
+    }
+    ysq[s] += __shfl_xor(ysq[s], 32);
+    top_sq = __builtin_fmaxf(top_sq, ysq[s]);
+  }
+#pragma unroll
+  for (int sh = 1; sh < 32; sh <<= 1)
+    top_sq = __builtin_fmaxf(top_sq, __shfl_xor(top_sq, sh));
+  if (lane == 0)
+    wave_norm[wave] = top_sq;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w)
+    top_sq = __builtin_fmaxf(top_sq, wave_norm[w]);
+
+  // ---- constants of the bound ------------------------------------------------
+  const float s_c = nf_scale(p.globals->max_bits);
+  const double scale2 = (double)s_c * (double)s_q;
+  const double r = (double)s_q / (double)s_c;
+  double rms = 1.0;
+  {
+    const unsigned rows = p.globals->rows;
+    const double mean = rows ? p.globals->sum_sq / rows : 0.0;
+    const double v = __builtin_sqrt(mean) * (double)s_c;
+    if (v > 9.765625e-4 && v < 1e7)
+      rms = v;
+  }
+  const double largest = __builtin_sqrt((double)top_sq) + 1e-3;
+  const double lambda = largest / rms;
+  const double eps = 1.0 / 1024.0 + (double)(d + 20) / 2097152.0;
+  const double delta = (double)(d + 20) / 2097152.0;
+  const double root_d = __builtin_sqrt((double)d) * 1.01;
+  float kappa;
+  {
+    const double k = r * (1.0 - delta) - eps * lambda -
+                     root_d / (32768.0 * rms);
+    kappa = (float)(k < 1e30 ? k : 1e30);
+  }
+  const double r_inv = (double)s_c / (double)s_q;
+  const double per_sq = eps / lambda - r_inv +
+                        (double)(d + 6) * (r_inv + 1.0) / 16777216.0;
+  const double constant = root_d * rms / 32768.0 + (double)d / 134217728.0;
+  // the largest s a row can have whose distance is not above `dist`
+  auto cut_of = [&](float dist, float sq) {
+    const double norm = (double)__builtin_sqrtf(sq) * 1.000001;
+    double c = scale2 * ((double)dist + (double)d * 5.7e-45) *
+                   (1.0 + (double)(d + 6) / 16777216.0) +
+               (double)sq * per_sq + root_d * norm / 8192.0 + constant;
+    c += __builtin_fabs(c) * 2.4e-7; // (the conversion rounds)
+    return c < (double)kNfCutLimit ? (float)c : kNfCutLimit;
+  };
+  // ... and the largest value its minimum of four can be kept as
+  auto kept_cut = [](float cut) {
+    return __builtin_fmaf(__builtin_fabsf(cut), 1.220703125e-4f, cut);
+  };
+
+  unsigned long long best[S];
+  float cut[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    best[s] = kNfNoKey;
+    cut[s] = kNfCutLimit;
+  }
+
+  // ---- one scan over rows c0 .. c1 of x ------------------------------------
+  auto request = [&](int c0, int t, int buf) {
+    const uint4 *src = p.pack + ((size_t)c0 + (size_t)t * TR) * RSU;
+    const uint32_t dst = (uint32_t)(uintptr_t)&tile_rows[buf][0];
+#pragma unroll
+    for (int e = 0; e < WAVE_PIECES; ++e) {
+      const int piece = wave + WAVES * e;
+      if (piece < PIECES) {
+        const uint4 *g = src + piece * kWave + lane;
+        const uint32_t base = dst + (uint32_t)piece * (kWave * 16);
+        // (M0 is written and used inside one statement)
+        asm volatile("s_mov_b32 m0, %1\n\t"
+                     "s_nop 0\n\t"
+                     "global_load_lds_dwordx4 %0, off"
+                     :
+                     : "v"(g), "s"(base)
+                     : "memory");
+      }
+    }
+  };
+  // the start value of the row's chains
+  auto weight_of = [&](int c0, int c1, int t) {
+    float w = kNfNothing;
+    const int row = c0 + t * TR + tid;
+    if (tid < TR && row < c1) {
+      const float v = p.weight[row];
+      if (v >= 0.0f)
+        w = __builtin_fminf(v * s_c * s_c * kappa, 1e37f);
+      else if (v == -1.0f)
+        w = kNfAlways;
+    }
+    return w;
+  };
+  // `visit(step, s, v, acc)` for every 32 rows, set of queries and four rows
+  auto scan = [&](int c0, int c1, auto &&visit) __attribute__((always_inline)) {
+    const int tiles = (c1 - c0 + TR - 1) / TR;
+    __syncthreads(); // (nobody reads an earlier scan's tiles any more)
+    request(c0, 0, 0);
+    float w = weight_of(c0, c1, 0);
+    if (tid < TR)
+      tile_weight[0][tid] = w;
+    for (int t = 0; t < tiles; ++t) {
+      const int buf = t & 1;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (t + 1 < tiles) {
+        w = weight_of(c0, c1, t + 1);
+        request(c0, t + 1, buf ^ 1);
+      }
+#pragma unroll 1
+      for (int i = 0; i < TR / 32; ++i) {
+        const uint4 *arow = &tile_rows[buf][(i * 32 + col) * RSU + half];
+        nf_f16x8_t a[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+          a[b] = __builtin_bit_cast(nf_f16x8_t, arow[2 * b]);
+        nf_acc_t start;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float4 w4 = *reinterpret_cast<const float4 *>(
+              &tile_weight[buf][i * 32 + 8 * v + 4 * half]);
+          start[4 * v] = w4.x;
+          start[4 * v + 1] = w4.y;
+          start[4 * v + 2] = w4.z;
+          start[4 * v + 3] = w4.w;
+        }
+        // the results of a set are looked at while the matrix cores work on
+        // the next one, four values per matrix instruction or so
+        nf_acc_t done = start;
+#pragma unroll
+        for (int s = 0; s <= S; ++s) {
+          nf_acc_t acc = start;
+#pragma unroll
+          for (int b = 0; b < NB; ++b) {
+            if (s < S)
+              acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                  a[b], yb[s < S ? s : 0][b], acc, 0, 0, 0);
+            if (s > 0) {
+#pragma unroll
+              for (int v = 0; v < 4; ++v)
+                if (v * NB / 4 == b)
+                  visit(t * (TR / 32) + i, s - 1, v, done);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          done = acc;
+        }
+      }
+      if (t + 1 < tiles && tid < TR)
+        tile_weight[buf ^ 1][tid] = w;
+    }
+  };
+
+  uint32_t keep_bits = ~kNfIndexMask; // (in a register)
+  asm volatile("" : "+v"(keep_bits));
+  float lowest = -__builtin_inff(); // (the compiler must not know)
+  asm volatile("" : "+s"(lowest));
+  for (int c0 = x_begin; c0 < x_end; c0 += kNfEpochRows) {
+    const int c1 = min(x_end, c0 + kNfEpochRows);
+    float top[S][3];
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      top[s][0] = top[s][1] = top[s][2] = kNfNothing;
+    scan(c0, c1, [&](int step, int s, int v, const nf_acc_t &acc)
+                     __attribute__((always_inline)) {
+      // (fmed3 with -inf is a minimum without the quieting of NaNs that fminf
+      // comes with; it is also the instruction that waits for the matrix
+      // cores, which the compiler sees to only for instructions of its own)
+      float m = __builtin_amdgcn_fmed3f(acc[4 * v], acc[4 * v + 1], lowest);
+      float t;
+      asm("v_min3_f32 %0, %1, %2, %3"
+          : "=v"(m)
+          : "v"(m), "v"(acc[4 * v + 2]), "v"(acc[4 * v + 3]));
+      asm("v_and_or_b32 %0, %1, %2, %3"
+          : "=v"(t)
+          : "v"(m), "v"(keep_bits), "s"(step * 4 + v));
+      top[s][2] = __builtin_amdgcn_fmed3f(top[s][1], top[s][2], t);
+      top[s][1] = __builtin_amdgcn_fmed3f(top[s][0], top[s][1], t);
+      asm("v_min_f32 %0, %1, %2" : "=v"(top[s][0]) : "v"(top[s][0]), "v"(t));
+    });
+
+    bool again = false;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int q = q0 + s * 32;
+      const float *row_y = p.y + (size_t)q * d;
+      // first row of the four behind a kept value
+      auto four_of = [&](float v, int h) {
+        const int index = (int)(__float_as_uint(v) & kNfIndexMask);
+        return c0 + (index >> 2) * 32 + (index & 3) * 8 + 4 * h;
+      };
+      const float other = __shfl_xor(top[s][0], 32);
+      const int owner =
+          half ? (other <= top[s][0] ? 0 : 1) : (top[s][0] <= other ? 0 : 1);
+      const float least = owner == half ? top[s][0] : other;
+      if (kind[s] == 1 && least <= cut[s]) {
+        // two of the four rows per lane
+        const int first = four_of(least, owner) + 2 * half;
+        const int rows[2] = {min(first, c1 - 1), min(first + 1, c1 - 1)};
+        float dist[2];
+        nf_exact<2>(row_y, p.x, rows, d, dist);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          best[s] = min(best[s], nf_key(dist[i], rows[i] - x_begin));
+      }
+      best[s] = min(best[s], (unsigned long long)__shfl_xor(best[s], 32));
+      if (kind[s] == 1) {
+        cut[s] = cut_of(best[s] != kNfNoKey
+                            ? __uint_as_float((uint32_t)(best[s] >> 32))
+                            : kNearestLimit,
+                        ysq[s]);
+        const float kept = kept_cut(cut[s]);
+        unsigned long long own = best[s];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          if (top[s][e] <= kept && !(e == 0 && owner == half)) {
+#pragma unroll 1
+            for (int i = 0; i < 4; ++i) {
+              const int rows[1] = {four_of(top[s][e], half) + i};
+              if (rows[0] < c1) {
+                float dist[1];
+                nf_exact<1>(row_y, p.x, rows, d, dist);
+                own = min(own, nf_key(dist[0], rows[0] - x_begin));
+              }
+            }
+          }
+        }
+        best[s] = own;
+        // (the lane goes through its rows again)
+        if (top[s][2] <= kept)
+          again = true;
+        else
+          cut[s] = -kNfCutLimit;
+      } else if (kind[s] == 2) {
+        again = true; // (with the cut that lets every row through)
+      } else {
+        cut[s] = -kNfCutLimit;
+      }
+    }
+
+    if (__syncthreads_or(again)) {
+      unsigned long long hits = 0; // 16 bits per set
+      scan(c0, c1, [&](int step, int s, int v, const nf_acc_t &acc)
+                       __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          hits |= acc[4 * v + i] <= cut[s] ? 1ull << (16 * s + 4 * v + i) : 0;
+        if (s < S - 1 || v < 3)
+          return;
+        while (hits != 0) {
+          const int at = __builtin_ctzll(hits);
+          hits &= hits - 1;
+          const int hit_s = at >> 4, hit_v = (at >> 2) & 3;
+          const int rows[1] = {c0 + step * 32 + 8 * hit_v + 4 * half +
+                               (at & 3)};
+          if (rows[0] < c1) {
+            float dist[1];
+            nf_exact<1>(p.y + (size_t)(q0 + hit_s * 32) * d, p.x, rows, d,
+                        dist);
+            const unsigned long long key = nf_key(dist[0], rows[0] - x_begin);
+#pragma unroll
+            for (int u = 0; u < S; ++u)
+              best[u] = u == hit_s ? min(best[u], key) : best[u];
+          }
+        }
+      });
+    }
+    // both lanes go on with the query's best row and a cut that follows it
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      best[s] = min(best[s], (unsigned long long)__shfl_xor(best[s], 32));
+      cut[s] = kNfCutLimit;
+      if (kind[s] == 1 && best[s] != kNfNoKey)
+        cut[s] = kept_cut(
+            cut_of(__uint_as_float((uint32_t)(best[s] >> 32)), ysq[s]));
+    }
+  }
+
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int q = q0 + s * 32;
+    if (half == 0 && q < y_end)
+      p.out[q] = best[s] != kNfNoKey
+                     ? (int64_t)x_begin +
+                           (int64_t)nearest_rel((uint32_t)best[s])
+                     : 0;
+  }
+}
+
+// |x|^2 of every row (or what it is instead, see NearestFeatParams), and the
+// largest component and the sum of the squares over the moderate rows.
+__global__ __launch_bounds__(kBlock) void nearest_feat_rows_kernel(
+    const float *__restrict__ x, int n, int d, float *__restrict__ weight,
+    NearestFeatGlobals *__restrict__ globals);
+
+// The fp16 operands of the rows, one thread per unit of 8 components; zeros
+// for rows the filter does not represent and for a tile of rows behind the
+// last one.
+template <int NB>
+__global__ __launch_bounds__(kBlock) void nearest_feat_pack_kernel(
+    const float *__restrict__ x, int n, int d,
+    const float *__restrict__ weight,
+    const NearestFeatGlobals *__restrict__ globals, uint4 *__restrict__ pack) {
+  constexpr int U = 2 * NB;
+  const size_t id = (size_t)blockIdx.x * kBlock + threadIdx.x;
+  if (id >= (size_t)(n + kNfTileRows) * U)
+    return;
+  const int row = (int)(id / U);
+  const int unit = (int)(id - (size_t)row * U);
+  uint4 out = make_uint4(0, 0, 0, 0);
+  if (row < n && weight[row] >= 0.0f) {
+    const float scale = nf_scale(globals->max_bits);
+    float v[8];
+    nf_load8(x + (size_t)row * d, 8 * unit, d, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      v[e] *= scale;
+    out = nf_pack8(v);
+  }
+  pack[(size_t)row * (U + 1) + unit] = out;
+}
+
+// One number of component blocks (two per translation unit).
+template <int NB>
+hipError_t launch_nearest_feat_blocks(const NearestFeatParams &p, int sets,
+                                      int grid, hipStream_t stream);
+// Sets of 32 queries per wave: as many as the registers hold.
+constexpr int nearest_feat_sets(int nb) { return nb <= 4 ? 4 : nb <= 6 ? 3 : 2; }
+
+#define PCA_NEAREST_FEAT_DEFINE(NB_)                                           \
+  template <>                                                                  \
+  hipError_t launch_nearest_feat_blocks<NB_>(const NearestFeatParams &p,       \
+                                             int sets, int grid,               \
+                                             hipStream_t stream) {             \
+    const size_t units = ((size_t)p.n + kNfTileRows) * (2 * NB_);              \
+    hipLaunchKernelGGL((nearest_feat_pack_kernel<NB_>),                        \
+                       dim3((unsigned)((units + kBlock - 1) / kBlock)),        \
+                       dim3(kBlock), 0, stream, p.x, p.n, p.d, p.weight,       \
+                       p.globals, const_cast<uint4 *>(p.pack));                \
+    if (sets == 1)                                                             \
+      hipLaunchKernelGGL((nearest_feat_kernel<NB_, 1>), dim3(grid),            \
+                         dim3(kBlock), 0, stream, p);                          \
+    else                                                                       \
+      hipLaunchKernelGGL((nearest_feat_kernel<NB_, nearest_feat_sets(NB_)>),   \
+                         dim3(grid), dim3(kBlock), 0, stream, p);              \
+    return hipGetLastError();                                                  \
+  }
+
+} // namespace pca
