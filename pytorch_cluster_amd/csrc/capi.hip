@@ -539,15 +539,37 @@ int knn_call(const void *x, const void *y, const int64_t *ptr_x,
   pca::SegmentSource src;
   const bool by_id = (edge_flags & PCA_SEGMENTS_BY_ID) != 0 && ptr_x != nullptr;
   int rc = PCA_OK;
+  const bool wave =
+      low_d && pca::knn_wave_supported((int)n, (int)m, (int)d,
+                                       (int)num_segments, (int)k, cosine != 0);
   if (by_id)
     src = segments_by_id(ptr_x, ptr_y, n, m, num_segments, take(lay.ptrs));
-  const bool plan_derives = by_id && num_segments <= kPlanDerivesExamples;
+  const bool plan_derives =
+      by_id && !wave && num_segments <= kPlanDerivesExamples;
   if (by_id && !plan_derives)
     rc = check_launch(
         pca::launch_segment_pointers(src, (int)num_segments, stream),
         "segment_pointers_kernel");
   if (rc != PCA_OK)
     return rc;
+  if (wave) {
+    pca::compact_counted(dense, (int)m, compact_ws,
+                         (edge_flags & PCA_EDGES_DROP_SELF) != 0);
+    const pca::SearchInput small{x,      y,      ptr_x,  ptr_y,
+                                 (int)n, (int)m, (int)d, (int)num_segments};
+    rc = check_launch(pca::launch_knn_wave(small, (int)k, dense, timer.start,
+                                           timer.stop, stream),
+                      "knn_wave_kernel");
+    timer.stop = nullptr;
+    if (rc != PCA_OK)
+      return rc;
+    return check_launch(
+        pca::launch_compact(dense, (int)m, edges, num_edges,
+                            static_cast<float *>(dist), compact_ws, stream,
+                            (edge_flags & PCA_EDGES_DROP_SELF) != 0,
+                            (edge_flags & PCA_EDGES_X_FIRST) != 0),
+        "compaction kernels");
+  }
   pca::KnnLowdConfig cfg = pca::knn_lowd_config(
       (int)d, (int)k, (int)n, (int)m, (int)num_segments, cosine != 0);
   // (the matrix-core kernels count the edges while they write their lists)

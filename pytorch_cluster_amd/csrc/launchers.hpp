@@ -26,6 +26,9 @@ struct DenseResult {
   unsigned long long *edge_sums = nullptr;
   int *self_pos = nullptr;
   int *kept = nullptr;
+  // self_pos / kept are filled and the call is small enough for the
+  // compaction to add up the counts themselves: no block sums (compact_counted)
+  bool counted = false;
 };
 
 struct SearchInput {
@@ -84,6 +87,11 @@ hipError_t launch_compact(const DenseResult &dense, int m, int64_t *edges,
 // counting pass.  Only for searches that fill them (the low-dimensional
 // matrix-core kernels, the one-kernel feature-space search).
 void compact_hints(DenseResult &dense, int m, void *workspace, bool drop_self);
+// The same for a search that fills self_pos / kept (with drop_self) and no
+// sums, of up to kCompactCountedQueries queries.
+constexpr int kCompactCountedQueries = 8192;
+void compact_counted(DenseResult &dense, int m, void *workspace,
+                     bool drop_self);
 // Queries per block sum.
 constexpr int kCompactBlockQueries = 256;
 
@@ -119,6 +127,17 @@ hipError_t launch_knn_lowd(const SearchInput &in, int k, bool cosine,
                            hipEvent_t time_start, hipEvent_t time_stop,
                            hipStream_t stream, int64_t *nearest_out = nullptr,
                            const SegmentSource *src = nullptr);
+
+// --- knn_wave.hip ------------------------------------------------------------
+
+// Small calls, one wave per query: fp32, up to 4 dimensions, Euclidean,
+// k <= 64, at most kCompactCountedQueries queries.  PCA_KNN_WAVE=0: never, 1:
+// whenever the shape fits.
+bool knn_wave_supported(int n, int m, int d, int num_segments, int k,
+                        bool cosine);
+hipError_t launch_knn_wave(const SearchInput &in, int k, const DenseResult &out,
+                           hipEvent_t time_start, hipEvent_t time_stop,
+                           hipStream_t stream);
 
 // --- knn_binned.hip --------------------------------------------------------
 

@@ -216,8 +216,9 @@ __device__ __forceinline__ int wave_inclusive_scan(int v, int lane) {
 
 // count: slots to write per query (without the self slot when self_pos is
 // given).  x_first: the x row goes to the first half of `edges`.
-// inline_scan: block_offsets holds the blocks' SUMS; this block adds up the
-// ones before it and all of them (block 0 also stores the total).
+// inline_scan 1: block_offsets holds the blocks' SUMS; this block adds up the
+// ones before it and all of them (block 0 also stores the total).  2: it adds
+// up the counts themselves.
 //
 // Bound by the latency of its reads -- counts and sums, then slots -- as long
 // as the device is not full: 1 << parts_log2 workgroups share a block of
@@ -247,11 +248,18 @@ __global__ __launch_bounds__(kBlock) void scatter_kernel(
   const int c = q < m ? count[q] : 0;
   const int self = self_pos && q < m ? self_pos[q] : -1;
   int64_t before = 0, all = 0;
-  if (inline_scan)
+  if (inline_scan == 1)
     for (int b = tid; b < num_blocks; b += kBlock) {
       const int64_t v = block_offsets[b];
       all += v;
       before += b < block ? v : 0;
+    }
+  else if (inline_scan == 2)
+#pragma unroll 4
+    for (int i = tid; i < m; i += kBlock) {
+      const int v = count[i];
+      all += v;
+      before += i < q0 ? v : 0;
     }
   const int inclusive = wave_inclusive_scan(c, lane);
   s_count[tid] = c;
@@ -373,6 +381,18 @@ void compact_hints(DenseResult &dense, int m, void *workspace, bool drop_self) {
   }
 }
 
+void compact_counted(DenseResult &dense, int m, void *workspace,
+                     bool drop_self) {
+  if (m > kCompactCountedQueries)
+    return;
+  dense.counted = true;
+  if (drop_self) {
+    dense.self_pos = static_cast<int *>(workspace);
+    dense.kept = reinterpret_cast<int *>(static_cast<char *>(workspace) +
+                                         align256(sizeof(int) * (size_t)m));
+  }
+}
+
 hipError_t launch_compact(const DenseResult &dense, int m, int64_t *edges,
                           int64_t *num_edges, float *dist_out, void *workspace,
                           hipStream_t stream, bool drop_self, bool x_first) {
@@ -399,6 +419,15 @@ hipError_t launch_compact(const DenseResult &dense, int m, int64_t *edges,
                        dense.slots, magic, x_first ? 1 : 0, parts_log2, blocks,
                        reinterpret_cast<const int64_t *>(dense.edge_sums),
                        num_edges, edges, dist_out, 1);
+    return hipGetLastError();
+  }
+  if (dense.counted) {
+    hipLaunchKernelGGL(scatter_kernel, scatter_grid, dim3(kBlock), 0, stream,
+                       dense.idx, dense.dist, drop_self ? dense.kept : count,
+                       drop_self ? dense.self_pos : (const int *)nullptr, m,
+                       dense.slots, magic, x_first ? 1 : 0, parts_log2, blocks,
+                       (const int64_t *)nullptr, num_edges, edges, dist_out,
+                       2);
     return hipGetLastError();
   }
   if (blocks <= kInlineScanBlocks) {
