@@ -824,12 +824,15 @@ int pca_radius(const void *x, const void *y, const int64_t *ptr_x,
     return fail(PCA_ERR_WORKSPACE, "workspace needs %zu bytes, 256-aligned",
                 radius_workspace(n, m, d, num_segments, slots, dtype));
 
-  const bool matrix_cores =
+  const bool short_examples =
       dtype == PCA_F32 &&
+      pca::radius_short_supported((int)d, (int)n, (int)m, (int)num_segments);
+  const bool matrix_cores =
+      !short_examples && dtype == PCA_F32 &&
       pca::radius_mc_supported((int)d, (int)n, (int)m, (int)num_segments);
   const int r16 = dtype == PCA_F16 ? 1 : (dtype == PCA_BF16 ? 2 : 0);
   const bool feature_space =
-      !matrix_cores && (dtype == PCA_F32 || r16 != 0) &&
+      !short_examples && !matrix_cores && (dtype == PCA_F32 || r16 != 0) &&
       pca::radius_feat_supported((int)n, (int)m, (int)d, (int)num_segments,
                                  (int)slots, r16);
   Carver ws(workspace);
@@ -857,7 +860,7 @@ int pca_radius(const void *x, const void *y, const int64_t *ptr_x,
     src = segments_by_id(ptr_x, ptr_y, n, m, num_segments,
                          ws.take<char>(segment_pointer_bytes(num_segments)));
   const bool plan_derives = by_id && num_segments <= kPlanDerivesExamples;
-  if (by_id && !plan_derives)
+  if (by_id && !plan_derives && !short_examples)
     rc = check_launch(
         pca::launch_segment_pointers(src, (int)num_segments, stream),
         "segment_pointers_kernel");
@@ -873,8 +876,9 @@ int pca_radius(const void *x, const void *y, const int64_t *ptr_x,
   const int per_item = matrix_cores    ? pca::kRadiusMcTileQueries
                        : feature_space ? pca::kMfmaTileQueries
                                        : pca::kRadiusQueriesPerWave;
-  // (the matrix-core path plans its work in the launch that packs the rows)
-  if (!matrix_cores)
+  // (the matrix-core path plans its work in the launch that packs the rows,
+  // short examples need no plan)
+  if (!matrix_cores && !short_examples)
     rc = check_launch(pca::launch_plan(ptr_y, (int)m, (int)num_segments,
                                        per_item, work_start, stream,
                                        plan_derives ? &src : nullptr),
@@ -885,9 +889,14 @@ int pca_radius(const void *x, const void *y, const int64_t *ptr_x,
       pca::plan_upper_bound((int)m, (int)num_segments, per_item);
   if (!matrix_cores && !feature_space)
     timer.begin();
-  if (matrix_cores || feature_space)
+  if (matrix_cores || feature_space || short_examples)
     pca::compact_hints(dense, (int)m, compact_ws, false);
-  if (feature_space) {
+  if (short_examples) {
+    rc = check_launch(pca::launch_radius_short(in, r2, ignore_same_index != 0,
+                                               dense, stream,
+                                               by_id ? &src : nullptr),
+                      "radius_short_kernel");
+  } else if (feature_space) {
     const pca::FeatRadius radius{
         r16 != 0 ? pca::narrow_r2_16bit(r * r, r16 == 2) : r2,
         ignore_same_index != 0};

@@ -338,6 +338,18 @@ hipError_t launch_radius_mc(const SearchInput &in, float r2,
                             hipStream_t stream,
                             const SegmentSource *src = nullptr);
 
+// --- radius_short.hip --------------------------------------------------------
+
+// Many short examples: fp32, up to 4 dimensions, a lane per query.  No plan and
+// no packed rows; with src the example ids are searched directly (the
+// pointers of `in` are not read).  Fills out.edge_sums.  PCA_RADIUS_SHORT=0:
+// never, 1: whenever the dimension fits.
+bool radius_short_supported(int d, int n, int m, int num_segments);
+hipError_t launch_radius_short(const SearchInput &in, float r2,
+                               bool ignore_same_index, const DenseResult &out,
+                               hipStream_t stream,
+                               const SegmentSource *src = nullptr);
+
 // --- radius.hip ------------------------------------------------------------
 
 constexpr int kRadiusQueriesPerWave = 8;
