@@ -67,6 +67,7 @@ hipError_t launch_radius_mc(const SearchInput &in, float r2,
   if (tiles_bound <= 0)
     return hipSuccess;
   RadiusMcParams p;
+  p.x = static_cast<const float *>(in.x);
   p.y = static_cast<const float *>(in.y);
   p.ptr_x = in.ptr_x;
   p.ptr_y = in.ptr_y;

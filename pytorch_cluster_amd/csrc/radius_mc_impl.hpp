@@ -10,8 +10,8 @@
 // moves: t - cut = w - 2 x.y - cut, cut = r^2 (1 + eps) - fl(|y|^2) (1 - eps),
 // comes out of one v_mfma_f32_32x32x16_bf16 per 32 rows x 32 queries
 // (split-bf16 operands, -cut in the two spare accumulation slots), the sign
-// bits of a lane's 16 results are gathered with funnel shifts, and a lane with
-// a non-zero mask parks (step, mask) in its LDS queue.  A candidate with an
+// bits of a lane's 16 results are gathered with funnel shifts, and a pair of
+// lanes with a row that passed parks (step, mask) in its LDS queue.  A candidate with an
 // exact distance below r^2 always has its sign bit set (error budget in
 // knn_lowd_mc_impl.hpp); whether a row with the bit set IS a neighbour is
 // decided by the exact distance (direct differences, one FMA per component in
@@ -19,10 +19,24 @@
 //
 // Lanes l and l + 32 share a query and see interleaved groups of four rows.
 // When a queue fills up or the tile ends, the lower lane of each pair walks
-// the parked rows of BOTH lanes in ascending row order and appends the
+// the parked rows in ascending order and appends the
 // neighbours to the query's slot row until it holds max_num_neighbors.  A
 // query that is full stops parking; a wave whose queries are all full skips
 // the matrix-core work, a workgroup whose waves are all done leaves the scan.
+//
+// A few queries far from everything would keep the whole workgroup scanning
+// (clustered points: after an eighth of the rows 85 % of the queries are
+// full, but hardly a wave is).  So from the first tile on at whose start at
+// most kRadiusFew queries are open, these are dealt to the four waves, and a
+// wave goes through the rows on its own, straight from memory, 256 at a time,
+// once for all its open queries: hits are found and numbered by ballots, in
+// row order as they are.  No barriers, no tiles, and a wave whose queries are
+// full leaves.
+//
+// 8 clouds of 16,384 clustered points, r = 0.05, 32 neighbours: kernel 228 ->
+// 132 us (the walk of parked rows without nested branches 20 us of that; 64
+// open queries instead of 32: 4 us more); two thirds of what is left are the
+// first three tiles, in which every query meets its neighbours one by one.
 //
 // A workgroup owns 128 queries of one segment and scans the whole segment
 // (rows must be reported in order, so the segment is not sliced).
@@ -32,7 +46,10 @@
 
 namespace pca {
 
+constexpr int kRadiusFew = 32; // open queries a workgroup deals to its waves
+
 struct RadiusMcParams {
+  const float *x;
   const float *y;
   const int64_t *ptr_x;
   const int64_t *ptr_y;
@@ -62,10 +79,12 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
   // (every 16-byte unit of a row in a plane of its own, as in
   // knn_lowd_mc_impl.hpp: conflict-free reads)
   __shared__ __attribute__((aligned(16))) uint4 rows_lds[REC][TX];
-  // parked steps: (step << 16) | mask of the lane's 16 rows that passed
+  // parked steps of the pairs of lanes: in the lower lane's column the mask of
+  // the 32 rows, in the upper lane's the step
   // (also carries, between the two barriers at the top of a tile, the four
-  // waves' "all my queries are full" flags: one more variable would take the
-  // workgroup past 40,960 bytes, the most that lets four of them share a CU)
+  // waves' numbers of open queries, and the last few open queries: one more
+  // variable would take the workgroup past 40,960 bytes, the most that lets
+  // four of them share a CU)
   __shared__ uint32_t queue[QCAP][kBlock];
 
   const int tid = threadIdx.x;
@@ -157,7 +176,9 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
   // the upper one after every drain); a query without a slot left is done
   int count = 0;
   bool done = !valid || slots <= 0;
-  int qn = 0; // parked steps of this lane: queue[0 .. qn)[tid]
+  int qn = 0; // parked steps of this pair: queue[0 .. qn)[lower, upper lane]
+  const bool ignore_same = p.ignore_same_index != 0;
+  int *const slot_row = p.out_idx + (size_t)(valid ? q : y_begin) * slots;
 
   // ---- tile staging -------------------------------------------------------
   uint4 stage[PT][REC];
@@ -191,78 +212,53 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
         rows_lds[i][r * kBlock + tid] = stage[r][i];
   };
 
-  // One lane's walk over parked rows (see knn_lowd_mc_kernel): peek returns
-  // the next row of queue column `column` (position in the tile) or a large
-  // number if none is left.
-  struct Walk {
-    int taken;
-    uint32_t pending;
-    int base;
-  };
-  auto peek = [&](Walk &w, int column, int entries, int row0) {
-    if (w.pending == 0 && w.taken < entries) {
-      const uint32_t word = queue[w.taken][column];
-      ++w.taken;
-      w.pending = word & 0xffffu;
-      w.base = (int)(word >> 16) * 32 + row0;
-    }
-    if (w.pending == 0)
-      return 1 << 30;
-    const int bit = 31 - __builtin_clz(w.pending);
-    const int v = 15 - bit;
-    return w.base + 2 * (v & 12) + (v & 3);
-  };
-  auto pop = [&](Walk &w) { // (only after a successful peek)
-    const int bit = 31 - __builtin_clz(w.pending);
-    w.pending &= ~(1u << bit);
-  };
-
   // Resolves the parked rows of the tile: the lower lane of every pair takes
-  // the rows of both lanes in ascending order.
+  // them in ascending order.  (No nested loops or branches but the refill: all
+  // lanes of a wave pass through every branch some lane takes.)
   auto drain = [&](int g_base, int rows) {
-    const auto both = __builtin_amdgcn_permlane32_swap((unsigned)qn,
-                                                       (unsigned)qn, false,
-                                                       false);
-    const int qn_upper = (int)both[1]; // of lane l + 32 (for the lower lanes)
-    Walk lo{0, 0u, 0}, hi{0, 0u, 0};
-    const bool worker = half == 0 && !done;
+    uint32_t pending = 0;
+    int base = 0, taken = 0;
+    const int entries = half == 0 && !done ? qn : 0;
     for (;;) {
-      int j = 1 << 30;
-      if (worker) {
-        const int a = peek(lo, tid, qn, 0);
-        const int b = peek(hi, tid + 32, qn_upper, 4);
-        j = min(a, b);
-        if (j < (1 << 30)) {
-          if (a <= b)
-            pop(lo);
-          else
-            pop(hi);
-        }
+      const bool refill = pending == 0 && taken < entries;
+      if (__any(refill)) {
+        const int at = min(taken, QCAP - 1);
+        const uint32_t mask = queue[at][tid];
+        const int step = (int)queue[at][min(tid + 32, kBlock - 1)];
+        pending = refill ? mask : pending;
+        base = refill ? step * 32 : base;
+        taken += refill ? 1 : 0;
       }
-      const bool has = j < rows; // (also drops padding rows)
-      if (!__any(j < (1 << 30)))
+      const bool has = pending != 0;
+      if (!__any(has))
         break;
-      if (has && count < slots) {
-        float row[XF];
+      const int v = __builtin_clz(pending | 1u);
+      const int j = base + v;
+      pending &= ~(0x80000000u >> v);
+      float row[XF];
 #pragma unroll
-        for (int e = 0; e < XF; e += 4) {
-          const uint4 q4 = rows_lds[NI + e / 4][j];
-          row[e] = __uint_as_float(q4.x);
-          row[e + 1] = __uint_as_float(q4.y);
-          row[e + 2] = __uint_as_float(q4.z);
-          row[e + 3] = __uint_as_float(q4.w);
-        }
-        const float d0 = row[0] - yq[0];
-        float dist = d0 * d0;
+      for (int e = 0; e < XF; e += 4) {
+        const uint4 q4 = rows_lds[NI + e / 4][min(j, TX - 1)];
+        row[e] = __uint_as_float(q4.x);
+        row[e + 1] = __uint_as_float(q4.y);
+        row[e + 2] = __uint_as_float(q4.z);
+        row[e + 3] = __uint_as_float(q4.w);
+      }
+      const float d0 = row[0] - yq[0];
+      float dist = d0 * d0;
 #pragma unroll
-        for (int c = 1; c < DIM; ++c) {
-          const float dc = row[c] - yq[c];
-          dist = __builtin_fmaf(dc, dc, dist);
-        }
-        const int g = g_base + j;
-        if (dist < r2 && !(p.ignore_same_index && g == q)) {
-          p.out_idx[(size_t)q * slots + count] = g;
-          ++count;
+      for (int c = 1; c < DIM; ++c) {
+        const float dc = row[c] - yq[c];
+        dist = __builtin_fmaf(dc, dc, dist);
+      }
+      const int g = g_base + j;
+      // (j < rows: no padding rows)
+      if (has && dist < r2 && j < rows && !(ignore_same && g == q)) {
+        slot_row[count] = g;
+        ++count;
+        if (count >= slots) {
+          pending = 0;
+          taken = entries;
         }
       }
     }
@@ -279,20 +275,29 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
   if (num_tiles > 0)
     load_tile(0);
   bool wave_done = false;
+  int few = 0, few_before = 0; // open queries, those of the waves before
+  int t = 0;
 
-  for (int t = 0; t < num_tiles; ++t) {
+  for (; t < num_tiles; ++t) {
     // one LDS buffer: the next tile waits in registers while this one is
     // scanned
     // (no lane has anything parked here)
+    const uint32_t open_queries = (uint32_t)__ballot(!done);
     if (lane == 0)
-      queue[0][wave * kWave] = wave_done ? 1u : 0u;
+      queue[0][wave * kWave] = (uint32_t)__builtin_popcount(open_queries);
     __syncthreads();
-    bool all_done = true;
+    int open = 0;
+    few_before = 0;
 #pragma unroll
-    for (int w = 0; w < kBlock / kWave; ++w)
-      all_done = all_done && queue[0][w * kWave] != 0;
-    if (all_done)
-      break; // (read between two barriers: the same for every thread)
+    for (int w = 0; w < kBlock / kWave; ++w) {
+      few_before = w == wave ? open : few_before;
+      open += (int)queue[0][w * kWave];
+    }
+    // (read between two barriers: the same for every thread)
+    if (open <= kRadiusFew) {
+      few = open;
+      break;
+    }
     store_tile();
     __syncthreads();
     if (t + 1 < num_tiles)
@@ -336,8 +341,16 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
       if (done)
         mask = 0;
       if (__any(mask != 0)) {
-        if (mask != 0) {
-          queue[qn][tid] = ((uint32_t)rt << 16) | mask;
+        // the rows of both lanes of a pair in order: nibbles of the lower and
+        // of the upper lane in turn, the first row in the highest bit
+        uint32_t rows_of = (mask | (mask << 8)) & 0x00ff00ffu;
+        rows_of = (rows_of | (rows_of << 4)) & 0x0f0f0f0fu;
+        rows_of <<= half == 0 ? 4 : 0;
+        const auto both = __builtin_amdgcn_permlane32_swap(rows_of, rows_of,
+                                                           false, false);
+        rows_of = both[0] | both[1];
+        if (rows_of != 0) {
+          queue[qn][tid] = half == 0 ? rows_of : (uint32_t)rt;
           ++qn;
         }
         if (__any(qn >= QCAP)) {
@@ -350,6 +363,114 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
     drain(g_base, rows);
     if (!__any(!done))
       wave_done = true;
+  }
+
+  if (few > 0) {
+    // entry e: query, slots filled, coordinates
+    constexpr int W = kBlock / kWave;
+    constexpr int MINE = (kRadiusFew + W - 1) / W;
+    static_assert(DIM * kRadiusFew <= kBlock && QCAP >= 4, "the queue's rows");
+    const uint32_t open_queries = (uint32_t)__ballot(!done);
+    const int entry =
+        few_before + __builtin_popcount(open_queries & ((1u << col) - 1u));
+    const bool mine = half == 0 && !done;
+    if (mine) {
+      queue[1][entry] = (uint32_t)q;
+      queue[2][entry] = (uint32_t)count;
+#pragma unroll
+      for (int c = 0; c < DIM; ++c)
+        queue[3][c * kRadiusFew + entry] = __float_as_uint(yq[c]);
+    }
+    __syncthreads();
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    auto uniform = [](uint32_t v) {
+      return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+    };
+    int of[MINE], filled[MINE];
+    float at[MINE][DIM];
+    uint32_t open = 0; // the wave's queries that are not full
+#pragma unroll
+    for (int i = 0; i < MINE; ++i) {
+      const int e = min(wave_u + W * i, few - 1);
+      of[i] = (int)uniform(queue[1][e]);
+      filled[i] = (int)uniform(queue[2][e]);
+#pragma unroll
+      for (int c = 0; c < DIM; ++c)
+        at[i][c] = __uint_as_float(uniform(queue[3][c * kRadiusFew + e]));
+      open |= wave_u + W * i < few ? 1u << i : 0u;
+    }
+    // the rows from the tile that waits in registers on, straight from memory,
+    // one round of G x 64 ahead of the one that is looked at
+    constexpr int G = DIM <= 4 ? 4 : 2;
+    float next[G][DIM];
+    auto load_rows = [&](int pos) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const int row = x_begin + min(pos + g * kWave + lane, c_count - 1);
+#pragma unroll
+        for (int c = 0; c < DIM; ++c)
+          next[g][c] = c < d_in ? p.x[(size_t)row * d_in + c] : 0.0f;
+      }
+    };
+    if (open != 0)
+      load_rows(t * TX);
+    for (int pos = t * TX; pos < c_count && open != 0; pos += G * kWave) {
+      float row[G][DIM];
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int c = 0; c < DIM; ++c)
+          row[g][c] = next[g][c];
+      if (pos + G * kWave < c_count)
+        load_rows(pos + G * kWave);
+#pragma unroll
+      for (int i = 0; i < MINE; ++i) {
+        if ((open & (1u << i)) == 0)
+          continue;
+        bool hit[G];
+        bool any = false;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const float d0 = row[g][0] - at[i][0];
+          float dist = d0 * d0;
+#pragma unroll
+          for (int c = 1; c < DIM; ++c) {
+            const float dc = row[g][c] - at[i][c];
+            dist = __builtin_fmaf(dc, dc, dist);
+          }
+          hit[g] = dist < r2;
+          any = any || hit[g];
+        }
+        if (!__any(any))
+          continue;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const int j = pos + g * kWave + lane;
+          const bool take = hit[g] && j < c_count &&
+                            !(p.ignore_same_index && x_begin + j == of[i]);
+          const uint64_t hits = __ballot(take);
+          const int slot =
+              filled[i] + (int)__builtin_amdgcn_mbcnt_hi(
+                              (uint32_t)(hits >> 32),
+                              __builtin_amdgcn_mbcnt_lo((uint32_t)hits, 0u));
+          if (take && slot < slots)
+            p.out_idx[(size_t)of[i] * slots + slot] = x_begin + j;
+          filled[i] += __builtin_popcountll(hits);
+        }
+        if (filled[i] >= slots) {
+          filled[i] = slots;
+          open &= ~(1u << i);
+        }
+      }
+    }
+    // the lanes that own the queries take the counts back
+#pragma unroll
+    for (int i = 0; i < MINE; ++i)
+      if (lane == 0 && wave_u + W * i < few)
+        queue[2][wave_u + W * i] = (uint32_t)filled[i];
+    __syncthreads();
+    if (mine)
+      count = (int)queue[2][entry];
   }
 
   if (valid && half == 0) {

@@ -1,0 +1,62 @@
+"""The matrix-core radius search where most queries of a workgroup are full
+early and the others go on by a wave each (csrc/radius_mc_impl.hpp), against
+the oracle: numbers of open queries around the switch and the waves' shares,
+rows around a tile and a wave, every compiled dimension."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from gpu_common import gpu_radius  # noqa: E402
+
+
+@pytest.fixture(autouse=True)
+def always(monkeypatch):
+    monkeypatch.setenv("PCA_RADIUS_MATRIX_CORES", "1")
+    monkeypatch.setenv("PCA_RADIUS_SHORT", "0")
+
+
+def check(oracle, x, y, ptr_x, ptr_y, r, limit, ignore_same=False):
+    want = oracle.radius_op(x, y, ptr_x, ptr_y, r, limit,
+                            ignore_same_index=ignore_same)
+    got = gpu_radius(x, y, ptr_x, ptr_y, r, limit, ignore_same)
+    assert got.shape == want.shape and (got == want).all()
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("open_queries", [1, 3, 4, 5, 31, 32, 33, 60])
+def test_open_queries(oracle, d, open_queries):
+    rng = np.random.default_rng(d * 100 + open_queries)
+    n = 3 * 1024 + 65
+    # rows near the origin, some near (3, ...): few and late, some nowhere
+    x = (0.1 * rng.random((n, d))).astype(np.float32)
+    x[1500::97] += 3
+    y = (0.1 * rng.random((140, d))).astype(np.float32)
+    far = rng.permutation(128)[:open_queries]
+    y[far] += 3
+    y[far[::3]] += 3
+    ptr_x, ptr_y = [0, n], [0, 140]
+    for limit in (1, 5, 20, 200):
+        check(oracle, x, y, ptr_x, ptr_y, 1.0, limit)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 256, 1023, 1024, 1025, 2100])
+@pytest.mark.parametrize("m", [1, 32, 33, 129, 160])
+def test_few_queries_from_the_start(oracle, n, m):
+    rng = np.random.default_rng(n + m)
+    x = rng.random((n, 3)).astype(np.float32)
+    y = rng.random((m, 3)).astype(np.float32)
+    for r, limit in ((0.3, 32), (2.0, 70), (0.05, 3)):
+        check(oracle, x, y, [0, n], [0, m], r, limit)
+
+
+def test_clustered_graph(oracle):
+    rng = np.random.default_rng(5)
+    sizes = [5000, 0, 1300, 2500]
+    ptr = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    centres = rng.random((12, 3))
+    x = (centres[rng.integers(0, 12, ptr[-1])]
+         + 0.02 * rng.standard_normal((ptr[-1], 3))).astype(np.float32)
+    x[7], x[1200, 1], x[6000] = np.nan, np.inf, 3e38
+    for r, limit in ((0.05, 32), (0.02, 8), (0.1, 64), (np.inf, 16)):
+        check(oracle, x, x, ptr, ptr, r, limit, ignore_same=True)
