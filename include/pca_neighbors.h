@@ -139,6 +139,32 @@ int pca_segment_pointers(const int64_t *ids_x, int64_t n, const int64_t *ids_y,
                          int64_t *ptr_y, void *stream);
 
 /*
+ * For `nearest` given example ids (sorted [n] / [m], at least one row each):
+ * the pointers of both sides ([num_segments + 1] each) and, in `report` (four
+ * numbers the caller has set to 0, in device-accessible host memory), what
+ * the reference checks before it searches (torch_cluster/nearest.py:7-91):
+ * [0] / [1] not 0 if ids_x / ids_y decrease somewhere, [2] not 0 if an example
+ * below num_segments has rows on one side only, [3] the largest id + 1.
+ */
+int pca_nearest_segments(const int64_t *ids_x, int64_t n, const int64_t *ids_y,
+                         int64_t m, int64_t num_segments, int64_t *ptr_x,
+                         int64_t *ptr_y, int64_t *report, void *stream);
+
+/*
+ * For fp32 `fps` given sorted example ids ([n]; NULL: one example, then
+ * num_segments is 1): ptr and out_ptr ([num_segments + 1] each) as pca_fps
+ * takes them, ceil(rows * ratio) samples per example in fp32
+ * (csrc/cuda/fps_cuda.cu:68-109), and in `report` (three numbers in
+ * device-accessible host memory, or NULL): [0] the number of samples, [1] the
+ * largest example, [2] the largest id + 1.  ptr_work: [num_segments + 1]
+ * scratch (NULL without ids).
+ */
+int pca_fps_segments(const int64_t *ids, int64_t n, int64_t num_segments,
+                     double ratio, int64_t *ptr, int64_t *ptr_work,
+                     int64_t *out_ptr, int64_t *report, void *stream);
+
+
+/*
  * For a caller that does not know the number of examples (the reference's
  * wrappers read it from the device, torch_cluster/knn.py:62-72: two
  * batch.max() reductions with a host wait each): the next call of the calling

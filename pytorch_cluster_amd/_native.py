@@ -43,6 +43,12 @@ C_ABI = {
                  ctypes.c_size_t, _vp]),
     "pca_segment_pointers": (ctypes.c_int,
                              [_vp, _i64, _vp, _i64, _i64, _vp, _vp, _vp]),
+    "pca_nearest_segments": (ctypes.c_int,
+                             [_vp, _i64, _vp, _i64, _i64, _vp, _vp, _vp,
+                              _vp]),
+    "pca_fps_segments": (ctypes.c_int,
+                         [_vp, _i64, _i64, ctypes.c_double, _vp, _vp, _vp,
+                          _vp, _vp]),
     "pca_knn_fixed_scratch": (ctypes.c_int,
                               [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64,
                                _i64, ctypes.c_int, ctypes.c_int, ctypes.c_int,

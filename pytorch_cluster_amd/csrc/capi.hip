@@ -415,6 +415,61 @@ int pca_segment_pointers(const int64_t *ids_x, int64_t n, const int64_t *ids_y,
       "segment_pointers_kernel");
 }
 
+int pca_nearest_segments(const int64_t *ids_x, int64_t n, const int64_t *ids_y,
+                         int64_t m, int64_t num_segments, int64_t *ptr_x,
+                         int64_t *ptr_y, int64_t *report, void *stream_) {
+  g_last_error[0] = 0;
+  if (n < 1 || m < 1 || n > kMaxRows || m > kMaxRows || num_segments < 1 ||
+      num_segments >= kMaxRows)
+    return fail(PCA_ERR_INVALID_ARGUMENT,
+                "bad sizes n=%lld m=%lld num_segments=%lld", (long long)n,
+                (long long)m, (long long)num_segments);
+  if (ids_x == nullptr || ids_y == nullptr || ptr_x == nullptr ||
+      ptr_y == nullptr || report == nullptr)
+    return fail(PCA_ERR_INVALID_ARGUMENT, "ids, pointers or report is NULL");
+  pca::SegmentSource src;
+  src.ids_x = ids_x;
+  src.ids_y = ids_y;
+  src.n = (int)n;
+  src.m = (int)m;
+  src.ptr_x = ptr_x;
+  src.ptr_y = ptr_y;
+  return check_launch(
+      pca::launch_two_sides(src, (int)num_segments, report,
+                            static_cast<hipStream_t>(stream_)),
+      "two_sides_kernel");
+}
+
+int pca_fps_segments(const int64_t *ids, int64_t n, int64_t num_segments,
+                     double ratio, int64_t *ptr, int64_t *ptr_work,
+                     int64_t *out_ptr, int64_t *report, void *stream_) {
+  g_last_error[0] = 0;
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  if (n < 1 || n > kMaxRows || num_segments < 1 || num_segments >= kMaxRows ||
+      (ids == nullptr && num_segments != 1))
+    return fail(PCA_ERR_INVALID_ARGUMENT, "bad sizes n=%lld num_segments=%lld",
+                (long long)n, (long long)num_segments);
+  if (ptr == nullptr || out_ptr == nullptr ||
+      (ids != nullptr && ptr_work == nullptr))
+    return fail(PCA_ERR_INVALID_ARGUMENT, "pointers are NULL");
+  if (ids != nullptr) {
+    pca::SegmentSource src;
+    src.ids_x = src.ids_y = ids;
+    src.n = src.m = (int)n;
+    src.ptr_x = ptr;
+    src.ptr_y = ptr_work;
+    const int rc = check_launch(
+        pca::launch_segment_pointers(src, (int)num_segments, stream),
+        "segment_pointers_kernel");
+    if (rc != PCA_OK)
+      return rc;
+  }
+  return check_launch(pca::launch_fps_sizes(ids, (int)n, (int)num_segments,
+                                            (float)ratio, ptr, out_ptr, report,
+                                            stream),
+                      "fps_sizes_kernel");
+}
+
 size_t pca_knn_workspace_bytes(int64_t n, int64_t m, int64_t d,
                                int64_t num_segments, int64_t k, int dtype) {
   if (num_segments < 1)

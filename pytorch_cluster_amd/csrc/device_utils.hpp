@@ -433,6 +433,40 @@ __device__ __forceinline__ void pointers_from_ids(const Src &src,
   }
 }
 
+// Number of rows of `ids` (sorted) below a[i], by the whole wave, both searches
+// side by side (the 65-fold narrowing of pointers_from_ids).
+__device__ __forceinline__ void wave_rows_below(const int64_t *__restrict__ ids,
+                                                int count,
+                                                const int64_t (&a)[2],
+                                                int lane, int (&out)[2]) {
+  int lo[2] = {0, 0}, hi[2] = {count, count};
+  while (hi[0] - lo[0] > 64 || hi[1] - lo[1] > 64) {
+    int64_t seen[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int64_t span = (int64_t)hi[i] - lo[i];
+      // (a finished search, span <= 64, probes rows inside its range too)
+      seen[i] = ids[max(lo[i] + (int)(span * (lane + 1) / 65) - 1, 0)];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int64_t span = (int64_t)hi[i] - lo[i];
+      const int below = __builtin_popcountll(__ballot(seen[i] < a[i]));
+      if (span > 64) {
+        const int base = lo[i];
+        lo[i] = below == 0 ? base : base + (int)(span * below / 65);
+        hi[i] = below == 64 ? hi[i]
+                            : base + (int)(span * (below + 1) / 65) - 1;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const bool below = lo[i] + lane < hi[i] && ids[lo[i] + lane] < a[i];
+    out[i] = lo[i] + __builtin_popcountll(__ballot(below));
+  }
+}
+
 } // namespace pca
 
 // experiment switch: -DPCA_NO_SWIZZLE maps workgroup ids to tiles directly

@@ -67,6 +67,16 @@ hipError_t launch_plan(const int64_t *ptr_y, int m, int num_segments,
 hipError_t launch_segment_pointers(const SegmentSource &src, int num_segments,
                                    hipStream_t stream);
 
+// `nearest`: the pointers of both sides and what its checks need (report: four
+// numbers, see two_sides_kernel); at least one row on each side.
+hipError_t launch_two_sides(const SegmentSource &src, int num_segments,
+                            int64_t *report, hipStream_t stream);
+// `fps`: out_ptr from ptr (ids NULL: one example of n rows, ptr written too;
+// num_segments 1) and its sizes (report: three numbers, or NULL).
+hipError_t launch_fps_sizes(const int64_t *ids, int n, int num_segments,
+                            float ratio, int64_t *ptr, int64_t *out_ptr,
+                            int64_t *report, hipStream_t stream);
+
 // Upper bound of work_start[num_segments] that needs no device data.
 inline int plan_upper_bound(int m, int num_segments, int per_item) {
   return m / per_item + num_segments;

@@ -44,6 +44,106 @@ __global__ __launch_bounds__(kBlock) void segment_pointers_kernel(
   pointers_from_ids(src, num_segments, (int)blockIdx.x, (int)gridDim.x);
 }
 
+// What `nearest` needs to know of its example ids before it may answer: the
+// pointers of both sides, whether a vector is not sorted (report[0] for x,
+// [1] for y), whether an example has rows on one side only ([2]), and the
+// number of examples the ids speak of ([3]).  report: four numbers set to 0
+// by the host, in memory it reads.  A wave per example, and all threads look
+// for a decrease; pointers of unsorted ids ascend too (a larger bound never
+// takes a search further to the left).
+__global__ __launch_bounds__(kBlock) void two_sides_kernel(
+    const int64_t *__restrict__ ids_x, int n,
+    const int64_t *__restrict__ ids_y, int m, int num_segments,
+    int64_t *__restrict__ ptr_x, int64_t *__restrict__ ptr_y,
+    int64_t *__restrict__ report) {
+  const int thread = blockIdx.x * kBlock + threadIdx.x;
+  const int threads = gridDim.x * kBlock;
+  const int lane = threadIdx.x & (kWave - 1);
+  if (thread == 0)
+    report[3] = max(max(ids_x[n - 1], ids_y[m - 1]), (int64_t)-1) + 1;
+  for (int b = thread / kWave; b <= num_segments; b += threads / kWave) {
+    const int64_t ends[2] = {(int64_t)b, (int64_t)b + 1};
+    int in_x[2], in_y[2];
+    wave_rows_below(ids_x, n, ends, lane, in_x);
+    wave_rows_below(ids_y, m, ends, lane, in_y);
+    if (lane == 0) {
+      // (searching rows beyond the last example: the last one's, as above)
+      ptr_x[b] = b == num_segments ? n : in_x[0];
+      ptr_y[b] = in_y[0];
+      if (b < num_segments && (in_x[1] > in_x[0]) != (in_y[1] > in_y[0]))
+        report[2] = 1;
+    }
+  }
+  bool falls = false;
+  for (int64_t i = thread; i < n - 1; i += threads)
+    falls = falls || ids_x[i + 1] < ids_x[i];
+  if (falls)
+    report[0] = 1;
+  falls = false;
+  for (int64_t i = thread; i < m - 1; i += threads)
+    falls = falls || ids_y[i + 1] < ids_y[i];
+  if (falls)
+    report[1] = 1;
+}
+
+// The samples of `fps`, ceil(rows * ratio) of every example in fp32 as the
+// host wrapper of the reference forms them (csrc/cuda/fps_cuda.cu:68-109):
+// out_ptr, and in report[0] their number, [1] the largest example, [2] the
+// examples the ids speak of.  One workgroup; ids NULL: one example of n rows,
+// whose pointers are written here too.
+__global__ __launch_bounds__(kPlanThreads) void fps_sizes_kernel(
+    const int64_t *__restrict__ ids, int n, int num_segments, float ratio,
+    int64_t *__restrict__ ptr, int64_t *__restrict__ out_ptr,
+    int64_t *__restrict__ report) {
+  __shared__ int64_t partial[kPlanThreads];
+  __shared__ int longest;
+  const int tid = threadIdx.x;
+  const int per_thread = (num_segments + kPlanThreads - 1) / kPlanThreads;
+  const int b0 = min(tid * per_thread, num_segments);
+  const int b1 = min(b0 + per_thread, num_segments);
+  auto rows_of = [&](int b) -> int64_t {
+    return ids != nullptr ? ptr[b + 1] - ptr[b] : (int64_t)n;
+  };
+  auto samples_of = [&](int64_t rows) {
+    return (int64_t)__builtin_ceilf((float)rows * ratio);
+  };
+  if (tid == 0)
+    longest = 0;
+  int64_t sum = 0;
+  int most = 0;
+  for (int b = b0; b < b1; ++b) {
+    const int64_t rows = rows_of(b);
+    sum += samples_of(rows);
+    most = max(most, (int)rows);
+  }
+  partial[tid] = sum;
+  __syncthreads();
+  atomicMax(&longest, most);
+  for (int off = 1; off < kPlanThreads; off <<= 1) {
+    const int64_t v = tid >= off ? partial[tid - off] : 0;
+    __syncthreads();
+    partial[tid] += v;
+    __syncthreads();
+  }
+  int64_t run = partial[tid] - sum;
+  for (int b = b0; b < b1; ++b) {
+    out_ptr[b] = run;
+    run += samples_of(rows_of(b));
+  }
+  if (tid == kPlanThreads - 1) {
+    out_ptr[num_segments] = partial[tid];
+    if (ids == nullptr) {
+      ptr[0] = 0;
+      ptr[1] = n;
+    }
+    if (report != nullptr) {
+      report[0] = partial[tid];
+      report[1] = longest;
+      report[2] = ids != nullptr ? max(ids[n - 1], (int64_t)-1) + 1 : 1;
+    }
+  }
+}
+
 // ---- compaction -----------------------------------------------------------
 
 constexpr int kCompactQueries = kBlock; // queries per workgroup
@@ -357,6 +457,28 @@ hipError_t launch_segment_pointers(const SegmentSource &src, int num_segments,
   const int blocks = std::min((searches + waves - 1) / waves, 4096);
   hipLaunchKernelGGL(segment_pointers_kernel, dim3(blocks), dim3(kBlock), 0,
                      stream, src, num_segments);
+  return hipGetLastError();
+}
+
+hipError_t launch_two_sides(const SegmentSource &src, int num_segments,
+                            int64_t *report, hipStream_t stream) {
+  // (a wave per example, some rows per thread)
+  const int waves = kBlock / kWave;
+  const int by_rows = (int)std::min<int64_t>(
+      ((int64_t)src.n + src.m) / (kBlock * 4), 2048);
+  const int blocks =
+      std::max(std::min((num_segments + waves) / waves, 4096), by_rows);
+  hipLaunchKernelGGL(two_sides_kernel, dim3(blocks), dim3(kBlock), 0, stream,
+                     src.ids_x, src.n, src.ids_y, src.m, num_segments,
+                     src.ptr_x, src.ptr_y, report);
+  return hipGetLastError();
+}
+
+hipError_t launch_fps_sizes(const int64_t *ids, int n, int num_segments,
+                            float ratio, int64_t *ptr, int64_t *out_ptr,
+                            int64_t *report, hipStream_t stream) {
+  hipLaunchKernelGGL(fps_sizes_kernel, dim3(1), dim3(kPlanThreads), 0, stream,
+                     ids, n, num_segments, ratio, ptr, out_ptr, report);
   return hipGetLastError();
 }
 

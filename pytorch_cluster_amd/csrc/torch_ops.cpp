@@ -22,10 +22,12 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <optional>
 #include <string>
+#include <tuple>
 
 #include "../../include/pca_neighbors.h"
 
@@ -736,6 +738,37 @@ at::Tensor nearest_host(at::Tensor x, at::Tensor y, at::Tensor ptr_x,
   return out;
 }
 
+// The search of `nearest` on checked rows [n, d], n >= 1, whose device is
+// current (px, py NULL: one example).
+void nearest_search(const at::Tensor &x, const at::Tensor &y,
+                    const int64_t *px, const int64_t *py, int64_t segments,
+                    at::Tensor &out, hipStream_t stream) {
+  const int64_t n = x.size(0), m = y.size(0), d = x.size(1);
+  const int dtype = dtype_code(x);
+  TORCH_CHECK(dtype != PCA_BF16,
+              "nearest is not implemented for 'BFloat16'");
+  // (the searched rows, y, are the ones a binned search orders)
+  const bool binned = bins_wanted(m, n, segments, kNearestCost) &&
+                      dtype == PCA_F32 && d <= 3 && m > 0 &&
+                      !being_captured(stream);
+  const size_t ws_bytes =
+      binned ? pca_nearest_binned_workspace_bytes(n, m, d, segments)
+             : pca_nearest_workspace_bytes(n, m, d, segments, dtype);
+  TORCH_CHECK(ws_bytes > 0, "problem size not supported");
+  auto workspace =
+      at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
+  if (binned) {
+    check_status(pca_nearest_binned(
+        x.data_ptr(), y.data_ptr(), px, py, n, m, d, segments,
+        out.data_ptr<int64_t>(), workspace.data_ptr(), ws_bytes, stream));
+    return;
+  }
+  check_status(pca_nearest(x.data_ptr(), m > 0 ? y.data_ptr() : nullptr, px,
+                           py, n, m, d, segments, dtype,
+                           out.data_ptr<int64_t>(), workspace.data_ptr(),
+                           ws_bytes, stream));
+}
+
 at::Tensor nearest(at::Tensor x, at::Tensor y, at::Tensor ptr_x,
                    at::Tensor ptr_y) {
   if (!x.device().is_cuda())
@@ -755,41 +788,118 @@ at::Tensor nearest(at::Tensor x, at::Tensor y, at::Tensor ptr_x,
   PCA_CHECK_INPUT(x.size(0) == 0 || y.size(0) == 0 ||
                   x.size(1) == y.size(1));
   auto out = at::empty({x.size(0)}, ptr_x.options().dtype(at::kLong));
-  const int64_t n = x.size(0), m = y.size(0);
-  if (n == 0)
+  if (x.size(0) == 0)
     return out;
-  const int64_t d = x.size(1);
   at::Tensor px = ptr_x.to(at::kLong).contiguous();
   at::Tensor py = ptr_y.to(at::kLong).contiguous();
-  const int64_t segments = px.numel() - 1;
-  const int dtype = dtype_code(x);
-  TORCH_CHECK(dtype != PCA_BF16,
-              "nearest is not implemented for 'BFloat16'");
-  // (the searched rows, y, are the ones a binned search orders)
-  const bool binned =
-      bins_wanted(m, n, segments, kNearestCost) &&
-      dtype == PCA_F32 && d <= 3 && m > 0 &&
-      !being_captured(
-          c10::hip::getCurrentHIPStream(x.get_device()).stream());
-  const size_t ws_bytes =
-      binned ? pca_nearest_binned_workspace_bytes(n, m, d, segments)
-             : pca_nearest_workspace_bytes(n, m, d, segments, dtype);
-  TORCH_CHECK(ws_bytes > 0, "problem size not supported");
-  auto workspace =
-      at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
-  hipStream_t stream = c10::hip::getCurrentHIPStream(x.get_device()).stream();
-  if (binned) {
-    check_status(pca_nearest_binned(
-        x.data_ptr(), y.data_ptr(), px.data_ptr<int64_t>(),
-        py.data_ptr<int64_t>(), n, m, d, segments, out.data_ptr<int64_t>(),
-        workspace.data_ptr(), ws_bytes, stream));
-    return out;
-  }
-  check_status(pca_nearest(x.data_ptr(), m > 0 ? y.data_ptr() : nullptr,
-                           px.data_ptr<int64_t>(), py.data_ptr<int64_t>(), n,
-                           m, d, segments, dtype, out.data_ptr<int64_t>(),
-                           workspace.data_ptr(), ws_bytes, stream));
+  nearest_search(x, y, px.data_ptr<int64_t>(), py.data_ptr<int64_t>(),
+                 px.numel() - 1, out,
+                 c10::hip::getCurrentHIPStream(x.get_device()).stream());
   return out;
+}
+
+// A mark in a stream the host can wait for while later work goes on.
+struct Mark {
+  hipEvent_t event = nullptr;
+  explicit Mark(hipStream_t stream) {
+    TORCH_CHECK(hipEventCreateWithFlags(&event, hipEventDisableTiming) ==
+                    hipSuccess,
+                "hipEventCreate failed");
+    if (hipEventRecord(event, stream) != hipSuccess) {
+      (void)hipEventDestroy(event);
+      TORCH_CHECK(false, "hipEventRecord failed");
+    }
+  }
+  ~Mark() { (void)hipEventDestroy(event); }
+  Mark(const Mark &) = delete;
+  Mark &operator=(const Mark &) = delete;
+  void wait() const {
+    TORCH_CHECK(hipEventSynchronize(event) == hipSuccess,
+                "hipEventSynchronize failed");
+    g_host_waits += 1;
+  }
+};
+
+// Numbers a kernel leaves for the host, set to 0.
+at::Tensor report_slot(int64_t count) {
+  return at::zeros({count}, at::TensorOptions().dtype(at::kLong).pinned_memory(
+                                true));
+}
+
+// `nearest` given the rows' sorted example ids (both or neither; at least one
+// row on each side): one launch derives the pointers and looks for what the
+// reference's wrapper checks with a dozen torch calls and two host reads
+// (torch_cluster/nearest.py:7-91), the search is queued behind it, and the
+// host waits for the first launch only.  The number of examples as in
+// with_examples.  Returns the rows and what is wrong with the ids: 0 nothing,
+// 1 / 2 batch_x / batch_y is not sorted, 3 an example has rows on one side
+// only.
+std::tuple<at::Tensor, int64_t>
+nearest_batched(at::Tensor x, at::Tensor y, std::optional<at::Tensor> batch_x,
+                std::optional<at::Tensor> batch_y) {
+  PCA_CHECK_GPU(x);
+  PCA_CHECK_GPU(y);
+  PCA_CHECK_INPUT(x.dim() >= 1 && y.dim() >= 1);
+  PCA_CHECK_INPUT(x.scalar_type() == y.scalar_type());
+  PCA_CHECK_INPUT(x.get_device() == y.get_device());
+  PCA_CHECK_INPUT(x.size(0) > 0 && y.size(0) > 0);
+  PCA_CHECK_INPUT(batch_x.has_value() == batch_y.has_value());
+  DeviceScope scope(x.get_device());
+  x = x.view({x.size(0), -1}).contiguous();
+  y = y.view({y.size(0), -1}).contiguous();
+  PCA_CHECK_INPUT(x.size(1) == y.size(1));
+  hipStream_t stream = c10::hip::getCurrentHIPStream(x.get_device()).stream();
+  // (with example ids the host reads from the device; without it could be
+  // captured, but so far `nearest` could not: the operator that takes
+  // pointers can)
+  TORCH_CHECK(!being_captured(stream),
+              "nearest cannot be captured into a graph (the operator that "
+              "takes pointers can)");
+  const int64_t n = x.size(0), m = y.size(0);
+  auto long_opts = x.options().dtype(at::kLong);
+  auto out = at::empty({n}, long_opts);
+  if (!batch_x.has_value()) {
+    nearest_search(x, y, nullptr, nullptr, 1, out, stream);
+    return {out, 0};
+  }
+  PCA_CHECK_GPU(batch_x.value());
+  PCA_CHECK_GPU(batch_y.value());
+  PCA_CHECK_INPUT(batch_x->dim() == 1 && batch_x->numel() == n);
+  PCA_CHECK_INPUT(batch_y->dim() == 1 && batch_y->numel() == m);
+  at::Tensor ids_x = batch_x->to(at::kLong).contiguous();
+  at::Tensor ids_y = batch_y->to(at::kLong).contiguous();
+  int64_t guess = g_examples_hint.load();
+  if (guess < 1) {
+    guess = std::max<int64_t>(std::max(ids_x[-1].item<int64_t>(),
+                                       ids_y[-1].item<int64_t>()) +
+                                  1,
+                              1);
+    g_host_waits += 1;
+  }
+  for (;;) {
+    auto slot = report_slot(4);
+    const int64_t *report = slot.data_ptr<int64_t>();
+    auto both = at::empty({2, guess + 1}, long_opts);
+    int64_t *px = both.data_ptr<int64_t>();
+    int64_t *py = px + (guess + 1);
+    SlotGuard guard(stream);
+    check_status(pca_nearest_segments(
+        ids_x.data_ptr<int64_t>(), n, ids_y.data_ptr<int64_t>(), m, guess, px,
+        py, slot.data_ptr<int64_t>(), stream));
+    const Mark mark(stream);
+    nearest_search(x, y, px, py, guess, out, stream);
+    mark.wait();
+    guard.armed = false;
+    const int64_t met = report[3];
+    g_examples_hint.store(std::max<int64_t>(met, 1));
+    const int64_t wrong = report[0] != 0   ? 1
+                          : report[1] != 0 ? 2
+                          : report[2] != 0 || met < 1 ? 3
+                                                      : 0;
+    if (wrong == 1 || wrong == 2 || met <= guess)
+      return {out, wrong};
+    guess = met;
+  }
 }
 
 // csrc/fps.cpp:22-36 -> fps_cuda (csrc/cuda/fps_cuda.cu:68-109): samples per
@@ -890,6 +1000,92 @@ at::Tensor fps(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
   return out;
 }
 
+// `fps` of fp32 rows given the sorted example ids (or none: one example) and
+// the ratio as a number: pointers, sizes and the largest example from two
+// launches and one host read (none for one example) instead of a dozen torch
+// calls with two.  Same numbers: ceil(rows * ratio) in fp32.  The number of
+// examples as in with_examples (batch_size < 1: not known).
+at::Tensor fps_batched(at::Tensor src, std::optional<at::Tensor> batch,
+                       int64_t batch_size, double ratio, bool random_start) {
+  PCA_CHECK_GPU(src);
+  PCA_CHECK_INPUT(src.dim() >= 1 && src.numel() > 0);
+  PCA_CHECK_INPUT(src.scalar_type() == at::kFloat);
+  DeviceScope scope(src.get_device());
+  src = src.view({src.size(0), -1}).contiguous();
+  const int64_t n = src.size(0), d = src.size(1);
+  hipStream_t stream =
+      c10::hip::getCurrentHIPStream(src.get_device()).stream();
+  refuse_capture(stream, "fps");
+  auto long_opts = src.options().dtype(at::kLong);
+  at::Tensor ptrs;
+  int64_t examples = 1, samples = 0, longest = n;
+  if (batch.has_value()) {
+    PCA_CHECK_GPU(batch.value());
+    PCA_CHECK_INPUT(batch->dim() == 1 && batch->numel() == n);
+    at::Tensor ids = batch->to(at::kLong).contiguous();
+    int64_t guess = batch_size >= 1 ? batch_size : g_examples_hint.load();
+    if (guess < 1) {
+      guess = std::max<int64_t>(ids[-1].item<int64_t>() + 1, 1);
+      g_host_waits += 1;
+    }
+    for (;;) {
+      auto slot = report_slot(3);
+      const int64_t *report = slot.data_ptr<int64_t>();
+      ptrs = at::empty({3, guess + 1}, long_opts);
+      int64_t *ptr = ptrs.data_ptr<int64_t>();
+      SlotGuard guard(stream);
+      check_status(pca_fps_segments(ids.data_ptr<int64_t>(), n, guess, ratio,
+                                    ptr, ptr + 2 * (guess + 1),
+                                    ptr + (guess + 1),
+                                    slot.data_ptr<int64_t>(), stream));
+      TORCH_CHECK(hipStreamSynchronize(stream) == hipSuccess,
+                  "hipStreamSynchronize failed");
+      g_host_waits += 1;
+      guard.armed = false;
+      samples = report[0];
+      longest = report[1];
+      examples = guess;
+      if (batch_size >= 1)
+        break;
+      const int64_t met = report[2];
+      PCA_CHECK_INPUT(met >= 1);
+      g_examples_hint.store(met);
+      examples = met; // (examples beyond it have no rows and no samples)
+      if (met <= guess)
+        break;
+      guess = met;
+    }
+  } else {
+    samples = (int64_t)std::ceil((float)n * (float)ratio);
+    ptrs = at::empty({3, 2}, long_opts);
+    int64_t *ptr = ptrs.data_ptr<int64_t>();
+    check_status(pca_fps_segments(nullptr, n, 1, ratio, ptr, nullptr, ptr + 2,
+                                  nullptr, stream));
+  }
+  const at::Tensor ptr = ptrs.select(0, 0), out_ptr = ptrs.select(0, 1);
+  at::Tensor start;
+  if (random_start) {
+    const auto deg =
+        ptr.narrow(0, 1, examples) - ptr.narrow(0, 0, examples);
+    start = at::rand({examples}, src.options());
+    start = (start * deg.toType(at::kFloat)).toType(at::kLong).contiguous();
+  }
+  auto out = at::empty({samples}, long_opts);
+  if (samples == 0)
+    return out;
+  const size_t ws_bytes =
+      pca_fps_workspace_bytes(n, d, examples, longest, PCA_F32);
+  TORCH_CHECK(ws_bytes > 0, "problem size not supported");
+  auto workspace =
+      at::empty({(int64_t)ws_bytes}, src.options().dtype(at::kByte));
+  check_status(pca_fps(src.data_ptr(), ptr.data_ptr<int64_t>(),
+                       out_ptr.data_ptr<int64_t>(),
+                       random_start ? start.data_ptr<int64_t>() : nullptr, n,
+                       d, examples, longest, PCA_F32, out.data_ptr<int64_t>(),
+                       workspace.data_ptr(), ws_bytes, stream));
+  return out;
+}
+
 // The stock loader of the reference package calls this
 // (torch_cluster/__init__.py:23, csrc/version.cpp:26-41).
 int64_t cuda_version() { return HIP_VERSION; }
@@ -930,6 +1126,12 @@ TORCH_LIBRARY(pytorch_cluster_amd, m) {
         "int batch_size, float r, int max_num_neighbors, "
         "bool ignore_same_index, bool x_first) -> Tensor",
         &radius_batched);
+  m.def("nearest_batched(Tensor x, Tensor y, Tensor? batch_x, "
+        "Tensor? batch_y) -> (Tensor, int)",
+        &nearest_batched);
+  m.def("fps_batched(Tensor src, Tensor? batch, int batch_size, float ratio, "
+        "bool random_start) -> Tensor",
+        &fps_batched);
   m.def("host_waits() -> int", &host_waits);
   m.def("set_search_strategy(str name) -> ()", &set_search_strategy);
   m.def("get_search_strategy() -> str", &get_search_strategy);

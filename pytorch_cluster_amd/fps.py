@@ -10,7 +10,7 @@ from typing import List, Optional, Union
 import torch
 from torch import Tensor
 
-from ._segments import batch_pointers
+from ._segments import batch_pointers, examples_or_unknown
 
 
 @torch.jit._overload  # noqa
@@ -63,6 +63,23 @@ def fps(  # noqa
     Returns the int64 row numbers of the samples, example after example, in
     sampling order.
     """
+    # fp32 rows with a plain ratio: pointers and numbers of samples on the
+    # device, without torch calls
+    if (ptr is None and src.is_cuda and src.dtype == torch.float32
+            and src.numel() > 0
+            and (batch_size is None or batch_size > 0)):
+        share_of: float = -1.0
+        if ratio is None:
+            share_of = 0.5
+        elif isinstance(ratio, float):
+            share_of = ratio
+        if share_of > 0.0 and share_of <= 1.0:
+            if batch is not None:
+                assert src.size(0) == batch.numel()
+            return torch.ops.pytorch_cluster_amd.fps_batched(
+                src, batch, examples_or_unknown(batch_size), share_of,
+                random_start)
+
     # the share of every example that is sampled, as the operator takes it: a
     # tensor (TorchScript resolves the three cases per overload, in this
     # order)

@@ -38,6 +38,16 @@ def _pointers(batch: Optional[torch.Tensor], rows: torch.Tensor,
     return torch.bucketize(ids, batch)
 
 
+def _refuse(unsorted_x: bool, unsorted_y: bool, mismatch: bool) -> None:
+    if unsorted_x:
+        raise ValueError("'batch_x' is not sorted")
+    if unsorted_y:
+        raise ValueError("'batch_y' is not sorted")
+    if mismatch:
+        raise ValueError("Some batch indices occur in 'batch_x' "
+                         "that do not occur in 'batch_y'")
+
+
 def nearest(
     x: torch.Tensor,
     y: torch.Tensor,
@@ -64,6 +74,14 @@ def nearest(
         assert x.size(0) == batch_x.numel()
     if batch_y is not None:
         assert y.size(0) == batch_y.numel()
+
+    if (x.is_cuda and x.numel() > 0 and y.numel() > 0
+            and (batch_x is None) == (batch_y is None)):
+        # ids and checks in one launch, in front of the search
+        rows, wrong = torch.ops.pytorch_cluster_amd.nearest_batched(
+            x, y, batch_x, batch_y)
+        _refuse(wrong == 1, wrong == 2, wrong == 3)
+        return rows
 
     # first read: the number of examples on each side (the last entry of a
     # sorted vector is its maximum; if it is not sorted the check below fails
@@ -93,12 +111,6 @@ def nearest(
         mismatch = torch.ones((), dtype=torch.bool, device=x.device)
     flags = torch.stack([_unsorted(batch_x, x), _unsorted(batch_y, y),
                          mismatch]).tolist()
-    if flags[0]:
-        raise ValueError("'batch_x' is not sorted")
-    if flags[1]:
-        raise ValueError("'batch_y' is not sorted")
-    if flags[2] or bad_sizes:
-        raise ValueError("Some batch indices occur in 'batch_x' "
-                         "that do not occur in 'batch_y'")
+    _refuse(flags[0], flags[1], flags[2] or bad_sizes)
 
     return torch.ops.torch_cluster.nearest(x, y, ptr_x, ptr_y)
