@@ -241,9 +241,9 @@ int pca_knn_fixed_scratch(const void *x, const void *y, const int64_t *ptr_x,
 /*
  * pca_knn for fp32 points of up to 3 dimensions, Euclidean distance and
  * k <= 64 (PCA_ERR_UNSUPPORTED otherwise) over spatially binned rows: the x
- * rows of every segment are ordered along a space-filling curve (the voxel
- * numbers of the reference's grid clustering, csrc/cuda/grid_cuda.cu:10-25,
- * bit-interleaved), cut into tiles with bounding boxes, and a query scans only
+ * rows of every segment are ordered along a space-filling curve through the
+ * voxels of the reference's grid clustering (csrc/cuda/grid_cuda.cu:10-25),
+ * cut into tiles with bounding boxes, and a query scans only
  * the tiles whose box is within its current k-th distance.  Stands under the
  * same operator as pca_knn (csrc/knn.cpp:22-40 -> csrc/cuda/knn_cuda.cu:86-135)
  * and returns the same edges, bit for bit, in the same order; only the work

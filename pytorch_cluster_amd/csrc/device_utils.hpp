@@ -467,6 +467,84 @@ __device__ __forceinline__ void wave_rows_below(const int64_t *__restrict__ ids,
   }
 }
 
+// 10 bits spread to every third position.
+__device__ __forceinline__ uint32_t spread3(uint32_t v) {
+  v &= 0x3ffu;
+  v = (v | (v << 16)) & 0x030000ffu;
+  v = (v | (v << 8)) & 0x0300f00fu;
+  v = (v | (v << 4)) & 0x030c30c3u;
+  v = (v | (v << 2)) & 0x09249249u;
+  return v;
+}
+
+// Place of a cell along a Hilbert curve through 2^bits cells per axis (up to
+// 10), D = 2 or 3 axes, by the exchanges and inversions of J. Skilling,
+// "Programming the Hilbert curve" (2004).  Consecutive cells are neighbours
+// everywhere on this curve; along the interleaved bits of the cells (Morton
+// order) runs jump, and the boxes of 32 or 64 consecutive rows are long: 18
+// of the boxes of 32 rows come nearer to a query of a LiDAR-like scan than its
+// 16th neighbour, on this curve 12 (one nearest row among 16,000: 9 and 5).
+template <int D>
+__device__ __forceinline__ uint32_t hilbert_place(uint32_t (&x)[3], int bits) {
+  static_assert(D == 2 || D == 3, "two or three axes");
+  for (uint32_t bit = (1u << bits) >> 1; bit > 1; bit >>= 1) {
+    const uint32_t low = bit - 1;
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      // invert the low bits of axis 0, or exchange them with axis i's
+      const bool set = (x[i] & bit) != 0;
+      const uint32_t differ = set ? 0u : (x[0] ^ x[i]) & low;
+      x[0] ^= set ? low : differ;
+      if (i > 0)
+        x[i] ^= differ;
+    }
+  }
+#pragma unroll
+  for (int i = 1; i < D; ++i)
+    x[i] ^= x[i - 1];
+  uint32_t flip = 0;
+  for (uint32_t bit = (1u << bits) >> 1; bit > 1; bit >>= 1)
+    flip ^= (x[D - 1] & bit) != 0 ? bit - 1 : 0u;
+  uint32_t place = 0;
+#pragma unroll
+  for (int i = 0; i < D; ++i)
+    place |= spread3(x[i] ^ flip) << (D - 1 - i);
+  return place;
+}
+
+// The curve's place of a point in the box lo .. hi of its example (d of its
+// axes, at most the first three; what lies outside the box, or is no number,
+// goes to its border).  An axis is cut into cells no narrower than a quarter
+// of the longest axis' cells: boxes of flat clouds would be needles otherwise
+// (1 x 1 x 0.05: 14 boxes nearer than the 16th neighbour, so 8; cells of equal
+// width 7, but 16 instead of 12 for the LiDAR-like scans, whose points crowd
+// in the middle of a flat box).
+__device__ __forceinline__ uint32_t curve_place(const float (&v)[3],
+                                                const float (&lo)[3],
+                                                const float (&hi)[3], int d,
+                                                int bits) {
+  float longest = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    if (c < d)
+      longest = __builtin_fmaxf(longest, hi[c] - lo[c]);
+  const float cells = (float)(1 << bits);
+  uint32_t cell[3] = {0u, 0u, 0u};
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    if (c < d) {
+      const float width = __builtin_fmaxf(hi[c] - lo[c], 0.25f * longest);
+      const float t = (v[c] - lo[c]) / width * cells;
+      // (NaN, also from an empty or flat box, fails the comparison)
+      cell[c] = t >= 0.0f ? (uint32_t)__builtin_fminf(t, cells - 1.0f) : 0u;
+    }
+  if (d >= 3)
+    return hilbert_place<3>(cell, bits);
+  if (d == 2)
+    return hilbert_place<2>(cell, bits);
+  return cell[0];
+}
+
 } // namespace pca
 
 // experiment switch: -DPCA_NO_SWIZZLE maps workgroup ids to tiles directly

@@ -537,16 +537,6 @@ __device__ __forceinline__ float fps_lower(const float (&q)[DIM],
   return dd;
 }
 
-// 10 bits spread to every third position
-__device__ __forceinline__ uint32_t fps_spread3(uint32_t v) {
-  v &= 0x3ffu;
-  v = (v | (v << 16)) & 0x030000ffu;
-  v = (v | (v << 8)) & 0x0300f00fu;
-  v = (v | (v << 4)) & 0x030c30c3u;
-  v = (v | (v << 2)) & 0x09249249u;
-  return v;
-}
-
 // Waits for this workgroup's LDS traffic and meets its other waves (global
 // stores stay in flight: what a wave stores only it reads again).
 __device__ __forceinline__ void fps_meet() {
@@ -610,19 +600,13 @@ fps_curve_order(const float *__restrict__ rows, int count, int d,
   for (int i = tid; i < n2; i += T) {
     uint32_t key = 0xffffffffu;
     if (i < count) {
-      uint32_t code = 0;
+      float v[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int c = 0; c < (DIM < 3 ? DIM : 3); ++c) {
-        uint32_t cell = 0;
-        if (c < d) {
-          const float cells = (float)(1 << AXIS_BITS);
-          const float t =
-              (rows[(size_t)i * d + c] - lo[c]) / (hi[c] - lo[c]) * cells;
-          // (NaN, also from a flat box, fails the comparison)
-          cell = t >= 0.0f ? (uint32_t)__builtin_fminf(t, cells - 1.0f) : 0u;
-        }
-        code |= fps_spread3(cell) << c;
-      }
+      for (int c = 0; c < (DIM < 3 ? DIM : 3); ++c)
+        if (c < d)
+          v[c] = rows[(size_t)i * d + c];
+      const uint32_t code =
+          curve_place(v, lo, hi, d < DIM ? d : DIM, AXIS_BITS);
       key = (code << REL_BITS) | (uint32_t)i;
     }
     keys[i] = key;
@@ -1119,8 +1103,10 @@ __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
 // several pieces to a bucket.
 //
 // Eight ragged LiDAR-like scans of 60,000 - 200,000 rows, 2 % sampled: 419.6 ->
-// 6.9 ms per call, 1.7 instead of 157 us per step of the longest scan (before:
-// fps_any_kernel, the whole scan through one compute unit in every step).
+// 5.7 ms per call, 1.4 instead of 157 us per step of the longest scan (before:
+// fps_any_kernel, the whole scan through one compute unit in every step; rows
+// in Morton instead of Hilbert order, 14 instead of 12 buckets per sample:
+// 6.8 ms).
 // Bound by the chain of a step: the trip to the L2 is a third of it.
 template <int W, int S, bool MANY>
 __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(

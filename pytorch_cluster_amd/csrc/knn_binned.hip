@@ -9,9 +9,9 @@
 // at rows near it.
 //
 // Per call: every segment's x rows are ordered along a space-filling curve
-// (30-bit Morton codes inside the segment's bounding box - the voxel number of
-// the reference's grid clustering, csrc/cuda/grid_cuda.cu:10-25, with its bits
-// interleaved - sorted by rocPRIM's radix sort), copied in that order together
+// (30-bit places on a Hilbert curve through the segment's bounding box, its
+// cells the voxels of the reference's grid clustering,
+// csrc/cuda/grid_cuda.cu:10-25, sorted by rocPRIM's radix sort), copied in that order together
 // with their row numbers, and cut into tiles of 32 rows with a bounding box
 // each.  The queries are ordered the same way, so the 64 queries of a wave
 // (one per lane) are neighbours in space and share one bounding box.
@@ -39,6 +39,10 @@
 // a row of EQUAL distance may still displace a neighbour with a larger row
 // number: a full list admits d <= its k-th distance and the 64-bit
 // (distance, row) keys decide.
+//
+// The curve decides how many boxes a query meets (hilbert_place).  Calls, us,
+// Morton / Hilbert order: kNN of 238,000 queries among 952,000 LiDAR-like rows,
+// k = 16, 713 / 649; nearest of 952,000 rows among 119,000 375 / 334.
 #include "device_utils.hpp"
 #include "knn_binned_mc_impl.hpp"
 #include "knn_lowd_impl.hpp"
@@ -169,20 +173,9 @@ __global__ __launch_bounds__(kBlock) void seg_box_kernel(
   }
 }
 
-// 10 bits spread to every third position
-__device__ __forceinline__ uint32_t spread3(uint32_t v) {
-  v &= 0x3ffu;
-  v = (v | (v << 16)) & 0x030000ffu;
-  v = (v | (v << 8)) & 0x0300f00fu;
-  v = (v | (v << 4)) & 0x030c30c3u;
-  v = (v | (v << 2)) & 0x09249249u;
-  return v;
-}
-
-// keys[i] = (segment << 3 axis_bits) | Morton code of row i inside its
-// segment's box of x rows, axis_bits bits per axis (coordinates outside the
-// box, NaN and missing axes go to its border); vals[i] = i.
-__global__ __launch_bounds__(kBlock) void morton_keys_kernel(
+// keys[i] = (segment << 3 axis_bits) | place of row i along the curve through
+// its segment's box of x rows, axis_bits bits per axis; vals[i] = i.
+__global__ __launch_bounds__(kBlock) void curve_keys_kernel(
     const float *__restrict__ pts, const int64_t *__restrict__ ptr, int count,
     int d, int num_segments, const int *__restrict__ seg_box,
     int axis_bits, uint32_t *__restrict__ keys,
@@ -206,21 +199,14 @@ __global__ __launch_bounds__(kBlock) void morton_keys_kernel(
     return;
   }
   const int seg = find_segment64(ptr, num_segments, i);
-  uint32_t code = 0;
+  float v[3], lo[3], hi[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    uint32_t cell = 0;
-    if (c < d) {
-      const float lo = from_ordered_int(seg_box[seg * 6 + c]);
-      const float hi = from_ordered_int(seg_box[seg * 6 + 3 + c]);
-      const float v = pts[(size_t)i * d + c];
-      const float cells = (float)(1 << axis_bits);
-      const float t = (v - lo) / (hi - lo) * cells;
-      // (NaN, also from an empty or flat box, fails the first comparison)
-      cell = t >= 0.0f ? (uint32_t)__builtin_fminf(t, cells - 1.0f) : 0u;
-    }
-    code |= spread3(cell) << c;
+    v[c] = c < d ? pts[(size_t)i * d + c] : 0.0f;
+    lo[c] = from_ordered_int(seg_box[seg * 6 + c]);
+    hi[c] = from_ordered_int(seg_box[seg * 6 + 3 + c]);
   }
+  const uint32_t code = curve_place(v, lo, hi, d, axis_bits);
   keys[i] = ((uint32_t)seg << (3 * axis_bits)) | code;
   vals[i] = (uint32_t)i;
 }
@@ -751,7 +737,7 @@ struct BinnedLayout {
   }
 };
 
-// Keys are 32 bits: the segment above the Morton code, whose bits per axis
+// Keys are 32 bits: the segment above the place on the curve, whose bits per axis
 // (at most 10) shrink as the segments get more (and with that smaller).
 int segment_bits(int num_segments) {
   int bits = 0;
@@ -1163,7 +1149,7 @@ hipError_t prepare_bins(const SearchInput &in, void *scratch, bool with_tasks,
   auto queries_chain = [&]() -> hipError_t {
     hipError_t e = hipSuccess;
     if (!self_search) {
-      hipLaunchKernelGGL(morton_keys_kernel,
+      hipLaunchKernelGGL(curve_keys_kernel,
                          dim3((in.m + kBlock - 1) / kBlock), dim3(kBlock), 0,
                          side, y, in.ptr_y, in.m, in.d, nseg, seg_box,
                          axis_bits(nseg), keys_b, vals_b, false);
@@ -1185,7 +1171,7 @@ hipError_t prepare_bins(const SearchInput &in, void *scratch, bool with_tasks,
   const bool queries_first = beside && in.m > in.n;
   if (queries_first && (err = queries_chain()) != hipSuccess)
     return err;
-  hipLaunchKernelGGL(morton_keys_kernel, dim3((in.n + kBlock - 1) / kBlock),
+  hipLaunchKernelGGL(curve_keys_kernel, dim3((in.n + kBlock - 1) / kBlock),
                      dim3(kBlock), 0, stream, x, in.ptr_x, in.n, in.d, nseg,
                      seg_box, axis_bits(nseg), keys_a, vals_a, true);
   if ((err = hipGetLastError()) != hipSuccess)
@@ -1305,7 +1291,7 @@ hipError_t launch_curve_order(const float *x, const int64_t *ptr, int n, int d,
                           std::min(num_segments, 65535)),
                      dim3(kBlock), 0, stream, x, ptr, n, d, num_segments,
                      seg_box);
-  hipLaunchKernelGGL(morton_keys_kernel, dim3((n + kBlock - 1) / kBlock),
+  hipLaunchKernelGGL(curve_keys_kernel, dim3((n + kBlock - 1) / kBlock),
                      dim3(kBlock), 0, stream, x, ptr, n, d, num_segments,
                      seg_box, axis_bits(num_segments), keys, vals, true);
   hipError_t err = hipGetLastError();
