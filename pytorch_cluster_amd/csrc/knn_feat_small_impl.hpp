@@ -71,9 +71,12 @@
 
 namespace pca {
 
-constexpr int kSmallStep = 32;        // rows per step and LDS tile
+constexpr int kSmallStep = 32;        // rows per step
 constexpr int kSmallSampleSteps = 64; // steps of an example the bound samples
 constexpr int kSmallQueue = 16;       // parked steps per lane
+// Values of rows that take part in the filter are below 3 x 128 x 2^22; those
+// of padding are 65504 x 2^15.
+constexpr float kSmallSampleLimit = 1.7e9f;
 // (a compiler vector: arrays of these are kept in registers where arrays of
 // float4, a class, end up in scratch memory)
 typedef float small_v4f __attribute__((ext_vector_type(4)));
@@ -190,7 +193,12 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
   typedef SmallChain<R16> Chain;
   typedef FeatShape<NB> S;
   constexpr int RSU = S::RSU;
-  constexpr int TILE = kSmallStep;
+  // fp32 rows: the filter's own upper bounds make the bound (see below), no
+  // rows are staged beside the packed ones, and a tile is two steps whose
+  // chains run side by side (half the barriers)
+  constexpr bool EXACT_SAMPLES = R16 == 1 || R16 == 2;
+  constexpr int SUBS = EXACT_SAMPLES ? 1 : 2; // steps per tile
+  constexpr int TILE = SUBS * kSmallStep;
   constexpr int TILE_UNITS = TILE * RSU;
   constexpr int PU = (TILE_UNITS + kBlock - 1) / kBlock; // packed units/thread
   constexpr int MAX_D = S::MAX_D;
@@ -199,14 +207,16 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
   constexpr int XS = (TILE * MAX_D + kBlock - 1) / kBlock;     // floats/thread
   constexpr int TQ = kFeatQueries;
   constexpr int SEEDS = K / 2;
-  constexpr int DEPTH = 4; // tiles in flight
-  static_assert(kSmallQueue % DEPTH == 0 && kSmallQueue >= 3 * DEPTH,
+  constexpr int DEPTH = 4 / SUBS; // tiles in flight
+  constexpr int LOOK = DEPTH * SUBS; // steps between looks at the queues
+  static_assert(kSmallQueue % LOOK == 0 && kSmallQueue >= 3 * LOOK,
                 "a queue outlasts two looks");
   static_assert(K % 8 == 0 && K <= 48, "list widths in steps of 8, up to 48");
   static_assert(kBlock == 256 && TQ == 128, "four waves of 32 queries");
 
   __shared__ __attribute__((aligned(16))) uint4 xs[2][TILE_UNITS];
-  __shared__ __attribute__((aligned(16))) float x32[2][TILE * ROW_F];
+  __shared__ __attribute__((aligned(16))) float
+      x32[EXACT_SAMPLES ? 2 : 1][EXACT_SAMPLES ? TILE * ROW_F : 4];
   __shared__ __attribute__((aligned(16))) float ys[TQ * ROW_F];
   // parked steps of the search: (step << 16) | mask of the lane's 16 rows
   __shared__ uint32_t queue[kSmallQueue][kBlock];
@@ -395,8 +405,8 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
 
   // the step's 32 x 32 values: s of row 8 (v / 4) + 4 half + v % 4 and the
   // lane's query in accumulator v
-  auto products = [&](int buf) {
-    const uint4 *arow = &xs[buf][col * RSU + half];
+  auto products = [&](int buf, int sub) {
+    const uint4 *arow = &xs[buf][(sub * kSmallStep + col) * RSU + half];
     feat_acc_t acc = {0};
 #pragma unroll
     for (int o = 0; o < NB; ++o)
@@ -425,7 +435,18 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
     }
     return acc;
   };
-  // row of the tile that accumulator v of this lane stands for
+  // smallest of a lane's 16 values
+  auto min16 = [](const feat_acc_t &a) {
+    float m0 = min3f(a[0], a[1], a[2]);
+    const float m1 = min3f(a[3], a[4], a[5]);
+    const float m2 = min3f(a[6], a[7], a[8]);
+    float m3 = min3f(a[9], a[10], a[11]);
+    const float m4 = min3f(a[12], a[13], a[14]);
+    m0 = min3f(m0, m1, m2);
+    m3 = min3f(m3, m4, a[15]);
+    return __builtin_fminf(m0, m3);
+  };
+  // row of the step that accumulator v of this lane stands for
   auto row_of = [&](int v) { return 8 * (v >> 2) + 4 * half + (v & 3); };
 
   // One pass over the example's tiles; body(t, buf, rows) with the tile in
@@ -482,43 +503,70 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
 #pragma unroll
     for (int j = 0; j < SEEDS; ++j)
       seed[j] = __builtin_inff();
-    auto sample_step = [&](int t, int buf, int rows) {
-      const feat_acc_t acc = products(buf);
-      // the smallest of the lane's 16 values, its accumulator number in the
-      // four lowest bits (which of two nearly equal rows is taken does not
-      // matter); rows behind the example's end do not count
-      float tagged[16];
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        tagged[v] = __uint_as_float((__float_as_uint(acc[v]) & ~15u) |
-                                    (uint32_t)v);
-        if (rows < TILE && row_of(v) >= rows)
-          tagged[v] = __builtin_inff();
-      }
-      float m0 = min3f(tagged[0], tagged[1], tagged[2]);
-      float m1 = min3f(tagged[3], tagged[4], tagged[5]);
-      float m2 = min3f(tagged[6], tagged[7], tagged[8]);
-      float m3 = min3f(tagged[9], tagged[10], tagged[11]);
-      float m4 = min3f(tagged[12], tagged[13], tagged[14]);
-      m0 = min3f(m0, m1, m2);
-      m3 = min3f(m3, m4, tagged[15]);
-      const float least = __builtin_fminf(m0, m3);
-      const int v = (int)(__float_as_uint(least) & 15u);
-      const int j = row_of(v);
-      const float e =
-          finish(exact(buf, j), min(x_begin + t * TILE + j, p.n - 1));
-      // (a padding row, a NaN or a distance beyond the limit is no sample)
-      const float sample =
-          (active && j < rows && least < __builtin_inff() && e < sentinel)
-              ? e
-              : __builtin_inff();
+    auto keep_sample = [&](float sample) {
 #pragma unroll
       for (int i = SEEDS - 1; i >= 1; --i)
         seed[i] = __builtin_amdgcn_fmed3f(seed[i - 1], seed[i], sample);
       seed[0] = __builtin_fminf(seed[0], sample);
     };
-    const int sampled = min(num_tiles, kSmallSampleSteps);
-    if (vec4)
+    auto sample_step = [&](int t, int buf, int rows) {
+      if constexpr (!EXACT_SAMPLES) {
+        // the smallest of the lane's 16 values is the sample; rows behind the
+        // example's end do not count, nor does padding
+        feat_acc_t acc[SUBS];
+#pragma unroll
+        for (int sub = 0; sub < SUBS; ++sub)
+          acc[sub] = products(buf, sub);
+#pragma unroll
+        for (int sub = 0; sub < SUBS; ++sub) {
+          feat_acc_t &a = acc[sub];
+          if (rows < TILE) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+              if (sub * kSmallStep + row_of(v) >= rows)
+                a[v] = __builtin_inff();
+          }
+          const float least = min16(a);
+          keep_sample(least < kSmallSampleLimit ? least : __builtin_inff());
+        }
+      } else {
+        const feat_acc_t acc = products(buf, 0);
+        // the smallest of the lane's 16 values, its accumulator number in the
+        // four lowest bits (which of two nearly equal rows is taken does not
+        // matter); rows behind the example's end do not count
+        float tagged[16];
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          tagged[v] = __uint_as_float((__float_as_uint(acc[v]) & ~15u) |
+                                      (uint32_t)v);
+          if (rows < TILE && row_of(v) >= rows)
+            tagged[v] = __builtin_inff();
+        }
+        float m0 = min3f(tagged[0], tagged[1], tagged[2]);
+        float m1 = min3f(tagged[3], tagged[4], tagged[5]);
+        float m2 = min3f(tagged[6], tagged[7], tagged[8]);
+        float m3 = min3f(tagged[9], tagged[10], tagged[11]);
+        float m4 = min3f(tagged[12], tagged[13], tagged[14]);
+        m0 = min3f(m0, m1, m2);
+        m3 = min3f(m3, m4, tagged[15]);
+        const float least = __builtin_fminf(m0, m3);
+        const int v = (int)(__float_as_uint(least) & 15u);
+        const int j = row_of(v);
+        const float e =
+            finish(exact(buf, j), min(x_begin + t * TILE + j, p.n - 1));
+        // (a padding row, a NaN or a distance beyond the limit is no sample)
+        const float sample =
+            (active && j < rows && least < __builtin_inff() && e < sentinel)
+                ? e
+                : __builtin_inff();
+        keep_sample(sample);
+      }
+    };
+    const int sampled = min(num_tiles, kSmallSampleSteps / SUBS);
+    if constexpr (!EXACT_SAMPLES)
+      for_tiles(sampled, std::false_type(), std::false_type(), sample_step,
+                [](int, bool) { return false; });
+    else if (vec4)
       for_tiles(sampled, std::true_type(), std::true_type(), sample_step,
                 [](int, bool) { return false; });
     else
@@ -536,7 +584,15 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
     const auto both = __builtin_amdgcn_permlane32_swap(
         __float_as_uint(own), __float_as_uint(own), false, false);
     const float partner = __uint_as_float(half ? both[0] : both[1]);
-    const float bound = __builtin_fmaxf(own, partner);
+    float bound = __builtin_fmaxf(own, partner);
+    if constexpr (!EXACT_SAMPLES) {
+      // F (knn_feat_impl.hpp): no row with this value or a smaller one is
+      // farther away
+      const double upper =
+          ((double)bound + fq.shift + fq.widen) * fq.grow / scale2;
+      bound = filtered && bound < kSmallSampleLimit ? feat_float_above(upper)
+                                                    : __builtin_inff();
+    }
     if (active && bound < sentinel) {
       shared = small_next_up(bound);
       thresh = __builtin_fminf(thresh, shared);
@@ -660,7 +716,7 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
         const uint32_t word = queue[taken][tid];
         ++taken;
         pending = word & 0xffffu;
-        step_row = (int)(word >> 16) * TILE;
+        step_row = (int)(word >> 16) * kSmallStep;
       }
       // (radius search: a lane that holds its k hits looks no further)
       on = pending != 0 && !(RADIUS && full);
@@ -751,27 +807,31 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
   };
   for_tiles(num_tiles, std::false_type(), std::false_type(),
             [&](int t, int buf, int rows) {
-    const feat_acc_t a = products(buf);
-    float m0 = min3f(a[0], a[1], a[2]);
-    float m1 = min3f(a[3], a[4], a[5]);
-    float m2 = min3f(a[6], a[7], a[8]);
-    float m3 = min3f(a[9], a[10], a[11]);
-    float m4 = min3f(a[12], a[13], a[14]);
-    m0 = min3f(m0, m1, m2);
-    m3 = min3f(m3, m4, a[15]);
-    const float least = __builtin_fminf(m0, m3);
+    feat_acc_t acc[SUBS];
+    float least[SUBS];
+#pragma unroll
+    for (int sub = 0; sub < SUBS; ++sub)
+      acc[sub] = products(buf, sub);
+#pragma unroll
+    for (int sub = 0; sub < SUBS; ++sub)
+      least[sub] = min16(acc[sub]);
     const bool all_rows = active && !filtered;
     const bool looking = !RADIUS || !full;
-    if (__any((least < cut || all_rows) && looking)) {
-      // the lane's rows under the cut: bit 15 - v for accumulator v
-      uint32_t mask = 0;
 #pragma unroll
-      for (int v = 0; v < 16; ++v)
-        if ((a[v] < cut || all_rows) && looking && row_of(v) < rows)
-          mask |= 0x8000u >> v;
-      if (mask != 0) {
-        queue[qn][tid] = ((uint32_t)t << 16) | mask;
-        ++qn;
+    for (int sub = 0; sub < SUBS; ++sub) {
+      const feat_acc_t &a = acc[sub];
+      if (__any((least[sub] < cut || all_rows) && looking)) {
+        // the lane's rows under the cut: bit 15 - v for accumulator v
+        uint32_t mask = 0;
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          if ((a[v] < cut || all_rows) && looking &&
+              sub * kSmallStep + row_of(v) < rows)
+            mask |= 0x8000u >> v;
+        if (mask != 0) {
+          queue[qn][tid] = ((uint32_t)(t * SUBS + sub) << 16) | mask;
+          ++qn;
+        }
       }
     }
   }, [&](int group, bool last) {
@@ -788,7 +848,7 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
       go = go || wave_says[(group & 1) ^ 1][w] != 0;
     if (go)
       drain();
-    const int want = __any(qn > kSmallQueue - 2 * DEPTH) ? 1 : 0;
+    const int want = __any(qn > kSmallQueue - 2 * LOOK) ? 1 : 0;
     if (lane == 0)
       wave_says[group & 1][wave] = want;
     if constexpr (RADIUS) {
