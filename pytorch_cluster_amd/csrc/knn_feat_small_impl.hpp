@@ -13,29 +13,33 @@
 // in knn_lowd_mc_impl.hpp) and goes over the example's rows TWICE, 32 rows at a
 // time.
 //
-//   1. Bound (the first 64 steps at most; the step's packed fp16 rows and its
-//      fp32 rows both in LDS).  One chain of v_mfma_f32_32x32x16_f16 per step
-//      gives a lane the values s of its 16 rows; it takes the row with the
-//      smallest one (accumulator number in the four lowest mantissa bits
-//      through a v_min3_f32 tree), evaluates THAT row exactly -- direct
-//      differences, one fused multiply-add per component in ascending order,
-//      the reference's chain -- and keeps the ceil(k / 2) smallest of these
-//      distances.  The rows are all different, and different from the partner
-//      lane's, so the larger of the two lanes' ceil(k / 2)-th samples is an
-//      upper bound tau of the query's k-th distance.
+//   1. Bound (the first 64 steps at most).  One chain of
+//      v_mfma_f32_32x32x16_f16 per step gives a lane the values s of its 16
+//      rows, and it keeps the ceil(k / 2) smallest of the steps' smallest ones.
+//      The rows are all different, and different from the partner lane's, so
+//      the larger of the two lanes' ceil(k / 2)-th values, as the upper bound
+//      F(l) of a distance (knn_feat_impl.hpp), is an upper bound tau of the
+//      query's k-th distance.  (F bounds an fp32 distance; of 16-bit rows it
+//      would have to allow for every rounding of the chain.  Their row of the
+//      smallest value, its accumulator number in the four lowest mantissa
+//      bits, is evaluated exactly instead, from fp32 rows in LDS.)
 //   2. Search (packed rows only).  The same chains again.  l = s + shift is a
 //      lower bound of the scaled distance e / sigma^2 the reference computes
 //      (knn_feat_impl.hpp), so every row with e below a bound has s <= bound /
 //      sigma^2 - shift =: cut.  A lane parks the rows under its cut (one word
 //      per step: step and 16-bit mask); when a queue is about to fill up,
-//      and at the end, all waves turn to their parked rows: in rounds of one
-//      row per lane the rows are fetched from global memory (four lanes per
+//      and at the end, all waves turn to their parked rows: in rounds of two
+//      rows per lane the rows are fetched from global memory (four lanes per
 //      64-byte line, handed to the owner through LDS), evaluated exactly, and
 //      enter the lane's sorted list of (distance, row) keys; the list's k-th distance and the partner's
 //      tighten the bound as in the low-dimensional kernel.  About 1.5 k rows
 //      per query get that far.  Nothing is approximate in what is KEPT, and
 //      every row that could be kept is looked at: no candidate list, no second
 //      stage, no proof of completeness to fail.
+//
+// 32 x 1,024 x 64, k = 20, call: 206 us with exact samples and one row per lane
+// and round, 182 with the filter's bounds and tiles of two steps, 171 with two
+// rows per lane; fp16 rows of 24 ragged examples 308 -> 292.
 //
 // A workgroup has its compute unit to itself (one wave per SIMD: 200+
 // registers for the lists, up to 157 KB of LDS), so nothing hides a wait but
@@ -638,11 +642,15 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
   // the query of lane l), the rows read from global memory.  A lane reading
   // its own row would touch a 64-byte line per 16-byte load; here four lanes
   // read one line of one row together (sixteen rows per load instruction,
-  // every line used in full), 64 components of all rows at a time (a
+  // every line used in full), 32 or 64 components of all rows at a time (a
   // "chunk": gather_chunk), and the pieces reach the lane that owns the row
   // through LDS, sixteen components at a time, in ascending order
   // (chain_chunk): the chain is the reference's.
-  auto gather_chunk = [&](small_v4f (&a)[4][4], int g, int f0) {
+  // of 16 components, per chunk: four where the lists leave the registers for
+  // them (32 x 1,024 x 64, k = 20: 171 us a call, with two 174; wider lists and
+  // rows went to scratch memory, and the fp16 chain is slower with four)
+  constexpr int PIECES = (R16 == 0 && !RADIUS && NB <= 5 && K <= 24) ? 4 : 2;
+  auto gather_chunk = [&](small_v4f (&a)[PIECES][4], int g, int f0) {
     const int quads = d >> 2;
     const small_v4f *x4 = reinterpret_cast<const small_v4f *>(p.x);
 #pragma unroll
@@ -650,37 +658,46 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
       // the row of lane 16 r + lane / 4: one of the four this lane helps with
       const size_t base = (size_t)__shfl(g, 16 * r + (lane >> 2)) * quads;
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int c = 0; c < PIECES; ++c)
         a[c][r] = x4[base + min(f0 + 4 * c + (lane & 3), quads - 1)];
     }
   };
-  auto chain_chunk = [&](const small_v4f (&a)[4][4], int f0, float acc) {
+  // (two rows per lane: their exchanges and chains fill each other's waits)
+  auto chain_chunk = [&](const small_v4f (&a)[2][PIECES][4], int f0,
+                         float (&acc)[2]) {
     const int quads = d >> 2;
     const small_v4f *y4 = reinterpret_cast<const small_v4f *>(my_y);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < PIECES; ++c) {
       if (f0 + 4 * c < quads) { // (uniform)
-        // (the wave is done reading the piece before)
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        small_v4f xv[2][4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          gathered[wave][16 * r + (lane >> 2)][lane & 3] = a[c][r];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (int w = 0; w < 2; ++w) {
+          // (the wave is done reading the piece before)
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            gathered[wave][16 * r + (lane >> 2)][lane & 3] = a[w][c][r];
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            xv[w][e] = gathered[wave][lane][e];
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           if (f0 + 4 * c + e < quads) {
-            const small_v4f xv = gathered[wave][lane][e];
             const small_v4f b = y4[f0 + 4 * c + e];
-            acc = Chain::step4(xv.x, xv.y, xv.z, xv.w, b.x, b.y, b.z, b.w,
-                               acc);
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+              acc[w] = Chain::step4(xv[w][e].x, xv[w][e].y, xv[w][e].z,
+                                    xv[w][e].w, b.x, b.y, b.z, b.w, acc[w]);
           }
         }
       }
     }
-    return acc;
   };
   // (d not a multiple of four: every lane reads its own row)
   auto exact_unaligned = [&](int g) {
@@ -747,40 +764,53 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
       }
       changed = true;
     };
-    int g;
-    bool on;
-    pop(g, on);
     if (vec4) {
-      // One chunk ahead: while a chunk goes through LDS and the chain, the
-      // next one (of the same rows, or the first of the next rows; after the
-      // last rows, one nobody looks at) is on its way from global memory.
-      // Two sets of registers take turns, and the fetch is unconditional
-      // (see load_tile).
+      // Two rows per lane at a time, one chunk ahead: while a chunk goes
+      // through LDS and the chains, the next one (of the same rows, or the
+      // first of the next rows; after the last rows, one nobody looks at) is
+      // on its way from global memory.  Two sets of registers take turns, and
+      // the fetch is unconditional (see load_tile).
       const int quads = d >> 2;
-      small_v4f set_a[4][4], set_b[4][4];
-      bool more = __any(on);
+      small_v4f set_a[2][PIECES][4], set_b[2][PIECES][4];
+      int g[2];
+      bool on[2];
+      pop(g[0], on[0]);
+      pop(g[1], on[1]);
+      bool more = __any(on[0]);
       int f0 = 0;
-      float acc = 0.0f;
-      auto chunk = [&](small_v4f (&now)[4][4], small_v4f (&next)[4][4]) {
-        const bool last = f0 + 16 >= quads; // (uniform)
-        int g_next = g;
-        bool on_next = on;
-        if (last)
-          pop(g_next, on_next);
-        const int f0_next = last ? 0 : f0 + 16;
-        gather_chunk(next, g_next, f0_next);
-        acc = chain_chunk(now, f0, acc);
+      float acc[2] = {0.0f, 0.0f};
+      auto chunk = [&](small_v4f (&now)[2][PIECES][4],
+                       small_v4f (&next)[2][PIECES][4]) {
+        const bool last = f0 + 4 * PIECES >= quads; // (uniform)
+        int g_next[2] = {g[0], g[1]};
+        bool on_next[2] = {on[0], on[1]};
         if (last) {
-          take(finish(acc, g), g, on);
-          acc = 0.0f;
-          more = __any(on_next);
+          pop(g_next[0], on_next[0]);
+          pop(g_next[1], on_next[1]);
         }
-        g = g_next;
-        on = on_next;
+        const int f0_next = last ? 0 : f0 + 4 * PIECES;
+        gather_chunk(next[0], g_next[0], f0_next);
+        gather_chunk(next[1], g_next[1], f0_next);
+        chain_chunk(now, f0, acc);
+        if (last) {
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            take(finish(acc[w], g[w]), g[w], on[w]);
+            acc[w] = 0.0f;
+          }
+          more = __any(on_next[0]);
+        }
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          g[w] = g_next[w];
+          on[w] = on_next[w];
+        }
         f0 = f0_next;
       };
-      if (more)
-        gather_chunk(set_a, g, 0);
+      if (more) {
+        gather_chunk(set_a[0], g[0], 0);
+        gather_chunk(set_a[1], g[1], 0);
+      }
       while (more) {
         chunk(set_a, set_b);
         if (!more)
@@ -788,6 +818,9 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
         chunk(set_b, set_a);
       }
     } else {
+      int g;
+      bool on;
+      pop(g, on);
       while (__any(on)) {
         take(finish(exact_unaligned(g), g), g, on);
         pop(g, on);
