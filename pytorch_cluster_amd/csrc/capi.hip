@@ -652,8 +652,13 @@ int knn_call(const void *x, const void *y, const int64_t *ptr_x,
     cfg.tile_queries = pca::kMfmaTileQueries;
   else if (!low_d)
     cfg.tile_queries = pca::kBlock; // any-dimension kernel: one query per lane
-  // (the low-dimensional path plans its work inside its own first launch)
-  if (!low_d)
+  // (the low-dimensional path plans its work inside its own first launch, the
+  // feature-space path beside its preparation)
+  pca::FeatPlan feat_plan;
+  feat_plan.work_start = work_start;
+  if (plan_derives)
+    feat_plan.src = src;
+  if (!low_d && !feat && !feat16)
     rc = check_launch(pca::launch_plan(ptr_y, (int)m, (int)num_segments,
                                        cfg.tile_queries, work_start, stream,
                                        plan_derives ? &src : nullptr),
@@ -675,13 +680,15 @@ int knn_call(const void *x, const void *y, const int64_t *ptr_x,
   } else if (feat) {
     rc = check_launch(pca::launch_knn_feat(in, (int)k, cosine != 0, work_start,
                                            lowd_scratch, dense, timer.start,
-                                           timer.stop, stream),
+                                           timer.stop, stream, 0, nullptr,
+                                           &feat_plan),
                       "knn_feat_kernel");
     timer.stop = nullptr;
   } else if (feat16) {
     rc = check_launch(pca::launch_knn_feat(in, (int)k, false, work_start,
                                            lowd_scratch, dense, timer.start,
-                                           timer.stop, stream, r16),
+                                           timer.stop, stream, r16, nullptr,
+                                           &feat_plan),
                       "knn_feat_small_kernel");
     timer.stop = nullptr;
   } else if (mfma) {
@@ -931,9 +938,13 @@ int pca_radius(const void *x, const void *y, const int64_t *ptr_x,
   const int per_item = matrix_cores    ? pca::kRadiusMcTileQueries
                        : feature_space ? pca::kMfmaTileQueries
                                        : pca::kRadiusQueriesPerWave;
-  // (the matrix-core path plans its work in the launch that packs the rows,
-  // short examples need no plan)
-  if (!matrix_cores && !short_examples)
+  // (the matrix-core path plans its work in the launch that packs the rows, the
+  // feature-space path beside its preparation, short examples need no plan)
+  pca::FeatPlan feat_plan;
+  feat_plan.work_start = work_start;
+  if (plan_derives)
+    feat_plan.src = src;
+  if (!matrix_cores && !feature_space && !short_examples)
     rc = check_launch(pca::launch_plan(ptr_y, (int)m, (int)num_segments,
                                        per_item, work_start, stream,
                                        plan_derives ? &src : nullptr),
@@ -957,7 +968,8 @@ int pca_radius(const void *x, const void *y, const int64_t *ptr_x,
         ignore_same_index != 0};
     rc = check_launch(pca::launch_knn_feat(in, (int)slots, false, work_start,
                                            packed_rows, dense, timer.start,
-                                           timer.stop, stream, r16, &radius),
+                                           timer.stop, stream, r16, &radius,
+                                           &feat_plan),
                       "knn_feat_small_kernel (radius)");
     timer.stop = nullptr;
   } else if (matrix_cores)

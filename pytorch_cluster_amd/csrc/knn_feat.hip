@@ -270,26 +270,48 @@ __global__ __launch_bounds__(kBlock) void feat_rows_kernel(
 // rows, unless a few rows (up to kFeatMaxOutliers of x and as many of y, and
 // never more than one in 64) are at least four times larger than all others --
 // then for the others, which keep their bits in fp16; the few are handled
-// exactly (see FeatGlobals).  One workgroup of 256 threads.
+// exactly (see FeatGlobals).  One workgroup.
 // (y_is_x: the queries are the rows of x, whose histogram stands for both)
-__global__ __launch_bounds__(256) void feat_scale_kernel(FeatGlobals *g, int n,
-                                                         int m, bool y_is_x) {
+// A second workgroup plans the search (plan.work_start not NULL): segment
+// pointers from example ids where the call has those, and the first work item
+// of every segment, which nothing before the search reads.  (In front of
+// everything, as a launch of its own, the plan took 10 us and a launch's gap.)
+__global__ __launch_bounds__(kPlanThreads) void feat_scale_kernel(
+    FeatGlobals *g, int n, int m, bool y_is_x, const int64_t *ptr_y,
+    int num_segments, FeatPlan plan) {
+  __shared__ int partial[kPlanThreads];
+  if (blockIdx.x == 1) {
+    if (plan.src.ids_x != nullptr) {
+      pointers_from_ids(plan.src, num_segments);
+      __syncthreads();
+    }
+    plan_segments(ptr_y, m, num_segments, kFeatQueries, plan.work_start,
+                  partial);
+    return;
+  }
   __shared__ unsigned hx[256], hy[256];
   __shared__ int need_x, need_y, top;
   const int t = threadIdx.x;
-  unsigned sum_x = 0, sum_y = 0;
-  for (int c = 0; c < kFeatHistCopies; ++c) {
-    sum_x += g->hist_x[c * 256 + t];
-    sum_y += g->hist_y[c * 256 + t];
+  if (t < 256) {
+    hx[t] = 0;
+    hy[t] = 0;
   }
-  if (y_is_x)
-    sum_y = sum_x;
-  hx[t] = sum_x;
-  hy[t] = sum_y;
   if (t == 0) {
     need_x = 255;
     need_y = 255;
     top = -1;
+  }
+  __syncthreads();
+  {
+    // (the copies of a bin by four threads)
+    unsigned sum_x = 0, sum_y = 0;
+    const int bin = t & 255;
+    for (int c = t >> 8; c < kFeatHistCopies; c += kPlanThreads / 256) {
+      sum_x += g->hist_x[c * 256 + bin];
+      sum_y += g->hist_y[c * 256 + bin];
+    }
+    atomicAdd(&hx[bin], sum_x);
+    atomicAdd(&hy[bin], y_is_x ? sum_x : sum_y);
   }
   __syncthreads();
   // rows with a larger exponent than t: one wave, four bins per lane, a
@@ -324,17 +346,19 @@ __global__ __launch_bounds__(256) void feat_scale_kernel(FeatGlobals *g, int n,
     }
   }
   __syncthreads();
-  const unsigned above_x = ax[t], above_y = ay[t];
-  const unsigned allow_x = (unsigned)min(kFeatMaxOutliers, n / 64);
-  const unsigned allow_y = (unsigned)min(kFeatMaxOutliers, m / 64);
-  // the smallest exponent that leaves at most that many rows above it (not
-  // below the smallest one in use: rows, not bins, are what is left out)
-  if (above_x <= allow_x && (hx[t] != 0 || above_x == 0))
-    atomicMin(&need_x, t);
-  if (above_y <= allow_y && (hy[t] != 0 || above_y == 0))
-    atomicMin(&need_y, t);
-  if (hx[t] != 0 || hy[t] != 0)
-    atomicMax(&top, t);
+  if (t < 256) {
+    const unsigned above_x = ax[t], above_y = ay[t];
+    const unsigned allow_x = (unsigned)min(kFeatMaxOutliers, n / 64);
+    const unsigned allow_y = (unsigned)min(kFeatMaxOutliers, m / 64);
+    // the smallest exponent that leaves at most that many rows above it (not
+    // below the smallest one in use: rows, not bins, are what is left out)
+    if (above_x <= allow_x && (hx[t] != 0 || above_x == 0))
+      atomicMin(&need_x, t);
+    if (above_y <= allow_y && (hy[t] != 0 || above_y == 0))
+      atomicMin(&need_y, t);
+    if (hx[t] != 0 || hy[t] != 0)
+      atomicMax(&top, t);
+  }
   __syncthreads();
   if (t == 0) {
     // (only the exponent of max_bits is used: the largest number of the
@@ -719,7 +743,8 @@ hipError_t launch_knn_feat(const SearchInput &in_given, int k, bool cosine,
                            const int *work_start, void *scratch,
                            const DenseResult &out, hipEvent_t time_start,
                            hipEvent_t time_stop, hipStream_t stream,
-                           int r16, const FeatRadius *radius) {
+                           int r16, const FeatRadius *radius,
+                           const FeatPlan *plan) {
   SearchInput in = in_given;
   if (radius != nullptr && cosine)
     return hipErrorInvalidValue;
@@ -803,6 +828,9 @@ hipError_t launch_knn_feat(const SearchInput &in_given, int k, bool cosine,
     (void)launch_row_norms(xf, in.n, in.d, x_norm, stream);
     (void)launch_row_norms(yf, in.m, in.d, y_norm, stream);
     // (no scale to make: the rows are normalised one by one)
+    if (plan != nullptr)
+      (void)launch_plan(in.ptr_y, in.m, in.num_segments, kFeatQueries,
+                        plan->work_start, stream, &plan->src);
     hipLaunchKernelGGL(feat_rows_kernel,
                        dim3((in.n + rows_per_block - 1) / rows_per_block),
                        dim3(kBlock), 0, stream, xf, in.n, in.d, x_class,
@@ -825,8 +853,10 @@ hipError_t launch_knn_feat(const SearchInput &in_given, int k, bool cosine,
                          dim3(kBlock), 0, stream, yf, in.m, in.d,
                          static_cast<float *>(nullptr), globals,
                          static_cast<unsigned *>(nullptr), globals->hist_y);
-    hipLaunchKernelGGL(feat_scale_kernel, dim3(1), dim3(256), 0, stream,
-                       globals, in.n, in.m, y_is_x);
+    hipLaunchKernelGGL(feat_scale_kernel, dim3(plan != nullptr ? 2 : 1),
+                       dim3(kPlanThreads), 0, stream, globals, in.n, in.m,
+                       y_is_x, in.ptr_y, in.num_segments,
+                       plan != nullptr ? *plan : FeatPlan{});
   }
   {
     hipError_t perr;

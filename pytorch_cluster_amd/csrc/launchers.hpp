@@ -221,13 +221,20 @@ hipError_t launch_nearest_feat(const SearchInput &in, int *work_start,
 // kernel (knn_feat_impl.hpp): fp32, 8 < d <= 512, k <= 100.
 bool knn_feat_supported(int d, int k, bool cosine);
 size_t knn_feat_scratch_bytes(int n, int m, int d, int num_segments, int k);
-// work_start: tiles of kMfmaTileQueries queries (planned by the caller).
+// work_start: tiles of kMfmaTileQueries queries, planned by the caller, or by
+// this call beside other work with `plan` (plan->work_start = work_start,
+// written; src: the example ids the segment pointers are derived from, or
+// none).
 // r16 = 1 / 2: x and y hold fp16 / bf16 rows (knn_feat16_supported shapes
 // only; scratch: knn_feat16_scratch_bytes); the results are those of the
 // reference's kernel for that element type.
 // radius: the radius search instead (radius_feat_supported shapes;
 // k = max_num_neighbors, out.dist NULL; scratch as for kNN with that k; r2
 // narrowed to the element type by the caller).
+struct FeatPlan {
+  SegmentSource src;
+  int *work_start = nullptr;
+};
 struct FeatRadius {
   float r2;
   bool ignore_same;
@@ -236,7 +243,8 @@ hipError_t launch_knn_feat(const SearchInput &in, int k, bool cosine,
                            const int *work_start, void *scratch,
                            const DenseResult &out, hipEvent_t time_start,
                            hipEvent_t time_stop, hipStream_t stream,
-                           int r16 = 0, const FeatRadius *radius = nullptr);
+                           int r16 = 0, const FeatRadius *radius = nullptr,
+                           const FeatPlan *plan = nullptr);
 // Feature-space radius search through the matrix-core filter
 // (knn_feat_small_impl.hpp): fp32 rows of 8 < d <= 128 components, fp16 and
 // bf16 rows of up to 128, at most 32 neighbours per query, and enough pairs to
