@@ -86,13 +86,13 @@ bool sizes_ok(int64_t n, int64_t m, int64_t d, int64_t num_segments) {
          d <= (1 << 20) && num_segments >= 1 && num_segments <= kMaxRows;
 }
 
-// two arrays of num_segments + 1 pointers (PCA_SEGMENTS_BY_ID)
 // Up to this many examples the launch that plans the work derives their
 // pointers itself, by the waves of one workgroup; more get a launch of their
 // own, one wave per pointer.  (A round of 16 searches takes ~1.3 us, the extra
 // launch ~5 us.)
 constexpr int64_t kPlanDerivesExamples = 32;
 
+// two arrays of num_segments + 1 pointers (PCA_SEGMENTS_BY_ID)
 size_t segment_pointer_bytes(int64_t num_segments) {
   return 2 * align256(sizeof(int64_t) * (size_t)(num_segments + 1));
 }
