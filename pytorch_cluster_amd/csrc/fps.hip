@@ -470,6 +470,13 @@ __global__ __launch_bounds__(T) void fps_reg_kernel(
 // touches are looked at side by side.
 
 constexpr uint32_t kFpsNoRow = 0xffffffffu; // its tie is the largest one
+// Largest minimum of a bucket before the first sample: a NaN, which no distance
+// is at or above, so that every bucket with rows is looked at and gets the
+// value of its rows (5e4 or less) there.  Against infinity a bucket at an
+// infinite distance -- rows without a finite coordinate on some axis, a first
+// sample with an infinite one, squared gaps beyond fp32 -- would be left alone
+// and keep the infinity.
+constexpr uint32_t kFpsUnseen = 0x7fc00000u;
 
 // What a wave hands over: the largest running minimum (bits of a float that
 // is not negative), the row that has it, and that row's coordinates.
@@ -722,8 +729,7 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
     perm[CAP] = 0xffffu;
   __syncthreads();
 
-  // lane = bucket: its box, and the best of its rows.  (Every minimum is 5e4
-  // before the first sample; the first test lets every bucket through.)
+  // lane = bucket: its box, and the best of its rows
   float blo[DIM], bhi[DIM], bx[DIM];
 #pragma unroll
   for (int c = 0; c < DIM; ++c) {
@@ -776,7 +782,7 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
     }
     __syncthreads();
   }
-  uint32_t val = lane < buckets ? __float_as_uint(__builtin_inff()) : 0u;
+  uint32_t val = lane < buckets ? kFpsUnseen : 0u;
   int place = CAP; // (of no row)
 
   float cur[DIM];
@@ -968,10 +974,8 @@ __global__ __launch_bounds__(W *kWave) void fps_bucket_kernel(
         bhi[c] = h;
       }
     }
-    // (before the first sample every minimum is 5e4: any value will do, the
-    // first test must let every bucket with rows through)
     if (lane == i && (i * W + wave) * kWave < count)
-      best.val = __float_as_uint(__builtin_inff());
+      best.val = kFpsUnseen;
     // (one bucket after the other: all loads and reductions at once would
     // take several times the registers the loop below needs)
     __builtin_amdgcn_sched_barrier(0);
@@ -1140,7 +1144,7 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
   for (int s = 0; s < S; ++s) {
     const int k = (s * kWave + lane) * W + wave;
     const bool any = k < buckets;
-    best[s].val = any ? __float_as_uint(__builtin_inff()) : 0u;
+    best[s].val = any ? kFpsUnseen : 0u;
     best[s].rel = kFpsNoRow;
 #pragma unroll
     for (int c = 0; c < DIM; ++c) {

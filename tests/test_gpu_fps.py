@@ -115,6 +115,49 @@ def test_skipped_rows_change_nothing(oracle, rows, d, kind):
     assert (got == want).all()
 
 
+# whole buckets (64 or 128 consecutive rows along the curve) at an infinite
+# distance: rows without a finite coordinate on an axis, rows and first samples
+# at infinity, squared gaps beyond the fp32 range
+@pytest.mark.parametrize("kind", ["nan", "nan_axis", "all_nan", "all_nan_axis",
+                                  "inf", "inf_start", "far", "mixed"])
+@pytest.mark.parametrize("rows,d", [(1025, 3), (4096, 4), (4097, 3), (4097, 4),
+                                    (8193, 2), (16385, 3), (20000, 1),
+                                    (262145, 3)])
+def test_rows_out_of_reach_keep_their_place(oracle, rows, d, kind):
+    rng = np.random.default_rng(rows + d)
+    begin, first = 70, 5
+    ptr = np.array([0, begin, begin + rows], dtype=np.int64)
+    x = rng.standard_normal((ptr[-1], d)).astype(np.float32)
+    some = begin + rng.permutation(rows)[:rows // 3]
+    if kind == "nan":
+        x[some] = np.nan
+    elif kind == "nan_axis":
+        x[some, d - 1] = np.nan
+    elif kind == "all_nan":
+        x[begin:] = np.nan
+    elif kind == "all_nan_axis":
+        x[begin:, 0] = np.nan
+    elif kind == "inf":
+        x[some, 0] = np.inf
+        x[some[:200], 0] = -np.inf
+        x[begin + first] = 0
+    elif kind == "inf_start":
+        x[begin + first, d - 1] = np.inf
+    elif kind == "far":
+        x[some] += np.float32(3e19)
+        x[begin + first] = 0
+    else:
+        x[some] = np.nan
+        x[some[:300]] = np.inf
+        x[some[300:]] *= np.float32(1e25)
+    share = np.array([0.1, 130.0 / rows])
+    start = np.array([0, first], dtype=np.int64)
+    got = gpu_fps(oracle, x, ptr, share, start)
+    assert got.min() >= 0 and (got[7:] >= begin).all()
+    assert got.max() < ptr[-1]
+    assert (got == oracle.fps_op(x, ptr, share, start)).all()
+
+
 def test_captured_into_a_graph(oracle):
     """While its stream is being captured the search does without the sort of
     the large examples; every replay samples the same rows."""
