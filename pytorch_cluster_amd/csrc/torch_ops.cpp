@@ -540,38 +540,51 @@ at::Tensor knn_edges(at::Tensor x, at::Tensor y,
 // of into pinned host memory, and the operator looks at it after the one wait
 // it has anyway (for the edge count): equal or smaller, the edges are right
 // (examples without rows); larger, the search runs once more with the right
-// number.  Only the first call of a process reads the ids' last entries up
-// front.
+// number.  A call that fails or is refused leaves the number as it was.
 std::atomic<int64_t> g_examples_hint{0};
+
+// What a call with these sorted ids starts with.  The first call of a process,
+// and one that has fewer rows than the previous call met examples, reads the
+// ids' last entries up front (known).
+struct ExamplesGuess {
+  int64_t examples;
+  bool known;
+};
+ExamplesGuess guess_examples(const at::Tensor &batch_x,
+                             const at::Tensor &batch_y) {
+  const int64_t hint = g_examples_hint.load();
+  if (hint >= 1 && hint <= batch_x.numel() + batch_y.numel())
+    return {hint, false};
+  int64_t last = -1;
+  if (batch_x.numel() > 0)
+    last = std::max(last, batch_x[-1].item<int64_t>());
+  if (batch_y.numel() > 0 && !batch_y.is_same(batch_x))
+    last = std::max(last, batch_y[-1].item<int64_t>());
+  g_host_waits += 1;
+  return {std::max<int64_t>(last + 1, 1), true};
+}
 
 template <typename Run>
 at::Tensor with_examples(const at::Tensor &batch_x, const at::Tensor &batch_y,
                          int64_t batch_size, Run run) {
   if (batch_size >= 1)
     return run(batch_size, nullptr);
-  int64_t guess = g_examples_hint.load();
-  if (guess < 1) {
-    // (sorted ids: the last ones are the largest)
-    int64_t last = -1;
-    if (batch_x.numel() > 0)
-      last = std::max(last, batch_x[-1].item<int64_t>());
-    if (batch_y.numel() > 0 && !batch_y.is_same(batch_x))
-      last = std::max(last, batch_y[-1].item<int64_t>());
-    g_host_waits += 1;
-    guess = std::max<int64_t>(last + 1, 1);
-    g_examples_hint.store(guess);
-    return run(guess, nullptr);
+  const ExamplesGuess guess = guess_examples(batch_x, batch_y);
+  if (guess.known) {
+    at::Tensor out = run(guess.examples, nullptr);
+    g_examples_hint.store(guess.examples);
+    return out;
   }
   auto slot = at::empty({1}, at::TensorOptions().dtype(at::kLong).pinned_memory(
                                  true));
   int64_t *in_use = slot.data_ptr<int64_t>();
   *in_use = 0;
-  at::Tensor out = run(guess, in_use);
+  at::Tensor out = run(guess.examples, in_use);
   // (run has waited for the stream: the number is there)
   const int64_t met = std::max<int64_t>(*in_use, 1);
-  g_examples_hint.store(met);
-  if (met > guess)
+  if (met > guess.examples)
     out = run(met, nullptr);
+  g_examples_hint.store(met);
   return out;
 }
 
@@ -868,14 +881,7 @@ nearest_batched(at::Tensor x, at::Tensor y, std::optional<at::Tensor> batch_x,
   PCA_CHECK_INPUT(batch_y->dim() == 1 && batch_y->numel() == m);
   at::Tensor ids_x = batch_x->to(at::kLong).contiguous();
   at::Tensor ids_y = batch_y->to(at::kLong).contiguous();
-  int64_t guess = g_examples_hint.load();
-  if (guess < 1) {
-    guess = std::max<int64_t>(std::max(ids_x[-1].item<int64_t>(),
-                                       ids_y[-1].item<int64_t>()) +
-                                  1,
-                              1);
-    g_host_waits += 1;
-  }
+  int64_t guess = guess_examples(ids_x, ids_y).examples;
   for (;;) {
     auto slot = report_slot(4);
     const int64_t *report = slot.data_ptr<int64_t>();
@@ -891,11 +897,12 @@ nearest_batched(at::Tensor x, at::Tensor y, std::optional<at::Tensor> batch_x,
     mark.wait();
     guard.armed = false;
     const int64_t met = report[3];
-    g_examples_hint.store(std::max<int64_t>(met, 1));
     const int64_t wrong = report[0] != 0   ? 1
                           : report[1] != 0 ? 2
                           : report[2] != 0 || met < 1 ? 3
                                                       : 0;
+    if (wrong == 0 && met <= guess)
+      g_examples_hint.store(met);
     if (wrong == 1 || wrong == 2 || met <= guess)
       return {out, wrong};
     guess = met;
@@ -1023,11 +1030,8 @@ at::Tensor fps_batched(at::Tensor src, std::optional<at::Tensor> batch,
     PCA_CHECK_GPU(batch.value());
     PCA_CHECK_INPUT(batch->dim() == 1 && batch->numel() == n);
     at::Tensor ids = batch->to(at::kLong).contiguous();
-    int64_t guess = batch_size >= 1 ? batch_size : g_examples_hint.load();
-    if (guess < 1) {
-      guess = std::max<int64_t>(ids[-1].item<int64_t>() + 1, 1);
-      g_host_waits += 1;
-    }
+    int64_t guess =
+        batch_size >= 1 ? batch_size : guess_examples(ids, ids).examples;
     for (;;) {
       auto slot = report_slot(3);
       const int64_t *report = slot.data_ptr<int64_t>();
@@ -1049,10 +1053,11 @@ at::Tensor fps_batched(at::Tensor src, std::optional<at::Tensor> batch,
         break;
       const int64_t met = report[2];
       PCA_CHECK_INPUT(met >= 1);
-      g_examples_hint.store(met);
       examples = met; // (examples beyond it have no rows and no samples)
-      if (met <= guess)
+      if (met <= guess) {
+        g_examples_hint.store(met);
         break;
+      }
       guess = met;
     }
   } else {

@@ -104,3 +104,54 @@ def test_fps_fewer_examples_than_ids():
     assert (pca.fps(x, ids, 0.5, False, 2) == want).all()
     with pytest.raises(RuntimeError):
         pca.fps(x, ids - 5, 0.5, False)
+
+
+@pytest.mark.parametrize("call", ["nearest", "nearest_mismatch", "fps", "knn",
+                                  "radius"])
+def test_a_refused_call_leaves_no_number_of_examples_behind(call):
+    """A call with one huge id fails; the next one, which starts with the
+    number of examples of an earlier call, must not start with that id."""
+    x = torch.rand(40, 3, device="cuda")
+    ids = torch.arange(4, device="cuda").repeat_interleave(10)
+    searches = [lambda: pca.nearest(x, x[::2], ids, ids[::2]),
+                lambda: pca.fps(x, ids, 0.5, random_start=False),
+                lambda: pca.knn_graph(x, 3, ids),
+                lambda: pca.radius_graph(x, 0.4, ids)]
+    want = [search() for search in searches]
+    bad = ids.clone()
+    bad[-1] = 10**12
+    with pytest.raises((RuntimeError, ValueError)):
+        if call == "nearest":
+            falls = bad.clone()
+            falls[3] = 2
+            pca.nearest(x, x[::2], falls, ids[::2])
+        elif call == "nearest_mismatch":
+            pca.nearest(x, x[10:20], bad, ids[10:20])
+        elif call == "fps":
+            pca.fps(x, bad, 0.5, random_start=False)
+        elif call == "knn":
+            pca.knn_graph(x, 3, bad)
+        else:
+            pca.radius_graph(x, 0.4, bad)
+    for search, rows in zip(searches, want):
+        assert (search() == rows).all()
+
+
+def test_examples_of_a_much_larger_batch_before():
+    many = torch.arange(5000, device="cuda").repeat_interleave(3)
+    x = torch.rand(15000, 3, device="cuda")
+    ids = torch.tensor([0] * 30 + [2] * 10, device="cuda")
+    y = torch.rand(40, 3, device="cuda")
+    want = [pca.knn_graph(y, 3, ids, batch_size=3),
+            pca.radius_graph(y, 0.4, ids, batch_size=3),
+            pca.fps(y, ids, 0.5, random_start=False, batch_size=3)]
+    waits = torch.ops.pytorch_cluster_amd.host_waits
+    for i, search in enumerate((lambda: pca.knn_graph(y, 3, ids),
+                                lambda: pca.radius_graph(y, 0.4, ids),
+                                lambda: pca.fps(y, ids, 0.5,
+                                                random_start=False))):
+        pca.radius_graph(x, 0.1, many)
+        pca.radius_graph(x, 0.1, many)
+        before = waits()
+        assert (search() == want[i]).all()
+        assert waits() - before == 2  # (more examples than rows: looked up)
