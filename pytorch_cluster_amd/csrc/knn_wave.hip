@@ -21,6 +21,8 @@
 #include "knn_lowd_impl.hpp"
 #include "launchers.hpp"
 
+#include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 namespace pca {
@@ -257,19 +259,33 @@ bool knn_wave_supported(int n, int m, int d, int num_segments, int k,
     if (env[0] == '1')
       return true;
   }
-  // us of the two kernels beyond what every call costs, as fitted to calls of
-  // knn_graph (this path / the matrix-core scan, us): one cloud of 1,024 points
-  // 26 / 55, of 4,096 45 / 93, of 8,192 96 / 126, of 16,384 263 / 151;
-  // 8 x 1,024 42 / 59, 16 x 1,024 60 / 61, 8 x 2,048 78 / 75 (k = 17; the scan
-  // is faster for short lists: one cloud of 8,192, k = 5, 90 / 83).  Lists
-  // beyond 32 entries go through the vector-ALU scan otherwise: k = 33, 1,024
-  // points 27 / 220, 16 x 4,096 316 / 468, 64 x 4,096 1,096 / 925.
-  const double rounds = (double)((n / num_segments + kWaveRows * kWave - 1) /
-                                 (kWaveRows * kWave));
-  const double here = (double)m / 1024.0 * (1.0 + rounds);
+  // us of a call both ways, fitted to 632 calls of one example and of batches
+  // (500 - 524,288 rows in all, 1 - 16,384 queries, k = 1 - 32).  The pick costs
+  // 0.2 % over the faster path on average and at most 8 % where the examples are
+  // of one size (batches with one example a hundred times longer: 28 %).
+  // Every query's wave goes through all rows of its example; the scan cuts long
+  // examples into slices, so it gains on this path as examples grow.  This path
+  // / the scan, us, k = 16: one cloud of 1,024 points 28 / 53, of 4,096 45 / 85,
+  // of 8,192 97 / 112, of 16,384 263 / 131; 4,000 queries among 20,000 rows
+  // 109 / 133, among 50,000 191 / 154, among 200,000 502 / 249; 64 queries among
+  // 16,384 66 / 118, among 200,000 285 / 206.
+  const double rows = (double)n / num_segments;
+  const double rounds = std::ceil(rows / (kWaveRows * kWave));
+  const double thousands = (double)m / 1024.0;
+  // Lists beyond 32 entries go through the vector-ALU scan otherwise: k = 33,
+  // 1,024 points 27 / 220, 16 x 4,096 316 / 468, 64 x 4,096 1,096 / 925.
   if (k > 32)
-    return here <= 400.0;
-  return here <= (k < 12 ? 0.55 : 0.9) * (24.0 + 12.0 * rounds);
+    return thousands * (1.0 + rounds) <= 400.0;
+  const double here =
+      26.0 + (num_segments > 1 ? 3.0 : 0.0) +
+      std::max(1.6 * rounds, thousands * (0.55 + 0.95 * rounds));
+  const int slices =
+      knn_lowd_config(d, k, n, m, num_segments, cosine).num_chunks;
+  const double scan = 37.0 + 0.8 * k +
+                      (4.3 + 0.16 * k) * rows / slices / 1024.0 +
+                      (slices > 1 ? 6.0 + 2.2 * k : 0.0) +
+                      (0.038 + 0.0025 * k) * 1e-6 * m * rows;
+  return here <= scan;
 }
 
 hipError_t launch_knn_wave(const SearchInput &in, int k, const DenseResult &out,

@@ -141,8 +141,9 @@ hipError_t launch_knn_lowd(const SearchInput &in, int k, bool cosine,
 // --- knn_wave.hip ------------------------------------------------------------
 
 // Small calls, one wave per query: fp32, up to 4 dimensions, Euclidean,
-// k <= 64, at most kCompactCountedQueries queries.  PCA_KNN_WAVE=0: never, 1:
-// whenever the shape fits.
+// k <= 64.  Any number of queries; beyond kCompactCountedQueries the
+// compaction counts the edges in a launch of its own.  PCA_KNN_WAVE=0: never,
+// 1: whenever the shape fits.
 bool knn_wave_supported(int n, int m, int d, int num_segments, int k,
                         bool cosine);
 hipError_t launch_knn_wave(const SearchInput &in, int k, const DenseResult &out,

@@ -80,3 +80,20 @@ def test_rows_without_a_distance(oracle):
     y[3, 0] = -np.inf
     for k in (3, 64):
         check(oracle, x, y, None, None, k)
+
+
+def test_graph_of_more_queries_than_the_compaction_adds_up(oracle):
+    # beyond 8,192 queries the edges are counted in a launch of their own
+    rng = np.random.default_rng(5)
+    sizes = rng.integers(1, 400, 60)
+    ptr = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    n = int(ptr[-1])
+    assert n > 8192
+    x = rng.integers(0, 6, (n, 3)).astype(np.float32)
+    got, _ = capi.knn_edges(dev(x), dev(x), dev(ptr), dev(ptr), 7,
+                            drop_self=True, x_first=True)
+    _, col, _ = oracle.knn_dense(x, x, ptr, ptr, 7, False, fma_mode=1)
+    col = col.reshape(n, 7)
+    keep = (col != -1) & (col != np.arange(n)[:, None])
+    rows = np.broadcast_to(np.arange(n)[:, None], (n, 7))[keep]
+    assert (got.cpu().numpy() == np.stack([col[keep], rows])).all()
