@@ -16,7 +16,23 @@
 // Bound by latency: ids, ~15 dependent probes of the searches, then a trip to
 // the L2 per eight rows, the eight rows of all lanes in flight together (sixteen
 // at a time measured the same: 38.8 / 39.9 us for 1,000 examples).
+//
+// The rule that takes a call here knows the mean length only, and of ids only
+// the number of examples an earlier call met, so an example may be of any
+// length.  Those of more than kShortRows rows are searched by the workgroups
+// that hold their queries, one example after the other: 512 rows at a time in
+// LDS, the distances of 64 rows x 64 queries of a wave by fp32 matrix
+// instructions.  Bound by that wave's chain -- operands from LDS, products,
+// gathered signs, the rows that pass one by one -- at one wave per SIMD: 12 ns
+// per row of the example (as plain fp32 instructions on broadcast rows the LDS
+// alone would take that).  Graphs of 1,000 examples of 35 rows and one of 2,000
+// / 20,000 / 60,000, r = 2, us a call (query after query by waves / so / the
+// matrix-core kernel with its pointers and plan): 381 / 4,113 / 12,250, now 82 /
+// 275 / 681, 232 / 354 / 785.  Only where few short examples share a call with
+// a long one that kernel is the faster one still: 300 of 35 rows and one of
+// 20,000 275 / 226.
 #include "device_utils.hpp"
+#include "knn_lowd_impl.hpp"
 #include "launchers.hpp"
 
 #include <cstdlib>
@@ -40,9 +56,16 @@ struct RadiusShortParams {
 };
 
 constexpr int kShortRound = 8; // rows per lane and round
-// a wave that meets a longer example takes its queries one after the other,
-// 64 rows at a time
-constexpr int kShortRows = 1024;
+// longest example a lane goes through by itself: 1,000 examples of 5 - 240
+// rows, r = 5, take 77 us a call, with those beyond 192 rows searched by their
+// workgroups 96 us; one of 1,000 rows among 1,000 of 35 takes 135 us by lanes
+// and 72 us by workgroups
+constexpr int kShortRows = 256;
+constexpr int kLongTile = 512; // rows of a longer one in LDS
+// start values of the filter's sum for rows and queries beyond its range
+constexpr float kLongNever = 3e38f;
+constexpr float kLongAlways = -3e38f;
+typedef float long_acc_t __attribute__((ext_vector_type(16)));
 
 template <int D>
 __device__ __forceinline__ float short_distance(const float (&row)[D],
@@ -61,7 +84,13 @@ template <int D>
 __global__ __launch_bounds__(kBlock) void radius_short_kernel(
     RadiusShortParams p) {
   constexpr int U = kShortRound;
-  __shared__ long long sums[kBlock / kWave];
+  constexpr int W = kBlock / kWave;
+  constexpr int K = D <= 3 ? 4 : 6;            // x .. | |x|^2 | 0
+  constexpr int AT_W = D;                      // plane of |x|^2
+  constexpr int STRIDE = kLongTile + 32;       // (both halves: other banks)
+  __shared__ float tile[K][STRIDE];
+  __shared__ int waiting_rows[W][2];
+  __shared__ long long sums[W];
   static_assert(kBlock == kCompactBlockQueries, "a block writes its own sum");
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -112,67 +141,227 @@ __global__ __launch_bounds__(kBlock) void radius_short_kernel(
   for (int c = 0; c < D; ++c)
     yq[c] = p.y[(size_t)q_in * D + c];
   int count = 0;
-  int longest = len;
+  // (no distance is below an r^2 of 0 or NaN, nor from a query that is not
+  // finite)
+  bool finite_query = true;
+#pragma unroll
+  for (int c = 0; c < D; ++c)
+    finite_query = finite_query && __builtin_fabsf(yq[c]) < __builtin_inff();
+  bool is_long = len > kShortRows && finite_query && p.r2 > 0.0f;
+  const int own = len > kShortRows ? 0 : len;
+  int longest = own;
 #pragma unroll
   for (int sh = 1; sh < kWave; sh <<= 1)
     longest = max(longest, __shfl_xor(longest, sh));
-  if (longest <= kShortRows) {
-    int *slot = p.out_idx + (size_t)q_in * p.slots;
-    for (int i0 = 0; i0 < longest; i0 += U) {
-      if (!__any(i0 < len && count < p.slots))
-        break;
-      float row[U][D];
+  int *slot = p.out_idx + (size_t)q_in * p.slots;
+  for (int i0 = 0; i0 < longest; i0 += U) {
+    if (!__any(i0 < own && count < p.slots))
+      break;
+    float row[U][D];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int at = min(x_begin + i0 + u, p.n - 1);
+    for (int u = 0; u < U; ++u) {
+      const int at = min(x_begin + i0 + u, p.n - 1);
 #pragma unroll
-        for (int c = 0; c < D; ++c)
-          row[u][c] = p.x[(size_t)at * D + c];
+      for (int c = 0; c < D; ++c)
+        row[u][c] = p.x[(size_t)at * D + c];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int g = x_begin + i0 + u;
+      const bool hit = short_distance<D>(row[u], yq) < p.r2 &&
+                       i0 + u < own && count < p.slots &&
+                       !(p.ignore_same_index && g == q);
+      if (hit) {
+        slot[count] = g;
+        ++count;
       }
+    }
+  }
+
+  // ---- long examples ----------------------------------------------------------
+  // With t = |x|^2 - 2 x.y + c, c = |y|^2 - r^2 - margin, from fp32 matrix
+  // instructions: a row with a computed distance below r^2 has t < 0.  (Such a
+  // row has |x|^2 <= 2 |y|^2 + 2 r^2 (1 + 2^-20); the roundings of |x|^2, |y|^2,
+  // c and of a sum of six terms are each within 2^-24 of |x|^2 + 2 |x| |y| +
+  // |y|^2 + r^2, 72 |y|^2 + 60 r^2 of them in all; the margin holds 128 of both,
+  // and 1e-36 for what is flushed to zero.)  Whether a row with t < 0 is a
+  // neighbour is decided by the distance.
+  if (__syncthreads_or(is_long)) {
+    const int wave = tid / kWave;
+    const int half = lane >> 5;
+    const int col = lane & 31;
+    // the queries of both halves of the wave: B operands and start values
+    float yb[2][K / 2], start[2];
+    {
+      float sq = 0.0f;
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int g = x_begin + i0 + u;
-        const bool hit = short_distance<D>(row[u], yq) < p.r2 &&
-                         i0 + u < len && count < p.slots &&
-                         !(p.ignore_same_index && g == q);
-        if (hit) {
-          slot[count] = g;
-          ++count;
+      for (int c = 0; c < D; ++c)
+        sq = __builtin_fmaf(yq[c], yq[c], sq);
+      // (a query beyond 1e30, or such an r^2: every row is looked at)
+      const bool moderate = sq <= kFilterNormLimit && p.r2 <= kFilterNormLimit;
+      float operand[K];
+#pragma unroll
+      for (int c = 0; c < K; ++c)
+        operand[c] = c < D ? (moderate ? -2.0f * yq[c < D ? c : 0] : 0.0f)
+                           : (c == AT_W ? 1.0f : 0.0f);
+      const float margin =
+          __builtin_fmaf(7.62939453125e-06f, sq + p.r2, 1e-36f);
+      const float begin = moderate ? (sq - p.r2) - margin : kLongAlways;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        start[s] = __shfl(begin, 32 * s + col);
+#pragma unroll
+        for (int i = 0; i < K / 2; ++i) {
+          const float lower = __shfl(operand[2 * i], 32 * s + col);
+          const float upper = __shfl(operand[2 * i + 1], 32 * s + col);
+          yb[s][i] = half ? upper : lower;
         }
       }
     }
-  } else {
-    for (int l = 0; l < kWave; ++l) {
-      const int rows = __builtin_amdgcn_readlane(len, l);
-      if (rows == 0)
-        continue;
-      const int first = __builtin_amdgcn_readlane(x_begin, l);
-      const int own = __builtin_amdgcn_readlane(q, l);
-      float of[D];
-#pragma unroll
-      for (int c = 0; c < D; ++c)
-        of[c] = __uint_as_float((uint32_t)__builtin_amdgcn_readlane(
-            (int)__float_as_uint(yq[c]), l));
-      int found = 0;
-      for (int i0 = 0; i0 < rows && found < p.slots; i0 += kWave) {
-        const int g = first + i0 + lane;
-        float row[D];
-#pragma unroll
-        for (int c = 0; c < D; ++c)
-          row[c] = p.x[(size_t)min(g, p.n - 1) * D + c];
-        const bool hit = short_distance<D>(row, of) < p.r2 &&
-                         i0 + lane < rows &&
-                         !(p.ignore_same_index && g == own);
-        const uint64_t hits = __ballot(hit);
-        const int at = found + (int)__builtin_amdgcn_mbcnt_hi(
-                                   (uint32_t)(hits >> 32),
-                                   __builtin_amdgcn_mbcnt_lo((uint32_t)hits, 0u));
-        if (hit && at < p.slots)
-          p.out_idx[(size_t)own * p.slots + at] = g;
-        found += __builtin_popcountll(hits);
+    for (;;) {
+      // the example of the workgroup's first query that waits (every wave has
+      // read the one before: at least one barrier per tile lies between)
+      const uint64_t waits = __ballot(is_long);
+      const int first = waits != 0 ? (int)__builtin_ctzll(waits) : 0;
+      if (lane == first) {
+        waiting_rows[wave][0] = x_begin;
+        waiting_rows[wave][1] = is_long ? x_end : x_begin;
       }
-      found = min(found, p.slots);
-      count = lane == l ? found : count;
+      __syncthreads();
+      int begin = 0, end = 0;
+#pragma unroll
+      for (int w = W - 1; w >= 0; --w)
+        if (waiting_rows[w][1] > waiting_rows[w][0]) {
+          begin = __builtin_amdgcn_readfirstlane(waiting_rows[w][0]);
+          end = __builtin_amdgcn_readfirstlane(waiting_rows[w][1]);
+        }
+      if (end <= begin)
+        break;
+      const bool mine = is_long && x_begin == begin && x_end == end;
+      is_long = is_long && !mine;
+      // a tile waits in registers while the one before it is searched
+      constexpr int PT = kLongTile / kBlock;
+      float staged[PT][D];
+      auto load = [&](int base) {
+#pragma unroll
+        for (int i = 0; i < PT; ++i) {
+          const int at = min(base + i * kBlock + tid, end - 1);
+#pragma unroll
+          for (int c = 0; c < D; ++c)
+            staged[i][c] = p.x[(size_t)at * D + c];
+        }
+      };
+      load(begin);
+      for (int base = begin; base < end; base += kLongTile) {
+        // (also: nobody reads the tile before any more)
+        if (!__syncthreads_or(mine && count < p.slots))
+          break;
+#pragma unroll
+        for (int i = 0; i < PT; ++i) {
+          const int at = i * kBlock + tid;
+          float sq = 0.0f;
+          bool finite = true;
+#pragma unroll
+          for (int c = 0; c < D; ++c) {
+            sq = __builtin_fmaf(staged[i][c], staged[i][c], sq);
+            finite = finite && __builtin_fabsf(staged[i][c]) < __builtin_inff();
+          }
+          // (rows that are not finite have no distance below r^2; those
+          // beyond 1e30 are always looked at, where they are)
+          const bool moderate = sq <= kFilterNormLimit;
+#pragma unroll
+          for (int c = 0; c < D; ++c)
+            tile[c][at] = moderate ? staged[i][c] : 0.0f;
+          tile[AT_W][at] = base + at >= end || !finite ? kLongNever
+                           : moderate                  ? sq
+                                                       : kLongAlways;
+#pragma unroll
+          for (int c = AT_W + 1; c < K; ++c)
+            tile[c][at] = 0.0f;
+        }
+        __syncthreads();
+        if (base + kLongTile < end)
+          load(base + kLongTile);
+        if (!__any(mine && count < p.slots))
+          continue;
+        // 64 rows at a time: the chains of four products fill each other's
+        // waits
+        const int steps = (min(kLongTile, end - base) + 63) / 64;
+        for (int step = 0; step < steps; ++step) {
+          uint32_t pending[2];
+          {
+            long_acc_t t[2][2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+              for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                  t[h][s][v] = start[s];
+#pragma unroll
+            for (int i = 0; i < K / 2; ++i)
+#pragma unroll
+              for (int h = 0; h < 2; ++h) {
+                const float a = tile[2 * i + half][step * 64 + 32 * h + col];
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+                  t[h][s] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                      a, yb[s][i], t[h][s], 0, 0, 0);
+              }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              uint32_t rows_of[2];
+#pragma unroll
+              for (int s = 0; s < 2; ++s) {
+                uint32_t mask = 0;
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                  mask = __builtin_amdgcn_alignbit(
+                      mask, __float_as_uint(t[h][s][v]), 31);
+                // the rows of the step in order, the first one in the highest
+                // bit: nibbles of the lower and of the upper lane in turn
+                uint32_t spread = (mask | (mask << 8)) & 0x00ff00ffu;
+                spread = (spread | (spread << 4)) & 0x0f0f0f0fu;
+                spread <<= half == 0 ? 4 : 0;
+                const auto both = __builtin_amdgcn_permlane32_swap(
+                    spread, spread, false, false);
+                rows_of[s] = both[0] | both[1];
+              }
+              pending[h] = half ? rows_of[1] : rows_of[0];
+            }
+          }
+          if (!mine || count >= p.slots)
+            pending[0] = pending[1] = 0;
+          while (__any((pending[0] | pending[1]) != 0)) {
+            const bool later = pending[0] == 0;
+            const uint32_t some = later ? pending[1] : pending[0];
+            const int v = __builtin_clz(some | 1u);
+            const int j = step * 64 + (later ? 32 : 0) + v;
+            const int g = base + j;
+            float row[D];
+#pragma unroll
+            for (int c = 0; c < D; ++c)
+              row[c] = tile[c][j];
+            if (tile[AT_W][j] == kLongAlways) {
+#pragma unroll
+              for (int c = 0; c < D; ++c)
+                row[c] = p.x[(size_t)min(g, end - 1) * D + c];
+            }
+            const bool hit = some != 0 && g < end &&
+                             short_distance<D>(row, yq) < p.r2 &&
+                             !(p.ignore_same_index && g == q);
+            const uint32_t rest = some & ~(0x80000000u >> v);
+            pending[0] = later ? 0 : rest;
+            pending[1] = later ? rest : pending[1];
+            if (hit) {
+              slot[count] = g;
+              ++count;
+              if (count >= p.slots)
+                pending[0] = pending[1] = 0;
+            }
+          }
+        }
+      }
     }
   }
 
@@ -191,7 +380,7 @@ __global__ __launch_bounds__(kBlock) void radius_short_kernel(
   if (tid == 0) {
     long long all = 0;
 #pragma unroll
-    for (int w = 0; w < kBlock / kWave; ++w)
+    for (int w = 0; w < W; ++w)
       all += sums[w];
     p.edge_sums[blockIdx.x] = (unsigned long long)all;
   }

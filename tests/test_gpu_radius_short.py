@@ -65,6 +65,64 @@ def test_one_long_example(oracle, longest):
         check(oracle, x, x, ptr, ptr, r, limit, ignore_same=True)
 
 
+# around the length up to which a lane searches by itself, and around one and
+# several tiles of 512 rows; short ones in between, queries of several long
+# examples in one workgroup, far fewer queries than rows
+@pytest.mark.parametrize("d", [1, 2, 3, 4])
+@pytest.mark.parametrize("sizes", [
+    [256, 257, 3, 511, 512, 513], [40, 300, 0, 300, 1, 290, 7],
+    [1, 1535, 64, 1537], [2300]])
+def test_long_examples(oracle, d, sizes):
+    rng = np.random.default_rng(d + len(sizes))
+    ptr = pointers(sizes)
+    x = rng.random((ptr[-1], d)).astype(np.float32)
+    for r, limit in ((0.1, 32), (0.02, 5), (3.0, 70)):
+        check(oracle, x, x, ptr, ptr, r, limit, ignore_same=limit == 32)
+    few = pointers([min(n, 11) for n in sizes])
+    y = rng.random((few[-1], d)).astype(np.float32)
+    check(oracle, x, y, ptr, few, 0.2, 16)
+    grid = rng.integers(0, 5, x.shape).astype(np.float32)
+    check(oracle, grid, grid, ptr, ptr, 1.0, 1000)  # (distances of r^2 itself)
+    check(oracle, grid * 3e4 + 1e6, grid * 3e4 + 1e6, ptr, ptr, 4e4, 9)
+
+
+@pytest.mark.parametrize("scale", [1e-25, 1e-12, 1e3, 1e14, 3e17])
+def test_long_example_at_the_edges_of_fp32(oracle, scale):
+    rng = np.random.default_rng(8)
+    ptr = pointers([5, 900, 30])
+    x = (rng.standard_normal((ptr[-1], 3)) * scale).astype(np.float32)
+    x[100], x[150, 1], x[200], x[250, 2] = np.nan, np.inf, 2e38, -np.inf
+    x[300:340] = np.float32(3e15)  # |x|^2 beyond 1e30
+    x[400] = x[401] = np.float32(1e19)
+    for r in (0.3 * scale, 3 * scale, np.inf, 0.0):
+        check(oracle, x, x, ptr, ptr, r, 20)
+
+
+def test_time_of_one_long_example(monkeypatch):
+    """Not much more than the kernel that gives an example its workgroups
+    (it was 18 times that; the bound leaves room for noise)."""
+    sizes = [35] * 300 + [20000]
+    ids = dev(ids_of(pointers(sizes)))
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.rand(sum(sizes), 3, generator=g, device="cuda") * 58
+
+    def least():
+        times = []
+        for _ in range(8):
+            begin, end = (torch.cuda.Event(enable_timing=True)
+                          for _ in range(2))
+            begin.record()
+            pca.radius_graph(x, 2.0, ids)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+
+    here = least()
+    monkeypatch.setenv("PCA_RADIUS_SHORT", "0")
+    assert here < 4 * least()
+
+
 def test_rows_without_a_distance(oracle):
     rng = np.random.default_rng(4)
     ptr = pointers([9, 30, 64, 17])
