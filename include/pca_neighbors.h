@@ -440,7 +440,8 @@ int pca_nearest_host(const void *x, const void *y, const int64_t *ptr_x,
  *            (it selects the kernel: fp32 points of up to 4 dimensions in
  *            segments of up to 16,384 rows are sampled on chip, larger ones
  *            of up to 3 dimensions from rows in curve order, everything else
- *            row by row), or 0 = unknown (row by row).
+ *            row by row), or 0 = unknown (row by row; also the faster choice
+ *            for a handful of samples from larger segments).
  * A stream that is being captured into a graph may be used: segments beyond
  * 16,384 rows are then sampled row by row (their sort clears its buffers with
  * memset nodes).

@@ -22,9 +22,10 @@
 // workgroup's (a step that several workgroups share costs two trips through
 // the L2).  Up to 1,024 rows of up to 4 dimensions fps_reg_kernel looks at
 // every row in every step, from registers.  Beyond that most rows are left
-// alone (see "rows in buckets" below): fps_lds_kernel keeps up to 8,192 rows in
-// LDS, fps_bucket_kernel up to 16,384 in registers, fps_stream_kernel any
-// number in memory (up to 3 dimensions).  fps_any_kernel (any size, dimension
+// alone (see "rows in buckets" below) where more than a few hundred samples
+// repay the sort: fps_lds_kernel keeps up to 8,192 rows in LDS,
+// fps_bucket_kernel up to 16,384 in registers, fps_stream_kernel any number in
+// memory (up to 3 dimensions).  fps_any_kernel (any size, dimension
 // and element type) streams the rows and a `dist` array from memory.
 #include "device_utils.hpp"
 #include "launchers.hpp"
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(kFpsThreads) void fps_any_kernel(
   }
 }
 
-// ---- fp32, up to 4 dimensions, up to 1,024 rows per example -------------------
+// ---- fp32, up to 4 dimensions: every row in every step -------------------------
 
 // T threads hold P rows each.  With T = 256 S, thread t has the rows
 // t / S + 256 * ((t % S) * P + i), i < P, of its example; a single wave
@@ -251,7 +252,7 @@ __global__ __launch_bounds__(kFpsThreads) void fps_any_kernel(
 // measured fastest for the row count.  The single wave needs neither the
 // hand-over through shared memory nor a barrier.
 template <int DIM, int P, int T>
-__global__ __launch_bounds__(T) void fps_reg_kernel(
+__device__ __forceinline__ void fps_every_row(
     const float *__restrict__ src, const int64_t *__restrict__ ptr,
     const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
     int d, int64_t *__restrict__ out) {
@@ -447,6 +448,14 @@ __global__ __launch_bounds__(T) void fps_reg_kernel(
     for (int c = 0; c < DIM; ++c)
       asm volatile("" : "+v"(cur[c]));
   }
+}
+
+template <int DIM, int P, int T>
+__global__ __launch_bounds__(T) void fps_reg_kernel(
+    const float *__restrict__ src, const int64_t *__restrict__ ptr,
+    const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
+    int d, int64_t *__restrict__ out) {
+  fps_every_row<DIM, P, T>(src, ptr, out_ptr, start, d, out);
 }
 
 // ---- fp32, up to 4 dimensions: rows in buckets, most of them left alone -------
@@ -654,6 +663,41 @@ fps_curve_order(const float *__restrict__ rows, int count, int d,
   }
 }
 
+// Putting the rows in buckets has to pay: with fewer samples than this every
+// row is looked at instead.  Kernel, us, all rows / buckets, per example 1, 128,
+// 256, 512 samples: 16 x 2,048 rows 14 / 33, 85 / 99, 159 / 162, 306 / 292;
+// 16 x 4,096 14 / 50, 97 / 127, 181 / 193, 349 / 319; 16 x 8,192 15 / 85,
+// 116 / 170, 217 / 243, 424 / 383; 8 x 16,384 16 / 155, 178 / 296, 342 / 398,
+// 669 / 584; 16 x 4,096 of 4 dimensions 14 / 57, 105 / 158, 196 / 240, 384 / 386.
+constexpr int fps_few(int dim) { return dim > 3 ? 480 : 340; }
+
+// Such an example by a workgroup of 1,024 threads.  Up to 8,192 rows half of
+// them hold the rows, which leaves fewer results to hand over per step; the
+// others only come to the barriers of fps_every_row (one before the first step
+// and one per step; 16 x 2,048 rows, 128 samples: 85 us, by all threads 111).
+template <int DIM, int CAP, int T>
+__device__ __forceinline__ void fps_few_samples(
+    const float *__restrict__ src, const int64_t *__restrict__ ptr,
+    const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
+    int d, int64_t *__restrict__ out, int count, int samples) {
+  static_assert(T == 1024 && (CAP == 4096 || CAP == 8192 || CAP == 16384),
+                "rows per thread");
+  if constexpr (CAP == 16384) {
+    fps_every_row<DIM, 16, T>(src, ptr, out_ptr, start, d, out);
+  } else {
+    if (threadIdx.x >= T / 2) {
+      for (int m = 0; m < samples; ++m)
+        __syncthreads();
+      return;
+    }
+    if (CAP == 4096 && count <= 2048)
+      fps_every_row<DIM, 4, T / 2>(src, ptr, out_ptr, start, d, out);
+    else
+      fps_every_row<DIM, CAP / (T / 2), T / 2>(src, ptr, out_ptr, start, d,
+                                               out);
+  }
+}
+
 // Examples of up to 4,096 R rows: everything a step needs of a bucket -- its
 // box and its best row -- is in one lane of EVERY wave's registers (64 buckets
 // of 64 R rows), the rows and their running minima are in LDS.  All waves see
@@ -697,6 +741,11 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
   const int64_t o_end = out_ptr[b + 1];
   if (o_begin >= o_end)
     return;
+  if (o_end - o_begin < fps_few(DIM) || count <= 0) {
+    fps_few_samples<DIM, CAP, T>(src, ptr, out_ptr, start, d, out, count,
+                                 (int)(o_end - o_begin));
+    return;
+  }
   const float *rows = src + (size_t)start_idx * d;
   const int buckets = (count + kWave * R - 1) / (kWave * R);
 
@@ -803,6 +852,10 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
     return (int)__builtin_ctzll(who);
   };
   const int steps = (int)(o_end - o_begin);
+  // (where the loop stands in the 32-byte windows of instruction fetch moves a
+  // step by 3 %: 16 x 4,096 rows, 1,024 samples, every other place in
+  // turn 562, 576, 577 and 560 us, the last of which this is)
+  asm volatile(".p2align 5\n\t.fill 6, 4, 0xbf800000"); // s_nop 0
   for (int m = 1; m < steps; ++m) {
     const int par = m & 1;
     const bool passes =
@@ -931,6 +984,11 @@ __global__ __launch_bounds__(W *kWave) void fps_bucket_kernel(
   const int64_t o_end = out_ptr[b + 1];
   if (o_begin >= o_end)
     return;
+  if (o_end - o_begin < fps_few(DIM) || count <= 0) {
+    fps_few_samples<DIM, CAP, T>(src, ptr, out_ptr, start, d, out, count,
+                                 (int)(o_end - o_begin));
+    return;
+  }
   const float *rows = src + (size_t)start_idx * d;
 
   fps_curve_order<W, DIM, REL_BITS>(rows, count, d, keys, part);

@@ -158,6 +158,44 @@ def test_rows_out_of_reach_keep_their_place(oracle, rows, d, kind):
     assert (got == oracle.fps_op(x, ptr, share, start)).all()
 
 
+# one sample more or fewer decides whether every row is looked at (up to 339
+# samples, of 4 dimensions 479) or the rows go into buckets; examples on both
+# sides in one call
+@pytest.mark.parametrize("rows,d,few", [
+    (1025, 3, 339), (2048, 2, 339), (2049, 3, 339), (4096, 4, 479),
+    (4096, 1, 339), (4097, 3, 339), (8192, 3, 339), (4097, 4, 479),
+    (8193, 3, 339), (16384, 2, 339)])
+def test_few_samples_and_many(oracle, rows, d, few):
+    rng = np.random.default_rng(rows + d)
+    ptr = np.cumsum([0, rows, 7, rows, rows // 2, rows]).astype(np.int64)
+    for grid in (False, True):
+        x = rng.standard_normal((ptr[-1], d)).astype(np.float32)
+        if grid:
+            x = rng.integers(0, 6, x.shape).astype(np.float32)
+        share = np.array([few / rows, 1.0, (few + 1) / rows, 0.01,
+                          1.0 / rows]).astype(np.float32)
+        start = np.array([rows - 1, 6, 0, 1, 5], dtype=np.int64)
+        got = gpu_fps(oracle, x, ptr, share, start)
+        assert (got == oracle.fps_op(x, ptr, share, start)).all()
+
+
+@pytest.mark.parametrize("rows,samples", [(16385, 8), (16385, 9), (16384, 8),
+                                          (60000, 3), (60000, 4), (140000, 1)])
+def test_a_handful_of_samples_from_large_examples(oracle, rows, samples):
+    rng = np.random.default_rng(rows)
+    x = rng.standard_normal((2 * rows, 3)).astype(np.float32)
+    ptr = np.array([0, rows, 2 * rows], dtype=np.int64)
+    ratio = (samples - 0.5) / rows
+    want = oracle.fps_op(x, ptr, ratio)
+    ids = torch.arange(2, device=DEV).repeat_interleave(rows)
+    got = pca.fps(dev(x), ids, ratio, random_start=False)
+    assert (got.cpu().numpy() == want).all()
+    got = pca.fps(dev(x), ptr=dev(ptr), ratio=ratio, random_start=False)
+    assert (got.cpu().numpy() == want).all()
+    one = pca.fps(dev(x[:rows]), None, ratio, random_start=False)
+    assert (one.cpu().numpy() == want[:samples]).all()
+
+
 def test_captured_into_a_graph(oracle):
     """While its stream is being captured the search does without the sort of
     the large examples; every replay samples the same rows."""
