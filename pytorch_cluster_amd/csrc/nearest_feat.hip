@@ -27,11 +27,11 @@ __global__ __launch_bounds__(kBlock) void nearest_feat_rows_kernel(
     NearestFeatGlobals *__restrict__ globals) {
   constexpr int W = kBlock / kWave;
   __shared__ unsigned s_bits[W], s_rows[W];
-  __shared__ double s_sum[W];
+  __shared__ double s_sum[W], s_log[W];
   const int tid = threadIdx.x;
   const int part = tid & 15;
   unsigned bits = 0, rows = 0;
-  double sum = 0.0;
+  double sum = 0.0, logs = 0.0;
   for (int row = blockIdx.x * (kBlock / 16) + (tid >> 4); row < n;
        row += gridDim.x * (kBlock / 16)) {
     const float *p = x + (size_t)row * d;
@@ -51,9 +51,10 @@ __global__ __launch_bounds__(kBlock) void nearest_feat_rows_kernel(
     const bool moderate = finite && sq <= kFilterNormLimit;
     if (part == 0) {
       weight[row] = moderate ? sq : finite ? -1.0f : -2.0f;
-      if (moderate) {
+      if (moderate && sq > 0.0f) {
         bits = max(bits, top);
         sum += (double)sq;
+        logs += (double)__builtin_log2f(sq);
         ++rows;
       }
     }
@@ -63,11 +64,13 @@ __global__ __launch_bounds__(kBlock) void nearest_feat_rows_kernel(
     bits = max(bits, (unsigned)__shfl_xor((int)bits, sh));
     rows += (unsigned)__shfl_xor((int)rows, sh);
     sum += __shfl_xor(sum, sh);
+    logs += __shfl_xor(logs, sh);
   }
   if ((tid & (kWave - 1)) == 0) {
     s_bits[tid / kWave] = bits;
     s_rows[tid / kWave] = rows;
     s_sum[tid / kWave] = sum;
+    s_log[tid / kWave] = logs;
   }
   __syncthreads();
   if (tid == 0) {
@@ -76,11 +79,13 @@ __global__ __launch_bounds__(kBlock) void nearest_feat_rows_kernel(
       bits = max(bits, s_bits[w]);
       rows += s_rows[w];
       sum += s_sum[w];
+      logs += s_log[w];
     }
     if (rows != 0) {
       atomicMax(&globals->max_bits, bits);
       atomicAdd(&globals->rows, rows);
       atomicAdd(&globals->sum_sq, sum);
+      atomicAdd(&globals->sum_log, logs);
     }
   }
 }
@@ -118,6 +123,7 @@ __global__ __launch_bounds__(kPlanThreads) void nearest_feat_plan_kernel(
     globals->max_bits = 0;
     globals->rows = 0;
     globals->sum_sq = 0.0;
+    globals->sum_log = 0.0;
   }
   plan_segments(ptr_y, m, num_segments, per_item, work_start, partial);
 }

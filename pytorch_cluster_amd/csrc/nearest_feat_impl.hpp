@@ -16,8 +16,10 @@
 //   * the accumulation: d + 16 terms, each within 2^-22 of a running magnitude
 //     below |kappa| |a|^2 + 1.01 |a| |b'|;
 //   * |a| |b'| <= l |a|^2 + |b|^2 / l with l = B / A, B the largest |b| of the
-//     workgroup and A the root mean square |a|, and |a| <= (|a|^2 / A + A) / 2,
-// so that  kappa = r (1 - delta) - eps l - 2^-15 sqrt(d) / A  and
+//     workgroup and A a typical |a|, and |a| <= (|a|^2 / A + A) / 2,
+// (any A > 0 will do; it is the root mean square of the |a|, or twice their
+// geometric mean where large rows bring the mean square above that) so that
+//     kappa = r (1 - delta) - eps l - 2^-15 sqrt(d) / A  and
 //     C = eps |b|^2 / l + 2^-15 sqrt(d) A + 2^-13 sqrt(d) |b| + d 2^-27
 // (each sqrt term times 1.01), eps = 2^-10 + (d + 20) 2^-21,
 // delta = (d + 20) 2^-21.
@@ -31,16 +33,31 @@
 // long from 48 components on.  After 4,096 rows the four rows of a query's
 // smallest minimum are evaluated exactly; their distance D gives the cut
 // below which s has to lie for a row to come before them; of the other
-// minima kept, those below the cut are evaluated too.  Only if even the third
-// lies below it (four fours of rows within the rounding margin of the nearest
-// one: duplicates, rows much larger than the others) there may be candidates
-// that were not kept: the workgroup then goes through these 4,096 rows again
-// and evaluates whatever lies below the cut.
+// minima kept, those below the cut are evaluated too.  Only if at the end of
+// the example a third minimum lies below the final cut (four fours of rows
+// within the rounding margin of the nearest one: duplicates, rows far from the
+// origin) there may be candidates that were not kept: the workgroup then goes
+// through such 4,096 rows again and evaluates whatever lies below the cut.
+//
+// One row or query far larger than the others must not set the scale, A or l for
+// all.  Rows of a norm beyond 4,096 times the geometric mean take part with
+// zeros for operands and s = r |a|^2 / 4 - B^2 / r, a lower bound as long as
+// |b| <= r |a| / 2 (otherwise they are always looked at).  Queries with a
+// component of 2^12 times the workgroup's mean are searched exactly, and where
+// the largest of the others is far beyond an ordinary one, l lies between the
+// two.  Calls of 100,000 queries x 4,096 rows x 64, 135 us: with one row a
+// million times the others 18,050 us without the limit, 162 with it; with every
+// thousandth query ten thousand times the others 4,660, now 162.  50,000 x
+// 8,192 x 128: the candidates of all scans but the one with the nearest row were
+// searched for again before its distance was known; 300 -> 240 us, 10 standard
+// deviations from the origin 1,004 -> 254.  What is left: an entry that occurs
+// 16 times or more brings the second pass to every query (654 us; the
+// kernel of knn_mfma_impl.hpp 553).
 //
 // Rows of x with a component that is not finite never qualify (their distance
 // is not below 1e38); finite ones of |x|^2 > 1e30 enter with s = -1e37, always
-// looked at.  Queries likewise: not finite, no candidate; too large, every
-// candidate is evaluated.
+// looked at.  Queries likewise: not finite, no candidate; |y|^2 > 1e30, searched
+// exactly.
 //
 // Mapping: a workgroup owns 4 waves x S x 32 queries of one segment; the query
 // operands stay in registers, packed rows of x (2 NB units of 16 bytes, an odd
@@ -70,10 +87,18 @@ constexpr float kNfNothing = 1.7e38f;  // s of a row that is none
 constexpr float kNfAlways = -1e37f;    // s of a row that is always looked at
 constexpr float kNfCutLimit = 1e38f;
 
+// What the rows' operands are made with.
+struct NfRows {
+  float typical;  // the A of the bound, unscaled
+  float limit_sq; // rows of a larger squared norm have no operands
+  float scale;
+};
 struct NearestFeatGlobals {
   unsigned max_bits; // largest |component| of the moderate rows of x
-  unsigned rows;     // moderate rows of x
+  unsigned rows;     // moderate rows of x that are not zero
   double sum_sq;     // of their squared norms
+  double sum_log;    // of log2 of those
+  NfRows rows_of_x;  // what follows from these (by the pack kernel)
 };
 
 struct NearestFeatParams {
@@ -96,6 +121,33 @@ __device__ __forceinline__ float nf_scale(unsigned max_bits) {
   int e = 137 - (int)((max_bits >> 23) & 0xffu);
   e = e > 100 ? 100 : (e < -100 ? -100 : e);
   return __uint_as_float((uint32_t)(e + 127) << 23);
+}
+
+__device__ __forceinline__ float nf_uniform(float v) {
+  return __uint_as_float(
+      (uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(v)));
+}
+__device__ __forceinline__ double nf_uniform(double v) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
+constexpr float kNfLargeRow = 4096.0f;
+constexpr int kNfLargeExponents = 12;
+__device__ __forceinline__ float nf_mean_norm(double sum_log, unsigned rows) {
+  return rows != 0 ? __builtin_exp2f((float)(0.5 * sum_log / (double)rows))
+                   : 1.0f;
+}
+__device__ __forceinline__ NfRows nf_rows(const NearestFeatGlobals *g) {
+  NfRows r;
+  const float mean = nf_mean_norm(g->sum_log, g->rows);
+  const float rms =
+      g->rows != 0 ? (float)__builtin_sqrt(g->sum_sq / (double)g->rows) : 1.0f;
+  r.typical = __builtin_fminf(rms, 2.0f * mean);
+  const float limit = __builtin_fminf(mean * kNfLargeRow, 1e18f);
+  r.limit_sq = limit * limit;
+  r.scale = nf_scale(min(g->max_bits, __float_as_uint(limit)));
+  return r;
 }
 
 __device__ __forceinline__ uint32_t nf_half(float v) {
@@ -189,8 +241,12 @@ nearest_feat_kernel(NearestFeatParams p) {
   static_assert(UNITS % kWave == 0, "whole pieces");
   __shared__ __attribute__((aligned(16))) uint4 tile_rows[2][UNITS];
   __shared__ __attribute__((aligned(16))) float tile_weight[2][TR];
-  __shared__ unsigned wave_bits[WAVES];
+  __shared__ unsigned wave_top[WAVES];
+  __shared__ unsigned wave_queries[WAVES];
   __shared__ float wave_norm[WAVES];
+  __shared__ unsigned long long wave_scans[WAVES];
+  __shared__ unsigned long long wave_best[2][WAVES];
+  __shared__ uint32_t alone[WAVES][S]; // queries searched exactly
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -212,13 +268,19 @@ nearest_feat_kernel(NearestFeatParams p) {
 
   // ---- queries ------------------------------------------------------------
   // 0: no query, or one no candidate is close enough to; 1: through the
-  // filter; 2: every candidate is evaluated
+  // filter; 2: searched exactly
   int kind[S];
+  uint32_t top_bits[S]; // largest component
   unsigned bits = 0;
+  // exponents of the queries that are not zero, added up, from bit 16 on their
+  // number, from bit 24 on that of the queries of the last kind (of a wave)
+  unsigned queries = 0;
+  static_assert(S <= 4, "sums over 128 queries");
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     const int q = q0 + s * 32;
     kind[s] = 0;
+    top_bits[s] = 0;
     if (q < y_end) {
       const float *row = p.y + (size_t)q * d;
       float sq = 0.0f;
@@ -236,19 +298,60 @@ nearest_feat_kernel(NearestFeatParams p) {
       sq += __shfl_xor(sq, 32);
       top = max(top, (unsigned)__shfl_xor((int)top, 32));
       kind[s] = top >= 0x7f800000u ? 0 : sq <= kFilterNormLimit ? 1 : 2;
-      if (kind[s] == 1)
+      top_bits[s] = top;
+      if (kind[s] == 1) {
         bits = max(bits, top);
+        queries += top != 0 ? (top >> 23) + 0x10000u : 0u;
+      } else if (kind[s] == 2) {
+        queries += 0x1000000u;
+      }
     }
   }
 #pragma unroll
-  for (int sh = 1; sh < 32; sh <<= 1)
+  for (int sh = 1; sh < 32; sh <<= 1) {
     bits = max(bits, (unsigned)__shfl_xor((int)bits, sh));
-  if (lane == 0)
-    wave_bits[wave] = bits;
+    queries += (unsigned)__shfl_xor((int)queries, sh);
+  }
+  if (lane == 0) {
+    wave_top[wave] = bits;
+    wave_queries[wave] = queries;
+  }
   __syncthreads();
+  unsigned exponents = 0, counted = 0;
+  bool any_alone = false;
 #pragma unroll
-  for (int w = 0; w < WAVES; ++w)
-    bits = max(bits, wave_bits[w]);
+  for (int w = 0; w < WAVES; ++w) {
+    bits = max(bits, wave_top[w]);
+    exponents += wave_queries[w] & 0xffffu;
+    counted += (wave_queries[w] >> 16) & 0xffu;
+    any_alone = any_alone || (wave_queries[w] >> 24) != 0;
+  }
+  // the mean exponent of the largest components
+  const int mean_exponent =
+      counted != 0 ? (int)((float)exponents / (float)counted) : 127;
+  if ((int)(bits >> 23) > mean_exponent + kNfLargeExponents) {
+    // a few queries far beyond the others' range (the same in all threads)
+    any_alone = true;
+    __syncthreads();
+    bits = 0;
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (kind[s] == 1) {
+        if ((int)(top_bits[s] >> 23) > mean_exponent + kNfLargeExponents)
+          kind[s] = 2;
+        else
+          bits = max(bits, top_bits[s]);
+      }
+#pragma unroll
+    for (int sh = 1; sh < 32; sh <<= 1)
+      bits = max(bits, (unsigned)__shfl_xor((int)bits, sh));
+    if (lane == 0)
+      wave_top[wave] = bits;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+      bits = max(bits, wave_top[w]);
+  }
   const float s_q = nf_scale(bits);
 
   nf_f16x8_t yb[S][NB];
@@ -285,32 +388,46 @@ nearest_feat_kernel(NearestFeatParams p) {
     top_sq = __builtin_fmaxf(top_sq, wave_norm[w]);
 
   // ---- constants of the bound ------------------------------------------------
-  const float s_c = nf_scale(p.globals->max_bits);
-  const double scale2 = (double)s_c * (double)s_q;
+  // (the same in every lane: kept in scalar registers)
+  const NfRows rows_of_x = p.globals->rows_of_x;
+  const float s_c = nf_uniform(rows_of_x.scale);
+  const float limit_sq = nf_uniform(rows_of_x.limit_sq);
+  const double scale2 = nf_uniform((double)s_c * (double)s_q);
   const double r = (double)s_q / (double)s_c;
-  double rms = 1.0;
+  double typical = (double)rows_of_x.typical * (double)s_c;
+  if (!(typical > 9.765625e-4 && typical < 1e7))
+    typical = 1.0;
+  // l: of the largest query, or of the geometric mean of it and of an ordinary
+  // one where it is much larger (2^e of the largest component and less times
+  // the root of d)
+  float largest = __builtin_sqrtf(top_sq) + 1e-3f;
   {
-    const unsigned rows = p.globals->rows;
-    const double mean = rows ? p.globals->sum_sq / rows : 0.0;
-    const double v = __builtin_sqrt(mean) * (double)s_c;
-    if (v > 9.765625e-4 && v < 1e7)
-      rms = v;
+    const float ordinary =
+        2.0f * __builtin_sqrtf((float)d) *
+        __uint_as_float((uint32_t)max(mean_exponent, 1) << 23) * s_q;
+    if (largest > ordinary)
+      largest = __builtin_sqrtf(largest) * __builtin_sqrtf(ordinary);
+    // (of queries whose components are all flushed: any number will do)
+    largest = __builtin_fmaxf(largest, 1e-3f);
   }
-  const double largest = __builtin_sqrt((double)top_sq) + 1e-3;
-  const double lambda = largest / rms;
+  const double lambda = (double)largest / typical;
   const double eps = 1.0 / 1024.0 + (double)(d + 20) / 2097152.0;
   const double delta = (double)(d + 20) / 2097152.0;
-  const double root_d = __builtin_sqrt((double)d) * 1.01;
+  const double root_d = nf_uniform(__builtin_sqrt((double)d) * 1.01);
   float kappa;
   {
     const double k = r * (1.0 - delta) - eps * lambda -
-                     root_d / (32768.0 * rms);
-    kappa = (float)(k < 1e30 ? k : 1e30);
+                     root_d / (32768.0 * typical);
+    kappa = nf_uniform((float)(k < 1e30 ? k : 1e30));
   }
   const double r_inv = (double)s_c / (double)s_q;
-  const double per_sq = eps / lambda - r_inv +
-                        (double)(d + 6) * (r_inv + 1.0) / 16777216.0;
-  const double constant = root_d * rms / 32768.0 + (double)d / 134217728.0;
+  const double per_sq = nf_uniform(
+      eps / lambda - r_inv + (double)(d + 6) * (r_inv + 1.0) / 16777216.0);
+  const double constant = nf_uniform(root_d * typical / 32768.0 +
+                                     (double)d / 134217728.0);
+  // (a factor beyond the fp32 range leaves no bound or the largest one)
+  const float large_gain = nf_uniform((float)(0.24 * r * s_c * s_c));
+  const float large_loss = nf_uniform((float)(1.01 * top_sq * r_inv));
   // the largest s a row can have whose distance is not above `dist`
   auto cut_of = [&](float dist, float sq) {
     const double norm = (double)__builtin_sqrtf(sq) * 1.000001;
@@ -323,6 +440,14 @@ nearest_feat_kernel(NearestFeatParams p) {
   // ... and the largest value its minimum of four can be kept as
   auto kept_cut = [](float cut) {
     return __builtin_fmaf(__builtin_fabsf(cut), 1.220703125e-4f, cut);
+  };
+
+  // the cut of a query whose best row so far is `best`
+  auto query_cut = [&](unsigned long long best_row, float sq) {
+    return cut_of(best_row != kNfNoKey
+                      ? __uint_as_float((uint32_t)(best_row >> 32))
+                      : kNearestLimit,
+                  sq);
   };
 
   unsigned long long best[S];
@@ -353,16 +478,23 @@ nearest_feat_kernel(NearestFeatParams p) {
       }
     }
   };
-  // the start value of the row's chains
+  // a row's weight, and the start value of its chains (apart: the load is on
+  // its way while a tile is searched)
   auto weight_of = [&](int c0, int c1, int t) {
-    float w = kNfNothing;
     const int row = c0 + t * TR + tid;
-    if (tid < TR && row < c1) {
-      const float v = p.weight[row];
-      if (v >= 0.0f)
-        w = __builtin_fminf(v * s_c * s_c * kappa, 1e37f);
-      else if (v == -1.0f)
-        w = kNfAlways;
+    return tid < TR && row < c1 ? p.weight[row] : -2.0f;
+  };
+  auto start_of = [&](float v) {
+    float w = __builtin_fminf(v * s_c * s_c * kappa, 1e37f);
+    // (negative ones compare as large ones; all waves wait for this)
+    const bool special = __float_as_uint(v) > __float_as_uint(limit_sq);
+    if (__any(special)) {
+      // a large row: 0.24 r |a|^2 is at least B^2 / r, or a bound of none
+      const float own = __builtin_fminf(v * large_gain, 1e37f);
+      const float large = __builtin_fmaxf(
+          (own >= large_loss ? own : 0.0f) - large_loss, -1e37f);
+      if (special)
+        w = v >= 0.0f ? large : v == -1.0f ? kNfAlways : kNfNothing;
     }
     return w;
   };
@@ -373,7 +505,7 @@ nearest_feat_kernel(NearestFeatParams p) {
     request(c0, 0, 0);
     float w = weight_of(c0, c1, 0);
     if (tid < TR)
-      tile_weight[0][tid] = w;
+      tile_weight[0][tid] = start_of(w);
     for (int t = 0; t < tiles; ++t) {
       const int buf = t & 1;
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -422,7 +554,7 @@ nearest_feat_kernel(NearestFeatParams p) {
         }
       }
       if (t + 1 < tiles && tid < TR)
-        tile_weight[buf ^ 1][tid] = w;
+        tile_weight[buf ^ 1][tid] = start_of(w);
     }
   };
 
@@ -430,6 +562,11 @@ nearest_feat_kernel(NearestFeatParams p) {
   asm volatile("" : "+v"(keep_bits));
   float lowest = -__builtin_inff(); // (the compiler must not know)
   asm volatile("" : "+s"(lowest));
+  unsigned long long scans = 0; // those with a third minimum below its cut
+  float third[S];               // smallest third minimum of the scans
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    third[s] = kNfNothing;
   for (int c0 = x_begin; c0 < x_end; c0 += kNfEpochRows) {
     const int c1 = min(x_end, c0 + kNfEpochRows);
     float top[S][3];
@@ -454,7 +591,6 @@ nearest_feat_kernel(NearestFeatParams p) {
       asm("v_min_f32 %0, %1, %2" : "=v"(top[s][0]) : "v"(top[s][0]), "v"(t));
     });
 
-    bool again = false;
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const int q = q0 + s * 32;
@@ -480,11 +616,7 @@ nearest_feat_kernel(NearestFeatParams p) {
       }
       best[s] = min(best[s], (unsigned long long)__shfl_xor(best[s], 32));
       if (kind[s] == 1) {
-        cut[s] = cut_of(best[s] != kNfNoKey
-                            ? __uint_as_float((uint32_t)(best[s] >> 32))
-                            : kNearestLimit,
-                        ysq[s]);
-        const float kept = kept_cut(cut[s]);
+        const float kept = kept_cut(query_cut(best[s], ysq[s]));
         unsigned long long own = best[s];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
@@ -501,19 +633,40 @@ nearest_feat_kernel(NearestFeatParams p) {
           }
         }
         best[s] = own;
-        // (the lane goes through its rows again)
         if (top[s][2] <= kept)
-          again = true;
-        else
-          cut[s] = -kNfCutLimit;
-      } else if (kind[s] == 2) {
-        again = true; // (with the cut that lets every row through)
-      } else {
-        cut[s] = -kNfCutLimit;
+          scans |= 1ull << min((c0 - x_begin) / kNfEpochRows, 63);
+        third[s] = __builtin_fminf(third[s], top[s][2]);
       }
+      // both lanes go on with the query's best row and a cut that follows it
+      best[s] = min(best[s], (unsigned long long)__shfl_xor(best[s], 32));
+      cut[s] = kind[s] == 1 ? kept_cut(query_cut(best[s], ysq[s])) : kNfCutLimit;
     }
+  }
 
-    if (__syncthreads_or(again)) {
+  // ---- queries that may have rows that were not kept ------------------------
+  // (a lane that doubts goes through its rows again, in scans some query of the
+  // workgroup has doubted in)
+  bool doubt = false;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const bool own = kind[s] == 1 && third[s] <= cut[s];
+    cut[s] = own ? query_cut(best[s], ysq[s]) : -kNfCutLimit;
+    doubt = doubt || own;
+  }
+  if (__syncthreads_or(doubt)) {
+#pragma unroll
+    for (int sh = 1; sh < kWave; sh <<= 1)
+      scans |= (unsigned long long)__shfl_xor(scans, sh);
+    if (lane == 0)
+      wave_scans[wave] = scans;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+      scans |= wave_scans[w];
+    for (int c0 = x_begin; c0 < x_end; c0 += kNfEpochRows) {
+      if (((scans >> min((c0 - x_begin) / kNfEpochRows, 63)) & 1) == 0)
+        continue;
+      const int c1 = min(x_end, c0 + kNfEpochRows);
       unsigned long long hits = 0; // 16 bits per set
       scan(c0, c1, [&](int step, int s, int v, const nf_acc_t &acc)
                        __attribute__((always_inline)) {
@@ -540,20 +693,59 @@ nearest_feat_kernel(NearestFeatParams p) {
         }
       });
     }
-    // both lanes go on with the query's best row and a cut that follows it
+  }
+  // ---- queries searched exactly: all threads share out the rows --------------
+  if (any_alone) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      best[s] = min(best[s], (unsigned long long)__shfl_xor(best[s], 32));
-      cut[s] = kNfCutLimit;
-      if (kind[s] == 1 && best[s] != kNfNoKey)
-        cut[s] = kept_cut(
-            cut_of(__uint_as_float((uint32_t)(best[s] >> 32)), ysq[s]));
+      const uint32_t queries = (uint32_t)__ballot(kind[s] == 2);
+      if (lane == 0)
+        alone[wave][s] = queries;
+    }
+    __syncthreads();
+    int turn = 0;
+#pragma unroll 1
+    for (int i = 0; i < WAVES * S; ++i) {
+      const int w = i / S, s = i % S;
+      uint32_t queries = alone[w][s];
+      while (queries != 0) {
+        const int at = __builtin_ctz(queries);
+        queries &= queries - 1;
+        const int q =
+            q0 - (wave * (S * 32) + col) + w * (S * 32) + s * 32 + at;
+        const float *row_y = p.y + (size_t)q * d;
+        unsigned long long key = kNfNoKey;
+#pragma unroll 1
+        for (int r0 = x_begin + tid; r0 < x_end; r0 += 2 * kBlock) {
+          const int rows[2] = {r0, min(r0 + kBlock, x_end - 1)};
+          float dist[2];
+          nf_exact<2>(row_y, p.x, rows, d, dist);
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            key = min(key, nf_key(dist[e], rows[e] - x_begin));
+        }
+#pragma unroll
+        for (int sh = 1; sh < kWave; sh <<= 1)
+          key = min(key, (unsigned long long)__shfl_xor(key, sh));
+        if (lane == 0)
+          wave_best[turn][wave] = key;
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < WAVES; ++u)
+          key = min(key, wave_best[turn][u]);
+        turn ^= 1;
+#pragma unroll
+        for (int u = 0; u < S; ++u)
+          if (u == s && w == wave && col == at)
+            best[u] = min(best[u], key);
+      }
     }
   }
 
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     const int q = q0 + s * 32;
+    best[s] = min(best[s], (unsigned long long)__shfl_xor(best[s], 32));
     if (half == 0 && q < y_end)
       p.out[q] = best[s] != kNfNoKey
                      ? (int64_t)x_begin +
@@ -563,19 +755,19 @@ nearest_feat_kernel(NearestFeatParams p) {
 }
 
 // |x|^2 of every row (or what it is instead, see NearestFeatParams), and the
-// largest component and the sum of the squares over the moderate rows.
+// largest component and the sum of log2 |x|^2 over the moderate rows.
 __global__ __launch_bounds__(kBlock) void nearest_feat_rows_kernel(
     const float *__restrict__ x, int n, int d, float *__restrict__ weight,
     NearestFeatGlobals *__restrict__ globals);
 
 // The fp16 operands of the rows, one thread per unit of 8 components; zeros
-// for rows the filter does not represent and for a tile of rows behind the
-// last one.
+// for rows the filter does not represent or that are far larger than the
+// others, and for a tile of rows behind the last one.
 template <int NB>
 __global__ __launch_bounds__(kBlock) void nearest_feat_pack_kernel(
     const float *__restrict__ x, int n, int d,
     const float *__restrict__ weight,
-    const NearestFeatGlobals *__restrict__ globals, uint4 *__restrict__ pack) {
+    NearestFeatGlobals *globals, uint4 *__restrict__ pack) {
   constexpr int U = 2 * NB;
   const size_t id = (size_t)blockIdx.x * kBlock + threadIdx.x;
   if (id >= (size_t)(n + kNfTileRows) * U)
@@ -583,8 +775,11 @@ __global__ __launch_bounds__(kBlock) void nearest_feat_pack_kernel(
   const int row = (int)(id / U);
   const int unit = (int)(id - (size_t)row * U);
   uint4 out = make_uint4(0, 0, 0, 0);
-  if (row < n && weight[row] >= 0.0f) {
-    const float scale = nf_scale(globals->max_bits);
+  const NfRows rows = nf_rows(globals);
+  if (id == 0)
+    globals->rows_of_x = rows;
+  if (row < n && weight[row] >= 0.0f && weight[row] <= rows.limit_sq) {
+    const float scale = rows.scale;
     float v[8];
     nf_load8(x + (size_t)row * d, 8 * unit, d, v);
 #pragma unroll
@@ -611,7 +806,8 @@ constexpr int nearest_feat_sets(int nb) { return nb <= 4 ? 4 : nb <= 6 ? 3 : 2; 
     hipLaunchKernelGGL((nearest_feat_pack_kernel<NB_>),                        \
                        dim3((unsigned)((units + kBlock - 1) / kBlock)),        \
                        dim3(kBlock), 0, stream, p.x, p.n, p.d, p.weight,       \
-                       p.globals, const_cast<uint4 *>(p.pack));                \
+                       const_cast<NearestFeatGlobals *>(p.globals),            \
+                       const_cast<uint4 *>(p.pack));                           \
     if (sets == 1)                                                             \
       hipLaunchKernelGGL((nearest_feat_kernel<NB_, 1>), dim3(grid),            \
                          dim3(kBlock), 0, stream, p);                          \

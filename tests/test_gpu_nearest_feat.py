@@ -88,6 +88,77 @@ def test_rows_the_filter_cannot_represent(oracle):
     check(oracle, x, np.zeros((40, 20), np.float32))
 
 
+# one scan of 4,096 rows and several; a handful of large ones and a third
+@pytest.mark.parametrize("factor", [50.0, 3e3, 1e5, 1e9])
+@pytest.mark.parametrize("n,m,d", [(700, 4096, 24), (300, 9000, 64),
+                                   (135000, 500, 20)])
+def test_rows_and_queries_far_larger_than_the_others(oracle, n, m, d, factor):
+    rng = np.random.default_rng(m)
+    y = rng.standard_normal((m, d)).astype(np.float32)
+    x = y[rng.integers(0, m, n)] + 0.5 * rng.standard_normal((n, d))
+    x = x.astype(np.float32)
+    few_x, few_y, many_x = x.copy(), y.copy(), x.copy()
+    few_x[::101] *= np.float32(factor)
+    few_y[::333] *= np.float32(factor)
+    many_x[::3] *= np.float32(factor)
+    if n > 1000:  # (all sets of queries per wave)
+        check(oracle, few_x, few_y)
+        return
+    check(oracle, few_x, y)
+    check(oracle, x, few_y)
+    check(oracle, few_x, few_y)
+    check(oracle, many_x, few_y)
+    near = few_y[rng.integers(0, m, n)] + rng.standard_normal((n, d))
+    check(oracle, near.astype(np.float32), few_y)
+    spread = np.exp(rng.standard_normal((m, 1)) * np.log(factor) / 3)
+    wide = (y * spread).astype(np.float32)
+    check(oracle, wide[rng.integers(0, m, n)] + x, wide)
+    every = (x * factor * 1e9).astype(np.float32)  # (|x|^2 beyond 1e30, too)
+    check(oracle, every, y)
+
+
+@pytest.mark.parametrize("d", [16, 70, 128])
+def test_candidates_that_were_not_kept_in_several_scans(oracle, d):
+    # dozens of rows within the margin of the nearest one, in the first, the
+    # last and the middle 4,096 rows
+    rng = np.random.default_rng(d)
+    y = (30 + rng.standard_normal((13000, d))).astype(np.float32)
+    for at in (100, 5000, 12500):
+        y[at:at + 60] = y[at] + (1e-3 * rng.standard_normal((60, d)))
+    x = np.concatenate([y[[100, 130, 5001, 5055, 12500, 12530]],
+                        30 + rng.standard_normal((200, d))])
+    check(oracle, x.astype(np.float32), y)
+    check(oracle, np.repeat(x[:3], 70, 0).astype(np.float32), y)
+
+
+def test_time_with_a_large_row_and_large_queries():
+    """One row of a code book a million times the others took 130 times as
+    long, a thousandth of the queries ten thousand times the others 35."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    y = torch.randn(4096, 64, generator=g, device="cuda")
+    x = y[torch.randint(0, 4096, (50000,), generator=g, device="cuda")]
+    x = x + 0.5 * torch.randn(50000, 64, generator=g, device="cuda")
+
+    def least(x, y):
+        times = []
+        for _ in range(6):
+            begin, end = (torch.cuda.Event(enable_timing=True)
+                          for _ in range(2))
+            begin.record()
+            capi.nearest_rows(x, y)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+
+    usual = least(x, y)
+    large_y, large_x = y.clone(), x.clone()
+    large_y[77] *= 1e6
+    large_x[::1000] *= 1e4
+    assert least(x, large_y) < 5 * usual
+    assert least(large_x, y) < 5 * usual
+
+
 def test_rows_far_from_the_origin(oracle):
     # |x - y|^2 far below the rounding margin of |x|^2 + |y|^2
     rng = np.random.default_rng(7)
