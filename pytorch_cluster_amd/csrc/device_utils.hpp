@@ -545,6 +545,26 @@ __device__ __forceinline__ uint32_t curve_place(const float (&v)[3],
   return cell[0];
 }
 
+// ---- operands of the fp16 filters (feature space) --------------------------
+
+// 1 / sigma: the power of two that brings `max_bits` into [2^10, 2^11).
+__device__ __forceinline__ float feat_inv_sigma(unsigned max_bits) {
+  if (max_bits == 0)
+    return 1.0f;
+  const int biased = (int)((max_bits >> 23) & 0xffu);
+  int e = 137 - biased;
+  e = e > 100 ? 100 : (e < -100 ? -100 : e);
+  return __uint_as_float((uint32_t)(e + 127) << 23);
+}
+
+// fp16 nearest-even with small values flushed to zero, as bits.
+__device__ __forceinline__ uint32_t feat_h(float v) {
+  if (!(__builtin_fabsf(v) >= 6.103515625e-05f)) // 2^-14 (NaN: zero)
+    return 0u;
+  const _Float16 h = (_Float16)v;
+  return (uint32_t)__builtin_bit_cast(unsigned short, h);
+}
+
 } // namespace pca
 
 // experiment switch: -DPCA_NO_SWIZZLE maps workgroup ids to tiles directly

@@ -114,15 +114,6 @@ struct NearestFeatParams {
   int64_t *out;
 };
 
-// The power of two that brings a largest component into [2^10, 2^11).
-__device__ __forceinline__ float nf_scale(unsigned max_bits) {
-  if (max_bits == 0)
-    return 1.0f;
-  int e = 137 - (int)((max_bits >> 23) & 0xffu);
-  e = e > 100 ? 100 : (e < -100 ? -100 : e);
-  return __uint_as_float((uint32_t)(e + 127) << 23);
-}
-
 __device__ __forceinline__ float nf_uniform(float v) {
   return __uint_as_float(
       (uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(v)));
@@ -146,21 +137,15 @@ __device__ __forceinline__ NfRows nf_rows(const NearestFeatGlobals *g) {
   r.typical = __builtin_fminf(rms, 2.0f * mean);
   const float limit = __builtin_fminf(mean * kNfLargeRow, 1e18f);
   r.limit_sq = limit * limit;
-  r.scale = nf_scale(min(g->max_bits, __float_as_uint(limit)));
+  r.scale = feat_inv_sigma(min(g->max_bits, __float_as_uint(limit)));
   return r;
-}
-
-__device__ __forceinline__ uint32_t nf_half(float v) {
-  if (!(__builtin_fabsf(v) >= 6.103515625e-05f)) // 2^-14
-    return 0u;
-  return (uint32_t)__builtin_bit_cast(unsigned short, (_Float16)v);
 }
 
 __device__ __forceinline__ uint4 nf_pack8(const float (&v)[8]) {
   uint32_t h[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e)
-    h[e] = nf_half(v[e]);
+    h[e] = feat_h(v[e]);
   return make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16),
                     h[4] | (h[5] << 16), h[6] | (h[7] << 16));
 }
@@ -352,7 +337,7 @@ nearest_feat_kernel(NearestFeatParams p) {
     for (int w = 0; w < WAVES; ++w)
       bits = max(bits, wave_top[w]);
   }
-  const float s_q = nf_scale(bits);
+  const float s_q = feat_inv_sigma(bits);
 
   nf_f16x8_t yb[S][NB];
   float ysq[S]; // |b|^2
