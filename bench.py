@@ -401,11 +401,11 @@ class Cases:
         return {"nearest: 1048576 x 64 features -> 4096 code vectors": {
             "ms": ms, "rows_per_s": feats.shape[0] / ms * 1e3,
             "roofline": _roofline(
-                "knn_mfma_kernel<5,8,nearest>", kms,
+                "nearest_feat_kernel<4,4>", kms,
                 2 * 64 * feats.shape[0] * 4096, PEAK_BF16_TFLOPS, "mfma",
-                "algorithmic 2*D flop per pair against the dense bf16 "
-                "matrix peak (this kernel forms three split-bf16 products "
-                "per pair and component)")}}
+                "algorithmic 2*D flop per pair against the dense fp16 "
+                "matrix peak, which is that of bf16 (one fp16 product per "
+                "pair and component, candidates evaluated in fp32)")}}
 
     # fps: the sampling step that precedes radius / knn in a set-abstraction
     # layer; a quarter of every cloud, first row as start
@@ -421,24 +421,21 @@ class Cases:
                 t, lambda: t.ops.torch_cluster.fps(pts, ptr, ratio, False),
                 reps or 5)
             # A sample step depends on the one before it, and a cloud is
-            # one workgroup's (its running minima stay in that compute
-            # unit's registers), so the floor is latency, not bandwidth:
-            # per step and row 3 subtractions, 3 multiply-adds, the minimum
-            # and two compare/selects for the running maximum = 9 vector
-            # instructions, 4 cycles each per wave of 64 on one of the
-            # unit's 4 SIMDs at 2.4 GHz; the two reductions across the
-            # workgroup come on top.
+            # one workgroup's, so the floor is latency, not bandwidth or
+            # rows (most rows are left alone in a step): about 100 vector
+            # instructions that wait for each other, 4 cycles each, and
+            # three trips to the LDS of 64 cycles, at 2.4 GHz.
             step_us = ms * 1e3 / (points // 4)
-            floor_us = points / 64.0 * 9 * 4 / 4 / 2400.0
+            floor_us = (100 * 4 + 3 * 64) / 2400.0
             report["fps %dx%d ratio 0.25" % (clouds, points)] = {
                 "ms": ms, "samples": int(out.numel()),
                 "us_per_sample_step": step_us,
                 "roofline": {
-                    "bound": "valu-latency", "unit": "us/step",
+                    "bound": "latency", "unit": "us/step",
                     "floor": floor_us, "achieved": step_us,
                     "frac": floor_us / step_us,
-                    "note": "vector-ALU time of one compute unit per "
-                            "sample step (9 instructions per row); "
+                    "note": "dependent instructions and LDS trips of a "
+                            "sample step that looks at one bucket of rows; "
                             "clouds run side by side, %d of the chip's "
                             "256 units busy" % clouds}}
         return report

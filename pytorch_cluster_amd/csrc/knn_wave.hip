@@ -279,12 +279,14 @@ bool knn_wave_supported(int n, int m, int d, int num_segments, int k,
   const double here =
       26.0 + (num_segments > 1 ? 3.0 : 0.0) +
       std::max(1.6 * rounds, thousands * (0.55 + 0.95 * rounds));
+  // (without its slices, which take a look at the environment)
+  const double least = 37.0 + 0.8 * k + (0.038 + 0.0025 * k) * 1e-6 * m * rows;
+  if (here <= least)
+    return true;
   const int slices =
       knn_lowd_config(d, k, n, m, num_segments, cosine).num_chunks;
-  const double scan = 37.0 + 0.8 * k +
-                      (4.3 + 0.16 * k) * rows / slices / 1024.0 +
-                      (slices > 1 ? 6.0 + 2.2 * k : 0.0) +
-                      (0.038 + 0.0025 * k) * 1e-6 * m * rows;
+  const double scan = least + (4.3 + 0.16 * k) * rows / slices / 1024.0 +
+                      (slices > 1 ? 6.0 + 2.2 * k : 0.0);
   return here <= scan;
 }
 
