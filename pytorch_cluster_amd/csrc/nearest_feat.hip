@@ -104,8 +104,9 @@ size_t pack_bytes(int n, int d) {
 // 1,048,576 queries x 4,096 rows, call (knn_mfma / this kernel, us): 16
 // components 1,271 / 396, 32: 1,540 / 453, 64: 2,208 / 679, 128: 4,094 / 1,274.
 // At 64 components the kernel takes 695 us under the profiler, 790 TFLOP/s
-// (hipBLASLt reaches 1,160 on 8,192^3 in fp16); below 48 the vector ALU bounds
-// it.
+// (hipBLASLt reaches 1,160 on 8,192^3 in fp16).  Vector ALU / matrix cores busy,
+// of the SIMD-cycles: 16 components 67 / 18 %, 32: 61 / 30, 64: 50 / 43, 128:
+// 36 / 44; two waves per SIMD wait for a tile, LDS or a barrier in the rest.
 //
 // Sets of queries per wave: all that fit the registers once that gives every
 // CU a workgroup, else one, for four times the workgroups.

@@ -29,8 +29,8 @@
 // MINIMA OF FOUR consecutive rows, the number of the four in the low nine bits
 // of the value (2^-14 of it, which the cut allows for).  That is 24 vector
 // instructions for 16 values; the matrix cores need 32 cycles per 16
-// components for them, and the vector ALU 4 cycles each: neither waits for
-// long from 48 components on.  After 4,096 rows the four rows of a query's
+// components for them, and the vector ALU 4 cycles each: alike from 48
+// components on, more for the vector ALU below.  After 4,096 rows the four rows of a query's
 // smallest minimum are evaluated exactly; their distance D gives the cut
 // below which s has to lie for a row to come before them; of the other
 // minima kept, those below the cut are evaluated too.  Only if at the end of
