@@ -15,8 +15,9 @@ namespace pca {
                                         int, hipStream_t);                     \
   template <>                                                                  \
   hipError_t launch_feat_pack<NB>(const float *, const float *,                \
-                                  const float *, const unsigned *, int, int,   \
-                                  bool, FeatGlobals *, uint4 *, hipStream_t);
+                                  const float *, const unsigned *,             \
+                                  const float *, int, int, bool,               \
+                                  FeatGlobals *, uint4 *, hipStream_t);
 PCA_DECLARE_FEAT_BLOCKS(3)
 PCA_DECLARE_FEAT_BLOCKS(5)
 PCA_DECLARE_FEAT_BLOCKS(9)
@@ -145,8 +146,69 @@ size_t feat_pack_bytes(int n, int d) {
   return align256(sizeof(uint4) * units * ((size_t)n + feat_tile_rows(d)));
 }
 
+// What the one-kernel search of fp32 rows subtracts from rows and queries: the
+// mean of 32 rows, if that at least halves their squares -- otherwise (rows
+// around the origin, a few large rows among the 32, components that are not
+// finite) zeros.  Up to 1e18, so that a difference is finite if its operands
+// are.  k = 20, us a call without / with the centre: 32 x 1,024 x 64 around the
+// origin 171 / 170, one standard deviation from it 173 / 167, 5 317 / 167, 20
+// 792 / 166; x 128 264 / 261, 272 / 257, 699 / 257, 1,528 / 258; uniform in
+// [0, 1) 300 / 259.  This kernel takes 1.5 us more, its readers less than before:
+// they load whole float4.
+__device__ void feat_centre(FeatGlobals *g, const float *__restrict__ x, int n,
+                            int d) {
+  constexpr int HALF = kFeatCentreSamples / 2;
+  __shared__ float sums[2][kFeatSmallMaxDim];
+  __shared__ float before[kBlock / kWave], after[kBlock / kWave];
+  static_assert(kBlock == 2 * kFeatSmallMaxDim, "half of the rows per thread");
+  const int tid = threadIdx.x;
+  const int c = tid & (kFeatSmallMaxDim - 1);
+  const int first = tid / kFeatSmallMaxDim * HALF;
+  float v[HALF];
+  float sum = 0.0f;
+#pragma unroll
+  for (int j = 0; j < HALF; ++j) {
+    const size_t row = (size_t)(first + j) * (size_t)n / kFeatCentreSamples;
+    v[j] = c < d ? x[row * d + c] : 0.0f;
+  }
+#pragma unroll
+  for (int j = 0; j < HALF; ++j)
+    sum += v[j];
+  sums[tid / kFeatSmallMaxDim][c] = sum;
+  __syncthreads();
+  const float mean = (sums[0][c] + sums[1][c]) * (1.0f / kFeatCentreSamples);
+  float sq = 0.0f, rest = 0.0f;
+#pragma unroll
+  for (int j = 0; j < HALF; ++j) {
+    sq = __builtin_fmaf(v[j], v[j], sq);
+    rest = __builtin_fmaf(v[j] - mean, v[j] - mean, rest);
+  }
+  if (!(__builtin_fabsf(mean) <= 1e18f))
+    rest = __builtin_inff();
+#pragma unroll
+  for (int sh = kWave / 2; sh >= 1; sh >>= 1) {
+    sq += __shfl_xor(sq, sh);
+    rest += __shfl_xor(rest, sh);
+  }
+  if ((tid & (kWave - 1)) == 0) {
+    before[tid / kWave] = sq;
+    after[tid / kWave] = rest;
+  }
+  __syncthreads();
+  sq = rest = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kBlock / kWave; ++w) {
+    sq += before[w];
+    rest += after[w];
+  }
+  if (tid < kFeatSmallMaxDim)
+    g->centre[c] = rest < 0.5f * sq ? mean : 0.0f;
+}
+
+// (centre_x: the rows whose centre the last workgroup makes, or null)
 __global__ __launch_bounds__(kBlock) void feat_init_kernel(
-    FeatGlobals *g, float *tau, int m, int *hit_count, int redo_cap,
+    const float *__restrict__ centre_x, int n, int d, FeatGlobals *g,
+    float *tau, int m, int *hit_count, int redo_cap,
     int *overflow, unsigned long long *edge_sums, int edge_blocks) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   // (the compaction's block sums, when the search counts the edges)
@@ -172,6 +234,8 @@ __global__ __launch_bounds__(kBlock) void feat_init_kernel(
     g->out_limit = 0xffffffffu;
     g->n_out = 0;
   }
+  if (centre_x != nullptr && blockIdx.x == gridDim.x - 1) // (uniform)
+    feat_centre(g, centre_x, n, d);
 }
 
 // slices of every segment's x rows of the second pass of the exact kernel
@@ -182,10 +246,11 @@ constexpr int kSecondPassChunks = 16;
 // largest finite |component| of the matrix.
 // big_out (or null): per row, the float bits of that largest |component|;
 // hist (or null): rows per binary exponent of it.
+// centre (or null): what is subtracted from every row first.
 __global__ __launch_bounds__(kBlock) void feat_rows_kernel(
     const float *__restrict__ x, int n, int d, float *__restrict__ sq_out,
     FeatGlobals *g, unsigned *__restrict__ big_out,
-    unsigned *__restrict__ hist) {
+    unsigned *__restrict__ hist, const float *__restrict__ centre) {
   __shared__ unsigned part[kBlock / kWave];
   __shared__ unsigned local_hist[256];
   static_assert(kBlock == 256, "one thread per exponent");
@@ -209,12 +274,16 @@ __global__ __launch_bounds__(kBlock) void feat_rows_kernel(
     if ((d & 3) == 0) {
       const float4 *p4 = reinterpret_cast<const float4 *>(p);
       for (int c = sub; c < d / 4; c += 16) {
-        const float4 v = p4[c];
+        float4 v = p4[c];
+        if (centre != nullptr) { // (uniform)
+          const float4 o = reinterpret_cast<const float4 *>(centre)[c];
+          v.x -= o.x, v.y -= o.y, v.z -= o.z, v.w -= o.w;
+        }
         take(v.x), take(v.y), take(v.z), take(v.w);
       }
     } else {
       for (int c = sub; c < d; c += 16)
-        take(p[c]);
+        take(centre != nullptr ? p[c] - centre[c] : p[c]);
     }
     // a row with an infinite or NaN component is nobody's neighbour
     // (csrc/cuda/knn_cuda.cu:48,68: its distances are infinite or NaN); it is
@@ -812,9 +881,13 @@ hipError_t launch_knn_feat(const SearchInput &in_given, int k, bool cosine,
   const bool small = r16 != 0 || radius != nullptr ||
                      feat_small_applies(in.n, in.m, in.d, in.num_segments, k,
                                         cosine);
-  hipLaunchKernelGGL(feat_init_kernel, dim3((in.m + kBlock - 1) / kBlock),
-                     dim3(kBlock), 0, stream, globals, tau, in.m, hit_count,
-                     redo_cap, overflow, small ? out.edge_sums : nullptr,
+  // (the one-kernel search of fp32 rows by Euclidean distance)
+  const bool centred = small && r16 == 0 && !cosine;
+  const float *centre = centred ? globals->centre : nullptr;
+  hipLaunchKernelGGL(feat_init_kernel,
+                     dim3((in.m + kBlock - 1) / kBlock + (centred ? 1 : 0)),
+                     dim3(kBlock), 0, stream, centred ? xf : nullptr, in.n,
+                     in.d, globals, tau, in.m, hit_count, redo_cap, overflow, small ? out.edge_sums : nullptr,
                      (in.m + kCompactBlockQueries - 1) / kCompactBlockQueries +
                          1);
   // squared norms that only classify the rows (NaN: a non-finite component);
@@ -836,7 +909,8 @@ hipError_t launch_knn_feat(const SearchInput &in_given, int k, bool cosine,
                        dim3(kBlock), 0, stream, xf, in.n, in.d, x_class,
                        static_cast<FeatGlobals *>(nullptr),
                        static_cast<unsigned *>(nullptr),
-                       static_cast<unsigned *>(nullptr));
+                       static_cast<unsigned *>(nullptr),
+                       static_cast<const float *>(nullptr));
   } else {
     // (the classification buffer is free here: it holds every row's largest
     // component)
@@ -844,7 +918,7 @@ hipError_t launch_knn_feat(const SearchInput &in_given, int k, bool cosine,
     hipLaunchKernelGGL(feat_rows_kernel,
                        dim3((in.n + rows_per_block - 1) / rows_per_block),
                        dim3(kBlock), 0, stream, xp, in.n, in.d, x_norm,
-                       globals, x_big, globals->hist_x);
+                       globals, x_big, globals->hist_x, centre);
     // (a cloud searched in itself: one pass over the rows serves both)
     const bool y_is_x = yf == xf && in.m == in.n;
     if (!y_is_x)
@@ -852,7 +926,8 @@ hipError_t launch_knn_feat(const SearchInput &in_given, int k, bool cosine,
                          dim3((in.m + rows_per_block - 1) / rows_per_block),
                          dim3(kBlock), 0, stream, yf, in.m, in.d,
                          static_cast<float *>(nullptr), globals,
-                         static_cast<unsigned *>(nullptr), globals->hist_y);
+                         static_cast<unsigned *>(nullptr), globals->hist_y,
+                         centre);
     hipLaunchKernelGGL(feat_scale_kernel, dim3(plan != nullptr ? 2 : 1),
                        dim3(kPlanThreads), 0, stream, globals, in.n, in.m,
                        y_is_x, in.ptr_y, in.num_segments,
@@ -862,24 +937,24 @@ hipError_t launch_knn_feat(const SearchInput &in_given, int k, bool cosine,
     hipError_t perr;
     switch (nb) {
     case 3:
-      perr = launch_feat_pack<3>(xp, x_norm, x_class, x_big, in.n, in.d,
-                                 cosine, globals, x_pack, stream);
+      perr = launch_feat_pack<3>(xp, x_norm, x_class, x_big, centre, in.n,
+                                 in.d, cosine, globals, x_pack, stream);
       break;
     case 5:
-      perr = launch_feat_pack<5>(xp, x_norm, x_class, x_big, in.n, in.d,
-                                 cosine, globals, x_pack, stream);
+      perr = launch_feat_pack<5>(xp, x_norm, x_class, x_big, centre, in.n,
+                                 in.d, cosine, globals, x_pack, stream);
       break;
     case 9:
-      perr = launch_feat_pack<9>(xp, x_norm, x_class, x_big, in.n, in.d,
-                                 cosine, globals, x_pack, stream);
+      perr = launch_feat_pack<9>(xp, x_norm, x_class, x_big, centre, in.n,
+                                 in.d, cosine, globals, x_pack, stream);
       break;
     case 17:
-      perr = launch_feat_pack<17>(xp, x_norm, x_class, x_big, in.n, in.d,
-                                  cosine, globals, x_pack, stream);
+      perr = launch_feat_pack<17>(xp, x_norm, x_class, x_big, centre, in.n,
+                                  in.d, cosine, globals, x_pack, stream);
       break;
     default:
-      perr = launch_feat_pack<33>(xp, x_norm, x_class, x_big, in.n, in.d,
-                                  cosine, globals, x_pack, stream);
+      perr = launch_feat_pack<33>(xp, x_norm, x_class, x_big, centre, in.n,
+                                  in.d, cosine, globals, x_pack, stream);
       break;
     }
     if (perr != hipSuccess)

@@ -75,6 +75,7 @@ constexpr int kFeatSlack = 16;    // list entries beyond k
 constexpr int kFeatDrainEvery = 64;
 constexpr int kFeatRoundPeriod = 8; // tiles between scheduled rounds
 constexpr int kFeatMaxDim = 512;    // components this path takes
+constexpr int kFeatSmallMaxDim = 128; // ... and its one-kernel search
 constexpr int kFeatRedoGroup = 32;  // queued queries per workgroup of the scan
 constexpr int kFeatMaxHits = 256;   // most rows the scan holds per query
 constexpr int kFeatRedoSlices = 32; // workgroups that share a group's rows
@@ -105,11 +106,17 @@ struct FeatGlobals {
   unsigned out_limit;
   int n_out;
   int out_rows[8];
+  // The one-kernel search of fp32 rows filters x - centre and y - centre
+  // (zeros: the rows as they are; feat_centre): the margins go with the norms,
+  // the distances do not, up to 2^-22 (|X|^2 + |Y|^2) for the roundings of the
+  // differences, which rho has room for.
+  alignas(16) float centre[kFeatSmallMaxDim];
   unsigned hist_x[32 * 256];
   unsigned hist_y[32 * 256];
 };
 constexpr int kFeatMaxOutliers = 8;
 constexpr int kFeatHistCopies = 32;
+constexpr int kFeatCentreSamples = 32; // rows the centre is the mean of
 
 // ---- constants of the error analysis (see the header) ----------------------
 // rho: 2^-9 up to 256 components, 2^-8 beyond (the accumulation error of the
@@ -185,10 +192,11 @@ struct FeatQuery {
 //   Euclid: `norm_in` unused.  cosine: the row's norm.
 //   R16 = 1 / 2: the row takes part in the filter with every component times
 //   chain_keep<R16> (device_utils.hpp), as the rows of x were packed.
-template <bool COSINE, int R16 = 0>
-__device__ __forceinline__ FeatQuery feat_query(const float *yrow, int d,
-                                                float inv_sigma,
-                                                float norm_in) {
+//   CENTRED: centre is subtracted from the row; both in aligned LDS.
+template <bool COSINE, int R16 = 0, bool CENTRED = false>
+__device__ __forceinline__ FeatQuery
+feat_query(const float *yrow, int d, float inv_sigma, float norm_in,
+           const float *centre = nullptr) {
   FeatQuery fq;
   if (COSINE) {
     // A query of zeros has no neighbours (0 / 0).  A norm of zero over
@@ -214,13 +222,25 @@ __device__ __forceinline__ FeatQuery feat_query(const float *yrow, int d,
   float chain = 0.0f; // classification as the old kernel does it
   double ysq = 0.0;
   float top = 0.0f;
-  for (int c = 0; c < d; ++c) {
-    const float v = yrow[c] * chain_keep<R16>(d, c);
+  auto take = [&](float v) {
     chain = __builtin_fmaf(v, v, chain);
     const float scaled = v * inv_sigma;
     top = __builtin_fmaxf(top, __builtin_fabsf(scaled));
     const double s = (double)scaled;
     ysq += s * s;
+  };
+  if constexpr (CENTRED) {
+    int c = 0;
+    for (; c + 4 <= d; c += 4) {
+      const float4 v = *reinterpret_cast<const float4 *>(yrow + c);
+      const float4 o = *reinterpret_cast<const float4 *>(centre + c);
+      take(v.x - o.x), take(v.y - o.y), take(v.z - o.z), take(v.w - o.w);
+    }
+    for (; c < d; ++c)
+      take(yrow[c] - centre[c]);
+  } else {
+    for (int c = 0; c < d; ++c)
+      take(yrow[c] * chain_keep<R16>(d, c));
   }
   fq.dead = chain != chain;
   // (a component beyond the range the scale was made for -- a query far
@@ -305,8 +325,9 @@ constexpr int feat_resident_groups(int nb, int kp) {
 template <int NB, bool COSINE>
 __global__ __launch_bounds__(kBlock) void feat_pack_kernel(
     const float *__restrict__ x, const float *__restrict__ norms,
-    const float *__restrict__ cls, const unsigned *__restrict__ big, int n,
-    int d, int spare, FeatGlobals *g, uint4 *__restrict__ out) {
+    const float *__restrict__ cls, const unsigned *__restrict__ big,
+    const float *__restrict__ centre, int n, int d, int spare, FeatGlobals *g,
+    uint4 *__restrict__ out) {
   typedef FeatShape<NB> S;
   const size_t id = (size_t)blockIdx.x * kBlock + threadIdx.x;
   if (id >= (size_t)(n + spare) * S::RSU)
@@ -356,10 +377,28 @@ __global__ __launch_bounds__(kBlock) void feat_pack_kernel(
     if (unit < S::UNITS - 2) {
       if (usable) {
         const int c0 = 8 * unit;
+        if (!COSINE && centre != nullptr && (d & 3) == 0) { // (uniform)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int c = c0 + e;
-          part[e] = c < d ? feat_h(x[(size_t)row * d + c] * scale) : 0u;
+          for (int e = 0; e < 8; e += 4) {
+            if (c0 + e < d) {
+              const float4 v = *reinterpret_cast<const float4 *>(
+                  x + (size_t)row * d + c0 + e);
+              const float4 o =
+                  *reinterpret_cast<const float4 *>(centre + c0 + e);
+              part[e] = feat_h((v.x - o.x) * scale);
+              part[e + 1] = feat_h((v.y - o.y) * scale);
+              part[e + 2] = feat_h((v.z - o.z) * scale);
+              part[e + 3] = feat_h((v.w - o.w) * scale);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int c = c0 + e;
+            const float o = !COSINE && centre != nullptr && c < d ? centre[c]
+                                                                  : 0.0f;
+            part[e] = c < d ? feat_h((x[(size_t)row * d + c] - o) * scale) : 0u;
+          }
         }
       }
     } else if (unit == S::UNITS - 2) {
@@ -1439,9 +1478,9 @@ hipError_t launch_knn_feat_blocks(const KnnFeatParams &p, int kp, bool cosine,
                                   int grid, hipStream_t stream);
 template <int NB>
 hipError_t launch_feat_pack(const float *x, const float *norms,
-                            const float *cls, const unsigned *big, int n,
-                            int d, bool cosine, FeatGlobals *g, uint4 *out,
-                            hipStream_t stream);
+                            const float *cls, const unsigned *big,
+                            const float *centre, int n, int d, bool cosine,
+                            FeatGlobals *g, uint4 *out, hipStream_t stream);
 
 #define PCA_KNN_FEAT_DEFINE(NB_)                                               \
   template <int KP>                                                            \
@@ -1485,19 +1524,20 @@ hipError_t launch_feat_pack(const float *x, const float *norms,
   template <>                                                                  \
   hipError_t launch_feat_pack<NB_>(const float *x, const float *norms,         \
                                    const float *cls, const unsigned *big,      \
-                                   int n, int d, bool cosine, FeatGlobals *g,  \
+                                   const float *centre, int n, int d,          \
+                                   bool cosine, FeatGlobals *g,                \
                                    uint4 *out, hipStream_t stream) {           \
     const int spare = FeatShape<NB_>::TILE;                                    \
     const size_t units = (size_t)(n + spare) * FeatShape<NB_>::RSU;            \
     const unsigned grid = (unsigned)((units + kBlock - 1) / kBlock);           \
     if (cosine)                                                                \
       hipLaunchKernelGGL((feat_pack_kernel<NB_, true>), dim3(grid),            \
-                         dim3(kBlock), 0, stream, x, norms, cls, nullptr, n,   \
-                         d, spare, g, out);                                    \
+                         dim3(kBlock), 0, stream, x, norms, cls, nullptr,      \
+                         nullptr, n, d, spare, g, out);                        \
     else                                                                       \
       hipLaunchKernelGGL((feat_pack_kernel<NB_, false>), dim3(grid),           \
-                         dim3(kBlock), 0, stream, x, norms, cls, big, n, d,    \
-                         spare, g, out);                                       \
+                         dim3(kBlock), 0, stream, x, norms, cls, big, centre,  \
+                         n, d, spare, g, out);                                 \
     return hipGetLastError();                                                  \
   }
 

@@ -50,6 +50,11 @@
 // sits under a condition (the compiler then counts loads in flight exactly
 // instead of waiting for all of them).
 //
+// The filter of fp32 rows by Euclidean distance works on x - centre and y -
+// centre (feat_centre): its margins grow with the squared norms, of rows 5
+// standard deviations from the origin 26 times beyond what the rows need.  The
+// exact distances are those of the rows as they are.
+//
 // Rows the filter cannot represent: NaN / infinite components are nobody's
 // neighbours (packed as padding); rows far larger than the rest (left out of
 // the scale, FeatGlobals::out_rows) are evaluated exactly for every query at
@@ -277,6 +282,12 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
       }
     }
   }
+  // the centre, where the gathered rows of the search will be (a pass over the
+  // tiles, with its barriers, comes between)
+  constexpr bool CENTRED = R16 == 0;
+  float *const centre = reinterpret_cast<float *>(&gathered[0][0][0]);
+  if (CENTRED && tid < MAX_D)
+    centre[tid] = p.globals->centre[tid];
   __syncthreads();
   const float *const my_y = &ys[(wave * 32 + col) * ROW_F];
 
@@ -285,7 +296,8 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
   const float ynorm = COSINE && valid ? p.y_norm[q] : 1.0f;
   const float inv_sigma =
       COSINE ? 1.0f : feat_inv_sigma(p.globals->max_bits);
-  const FeatQuery fq = feat_query<COSINE, R16>(my_y, d, inv_sigma, ynorm);
+  const FeatQuery fq = feat_query<COSINE, R16, CENTRED>(
+      my_y, d, inv_sigma, ynorm, centre);
   // active: the query searches (a NaN component: no neighbours).  filtered:
   // it does so with the fp16 lower bound; if the filter cannot take the query
   // (a component beyond the range the scale was made for) or some row of x
@@ -316,12 +328,26 @@ __global__ __launch_bounds__(kBlock, 1) void knn_feat_small_kernel(
     uint32_t hb[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (i < NB - 1) {
       const int cb = 16 * i + 8 * half;
+      if constexpr (CENTRED) {
+        // (what lies behind the row's d components is read and not used)
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        hb[e] = (filtered && cb + e < d)
-                    ? feat_h(my_y[min(cb + e, d - 1)] *
-                             chain_keep<R16>(d, min(cb + e, d - 1)) * y_scale)
-                    : 0u;
+        for (int e = 0; e < 8; e += 4) {
+          const small_v4f v =
+              *reinterpret_cast<const small_v4f *>(my_y + cb + e) -
+              *reinterpret_cast<const small_v4f *>(centre + cb + e);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            hb[e + j] =
+                filtered && cb + e + j < d ? feat_h(v[j] * y_scale) : 0u;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          hb[e] = (filtered && cb + e < d)
+                      ? feat_h(my_y[min(cb + e, d - 1)] *
+                               chain_keep<R16>(d, min(cb + e, d - 1)) * y_scale)
+                      : 0u;
+      }
     } else if (half == 0 && filtered) {
       hb[0] = 0x7800u; // 2^15
       hb[1] = 0x4c00u; // 2^4

@@ -468,3 +468,45 @@ def test_16bit_chain_against_the_real_distance(bf16, kind):
         # and the bound is not vacuous: the chain does lose something
         if kind in ("normal", "decreasing"):
             assert (H[finite] < D[finite]).any()
+
+
+def check_centred(x, y, centre):
+    """The same bounds with rows and queries less `centre` in the filter
+    (feat_centre of knn_feat.hip) and the distances of the rows as they are."""
+    x = np.ascontiguousarray(x, dtype=np.float32)
+    y = np.ascontiguousarray(y, dtype=np.float32)
+    d = x.shape[1]
+    rho = rho_of(d)
+    u, v = x - centre, y - centre  # (fp32, rounded)
+    inv = inv_sigma(max(np.abs(u).max(), np.abs(v).max()))
+    scale2 = inv * inv
+    c0 = d / 4096.0 + d * 2.0 ** -149 * scale2
+    us = u * np.float32(inv)
+    vs = v * np.float32(inv)
+    usq32 = np.zeros(len(u), dtype=np.float32)
+    for c in range(d):
+        usq32 = (u[:, c].astype(np.float64) ** 2 + usq32).astype(np.float32)
+    w = np.array([w_parts(float(s) * scale2 * (1.0 - rho)) for s in usq32])
+    s = w[None, :] + h(-2.0 * vs.astype(np.float64)) @ h(us).T
+    vsq = (vs.astype(np.float64) ** 2).sum(1)
+    lower = s + (vsq * (1.0 - rho) - c0)[:, None]
+    upper = (lower + (6.0 * rho * vsq + 2.0 * c0)[:, None]) * (1.0 + 4.1 * rho)
+    e = reference_distances(x, y) * scale2
+    norms = (us.astype(np.float64) ** 2).sum(1)[None, :] + vsq[:, None]
+    room = max(0.15, (d + 16) * 2.01 / 4096.0) * 2.0 ** -10 * norms
+    assert (lower + room <= e + 1e-300).all()
+    assert (e <= upper - room).all()
+
+
+@pytest.mark.parametrize("d", [9, 64, 128])
+@pytest.mark.parametrize("offset", [0.0, 1.0, 5.0, 1000.0, 3e17])
+def test_rows_less_a_centre(d, offset):
+    rng = np.random.default_rng(d)
+    x = (rng.standard_normal((200, d)) + offset).astype(np.float32)
+    mean = x[:32].mean(0, dtype=np.float32)
+    check_centred(x, x[:40], mean)
+    check_centred(x, (rng.standard_normal((40, d)) + offset), mean)
+    # a centre far from the rows, and rows at rounding midpoints about one
+    check_centred(x, x[:40], mean * np.float32(-3.0))
+    x = midpoint_rows(rng, 200, d, 0, 1) + np.float32(offset % 1e6)
+    check_centred(x, x[:40], np.full(d, offset % 1e6, dtype=np.float32))
