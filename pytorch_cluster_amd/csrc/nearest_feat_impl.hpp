@@ -5,7 +5,8 @@
 // ONE fp16 product per pair and component on the matrix cores ranks a query's
 // candidates, and a few of them are evaluated exactly afterwards.  With
 // a = s_c x, b = s_q y (s_c, s_q powers of two, of the call and of the
-// workgroup's queries, that bring the largest component into [2^10, 2^11)) and
+// workgroup's queries, that bring the largest component near the end of the fp16
+// range) and
 // r = s_q / s_c, a chain of v_mfma_f32_32x32x16_f16 that starts from
 // kappa |a|^2 gives
 //     s = kappa |a|^2 + sum_c h(a_c) h(-2 b_c),    h: fp16, |h| < 2^-14 flushed,
@@ -123,6 +124,16 @@ __device__ __forceinline__ double nf_uniform(double v) {
                           __builtin_amdgcn_readfirstlane(__double2loint(v)));
 }
 
+// Largest components after scaling: rows in [2^14, 2^15), queries in [2^13,
+// 2^14), as -2 b has to be an fp16 number too.  What is flushed below 2^-14 is
+// that much less of a small row or query than with feat_inv_sigma alone ([2^10,
+// 2^11)).  Norms of both log-normal with sigma 2, us a call, with the second
+// term of per_sq (below) taken for r_inv + 1 / as it is, scaled so: 100,000 x
+// 4,096 x 64 342 / 221, 50,000 x 4,096 x 128 489 / 305; of the rows with sigma 3
+// 476 / 192 and 7,469 / 247.
+constexpr float kNfRowScale = 16.0f;
+constexpr float kNfQueryScale = 8.0f;
+
 constexpr float kNfLargeRow = 4096.0f;
 constexpr int kNfLargeExponents = 12;
 __device__ __forceinline__ float nf_mean_norm(double sum_log, unsigned rows) {
@@ -137,7 +148,8 @@ __device__ __forceinline__ NfRows nf_rows(const NearestFeatGlobals *g) {
   r.typical = __builtin_fminf(rms, 2.0f * mean);
   const float limit = __builtin_fminf(mean * kNfLargeRow, 1e18f);
   r.limit_sq = limit * limit;
-  r.scale = feat_inv_sigma(min(g->max_bits, __float_as_uint(limit)));
+  r.scale = kNfRowScale *
+            feat_inv_sigma(min(g->max_bits, __float_as_uint(limit)));
   return r;
 }
 
@@ -337,7 +349,7 @@ nearest_feat_kernel(NearestFeatParams p) {
     for (int w = 0; w < WAVES; ++w)
       bits = max(bits, wave_top[w]);
   }
-  const float s_q = feat_inv_sigma(bits);
+  const float s_q = kNfQueryScale * feat_inv_sigma(bits);
 
   nf_f16x8_t yb[S][NB];
   float ysq[S]; // |b|^2
@@ -407,7 +419,9 @@ nearest_feat_kernel(NearestFeatParams p) {
   }
   const double r_inv = (double)s_c / (double)s_q;
   const double per_sq = nf_uniform(
-      eps / lambda - r_inv + (double)(d + 6) * (r_inv + 1.0) / 16777216.0);
+      eps / lambda - r_inv +
+      // (|b|^2 is a sum in fp32)
+      (double)(d + 6) * (r_inv + eps / lambda) / 16777216.0);
   const double constant = nf_uniform(root_d * typical / 32768.0 +
                                      (double)d / 134217728.0);
   // (a factor beyond the fp32 range leaves no bound or the largest one)

@@ -41,12 +41,12 @@ def rows_of_x(x):
     sq = squares(x)
     some = sq[sq > 0]
     if len(some) == 0:
-        return 1.0, 1e36, inv_sigma(0)
+        return 1.0, 1e36, 16.0 * inv_sigma(0)
     mean = 2.0 ** (0.5 * np.log2(some).mean())
     limit = min(mean * LARGE_ROW, 1e18)
     top = np.abs(x[sq > 0]).max()
     return (min(math.sqrt(some.mean()), 2.0 * mean), limit ** 2,
-            inv_sigma(min(top, limit)))
+            16.0 * inv_sigma(min(top, limit)))
 
 
 def exponent(v):
@@ -66,7 +66,7 @@ def check(x, y):
     ours = np.array([exponent(t) <= mean + LARGE_EXPONENTS for t in tops])
     assert ours.any()
     y = y[ours]  # (the others are searched exactly)
-    s_q = inv_sigma(np.abs(y).max())
+    s_q = 8.0 * inv_sigma(np.abs(y).max())
     a = x.astype(np.float64) * s_c
     b = y.astype(np.float64) * s_q
     large = squares(x) > limit_sq
@@ -96,7 +96,8 @@ def check(x, y):
     start = np.minimum(start, 1e37)
     s = start[:, None] + ha @ hb.T
     dist = distances(x, y).astype(np.float64)
-    per_sq = eps / lam - 1.0 / r + (d + 6) * (1.0 / r + 1.0) * 2.0 ** -24
+    per_sq = (eps / lam - 1.0 / r +
+              (d + 6) * (1.0 / r + eps / lam) * 2.0 ** -24)
     cut = (s_c * s_q * (dist + d * 5.7e-45) * (1.0 + (d + 6) * 2.0 ** -24) +
            ysq * per_sq + root_d * np.sqrt(ysq) / 8192.0 +
            root_d * A / 32768.0 + d * 2.0 ** -27)
