@@ -43,7 +43,7 @@
 // One row or query far larger than the others must not set the scale, A or l for
 // all.  Rows of a norm beyond 4,096 times the geometric mean take part with
 // zeros for operands and s = r |a|^2 / 4 - B^2 / r, a lower bound as long as
-// |b| <= r |a| / 2 (otherwise they are always looked at).  Queries with a
+// |b| <= r |a| / 2 (otherwise they are left to a second pass).  Queries with a
 // component of 2^12 times the workgroup's mean are searched exactly, and where
 // the largest of the others is far beyond an ordinary one, l lies between the
 // two.  Calls of 100,000 queries x 4,096 rows x 64, 135 us: with one row a
@@ -52,8 +52,8 @@
 // 8,192 x 128: the candidates of all scans but the one with the nearest row were
 // searched for again before its distance was known; 300 -> 240 us, 10 standard
 // deviations from the origin 1,004 -> 254.  What is left: an entry that occurs
-// 16 times or more brings the second pass to every query (654 us; the
-// kernel of knn_mfma_impl.hpp 553).
+// 16 times or more brings the second pass to every query (640 us; the
+// kernel of knn_mfma_impl.hpp 407).
 //
 // Rows of x with a component that is not finite never qualify (their distance
 // is not below 1e38); finite ones of |x|^2 > 1e30 enter with s = -1e37, always
@@ -483,7 +483,14 @@ nearest_feat_kernel(NearestFeatParams p) {
     const int row = c0 + t * TR + tid;
     return tid < TR && row < c1 ? p.weight[row] : -2.0f;
   };
-  auto start_of = [&](float v) {
+  // (in the first pass a large row that every query would have to look at is left
+  // out: with a dozen of them the three minima that a query keeps were all
+  // theirs, their distances gave the cut, and the second pass looked at every
+  // row.  Norms of rows and queries log-normal with sigma 3, us a call: 100,000
+  // x 4,096 x 64 2,778 / 723, 50,000 x 4,096 x 128 4,146 / 1,058, 100,000 x
+  // 4,096 x 16 942 / 214)
+  bool left_out = false;
+  auto start_of = [&](float v, bool first) {
     float w = __builtin_fminf(v * s_c * s_c * kappa, 1e37f);
     // (negative ones compare as large ones; all waves wait for this)
     const bool special = __float_as_uint(v) > __float_as_uint(limit_sq);
@@ -492,19 +499,25 @@ nearest_feat_kernel(NearestFeatParams p) {
       const float own = __builtin_fminf(v * large_gain, 1e37f);
       const float large = __builtin_fmaxf(
           (own >= large_loss ? own : 0.0f) - large_loss, -1e37f);
+      const bool later =
+          first && special && v >= 0.0f && own < large_loss;
+      left_out = left_out || later;
       if (special)
-        w = v >= 0.0f ? large : v == -1.0f ? kNfAlways : kNfNothing;
+        w = v >= 0.0f    ? (later ? kNfNothing : large)
+            : v == -1.0f ? kNfAlways
+                         : kNfNothing;
     }
     return w;
   };
   // `visit(step, s, v, acc)` for every 32 rows, set of queries and four rows
-  auto scan = [&](int c0, int c1, auto &&visit) __attribute__((always_inline)) {
+  auto scan = [&](int c0, int c1, bool first, auto &&visit)
+                  __attribute__((always_inline)) {
     const int tiles = (c1 - c0 + TR - 1) / TR;
     __syncthreads(); // (nobody reads an earlier scan's tiles any more)
     request(c0, 0, 0);
     float w = weight_of(c0, c1, 0);
     if (tid < TR)
-      tile_weight[0][tid] = start_of(w);
+      tile_weight[0][tid] = start_of(w, first);
     for (int t = 0; t < tiles; ++t) {
       const int buf = t & 1;
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -553,7 +566,7 @@ nearest_feat_kernel(NearestFeatParams p) {
         }
       }
       if (t + 1 < tiles && tid < TR)
-        tile_weight[buf ^ 1][tid] = start_of(w);
+        tile_weight[buf ^ 1][tid] = start_of(w, first);
     }
   };
 
@@ -563,6 +576,7 @@ nearest_feat_kernel(NearestFeatParams p) {
   asm volatile("" : "+s"(lowest));
   unsigned long long scans = 0; // those with a third minimum below its cut
   float third[S];               // smallest third minimum of the scans
+  bool any_left_out = false;
 #pragma unroll
   for (int s = 0; s < S; ++s)
     third[s] = kNfNothing;
@@ -572,8 +586,8 @@ nearest_feat_kernel(NearestFeatParams p) {
 #pragma unroll
     for (int s = 0; s < S; ++s)
       top[s][0] = top[s][1] = top[s][2] = kNfNothing;
-    scan(c0, c1, [&](int step, int s, int v, const nf_acc_t &acc)
-                     __attribute__((always_inline)) {
+    scan(c0, c1, true, [&](int step, int s, int v, const nf_acc_t &acc)
+                           __attribute__((always_inline)) {
       // (fmed3 with -inf is a minimum without the quieting of NaNs that fminf
       // comes with; it is also the instruction that waits for the matrix
       // cores, which the compiler sees to only for instructions of its own)
@@ -640,15 +654,20 @@ nearest_feat_kernel(NearestFeatParams p) {
       best[s] = min(best[s], (unsigned long long)__shfl_xor(best[s], 32));
       cut[s] = kind[s] == 1 ? kept_cut(query_cut(best[s], ysq[s])) : kNfCutLimit;
     }
+    if (left_out)
+      scans |= 1ull << min((c0 - x_begin) / kNfEpochRows, 63);
+    any_left_out = any_left_out || left_out;
+    left_out = false;
   }
 
   // ---- queries that may have rows that were not kept ------------------------
   // (a lane that doubts goes through its rows again, in scans some query of the
-  // workgroup has doubted in)
+  // workgroup has doubted in; all of them where a row was left out)
   bool doubt = false;
+  const bool everyone = __syncthreads_or(any_left_out) != 0;
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const bool own = kind[s] == 1 && third[s] <= cut[s];
+    const bool own = kind[s] == 1 && (everyone || third[s] <= cut[s]);
     cut[s] = own ? query_cut(best[s], ysq[s]) : -kNfCutLimit;
     doubt = doubt || own;
   }
@@ -667,8 +686,8 @@ nearest_feat_kernel(NearestFeatParams p) {
         continue;
       const int c1 = min(x_end, c0 + kNfEpochRows);
       unsigned long long hits = 0; // 16 bits per set
-      scan(c0, c1, [&](int step, int s, int v, const nf_acc_t &acc)
-                       __attribute__((always_inline)) {
+      scan(c0, c1, false, [&](int step, int s, int v, const nf_acc_t &acc)
+                              __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           hits |= acc[4 * v + i] <= cut[s] ? 1ull << (16 * s + 4 * v + i) : 0;

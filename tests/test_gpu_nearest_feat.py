@@ -117,6 +117,26 @@ def test_rows_and_queries_far_larger_than_the_others(oracle, n, m, d, factor):
     check(oracle, every, y)
 
 
+@pytest.mark.parametrize("m,d", [(4096, 24), (9000, 64), (4500, 128)])
+def test_norms_over_many_magnitudes(oracle, m, d):
+    # large rows that a large query of the workgroup could have for its nearest
+    # one are left out of the first pass; in the third example every row is one
+    rng = np.random.default_rng(m)
+
+    def norms(rows):
+        return np.exp(3 * rng.standard_normal((rows, 1)))
+
+    y = rng.standard_normal((m, d)) * norms(m)
+    x = rng.standard_normal((700, d)) * norms(700)
+    check(oracle, x.astype(np.float32), y.astype(np.float32))
+    near = y[rng.integers(0, m, 700)] * (1 + 0.1 * rng.standard_normal((700, d)))
+    check(oracle, near.astype(np.float32), y.astype(np.float32))
+    y[-40:] = 1e4 * rng.standard_normal((40, d))
+    near[-300:] = 1e3 * rng.standard_normal((300, d)) * norms(300)
+    check(oracle, near.astype(np.float32), y.astype(np.float32),
+          [0, 300, 400, 700], [0, 50, m - 40, m])
+
+
 @pytest.mark.parametrize("d", [16, 70, 128])
 def test_candidates_that_were_not_kept_in_several_scans(oracle, d):
     # dozens of rows within the margin of the nearest one, in the first, the
