@@ -20,7 +20,8 @@
 // The sampling is a chain of dependent steps, each an arg-max over the
 // example's rows, so the time per sample is what counts, and an example is one
 // workgroup's (a step that several workgroups share costs two trips through
-// the L2).  Up to 1,024 rows of up to 4 dimensions fps_reg_kernel looks at
+// the L2).  fps_stream_kernel has several samples per step (see "several samples
+// per step").  Up to 1,024 rows of up to 4 dimensions fps_reg_kernel looks at
 // every row in every step, from registers.  Beyond that most rows are left
 // alone (see "rows in buckets" below) where more than a few hundred samples
 // repay the sort: fps_lds_kernel keeps up to 8,192 rows in LDS,
@@ -83,6 +84,14 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
   PCA_DPP_UMAX(v, 0x142, 0xa); // row_bcast:15 into rows 1 and 3
   PCA_DPP_UMAX(v, 0x143, 0xc); // row_bcast:31 into rows 2 and 3
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+// Every lane gets the largest value of its row of 16 lanes.
+__device__ __forceinline__ uint32_t row16_umax_all(uint32_t v) {
+  PCA_DPP_UMAX(v, 0x128, 0xf); // row_ror:8
+  PCA_DPP_UMAX(v, 0x124, 0xf); // row_ror:4
+  PCA_DPP_UMAX(v, 0x122, 0xf); // row_ror:2
+  PCA_DPP_UMAX(v, 0x121, 0xf); // row_ror:1
+  return v;
 }
 // U waves' worth of values at once: their steps fill each other's wait states.
 template <int U> __device__ __forceinline__ void wave_umax_of(uint32_t (&v)[U]) {
@@ -554,10 +563,91 @@ __device__ __forceinline__ float fps_lower(const float (&q)[DIM],
   return dd;
 }
 
+// ---- several samples per step ---------------------------------------------------
+//
+// The rows of an example are in 64 groups; of each group an entry of a table in
+// LDS has the largest running minimum, the row that has it (its number and
+// its coordinates), and `rest`, no smaller than any other minimum of
+// the group.  The next sample is the entry that comes first (largest value, equal
+// ones in the reference's order).  A sample lowers minima only: while an entry's
+// row is at least its value away from all samples of the step before it, it
+// still has that value and is still the first of its group; and while the value
+// is above the `rest` of those samples' groups, no other row can be before it.
+// So the entries are ranked, and the samples of a step are the longest run of
+// first ones of which that holds for every pair -- the same samples, in the same
+// order, as one by one.  (A sample that does not lower its own minimum -- a row
+// without a finite distance to itself, or a minimum of 0 -- is the next sample
+// again: the run ends with it.)
+constexpr int kFpsBatch = 8; // at most; 8 x 8 pairs are a wave's lanes
+
+struct FpsTable {
+  float4 head[kWave];   // value, row, x, y
+  float2 tail[kWave];   // z, rest
+  float4 first[kFpsBatch]; // of rank i: x, y, z, value
+  float2 more[kFpsBatch];  // its rest and row
+};
+
 // Waits for this workgroup's LDS traffic and meets its other waves (global
-// stores stay in flight: what a wave stores only it reads again).
+// stores stay in flight: for them __syncthreads).
 __device__ __forceinline__ void fps_meet() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Entries to samples, by a workgroup of 64 / OWN waves, after the entries of
+// this step are written; wave w ranks entries OWN w ...  Returns the number of
+// samples, the same for all waves; lane i % 8 holds the i-th: coordinates and
+// row of the example.
+template <int OWN>
+__device__ __forceinline__ int fps_rank(FpsTable &t, int wave, float (&sx)[3],
+                                        uint32_t &row) {
+  const int lane = threadIdx.x & (kWave - 1);
+  fps_meet();
+  const uint32_t v = __float_as_uint(t.head[lane].x);
+  const int own = wave * OWN + (lane & (OWN - 1));
+  const float4 h = t.head[own];
+  const float2 g = t.tail[own];
+  int before[OWN], equal = 0;
+#pragma unroll
+  for (int e = 0; e < OWN; ++e) {
+    const uint32_t mine = lane_value(v, wave * OWN + e);
+    before[e] = __builtin_popcountll(__ballot(v > mine));
+    equal += __builtin_popcountll(__ballot(v >= mine)) - before[e];
+  }
+  if (__builtin_expect(equal != OWN, 0)) {
+    const uint32_t tie = fps_tie(__float_as_uint(t.head[lane].y));
+#pragma unroll
+    for (int e = 0; e < OWN; ++e) {
+      const uint32_t mine = lane_value(v, wave * OWN + e);
+      const uint32_t mine_tie = lane_value(tie, wave * OWN + e);
+      before[e] += __builtin_popcountll(
+          __ballot(v == mine && (tie < mine_tie ||
+                                 (tie == mine_tie && lane < wave * OWN + e))));
+    }
+  }
+  int rank = before[0];
+#pragma unroll
+  for (int e = 1; e < OWN; ++e)
+    rank = (lane & (OWN - 1)) == e ? before[e] : rank;
+  if (lane < OWN && rank < kFpsBatch) {
+    t.first[rank] = make_float4(h.z, h.w, g.x, h.x);
+    t.more[rank] = make_float2(g.y, h.y);
+  }
+  fps_meet();
+  const int a = lane & (kFpsBatch - 1), b = lane / kFpsBatch;
+  const float4 ra = t.first[a], rb = t.first[b];
+  const float2 ma = t.more[a];
+  const float d0 = ra.x - rb.x, d1 = ra.y - rb.y, d2 = ra.z - rb.z;
+  float dd = d0 * d0;
+  dd = __builtin_fmaf(d1, d1, dd);
+  dd = __builtin_fmaf(d2, d2, dd);
+  // (infinite: one of the two has no distance to itself)
+  const bool apart = dd >= rb.w && dd < __builtin_inff() && ma.x < rb.w;
+  const uint64_t ends = __ballot(a < b && !apart);
+  sx[0] = ra.x;
+  sx[1] = ra.y;
+  sx[2] = ra.z;
+  row = __float_as_uint(ma.y);
+  return ends != 0 ? (int)__builtin_ctzll(ends) / kFpsBatch : kFpsBatch;
 }
 
 // The rows of an example in curve order, by one workgroup: afterwards keys[i],
@@ -1108,40 +1198,41 @@ __global__ __launch_bounds__(W *kWave) void fps_bucket_kernel(
 
 // ---- fp32, up to 3 dimensions, larger examples ---------------------------------
 
-// Rows in curve order: (x, y, z, row of the example), their running minima,
-// and the box of every piece of 64 rows.  Piece i of example b has the number
-// ptr[b] / 64 + b + i (no two examples meet).  A wave per piece.
+// Rows in curve order, (x, y, z, row of the example), their running minima, and
+// the box of every piece of 64 rows.  The pieces of an example, a multiple of four
+// (places beyond the last row: minimum 0 and the last of all ties), follow piece
+// number ptr[b] / 64 + 4 b, so that no two examples meet.  A wave per piece.
 struct FpsPieces {
-  float4 *rows;   // [n]
-  float *minima;  // [n]
-  float *boxes;   // [pieces][8]: lower corner, -, upper corner, -
+  float4 *rows;  // [pieces][64]
+  float *minima; // [pieces][64]
+  float *boxes;  // [pieces][8]: lower corner, -, upper corner, -
 };
-__device__ __forceinline__ int64_t fps_first_piece(int64_t begin, int b) {
-  return begin / kWave + b;
+constexpr int kFpsPieces = 4;
+static_assert(kFpsPieces == kBlock / kWave, "a block of the kernel below");
+__host__ __device__ constexpr int64_t fps_first_piece(int64_t begin, int b) {
+  return begin / kWave + (int64_t)kFpsPieces * b;
 }
 __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
     const float *__restrict__ src, const int64_t *__restrict__ ptr, int d,
     int first_segment, const uint32_t *__restrict__ perm, FpsPieces out) {
   const int b = first_segment + blockIdx.y;
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t piece = (int64_t)blockIdx.x * (kBlock / kWave) +
-                        threadIdx.x / kWave;
   const int64_t begin = ptr[b], end = ptr[b + 1];
-  if (begin + piece * kWave >= end)
+  if (begin + (int64_t)blockIdx.x * kBlock >= end)
     return;
-  const int64_t at = begin + piece * kWave + lane;
-  const bool ok = at < end;
-  const int64_t id = ok ? (int64_t)perm[at] : begin;
+  const int64_t rel = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const bool ok = begin + rel < end;
+  const int64_t id = ok ? (int64_t)perm[begin + rel] : begin;
   float v[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c)
-    v[c] = c < d ? src[(size_t)id * d + c] : 0.0f;
-  if (ok) {
-    out.rows[at] =
-        make_float4(v[0], v[1], v[2], __uint_as_float((uint32_t)(id - begin)));
-    out.minima[at] = 5e4f;
-  }
-  float *box = out.boxes + (size_t)(fps_first_piece(begin, b) + piece) * 8;
+    v[c] = ok && c < d ? src[(size_t)id * d + c] : 0.0f;
+  const int64_t first = fps_first_piece(begin, b);
+  out.rows[first * kWave + rel] = make_float4(
+      v[0], v[1], v[2],
+      __uint_as_float(ok ? (uint32_t)(id - begin) : kFpsNoRow));
+  out.minima[first * kWave + rel] = ok ? 5e4f : 0.0f;
+  float *box = out.boxes + (first + rel / kWave) * 8;
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     // (fminf / fmaxf drop a NaN; such a row's minimum never changes)
@@ -1159,28 +1250,46 @@ __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
   }
 }
 
-// Bucket k of an example belongs to wave k % W: its box and its best row are in
-// lane (k / W) % 64, slot k / W / 64, of that wave; the rows and their running
-// minima stay in memory, that is in the L2 of the workgroup's XCD.  S slots
-// hold buckets of one piece for up to 65,536 S rows; MANY: more than that,
-// several pieces to a bucket.
+// A bucket has R pieces of 64 rows (MANY: a multiple of that) and belongs to a
+// lane of the workgroup: its box and its best row are in that lane's registers; the
+// rows and their running minima stay in memory, that is in the L2 of the
+// workgroup's XCD.  The groups of the samples' table are rows of 16 lanes.  A step
+// of up to eight samples: every wave tests its buckets (those samples only that
+// are near to any of them), the buckets that pass go on a list, all waves share
+// the list, the owners take the results, the entries are ranked.
 //
-// Eight ragged LiDAR-like scans of 60,000 - 200,000 rows, 2 % sampled: 419.6 ->
-// 5.7 ms per call, 1.4 instead of 157 us per step of the longest scan (before:
-// fps_any_kernel, the whole scan through one compute unit in every step; rows
-// in Morton instead of Hilbert order, 14 instead of 12 buckets per sample:
-// 6.8 ms).
-// Bound by the chain of a step: a wave waits in 65 % of its cycles (its SIMD's
-// other three, the rows of a bucket from the L2, LDS, the barrier), the vector
-// ALU is busy in 56 % of the cycles of the compute unit.
-template <int W, int S, bool MANY>
+// Eight ragged LiDAR-like scans of 60,000 - 200,000 rows, 2 % sampled: 5.75 ->
+// 2.79 ms per call, 1.47 -> 0.71 us per sample of the longest scan (before: one
+// sample per step).  Uniform rows, samples: 8 x 20,000, 2,000 each 2.22 -> 1.16
+// ms; 8 x 60,000, 600 each 1.27 -> 0.83; 2 x 300,000, 900 each 4.54 -> 2.93.
+// Where nearly every maximum is a tie (200,000 rows on 33^3 places) groups hold
+// several rows of the largest value and a step ends with its first sample: 5.2
+// -> 6.1 ms.
+// Bound by the chain of a step, about 7,000 cycles for five samples of a scan of
+// 200,000 rows: 1,400 to the list, 2,500 + 1,200 for the 21 buckets of the list
+// (their rows at the 64 bytes per clock that a compute unit gets from the L2, and
+// the wait for the slowest wave), 1,800 for entries and ranks, of which most is
+// instructions that all sixteen waves execute.  Figures behind the choices, on
+// the scans: with the owners looking at their own buckets 3.1 ms, two thirds of
+// it waits for the wave with the most; minima stored where nothing changed 3.4;
+// up to four samples per step 3.7; buckets of 128 rows 2.9 (16-lane groups of
+// 64 rows could not hold 200,000).
+template <int W, int R, bool MANY>
 __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
     const float *__restrict__ src, const int64_t *__restrict__ ptr,
     const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
     int d, FpsPieces p, int64_t *__restrict__ out) {
   constexpr int DIM = 3;
-  __shared__ FpsBest<DIM> table[2][W];
-  __shared__ uint32_t sampled[kWave];
+  static_assert(W * 4 == kWave, "a group per row of 16 lanes");
+  static_assert(kFpsPieces % R == 0, "whole buckets");
+  __shared__ FpsTable table;
+  // the buckets of a step, with the samples that they are near to, and what was
+  // found in them
+  __shared__ uint32_t list[kWave * W];
+  __shared__ float4 found_head[kWave * W]; // value, row, x, y
+  __shared__ float2 found_tail[kWave * W]; // z, rest
+  __shared__ int items[2];
+  __shared__ uint32_t sampled[2 * kWave];
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -1189,188 +1298,322 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
   const int count = (int)(ptr[b + 1] - start_idx);
   const int64_t o_begin = out_ptr[b];
   const int64_t o_end = out_ptr[b + 1];
-  if (o_begin >= o_end)
+  if (o_begin >= o_end || count <= 0)
     return;
-  float4 *rows = p.rows + start_idx;
-  float *minima = p.minima + start_idx;
-  // (MANY: examples of more than 64 W S pieces, several of them to a bucket)
+  const int64_t first_piece = fps_first_piece(start_idx, b);
+  const float4 *rows = p.rows + first_piece * kWave;
+  float *minima = p.minima + first_piece * kWave;
   const int pieces = (count + kWave - 1) / kWave;
   const int chunks =
-      MANY ? max(1, (pieces + kWave * W * S - 1) / (kWave * W * S)) : 1;
-  const int buckets = (pieces + chunks - 1) / chunks;
+      MANY ? max(1, (pieces + kWave * W * R - 1) / (kWave * W * R)) : 1;
+  const int per_bucket = chunks * R;
+  const int buckets = (pieces + per_bucket - 1) / per_bucket;
+  const int last = (pieces - 1) / R * (R * kWave) + lane;
+  // The buckets of a wave follow each other along the curve, so that most
+  // samples are far from all of them; neighbours, of which one sample often
+  // changes several, are in different groups.
+  const int run = (buckets + W - 1) / W;
+  const int slot = (lane & 15) * 4 + lane / 16;
+  const int bucket = wave * run + slot;
 
-  float blo[S][DIM], bhi[S][DIM];
-  FpsBest<DIM> best[S];
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const int k = (s * kWave + lane) * W + wave;
-    const bool any = k < buckets;
-    best[s].val = any ? kFpsUnseen : 0u;
-    best[s].rel = kFpsNoRow;
+  float blo[DIM], bhi[DIM], bx[DIM];
+  uint32_t val, rest = 0u, rel = kFpsNoRow;
+  {
+    const int k = bucket;
+    const bool any = slot < run && k < buckets;
+    val = any ? kFpsUnseen : 0u;
 #pragma unroll
     for (int c = 0; c < DIM; ++c) {
-      blo[s][c] = __builtin_inff();
-      bhi[s][c] = -__builtin_inff();
-      best[s].x[c] = 0.0f;
+      blo[c] = __builtin_inff();
+      bhi[c] = -__builtin_inff();
+      bx[c] = 0.0f;
     }
-    const float *box =
-        p.boxes + (size_t)(fps_first_piece(start_idx, b) + k * chunks) * 8;
-    for (int i = 0; any && i < chunks && k * chunks + i < pieces; ++i) {
+    const float *box = p.boxes + (first_piece + (int64_t)k * per_bucket) * 8;
+    for (int i = 0; any && i < per_bucket && k * per_bucket + i < pieces; ++i) {
 #pragma unroll
       for (int c = 0; c < DIM; ++c) {
-        blo[s][c] = __builtin_fminf(blo[s][c], box[i * 8 + c]);
-        bhi[s][c] = __builtin_fmaxf(bhi[s][c], box[i * 8 + 4 + c]);
+        blo[c] = __builtin_fminf(blo[c], box[i * 8 + c]);
+        bhi[c] = __builtin_fmaxf(bhi[c], box[i * 8 + 4 + c]);
       }
     }
   }
 
-  float cur[DIM];
+  // of all buckets of the wave: box, largest value
+  float wlo[DIM], whi[DIM];
+  uint32_t wave_val = kFpsUnseen;
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) {
+    wlo[c] = blo[c];
+    whi[c] = bhi[c];
+#pragma unroll
+    for (int sh = 1; sh < kWave; sh <<= 1) {
+      wlo[c] = __builtin_fminf(wlo[c], __shfl_xor(wlo[c], sh));
+      whi[c] = __builtin_fmaxf(whi[c], __shfl_xor(whi[c], sh));
+    }
+  }
+  if (tid < 2)
+    items[tid] = 0;
+  __syncthreads();
+  float sx[DIM]; // lane i: sample i of the step
+  int got = 1, turn = 0;
   {
     const int64_t first = start_idx + (start ? start[b] : 0);
     if (tid == 0)
       out[o_begin] = first;
 #pragma unroll
     for (int c = 0; c < DIM; ++c)
-      cur[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
+      sx[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
   }
 
-  int own = 0; // lane of the wave's best
-  FpsBest<DIM> mine = best[0];
-  const int64_t steps = o_end - o_begin;
-  for (int64_t m = 1; m < steps; ++m) {
-    const int par = (int)(m & 1);
-    uint64_t pass[S], any = 0;
+  const int steps = (int)(o_end - o_begin);
+  int m = 1;
+  while (m < steps) {
+    uint32_t hits = 0; // bit i: sample i may lower a minimum of this bucket
+    uint32_t near = (uint32_t)__ballot(
+        lane < got && !(fps_box_distance<DIM>(sx, wlo, whi) >=
+                        __uint_as_float(wave_val)));
+    while (near != 0) {
+      const int i = __builtin_ctz(near);
+      near &= near - 1;
+      float q[DIM];
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      pass[s] = __ballot(!(fps_box_distance<DIM>(cur, blo[s], bhi[s]) >=
-                           __uint_as_float(best[s].val)));
-      any |= pass[s];
+      for (int c = 0; c < DIM; ++c)
+        q[c] = lane_value(sx[c], i);
+      const bool passes =
+          !(fps_box_distance<DIM>(q, blo, bhi) >= __uint_as_float(val));
+      hits |= passes ? 1u << i : 0u;
     }
-    if (any != 0) {
+    // the buckets to look at, for all waves
+    const uint64_t pass = __ballot(hits != 0);
+    int item = 0;
+    if (pass != 0) {
+      int base = 0;
+      if (lane == 0)
+        base = atomicAdd(&items[turn], __builtin_popcountll(pass));
+      item = __builtin_amdgcn_readfirstlane(base) +
+             __builtin_amdgcn_mbcnt_hi(
+                 (uint32_t)(pass >> 32),
+                 __builtin_amdgcn_mbcnt_lo((uint32_t)pass, 0u));
+      if (hits != 0)
+        list[item] = (uint32_t)bucket | hits << 16;
+    }
+    // (with the rows' minima of the step before, which any wave may read now)
+    __syncthreads();
+    const int total = __builtin_amdgcn_readfirstlane(items[turn]);
+    turn ^= 1;
+    if (tid == 0)
+      items[turn] = 0;
+    // U buckets at a time, so that their rows are on the way together
+    auto look = [&](auto many, const int first_item) {
+      constexpr int U = decltype(many)::value;
+      uint32_t todo[U];
+      int bucket[U];
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
-        // U buckets at a time, so that their rows are on the way together
-        auto look = [&](auto many, const int (&at_lane)[decltype(many)::value]) {
-          constexpr int U = decltype(many)::value;
-          FpsBest<DIM> found[U];
+      for (int u = 0; u < U; ++u) {
+        const uint32_t what = (uint32_t)__builtin_amdgcn_readfirstlane(
+            (int)list[first_item + u * W]);
+        bucket[u] = (int)(what & 0xffffu);
+        todo[u] = what >> 16;
+      }
+      // a lane's largest minimum of each bucket and the second
+      uint32_t f_val[U], f_rest[U], f_rel[U];
+      float f_x[U][DIM];
+      int i_last[U];
+      float4 v[U][R];
+      float low[U][R];
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            found[u].val = 0u;
-            found[u].rel = kFpsNoRow;
+      for (int u = 0; u < U; ++u) {
+        i_last[u] = (pieces - 1) / R - bucket[u] * chunks;
+        f_val[u] = 0u;
+        f_rest[u] = 0u;
+      }
+      for (int i = 0; i < chunks; ++i) {
+        float was[U][R];
+        int at[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          at[u] = (bucket[u] * chunks + i) * (R * kWave) + lane;
+          // (MANY: the pieces may end inside the bucket; then the last ones
+          // again, which are not looked at below)
+          if (MANY)
+            at[u] = min(at[u], last);
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+          {
+            v[u][r] = rows[at[u] + r * kWave];
+            was[u][r] = minima[at[u] + r * kWave];
+            low[u][r] = was[u][r];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          uint32_t some = todo[u];
+          do {
+            float q[DIM];
 #pragma unroll
             for (int c = 0; c < DIM; ++c)
-              found[u].x[c] = 0.0f;
-          }
-          for (int i = 0; i < chunks; ++i) {
-            float4 v[U];
-            float low[U];
-            int at[U];
+              q[c] = lane_value(sx[c], __builtin_ctz(some));
+            some &= some - 1;
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-              const int k = (s * kWave + at_lane[u]) * W + wave;
-              at[u] = (k * chunks + i) * kWave + lane;
-              const int in = min(at[u], count - 1);
-              v[u] = rows[in];
-              low[u] = minima[in];
+            for (int r = 0; r < R; ++r) {
+              const float x[DIM] = {v[u][r].x, v[u][r].y, v[u][r].z};
+              low[u][r] = fps_lower<DIM>(q, x, low[u][r]);
             }
+          } while (some != 0);
+        }
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-              const float x[DIM] = {v[u].x, v[u].y, v[u].z};
-              low[u] = fps_lower<DIM>(cur, x, low[u]);
-              const bool ok = at[u] < count;
-              if (ok)
-                minima[at[u]] = low[u];
-              const uint32_t bits = ok ? __float_as_uint(low[u]) : 0u;
-              const uint32_t rel = ok ? __float_as_uint(v[u].w) : kFpsNoRow;
-              // (a lane's rows of a bucket of several pieces)
-              const bool take =
-                  !MANY || i == 0 || bits > found[u].val ||
-                  (bits == found[u].val && fps_tie(rel) < fps_tie(found[u].rel));
-              found[u].val = take ? bits : found[u].val;
-              found[u].rel = take ? rel : found[u].rel;
+        for (int u = 0; u < U; ++u) {
+          const uint32_t before = f_val[u];
 #pragma unroll
-              for (int c = 0; c < DIM; ++c)
-                found[u].x[c] = take ? x[c] : found[u].x[c];
+          for (int r = 0; r < R; ++r) {
+            if (low[u][r] < was[u][r])
+              minima[at[u] + r * kWave] = low[u][r];
+            const uint32_t bits =
+                !MANY || i <= i_last[u] ? __float_as_uint(low[u][r]) : 0u;
+            // (the middle one of three: the second largest is not below it)
+            f_rest[u] = max(f_rest[u], min(f_val[u], bits));
+            f_val[u] = max(f_val[u], bits);
+          }
+          // which row it is (the last one of equal ones)
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            const bool is = __float_as_uint(low[u][r]) == f_val[u] &&
+                            (!MANY || f_val[u] > before);
+            if (r == 0 && !MANY) {
+              f_rel[u] = __float_as_uint(v[u][r].w);
+              f_x[u][0] = v[u][r].x;
+              f_x[u][1] = v[u][r].y;
+              f_x[u][2] = v[u][r].z;
+            } else {
+              f_rel[u] = is ? __float_as_uint(v[u][r].w) : f_rel[u];
+              f_x[u][0] = is ? v[u][r].x : f_x[u][0];
+              f_x[u][1] = is ? v[u][r].y : f_x[u][1];
+              f_x[u][2] = is ? v[u][r].z : f_x[u][2];
             }
           }
-          uint32_t top[U];
-#pragma unroll
-          for (int u = 0; u < U; ++u)
-            top[u] = found[u].val;
-          wave_umax_of<U>(top);
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const int at =
-                fps_first(__ballot(found[u].val == top[u]), found[u].rel);
-            const uint32_t row = lane_value(found[u].rel, at);
-            float at_x[DIM];
-#pragma unroll
-            for (int c = 0; c < DIM; ++c)
-              at_x[c] = lane_value(found[u].x[c], at);
-            const bool here = lane == at_lane[u];
-            best[s].val = here ? top[u] : best[s].val;
-            best[s].rel = here ? row : best[s].rel;
-#pragma unroll
-            for (int c = 0; c < DIM; ++c)
-              best[s].x[c] = here ? at_x[c] : best[s].x[c];
-          }
-        };
-        uint64_t left = pass[s];
-        while (left != 0) {
-          int id[4];
-          id[0] = (int)__builtin_ctzll(left);
-          left &= left - 1;
-          if (left == 0) {
-            const int one[1] = {id[0]};
-            look(std::integral_constant<int, 1>{}, one);
-            break;
-          }
-          // (fewer than four: the first one again, which changes nothing)
-#pragma unroll
-          for (int u = 1; u < 4; ++u) {
-            id[u] = left != 0 ? (int)__builtin_ctzll(left) : id[0];
-            left &= left - 1;
-          }
-          look(std::integral_constant<int, 4>{}, id);
         }
       }
-      mine = best[0];
+      uint32_t top[U], next[U];
+      uint64_t who[U];
 #pragma unroll
-      for (int s = 1; s < S; ++s) {
-        const bool take = best[s].val > mine.val ||
-                          (best[s].val == mine.val &&
-                           fps_tie(best[s].rel) < fps_tie(mine.rel));
-        mine.val = take ? best[s].val : mine.val;
-        mine.rel = take ? best[s].rel : mine.rel;
+      for (int u = 0; u < U; ++u)
+        top[u] = f_val[u];
+      wave_umax_of<U>(top);
 #pragma unroll
-        for (int c = 0; c < DIM; ++c)
-          mine.x[c] = take ? best[s].x[c] : mine.x[c];
+      for (int u = 0; u < U; ++u) {
+        const bool is = f_val[u] == top[u];
+        who[u] = __ballot(is);
+        next[u] = is ? f_rest[u] : f_val[u];
       }
-      const uint32_t top = wave_umax(mine.val);
-      own = fps_first(__ballot(mine.val == top), mine.rel);
-    }
-    if (lane == own)
-      table[par][wave] = mine;
-    fps_meet();
-    FpsBest<DIM> e = table[par][lane & (W - 1)];
-    static_assert(W == 16, "one row of 16 lanes looks at the waves' bests");
-    const uint32_t top =
-        (uint32_t)__builtin_amdgcn_readlane((int)row16_umax(e.val), 15);
-    const int at = fps_first(__ballot(e.val == top) & 0xffffull, e.rel);
+      wave_umax_of<U>(next);
 #pragma unroll
-    for (int c = 0; c < DIM; ++c)
-      cur[c] = lane_value(e.x[c], at);
+      for (int u = 0; u < U; ++u) {
+        int at = (int)__builtin_ctzll(who[u]);
+        if (__builtin_expect((who[u] & (who[u] - 1)) != 0 || next[u] == top[u],
+                             0)) {
+          // rows of equal value: the one that comes first in the reference's
+          // order
+          next[u] = top[u];
+          uint32_t first = 0u; // (the complement of the smallest tie)
+          auto among = [&](const float4(&row)[R], const float(&m)[R]) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              const bool is = __float_as_uint(m[r]) == top[u];
+              const uint32_t t = is ? ~fps_tie(__float_as_uint(row[r].w)) : 0u;
+              const bool take = t > first;
+              first = max(first, t);
+              f_rel[u] = take ? __float_as_uint(row[r].w) : f_rel[u];
+              f_x[u][0] = take ? row[r].x : f_x[u][0];
+              f_x[u][1] = take ? row[r].y : f_x[u][1];
+              f_x[u][2] = take ? row[r].z : f_x[u][2];
+            }
+          };
+          if (R > 1 && !MANY) {
+            among(v[u], low[u]);
+          } else {
+#pragma unroll 1
+            for (int i = 0; i < chunks; ++i) {
+              float4 row[R];
+              float m[R];
+              const int to = min(
+                  (bucket[u] * chunks + i) * (R * kWave) + lane, last);
+#pragma unroll
+              for (int r = 0; r < R; ++r) {
+                row[r] = rows[to + r * kWave];
+                m[r] = minima[to + r * kWave];
+              }
+              among(row, m);
+            }
+          }
+          const uint32_t most = wave_umax(first);
+          at = (int)__builtin_ctzll(__ballot(first == most));
+        }
+        if (lane == at) {
+          found_head[first_item + u * W] =
+              make_float4(__uint_as_float(top[u]), __uint_as_float(f_rel[u]),
+                          f_x[u][0], f_x[u][1]);
+          found_tail[first_item + u * W] =
+              make_float2(f_x[u][2], __uint_as_float(next[u]));
+        }
+      }
+    };
+    int i = wave;
+    for (; i + W < total; i += 2 * W)
+      look(std::integral_constant<int, 2>{}, i);
+    if (i < total)
+      look(std::integral_constant<int, 1>{}, i);
+    fps_meet();
+    if (hits != 0) {
+      const float4 h = found_head[item];
+      const float2 t = found_tail[item];
+      val = __float_as_uint(h.x);
+      rel = __float_as_uint(h.y);
+      bx[0] = h.z;
+      bx[1] = h.w;
+      bx[2] = t.x;
+      rest = __float_as_uint(t.y);
+    }
+    if (pass != 0 || m == 1) {
+      // the best of every group
+      const uint32_t top = row16_umax_all(val);
+      bool is = val == top;
+      uint32_t next = row16_umax_all(is ? rest : val);
+      const uint64_t who = __ballot(is);
+      if (__builtin_expect(__builtin_popcountll(who) > 4, 0)) {
+        // several of a group (at most `top` is left without the first one)
+        const uint32_t t = is ? ~fps_tie(rel) : 0u;
+        const uint32_t first = row16_umax_all(t);
+        const uint64_t mine = who >> (lane & 48) & 0xffffull;
+        next = (mine & (mine - 1)) != 0 ? top : next;
+        is = is && t == first;
+      }
+      wave_val = max(max(lane_value(top, 0), lane_value(top, 16)),
+                     max(lane_value(top, 32), lane_value(top, 48)));
+      if (is) {
+        table.head[wave * 4 + lane / 16] =
+            make_float4(__uint_as_float(top), __uint_as_float(rel), bx[0],
+                        bx[1]);
+        table.tail[wave * 4 + lane / 16] =
+            make_float2(bx[2], __uint_as_float(next));
+      }
+    }
+    uint32_t chosen;
+    got = fps_rank<kWave / W>(table, wave, sx, chosen);
+    got = min(got, steps - m);
     if (wave == 0) {
       // (64 samples are written out at a time)
-      const uint32_t chosen = lane_value(e.rel, at);
-      if (lane == 0)
-        sampled[m & (kWave - 1)] = chosen;
-      if ((m & (kWave - 1)) == kWave - 1 || m == steps - 1) {
-        const int64_t to = (m & ~(int64_t)(kWave - 1)) + lane;
-        if (to <= m && to > 0)
-          out[o_begin + to] = start_idx + (int64_t)sampled[lane];
+      if (lane < got)
+        sampled[(m + lane) & (2 * kWave - 1)] = chosen;
+      const int from = m & ~(kWave - 1), to = m + got;
+      if (to >= from + kWave || to == steps) {
+        // (the last step may end one block of samples and begin another)
+        for (int k = from + lane; k < to; k += kWave)
+          if (k > 0 && (k < from + kWave || to == steps))
+            out[o_begin + k] =
+                start_idx + (int64_t)sampled[k & (2 * kWave - 1)];
       }
     }
+    m += got;
   }
 }
 
@@ -1435,10 +1678,10 @@ size_t fps_scratch_bytes(int dtype, int n, int d, int num_segments,
   const size_t dist = fps_align(sizeof(double) * (size_t)n);
   if (!fps_streams(dtype, d, max_rows))
     return dist;
-  const size_t pieces = (size_t)n / kWave + (size_t)num_segments + 1;
+  const size_t pieces = (size_t)fps_first_piece(n, num_segments);
   // (a stream that is being captured takes fps_any_kernel and its `dist`)
-  return std::max(dist, fps_align(sizeof(float4) * (size_t)n) +
-                            fps_align(sizeof(float) * (size_t)n) +
+  return std::max(dist, fps_align(sizeof(float4) * kWave * pieces) +
+                            fps_align(sizeof(float) * kWave * pieces) +
                             fps_align(sizeof(float) * 8 * pieces) +
                             curve_order_bytes(n, num_segments));
 }
@@ -1455,32 +1698,33 @@ hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
     return static_cast<void *>(piece);
   };
   FpsPieces p;
-  p.rows = static_cast<float4 *>(take(sizeof(float4) * (size_t)n));
-  p.minima = static_cast<float *>(take(sizeof(float) * (size_t)n));
-  p.boxes = static_cast<float *>(
-      take(sizeof(float) * 8 *
-           ((size_t)n / kWave + (size_t)num_segments + 1)));
+  const size_t pieces = (size_t)fps_first_piece(n, num_segments);
+  p.rows = static_cast<float4 *>(take(sizeof(float4) * kWave * pieces));
+  p.minima = static_cast<float *>(take(sizeof(float) * kWave * pieces));
+  p.boxes = static_cast<float *>(take(sizeof(float) * 8 * pieces));
   const uint32_t *perm = nullptr;
   hipError_t err = launch_curve_order(src, ptr, n, d, num_segments, cursor,
                                       &perm, stream);
   if (err != hipSuccess)
     return err;
-  const int per_block = kWave * (kBlock / kWave);
   const int64_t rows = std::min(max_rows, (int64_t)n);
   for (int b0 = 0; b0 < num_segments; b0 += 65535) {
     const int some = std::min(65535, num_segments - b0);
     hipLaunchKernelGGL(fps_gather_kernel,
-                       dim3((unsigned)((rows + per_block - 1) / per_block),
-                            some),
-                       dim3(kBlock), 0, stream, src, ptr, d, b0, perm, p);
+                       dim3((unsigned)((rows + kBlock - 1) / kBlock), some),
+                       dim3(kBlock), 0, stream, src, ptr, d, b0, perm,
+                       p);
   }
+  // (half as many rows to a bucket where the lanes suffice: 8 x 60,000 rows, 600
+  // samples each, R = 1 / 2 910 / 840 us, 8 x 20,000 1,160 / 1,240; the scans, at
+  // most 200,000 rows, R = 4 2.8 ms, 2 x 4 2.9)
 #define PCA_FPS_STREAM(S_, MANY_)                                              \
   hipLaunchKernelGGL((fps_stream_kernel<kFpsWaves, S_, MANY_>),                \
                      dim3(num_segments), dim3(kFpsThreads), 0, stream, src,    \
                      ptr, out_ptr, start, d, p, out)
-  if (rows <= 1 * kWave * kFpsThreads)
+  if (rows <= kWave * kFpsThreads / 2)
     PCA_FPS_STREAM(1, false);
-  else if (rows <= 2 * kWave * kFpsThreads)
+  else if (rows <= kWave * kFpsThreads)
     PCA_FPS_STREAM(2, false);
   else if (rows <= 4 * kWave * kFpsThreads)
     PCA_FPS_STREAM(4, false);

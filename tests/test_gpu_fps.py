@@ -115,6 +115,31 @@ def test_skipped_rows_change_nothing(oracle, rows, d, kind):
     assert (got == want).all()
 
 
+# 32,768 / 65,536 / 262,144: buckets of one, two, four pieces of 64 rows and of
+# several times four; hundreds of samples, most of them several to a step
+@pytest.mark.parametrize("kind", ["uniform", "grid", "copies", "clusters"])
+@pytest.mark.parametrize("rows", [16385, 32769, 65537, 262145])
+def test_several_samples_per_step_are_those_one_by_one(oracle, rows, kind):
+    rng = np.random.default_rng(rows)
+    ptr = np.cumsum([0, 40, rows, 17000]).astype(np.int64)
+    n = ptr[-1]
+    if kind == "uniform":
+        x = rng.random((n, 3))
+    elif kind == "grid":  # most largest minima are ties
+        x = rng.integers(0, 24, (n, 3))
+    elif kind == "copies":  # samples whose neighbours come to a minimum of 0
+        x = rng.random((700, 3))[rng.integers(0, 700, n)]
+    else:
+        x = rng.random((12, 3))[rng.integers(0, 12, n)]
+        x = x + 0.003 * rng.standard_normal((n, 3))
+    x = x.astype(np.float32)
+    share = np.array([1.0, 750.0 / rows, 800.0 / 17000])
+    start = np.array([7, rows - 1, 0], dtype=np.int64)
+    got = gpu_fps(oracle, x, ptr, share, start)
+    want = oracle.fps_op(x, ptr, share, start)
+    assert (got == want).all()
+
+
 # whole buckets (64 or 128 consecutive rows along the curve) at an infinite
 # distance: rows without a finite coordinate on an axis, rows and first samples
 # at infinity, squared gaps beyond the fp32 range
