@@ -571,8 +571,8 @@ __device__ __forceinline__ float fps_lower(const float (&q)[DIM],
 // the group.  The next sample is the entry that comes first (largest value, equal
 // ones in the reference's order).  A sample lowers minima only: while an entry's
 // row is at least its value away from all samples of the step before it, it
-// still has that value and is still the first of its group; and while the value
-// is above the `rest` of those samples' groups, no other row can be before it.
+// still has that value and is still the first of its group; and while it comes
+// before the `rest` of those samples' groups, no other row can be before it.
 // So the entries are ranked, and the samples of a step are the longest run of
 // first ones of which that holds for every pair -- the same samples, in the same
 // order, as one by one.  (A sample that does not lower its own minimum -- a row
@@ -581,11 +581,25 @@ __device__ __forceinline__ float fps_lower(const float (&q)[DIM],
 constexpr int kFpsBatch = 8; // at most; 8 x 8 pairs are a wave's lanes
 
 struct FpsTable {
-  float4 head[kWave];   // value, row, x, y
-  float2 tail[kWave];   // z, rest
-  float4 first[kFpsBatch]; // of rank i: x, y, z, value
-  float2 more[kFpsBatch];  // its rest and row
+  float4 head[kWave];      // value, row, first two coordinates
+  float4 tail[kWave];      // the other coordinates, rest, its tie
+  float4 first[kFpsBatch]; // of rank i: value, coordinates
+  float4 more[kFpsBatch];  // fourth coordinate, rest, row, tie of rest
 };
+// Among rows of the value `rest` of a group the complement of the smallest tie;
+// where nobody looked for it, a number that is before all others.
+constexpr uint32_t kFpsAnyTie = 0xffffffffu;
+template <int DIM>
+__device__ __forceinline__ void
+fps_enter(FpsTable &t, int group, uint32_t val, uint32_t row,
+          const float (&x)[DIM], uint32_t rest, uint32_t rest_tie) {
+  t.head[group] = make_float4(__uint_as_float(val), __uint_as_float(row), x[0],
+                              DIM > 1 ? x[DIM > 1 ? 1 : 0] : 0.0f);
+  t.tail[group] = make_float4(DIM > 2 ? x[DIM > 2 ? 2 : 0] : 0.0f,
+                              DIM > 3 ? x[DIM > 3 ? 3 : 0] : 0.0f,
+                              __uint_as_float(rest),
+                              __uint_as_float(rest_tie));
+}
 
 // Waits for this workgroup's LDS traffic and meets its other waves (global
 // stores stay in flight: for them __syncthreads).
@@ -596,16 +610,16 @@ __device__ __forceinline__ void fps_meet() {
 // Entries to samples, by a workgroup of 64 / OWN waves, after the entries of
 // this step are written; wave w ranks entries OWN w ...  Returns the number of
 // samples, the same for all waves; lane i % 8 holds the i-th: coordinates and
-// row of the example.
-template <int OWN>
-__device__ __forceinline__ int fps_rank(FpsTable &t, int wave, float (&sx)[3],
-                                        uint32_t &row) {
+// `row`.  `rel`: from an entry's row to its number in the example.
+template <int OWN, int DIM, typename Rel>
+__device__ __forceinline__ int fps_rank(FpsTable &t, int wave, Rel rel,
+                                        float (&sx)[DIM], uint32_t &row) {
   const int lane = threadIdx.x & (kWave - 1);
   fps_meet();
   const uint32_t v = __float_as_uint(t.head[lane].x);
   const int own = wave * OWN + (lane & (OWN - 1));
   const float4 h = t.head[own];
-  const float2 g = t.tail[own];
+  const float4 g = t.tail[own];
   int before[OWN], equal = 0;
 #pragma unroll
   for (int e = 0; e < OWN; ++e) {
@@ -614,7 +628,7 @@ __device__ __forceinline__ int fps_rank(FpsTable &t, int wave, float (&sx)[3],
     equal += __builtin_popcountll(__ballot(v >= mine)) - before[e];
   }
   if (__builtin_expect(equal != OWN, 0)) {
-    const uint32_t tie = fps_tie(__float_as_uint(t.head[lane].y));
+    const uint32_t tie = fps_tie(rel(__float_as_uint(t.head[lane].y)));
 #pragma unroll
     for (int e = 0; e < OWN; ++e) {
       const uint32_t mine = lane_value(v, wave * OWN + e);
@@ -629,24 +643,34 @@ __device__ __forceinline__ int fps_rank(FpsTable &t, int wave, float (&sx)[3],
   for (int e = 1; e < OWN; ++e)
     rank = (lane & (OWN - 1)) == e ? before[e] : rank;
   if (lane < OWN && rank < kFpsBatch) {
-    t.first[rank] = make_float4(h.z, h.w, g.x, h.x);
-    t.more[rank] = make_float2(g.y, h.y);
+    t.first[rank] = make_float4(h.x, h.z, h.w, g.x);
+    t.more[rank] = make_float4(g.y, g.z, h.y, g.w);
   }
   fps_meet();
   const int a = lane & (kFpsBatch - 1), b = lane / kFpsBatch;
   const float4 ra = t.first[a], rb = t.first[b];
-  const float2 ma = t.more[a];
-  const float d0 = ra.x - rb.x, d1 = ra.y - rb.y, d2 = ra.z - rb.z;
-  float dd = d0 * d0;
-  dd = __builtin_fmaf(d1, d1, dd);
-  dd = __builtin_fmaf(d2, d2, dd);
-  // (infinite: one of the two has no distance to itself)
-  const bool apart = dd >= rb.w && dd < __builtin_inff() && ma.x < rb.w;
+  const float4 ma = t.more[a];
+  const float xa[4] = {ra.y, ra.z, ra.w, ma.x};
+  const float xb[4] = {rb.y, rb.z, rb.w, DIM > 3 ? t.more[b].x : 0.0f};
+  float dd = 0.0f;
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) {
+    const float df = xa[c] - xb[c];
+    dd = c == 0 ? df * df : __builtin_fmaf(df, df, dd);
+    sx[c] = xa[c];
+  }
+  row = __float_as_uint(ma.z);
+  // (infinite: one of the two has no distance to itself; 0: nor is a minimum of 0
+  // lowered by its own sample)
+  bool apart = dd >= rb.x && dd < __builtin_inff() && ma.y <= rb.x &&
+               rb.x > 0.0f;
+  const bool equal_rest = a < b && apart && ma.y == rb.x;
+  if (__builtin_expect(__ballot(equal_rest) != 0, 0)) {
+    // the next row of that group comes after this one
+    const uint32_t tie = ~fps_tie(rel(__float_as_uint(t.more[b].z)));
+    apart = apart && (!equal_rest || __float_as_uint(ma.w) < tie);
+  }
   const uint64_t ends = __ballot(a < b && !apart);
-  sx[0] = ra.x;
-  sx[1] = ra.y;
-  sx[2] = ra.z;
-  row = __float_as_uint(ma.y);
   return ends != 0 ? (int)__builtin_ctzll(ends) / kFpsBatch : kFpsBatch;
 }
 
@@ -755,12 +779,15 @@ fps_curve_order(const float *__restrict__ rows, int count, int d,
 }
 
 // Putting the rows in buckets has to pay: with fewer samples than this every
-// row is looked at instead.  Kernel, us, all rows / buckets, per example 1, 128,
-// 256, 512 samples: 16 x 2,048 rows 14 / 33, 85 / 99, 159 / 162, 306 / 292;
-// 16 x 4,096 14 / 50, 97 / 127, 181 / 193, 349 / 319; 16 x 8,192 15 / 85,
-// 116 / 170, 217 / 243, 424 / 383; 8 x 16,384 16 / 155, 178 / 296, 342 / 398,
-// 669 / 584; 16 x 4,096 of 4 dimensions 14 / 57, 105 / 158, 196 / 240, 384 / 386.
-constexpr int fps_few(int dim) { return dim > 3 ? 480 : 340; }
+// row is looked at instead.  Kernel, us, all rows / buckets, 16 examples of 100,
+// 220, 300 samples each, from LDS: 1,100 rows 59 / 93, 126 / 137, 171 / 163; 2,048
+// rows 59 / 101, 127 / 144, 171 / 170; 4,096 69 / 118, 149 / 163, 202 / 185; 8,192
+// 85 / 168, 182 / 219, 247 / 247; 4,096 of 4 dimensions 76 / 142, 160 / 195, 218 /
+// 229.  From registers (fps_bucket_kernel), 256 and 512 samples: 8 x 16,384 342 /
+// 398, 669 / 584; 16 x 4,096 of 4 dimensions 196 / 240, 384 / 386.
+constexpr int fps_few(int dim, bool lds) {
+  return lds ? (dim > 3 ? 340 : 280) : (dim > 3 ? 480 : 340);
+}
 
 // Such an example by a workgroup of 1,024 threads.  Up to 8,192 rows half of
 // them hold the rows, which leaves fewer results to hand over per step; the
@@ -789,20 +816,17 @@ __device__ __forceinline__ void fps_few_samples(
   }
 }
 
-// Examples of up to 4,096 R rows: everything a step needs of a bucket -- its
-// box and its best row -- is in one lane of EVERY wave's registers (64 buckets
-// of 64 R rows), the rows and their running minima are in LDS.  All waves see
-// the same buckets pass, so they share them out without asking each other,
-// whichever wave is free of work taking part; the new best of a bucket
-// reaches the other waves through LDS, one barrier per step.
+// Examples of up to 4,096 R rows in LDS: 64 buckets of 64 R rows, which are the
+// groups of the samples' table.  A step: wave i tests all boxes against sample i,
+// the waves share the buckets that some sample is near to, the entries are ranked.
 //
-// 16 uniform clouds, a quarter sampled, per step (before: every row of a cloud
-// from the registers of 8 waves): 2,048 rows 0.60 -> 0.57 us, 4,096 0.68 ->
-// 0.58, 8,192 0.84 -> 0.65.  About 0.55 us of that is the chain of a step with a
-// single bucket, ~100 dependent instructions and three LDS round trips; at
-// 1,024 rows fps_reg_kernel's chain is as short.  16 waves measured faster
-// than 8 (0.62 us at 4,096 rows) and 4 (0.83): a wave rarely meets two of the
-// 9 buckets that pass.
+// 16 uniform clouds, a quarter sampled, calls (before: one sample per step): 2,048
+// rows 274 -> 231 us, 4,096 552 -> 365, 8,192 1,175 -> 687; 4,096 rows of 4
+// dimensions 646 -> 458; on 33^3 places (ties) 4,096 rows 727 -> 499, 8,192 1,588 ->
+// 960.  Of the 365 us 50 are the order of the rows; the rest are some 200 steps of
+// about 3,700 cycles, a chain of three barriers with five LDS trips between them.
+// 16 waves measured faster than 8 (452 us): two or more of the 20 buckets of a step
+// then fall to one wave.
 template <int DIM, int W, int R>
 __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
     const float *__restrict__ src, const int64_t *__restrict__ ptr,
@@ -818,8 +842,9 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
   __shared__ __align__(16) float rows_lds[CAP * STRIDE];
   __shared__ uint16_t perm[CAP + 2];
   __shared__ float part[2 * 3][W];
-  __shared__ __align__(16) float table[2][kWave][8]; // value, place, x ...
-  __shared__ uint16_t sampled[kWave];
+  __shared__ FpsTable table;
+  __shared__ uint32_t hits_of[2][kWave]; // bit i: sample i is near to the bucket
+  __shared__ uint16_t sampled[2 * kWave];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -832,7 +857,7 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
   const int64_t o_end = out_ptr[b + 1];
   if (o_begin >= o_end)
     return;
-  if (o_end - o_begin < fps_few(DIM) || count <= 0) {
+  if (o_end - o_begin < fps_few(DIM, true) || count <= 0) {
     fps_few_samples<DIM, CAP, T>(src, ptr, out_ptr, start, d, out, count,
                                  (int)(o_end - o_begin));
     return;
@@ -870,14 +895,14 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
   __syncthreads();
 
   // lane = bucket: its box, and the best of its rows
-  float blo[DIM], bhi[DIM], bx[DIM];
+  float blo[DIM], bhi[DIM];
 #pragma unroll
   for (int c = 0; c < DIM; ++c) {
     blo[c] = __builtin_inff();
     bhi[c] = -__builtin_inff();
-    bx[c] = 0.0f;
   }
   {
+    float *low_of = &table.head[0].x, *high_of = &table.tail[0].x;
     // (a wave goes through its share of the buckets, a row per lane; the
     // boxes then travel through the table)
     for (int i = wave; i < buckets; i += W) {
@@ -907,8 +932,8 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
           h[c] = __builtin_fmaxf(h[c], __shfl_xor(h[c], sh));
         }
         if (lane == 0) {
-          table[0][i][c] = l[c];
-          table[1][i][c] = h[c];
+          low_of[i * 4 + c] = l[c];
+          high_of[i * 4 + c] = h[c];
         }
       }
     }
@@ -916,49 +941,58 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
     if (lane < buckets) {
 #pragma unroll
       for (int c = 0; c < DIM; ++c) {
-        blo[c] = table[0][lane][c];
-        bhi[c] = table[1][lane][c];
+        blo[c] = low_of[lane * 4 + c];
+        bhi[c] = high_of[lane * 4 + c];
       }
     }
     __syncthreads();
   }
-  uint32_t val = lane < buckets ? kFpsUnseen : 0u;
-  int place = CAP; // (of no row)
-
-  float cur[DIM];
+  // lane i: sample i of the step
+  float sx[DIM];
+  int got = 1;
   {
     const int64_t first = start_idx + (start ? start[b] : 0);
     if (tid == 0)
       out[o_begin] = first;
 #pragma unroll
     for (int c = 0; c < DIM; ++c)
-      cur[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
+      sx[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
   }
+  if (wave == 0) {
+    const float none[DIM] = {};
+    fps_enter<DIM>(table, lane, lane < buckets ? kFpsUnseen : 0u, CAP, none, 0u,
+                   kFpsAnyTie);
+    hits_of[0][lane] = 0u;
+    hits_of[1][lane] = 0u;
+  }
+  __syncthreads();
 
-  // of the lanes `who` of equal value the one whose place holds the row that
-  // comes first in the reference's order
-  auto first_of = [&](uint64_t who, int at_place) -> int {
-    if (__builtin_expect((who & (who - 1)) != 0, 0))
-      return fps_first(who, perm[at_place]);
-    return (int)__builtin_ctzll(who);
-  };
   const int steps = (int)(o_end - o_begin);
-  // (where the loop stands in the 32-byte windows of instruction fetch moves a
-  // step by 3 %: 16 x 4,096 rows, 1,024 samples, every other place in
-  // turn 562, 576, 577 and 560 us, the last of which this is)
-  asm volatile(".p2align 5\n\t.fill 6, 4, 0xbf800000"); // s_nop 0
-  for (int m = 1; m < steps; ++m) {
-    const int par = m & 1;
-    const bool passes =
-        !(fps_box_distance<DIM>(cur, blo, bhi) >= __uint_as_float(val));
-    const uint64_t pass = __ballot(passes);
+  int m = 1, par = 0;
+  while (m < steps) {
+    // sample i against the boxes by wave i
+    static_assert(W >= kFpsBatch, "a wave per sample");
+    if (wave < got) {
+      float q[DIM];
+#pragma unroll
+      for (int c = 0; c < DIM; ++c)
+        q[c] = lane_value(sx[c], wave);
+      if (!(fps_box_distance<DIM>(q, blo, bhi) >= table.head[lane].x))
+        atomicOr(&hits_of[par][lane], 1u << wave);
+    }
+    fps_meet();
+    const uint32_t hits = hits_of[par][lane];
+    par ^= 1;
+    if (wave == 0)
+      hits_of[par][lane] = 0u;
+    const uint64_t pass = __ballot(hits != 0);
     const int passing = __builtin_popcountll(pass);
     // (how many passing buckets come before this lane's)
     const int before = __builtin_amdgcn_mbcnt_hi(
         (uint32_t)(pass >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)pass, 0u));
-    const int rank = passes ? before : -1;
+    const int item = hits != 0 ? before : -1;
     for (int j = wave; j < passing; j += W) {
-      const int bucket = (int)__builtin_ctzll(__ballot(rank == j));
+      const int bucket = (int)__builtin_ctzll(__ballot(item == j));
       float x[R][DIM], low[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -978,71 +1012,81 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
           low[r] = row[AT_M];
         }
       }
+      uint32_t some = lane_value(hits, bucket);
+      do {
+        float q[DIM];
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        low[r] = fps_lower<DIM>(cur, x[r], low[r]);
+        for (int c = 0; c < DIM; ++c)
+          q[c] = lane_value(sx[c], __builtin_ctz(some));
+        some &= some - 1;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          low[r] = fps_lower<DIM>(q, x[r], low[r]);
+      } while (some != 0);
+#pragma unroll
+      for (int r = 0; r < R; ++r)
         rows_lds[((bucket * R + r) * kWave + lane) * STRIDE + AT_M] = low[r];
-      }
-      uint32_t most = __float_as_uint(low[0]);
-      if (R == 2)
-        most = max(most, __float_as_uint(low[R - 1]));
-      const uint32_t top = wave_umax(most);
-      // which of a lane's two rows has the value; both: the earlier one
-      int at_place = bucket * R * kWave + lane;
-      int r = 0;
+      // a lane's largest minimum and the other one
+      uint32_t most = __float_as_uint(low[0]), less = 0u;
+      int at_r = 0;
       if (R == 2) {
-        r = __float_as_uint(low[0]) == top ? 0 : 1;
-        const bool both = r == 0 && __float_as_uint(low[R - 1]) == top;
-        if (__builtin_expect(__ballot(both) != 0, 0)) {
-          if (both && fps_tie(perm[at_place + kWave]) < fps_tie(perm[at_place]))
-            r = 1;
+        const uint32_t other = __float_as_uint(low[R - 1]);
+        at_r = other > most ? 1 : 0;
+        less = min(most, other);
+        most = max(most, other);
+      }
+      const uint32_t top = wave_umax(most);
+      const bool is = most == top;
+      const uint64_t who = __ballot(is);
+      uint32_t next = wave_umax(is ? less : most);
+      uint32_t next_tie = kFpsAnyTie;
+      int at = (int)__builtin_ctzll(who);
+      if (__builtin_expect((who & (who - 1)) != 0 || next == top, 0)) {
+        // rows of equal value: the one that comes first in the reference's order
+        next = top;
+        uint32_t first = 0u, second = 0u; // (complements of the smallest ties)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const bool equal = __float_as_uint(low[r]) == top;
+          const uint32_t t =
+              equal ? ~fps_tie(perm[(bucket * R + r) * kWave + lane]) : 0u;
+          at_r = t > first ? r : at_r;
+          second = max(second, min(first, t));
+          first = max(first, t);
         }
-        at_place += r * kWave;
+        const uint32_t t_top = wave_umax(first);
+        at = (int)__builtin_ctzll(__ballot(first == t_top));
+        next_tie = wave_umax(lane == at ? second : first);
       }
-      const int at = first_of(__ballot(most == top), at_place);
       if (lane == at) {
-        float *e = table[par][bucket];
-        float4 head;
-        head.x = __uint_as_float(top);
-        head.y = __int_as_float(at_place);
-        head.z = r ? x[R - 1][0] : x[0][0];
-        head.w = r ? x[R - 1][DIM > 1 ? 1 : 0] : x[0][DIM > 1 ? 1 : 0];
-        *reinterpret_cast<float4 *>(e) = head;
+        float best[DIM];
 #pragma unroll
-        for (int c = 2; c < DIM; ++c)
-          e[2 + c] = r ? x[R - 1][c] : x[0][c];
+        for (int c = 0; c < DIM; ++c)
+          best[c] = R == 2 && at_r ? x[R - 1][c] : x[0][c];
+        fps_enter<DIM>(table, bucket, top,
+                       (uint32_t)((bucket * R + at_r) * kWave + lane), best,
+                       next, next_tie);
       }
     }
-    fps_meet();
-    if (passes) {
-      const float *e = table[par][lane];
-      const float4 head = *reinterpret_cast<const float4 *>(e);
-      val = __float_as_uint(head.x);
-      place = __float_as_int(head.y);
-      bx[0] = head.z;
-      if (DIM > 1)
-        bx[DIM > 1 ? 1 : 0] = head.w;
-#pragma unroll
-      for (int c = 2; c < DIM; ++c)
-        bx[c] = e[2 + c];
-    }
-    const uint32_t top = wave_umax(val);
-    const int at = first_of(__ballot(val == top), place);
-#pragma unroll
-    for (int c = 0; c < DIM; ++c)
-      cur[c] = lane_value(bx[c], at);
+    uint32_t chosen;
+    got = fps_rank<kWave / W, DIM>(
+        table, wave, [&](uint32_t place) { return (uint32_t)perm[place]; }, sx,
+        chosen);
+    got = min(got, steps - m);
     if (wave == 0) {
       // (64 samples are written out at a time: the store's way to memory is
       // then no part of a step)
-      const int chosen = (int)lane_value((uint32_t)place, at);
-      if (lane == 0)
-        sampled[m & (kWave - 1)] = (uint16_t)chosen;
-      if ((m & (kWave - 1)) == kWave - 1 || m == steps - 1) {
-        const int from = m & ~(kWave - 1);
-        if (from + lane <= m && from + lane > 0)
-          out[o_begin + from + lane] = start_idx + perm[sampled[lane]];
+      if (lane < got)
+        sampled[(m + lane) & (2 * kWave - 1)] = (uint16_t)chosen;
+      const int from = m & ~(kWave - 1), to = m + got;
+      if (to >= from + kWave || to == steps) {
+        // (the last step may end one block of samples and begin another)
+        for (int k = from + lane; k < to; k += kWave)
+          if (k > 0 && (k < from + kWave || to == steps))
+            out[o_begin + k] = start_idx + perm[sampled[k & (2 * kWave - 1)]];
       }
     }
+    m += got;
   }
 }
 
@@ -1075,7 +1119,7 @@ __global__ __launch_bounds__(W *kWave) void fps_bucket_kernel(
   const int64_t o_end = out_ptr[b + 1];
   if (o_begin >= o_end)
     return;
-  if (o_end - o_begin < fps_few(DIM) || count <= 0) {
+  if (o_end - o_begin < fps_few(DIM, false) || count <= 0) {
     fps_few_samples<DIM, CAP, T>(src, ptr, out_ptr, start, d, out, count,
                                  (int)(o_end - o_begin));
     return;
@@ -1262,9 +1306,9 @@ __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
 // 2.79 ms per call, 1.47 -> 0.71 us per sample of the longest scan (before: one
 // sample per step).  Uniform rows, samples: 8 x 20,000, 2,000 each 2.22 -> 1.16
 // ms; 8 x 60,000, 600 each 1.27 -> 0.83; 2 x 300,000, 900 each 4.54 -> 2.93.
-// Where nearly every maximum is a tie (200,000 rows on 33^3 places) groups hold
-// several rows of the largest value and a step ends with its first sample: 5.2
-// -> 6.1 ms.
+// Where nearly every maximum is a tie (4 x 200,000 rows on 33^3 places, 2,000 samples
+// each) 5.2 -> 3.2 ms; without the tie of `rest` a step there ends with its first
+// sample (6.0 ms).
 // Bound by the chain of a step, about 7,000 cycles for five samples of a scan of
 // 200,000 rows: 1,400 to the list, 2,500 + 1,200 for the 21 buckets of the list
 // (their rows at the 64 bytes per clock that a compute unit gets from the L2, and
@@ -1287,7 +1331,7 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
   // found in them
   __shared__ uint32_t list[kWave * W];
   __shared__ float4 found_head[kWave * W]; // value, row, x, y
-  __shared__ float2 found_tail[kWave * W]; // z, rest
+  __shared__ float4 found_tail[kWave * W]; // z, rest, its tie, -
   __shared__ int items[2];
   __shared__ uint32_t sampled[2 * kWave];
   const int tid = threadIdx.x;
@@ -1317,7 +1361,7 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
   const int bucket = wave * run + slot;
 
   float blo[DIM], bhi[DIM], bx[DIM];
-  uint32_t val, rest = 0u, rel = kFpsNoRow;
+  uint32_t val, rest = 0u, rest_tie = kFpsAnyTie, rel = kFpsNoRow;
   {
     const int k = bucket;
     const bool any = slot < run && k < buckets;
@@ -1508,19 +1552,21 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
       wave_umax_of<U>(next);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
+        uint32_t next_tie = kFpsAnyTie;
         int at = (int)__builtin_ctzll(who[u]);
         if (__builtin_expect((who[u] & (who[u] - 1)) != 0 || next[u] == top[u],
                              0)) {
           // rows of equal value: the one that comes first in the reference's
           // order
           next[u] = top[u];
-          uint32_t first = 0u; // (the complement of the smallest tie)
+          uint32_t first = 0u, second = 0u; // (complements of smallest ties)
           auto among = [&](const float4(&row)[R], const float(&m)[R]) {
 #pragma unroll
             for (int r = 0; r < R; ++r) {
               const bool is = __float_as_uint(m[r]) == top[u];
               const uint32_t t = is ? ~fps_tie(__float_as_uint(row[r].w)) : 0u;
               const bool take = t > first;
+              second = max(second, min(first, t));
               first = max(first, t);
               f_rel[u] = take ? __float_as_uint(row[r].w) : f_rel[u];
               f_x[u][0] = take ? row[r].x : f_x[u][0];
@@ -1547,13 +1593,15 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
           }
           const uint32_t most = wave_umax(first);
           at = (int)__builtin_ctzll(__ballot(first == most));
+          next_tie = wave_umax(lane == at ? second : first);
         }
         if (lane == at) {
           found_head[first_item + u * W] =
               make_float4(__uint_as_float(top[u]), __uint_as_float(f_rel[u]),
                           f_x[u][0], f_x[u][1]);
           found_tail[first_item + u * W] =
-              make_float2(f_x[u][2], __uint_as_float(next[u]));
+              make_float4(f_x[u][2], __uint_as_float(next[u]),
+                          __uint_as_float(next_tie), 0.0f);
         }
       }
     };
@@ -1565,40 +1613,42 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
     fps_meet();
     if (hits != 0) {
       const float4 h = found_head[item];
-      const float2 t = found_tail[item];
+      const float4 t = found_tail[item];
       val = __float_as_uint(h.x);
       rel = __float_as_uint(h.y);
       bx[0] = h.z;
       bx[1] = h.w;
       bx[2] = t.x;
       rest = __float_as_uint(t.y);
+      rest_tie = __float_as_uint(t.z);
     }
     if (pass != 0 || m == 1) {
       // the best of every group
       const uint32_t top = row16_umax_all(val);
       bool is = val == top;
       uint32_t next = row16_umax_all(is ? rest : val);
-      const uint64_t who = __ballot(is);
-      if (__builtin_expect(__builtin_popcountll(who) > 4, 0)) {
-        // several of a group (at most `top` is left without the first one)
+      uint32_t next_tie = next == top ? rest_tie : kFpsAnyTie;
+      if (__builtin_expect(__builtin_popcountll(__ballot(is)) > 4, 0)) {
+        // several of a group
         const uint32_t t = is ? ~fps_tie(rel) : 0u;
         const uint32_t first = row16_umax_all(t);
-        const uint64_t mine = who >> (lane & 48) & 0xffffull;
-        next = (mine & (mine - 1)) != 0 ? top : next;
-        is = is && t == first;
+        const bool it = is && t == first;
+        const uint32_t other =
+            row16_umax_all(it ? (rest == top ? rest_tie : 0u) : t);
+        next = other != 0u ? top : next;
+        next_tie = other != 0u ? other : next_tie;
+        is = it;
       }
       wave_val = max(max(lane_value(top, 0), lane_value(top, 16)),
                      max(lane_value(top, 32), lane_value(top, 48)));
       if (is) {
-        table.head[wave * 4 + lane / 16] =
-            make_float4(__uint_as_float(top), __uint_as_float(rel), bx[0],
-                        bx[1]);
-        table.tail[wave * 4 + lane / 16] =
-            make_float2(bx[2], __uint_as_float(next));
+        fps_enter<DIM>(table, wave * 4 + lane / 16, top, rel, bx, next,
+                       next_tie);
       }
     }
     uint32_t chosen;
-    got = fps_rank<kWave / W>(table, wave, sx, chosen);
+    got = fps_rank<kWave / W, DIM>(
+        table, wave, [](uint32_t row) { return row; }, sx, chosen);
     got = min(got, steps - m);
     if (wave == 0) {
       // (64 samples are written out at a time)

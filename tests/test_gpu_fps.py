@@ -115,25 +115,29 @@ def test_skipped_rows_change_nothing(oracle, rows, d, kind):
     assert (got == want).all()
 
 
-# 32,768 / 65,536 / 262,144: buckets of one, two, four pieces of 64 rows and of
-# several times four; hundreds of samples, most of them several to a step
+# 1,025 / 4,097: buckets of 64 and 128 rows in LDS; 32,768 / 65,536 / 262,144:
+# of one, two, four pieces of 64 rows in memory and of several times four; hundreds
+# of samples, most of them several to a step
 @pytest.mark.parametrize("kind", ["uniform", "grid", "copies", "clusters"])
-@pytest.mark.parametrize("rows", [16385, 32769, 65537, 262145])
-def test_several_samples_per_step_are_those_one_by_one(oracle, rows, kind):
+@pytest.mark.parametrize("rows,d", [(1025, 3), (2048, 2), (4096, 4), (4097, 1),
+                                    (8192, 3), (16385, 3), (32769, 3),
+                                    (65537, 2), (262145, 3)])
+def test_several_samples_per_step_are_those_one_by_one(oracle, rows, d, kind):
     rng = np.random.default_rng(rows)
-    ptr = np.cumsum([0, 40, rows, 17000]).astype(np.int64)
+    second = max(1000, rows // 16)
+    ptr = np.cumsum([0, 40, rows, second]).astype(np.int64)
     n = ptr[-1]
     if kind == "uniform":
-        x = rng.random((n, 3))
+        x = rng.random((n, d))
     elif kind == "grid":  # most largest minima are ties
-        x = rng.integers(0, 24, (n, 3))
+        x = rng.integers(0, 24, (n, d))
     elif kind == "copies":  # samples whose neighbours come to a minimum of 0
-        x = rng.random((700, 3))[rng.integers(0, 700, n)]
+        x = rng.random((700, d))[rng.integers(0, 700, n)]
     else:
-        x = rng.random((12, 3))[rng.integers(0, 12, n)]
-        x = x + 0.003 * rng.standard_normal((n, 3))
+        x = rng.random((12, d))[rng.integers(0, 12, n)]
+        x = x + 0.003 * rng.standard_normal((n, d))
     x = x.astype(np.float32)
-    share = np.array([1.0, 750.0 / rows, 800.0 / 17000])
+    share = np.array([1.0, 750.0 / rows, 800.0 / second])
     start = np.array([7, rows - 1, 0], dtype=np.int64)
     got = gpu_fps(oracle, x, ptr, share, start)
     want = oracle.fps_op(x, ptr, share, start)
