@@ -10,19 +10,12 @@
  *
  * What the library keeps between calls:
  *   - per calling thread: pca_last_error's text, the one-shot
- *     pca_time_next_search request, the last size query of the binned
- *     searches' sort;
- *   - per device, from the first call that needs them until the process ends:
- *     the address of the fixed scratch of pca_knn_fixed_scratch, and -- for
- *     the *_binned entry points with 131,072 queries or more -- one extra
- *     stream and two events: the queries are ordered on that stream beside
- *     the rows on the caller's (forked and joined with events inside the
- *     call).  Calls on one device queue that part of their work under a mutex,
- *     one after the other; PCA_BINNED_SIDE_STREAM=0 in the environment keeps
- *     everything on the caller's stream.
+ *     pca_time_next_search request;
+ *   - per device, from the first call that needs it until the process ends:
+ *     the address of the fixed scratch of pca_knn_fixed_scratch.
  * Stream capture: the *_binned entry points refuse a stream that is being
- * captured into a graph (PCA_ERR_UNSUPPORTED: their sorts clear buffers with
- * memset nodes); all other device entry points record kernels only.
+ * captured into a graph (PCA_ERR_UNSUPPORTED; the scanning entry points take
+ * it); all other device entry points record kernels only.
  *
  * The reference (rusty1s/pytorch_cluster 1.6.3) has no C ABI: its boundary is
  * the TorchScript operator registry.  Each entry point below names the

@@ -277,9 +277,8 @@ size_t nearest_workspace(int64_t n, int64_t m, int64_t d,
   return bytes;
 }
 
-// The binned entry points sort with rocPRIM, whose clears of histograms are
-// memset nodes in a captured graph: they are refused while `stream` is being
-// captured (the scanning entry points can be captured).
+// The binned entry points are refused while `stream` is being captured (the
+// scanning entry points can be captured, and the operators take those then).
 bool being_captured(hipStream_t stream) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
@@ -291,8 +290,8 @@ bool being_captured(hipStream_t stream) {
 
 int refuse_capture(const char *entry) {
   return fail(PCA_ERR_UNSUPPORTED,
-              "%s cannot be captured into a graph (its sorts clear their "
-              "buffers with memset nodes); use the scanning entry point",
+              "%s cannot be captured into a graph; use the scanning entry "
+              "point",
               entry);
 }
 

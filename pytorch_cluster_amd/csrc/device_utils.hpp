@@ -319,6 +319,15 @@ __device__ __forceinline__ int find_segment64(const int64_t *__restrict__ ptr,
   return lo;
 }
 
+// floats as integers of the same order (for atomic min / max)
+__device__ __forceinline__ int ordered_int(float f) {
+  const int i = __float_as_int(f);
+  return i >= 0 ? i : i ^ 0x7fffffff;
+}
+__device__ __forceinline__ float from_ordered_int(int i) {
+  return __int_as_float(i >= 0 ? i : i ^ 0x7fffffff);
+}
+
 // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  This
 // maps the hardware block id to a logical one such that blocks with
 // neighbouring logical ids (which scan the same segment of x) land on the same
@@ -330,11 +339,13 @@ __device__ __forceinline__ int xcd_swizzle(int block, int grid) {
 // Work items of ragged segments, by a single workgroup of kPlanThreads
 // threads: work_start[b] = exclusive scan of ceil(rows of segment b /
 // per_item), work_start[num_segments] = their total.  ptr == nullptr: one
-// segment of m rows.  `partial`: kPlanThreads ints of LDS.
+// segment of m rows.  Segments of at most `above` rows count none.  `partial`:
+// kPlanThreads ints of LDS.
 constexpr int kPlanThreads = 1024;
 __device__ __forceinline__ void
 plan_segments(const int64_t *__restrict__ ptr, int m, int num_segments,
-              int per_item, int *__restrict__ work_start, int *partial) {
+              int per_item, int *__restrict__ work_start, int *partial,
+              int above = 0) {
   const int tid = threadIdx.x;
   // contiguous chunk of segments per thread
   const int per_thread = (num_segments + kPlanThreads - 1) / kPlanThreads;
@@ -346,7 +357,7 @@ plan_segments(const int64_t *__restrict__ ptr, int m, int num_segments,
     const int64_t lo = ptr ? ptr[b] : 0;
     const int64_t hi = ptr ? ptr[b + 1] : m;
     const int len = (int)max((int64_t)0, hi - lo);
-    sum += (len + per_item - 1) / per_item;
+    sum += len > above ? (len + per_item - 1) / per_item : 0;
   }
   partial[tid] = sum;
   __syncthreads();
@@ -363,7 +374,7 @@ plan_segments(const int64_t *__restrict__ ptr, int m, int num_segments,
     const int64_t lo = ptr ? ptr[b] : 0;
     const int64_t hi = ptr ? ptr[b + 1] : m;
     const int len = (int)max((int64_t)0, hi - lo);
-    run += (len + per_item - 1) / per_item;
+    run += len > above ? (len + per_item - 1) / per_item : 0;
   }
   if (tid == kPlanThreads - 1)
     work_start[num_segments] = partial[tid];

@@ -11,7 +11,7 @@
 // Per call: every segment's x rows are ordered along a space-filling curve
 // (30-bit places on a Hilbert curve through the segment's bounding box, its
 // cells the voxels of the reference's grid clustering,
-// csrc/cuda/grid_cuda.cu:10-25, sorted by rocPRIM's radix sort), copied in that order together
+// csrc/cuda/grid_cuda.cu:10-25, sorted by curve_order.hip), copied in that order together
 // with their row numbers, and cut into tiles of 32 rows with a bounding box
 // each.  The queries are ordered the same way, so the 64 queries of a wave
 // (one per lane) are neighbours in space and share one bounding box.
@@ -51,10 +51,7 @@
 #include <climits>
 #include <cstdlib>
 #include <cstring>
-#include <mutex>
 #include <type_traits>
-
-#include <rocprim/device/device_radix_sort.hpp>
 
 namespace pca {
 
@@ -64,55 +61,71 @@ constexpr int kBinQueueCap = 16;  // parked rows per lane
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// floats as integers of the same order (for atomic min / max)
-__device__ __forceinline__ int ordered_int(float f) {
-  const int i = __float_as_int(f);
-  return i >= 0 ? i : i ^ 0x7fffffff;
-}
-__device__ __forceinline__ float from_ordered_int(int i) {
-  return __int_as_float(i >= 0 ? i : i ^ 0x7fffffff);
-}
-
 // The first launch of a binned search (a call starts with kernels so short
-// that the host's launch rate sets the pace: one launch instead of five):
-// workgroups 0-3 count the work items of the segments - tiles and groups of
-// tiles of x, tasks of 64 and of 32 queries of y -, the others empty the
-// segment boxes and the extra task slots.  seg_box: [num_segments][6] = lower
-// corner, upper corner (ordered integers).
+// that the host's launch rate sets the pace: one launch instead of many): a
+// workgroup per plan counts the work items of the segments - tiles and groups of
+// tiles of x, tasks of 64 and of 32 queries of y, the sort's -, the others empty
+// the segment boxes, the buckets and the extra task slots.  seg_box:
+// [num_segments][6] = lower corner, upper corner (ordered integers).
 struct BinsSetup {
-  const int64_t *ptr_x, *ptr_y;
-  int n, m, num_segments;
-  int *tile_start, *group_start, *wave_start, *half_start;
+  struct Plan {
+    const int64_t *ptr;
+    int rows, per_item;
+    int *start;
+    int above; // segments of at most so many rows count none
+  } plan[10];
+  int plans, num_segments;
   int *seg_box;
-  // task slots (task_span_kernel's; task_extra == 0: no tasks wanted)
+  uint32_t *total[2]; // the sort's buckets
+  int totals[2];
+  // task slots (task_spans'; task_extra == 0: no tasks wanted)
   int task_blocks, task_extra;
   int *extra_used;
   int2 *task_desc;
+
+  void add(const int64_t *ptr, int rows, int per_item, int *start,
+           int above = 0) {
+    plan[plans++] = {ptr, rows, per_item, start, above};
+  }
+  void add_sort(int side, const int64_t *ptr, int rows, void *scratch) {
+    const CurveSortPlan s = curve_sort_plan(scratch, rows, num_segments);
+    add(ptr, rows, s.bucket_rows, s.bucket_start);
+    add(ptr, rows, s.tile_rows, s.tile_start, s.bucket_rows);
+    add(ptr, rows, s.chunk_rows, s.chunk_start, s.bucket_rows);
+    total[side] = s.total;
+    totals[side] = s.buckets;
+  }
 };
 __global__ __launch_bounds__(kPlanThreads) void bins_setup_kernel(BinsSetup s) {
   __shared__ int partial[kPlanThreads];
   const int job = blockIdx.x; // (uniform over the workgroup)
-  if (job == 0) {
-    plan_segments(s.ptr_x, s.n, s.num_segments, kBinTile, s.tile_start,
-                  partial);
-  } else if (job == 1) {
-    plan_segments(s.ptr_x, s.n, s.num_segments, kBinTile * kBinGroup,
-                  s.group_start, partial);
-  } else if (job == 2) {
-    plan_segments(s.ptr_y, s.m, s.num_segments, kWave, s.wave_start, partial);
-  } else if (job == 3) {
-    plan_segments(s.ptr_y, s.m, s.num_segments, kWave / 2, s.half_start,
-                  partial);
+  if (job < s.plans) {
+    const BinsSetup::Plan p = s.plan[job];
+    plan_segments(p.ptr, p.rows, s.num_segments, p.per_item, p.start, partial,
+                  p.above);
   } else {
-    const int i = (job - 4) * kPlanThreads + (int)threadIdx.x;
+    const int i = (job - s.plans) * kPlanThreads + (int)threadIdx.x;
     if (i < 6 * s.num_segments)
       s.seg_box[i] = (i % 6) < 3 ? INT_MAX : INT_MIN;
+#pragma unroll
+    for (int side = 0; side < 2; ++side)
+      if (i < s.totals[side])
+        s.total[side][i] = 0u;
     // the extra task slots start out unused
     if (i == 0 && s.extra_used != nullptr)
       *s.extra_used = 0;
     if (i < s.task_extra)
       s.task_desc[s.task_blocks + i] = make_int2(0, 0);
   }
+}
+hipError_t launch_bins_setup(const BinsSetup &s, hipStream_t stream) {
+  const int resets = std::max(std::max(6 * s.num_segments, s.task_extra),
+                              std::max(s.totals[0], s.totals[1]));
+  hipLaunchKernelGGL(
+      bins_setup_kernel,
+      dim3(s.plans + (resets + kPlanThreads - 1) / kPlanThreads),
+      dim3(kPlanThreads), 0, stream, s);
+  return hipGetLastError();
 }
 
 // Bounding box of the finite coordinates of every segment; grid (parts,
@@ -130,17 +143,24 @@ __global__ __launch_bounds__(kBlock) void seg_box_kernel(
       lo[c] = __builtin_inff();
       hi[c] = -__builtin_inff();
     }
+    // (eight rows at a time, the last one again beyond the end)
+    const int64_t step = (int64_t)gridDim.x * kBlock;
     for (int64_t i = begin + (int64_t)blockIdx.x * kBlock + threadIdx.x;
-         i < end; i += (int64_t)gridDim.x * kBlock) {
+         i < end; i += 8 * step) {
+      float v[8][3];
 #pragma unroll
-      for (int c = 0; c < 3; ++c)
-        if (c < d) {
-          const float v = x[(size_t)i * d + c];
-          if (__builtin_fabsf(v) < __builtin_inff()) {
-            lo[c] = __builtin_fminf(lo[c], v);
-            hi[c] = __builtin_fmaxf(hi[c], v);
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          v[u][c] = c < d ? x[(size_t)min(i + u * step, end - 1) * d + c] : 0.0f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          if (__builtin_fabsf(v[u][c]) < __builtin_inff()) {
+            lo[c] = __builtin_fminf(lo[c], v[u][c]);
+            hi[c] = __builtin_fmaxf(hi[c], v[u][c]);
           }
-        }
     }
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
@@ -173,56 +193,19 @@ __global__ __launch_bounds__(kBlock) void seg_box_kernel(
   }
 }
 
-// keys[i] = (segment << 3 axis_bits) | place of row i along the curve through
-// its segment's box of x rows, axis_bits bits per axis; vals[i] = i.
-__global__ __launch_bounds__(kBlock) void curve_keys_kernel(
-    const float *__restrict__ pts, const int64_t *__restrict__ ptr, int count,
-    int d, int num_segments, const int *__restrict__ seg_box,
-    int axis_bits, uint32_t *__restrict__ keys,
-    uint32_t *__restrict__ vals, bool searched_side) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= count)
-    return;
-  // rows of x behind the last pointer belong to no segment (a caller's
-  // batch_size below the ids in use: the reference never searches them,
-  // csrc/cuda/utils.cuh:11-19): they sort behind every segment's rows
-  if (searched_side && ptr != nullptr && (int64_t)i >= ptr[num_segments]) {
-    keys[i] = 0xffffffffu;
-    vals[i] = (uint32_t)i;
-    return;
-  }
-  // rows in front of the first pointer sort in front (the sort is stable and
-  // their numbers are the lowest)
-  if (searched_side && ptr != nullptr && (int64_t)i < ptr[0]) {
-    keys[i] = 0u;
-    vals[i] = (uint32_t)i;
-    return;
-  }
-  const int seg = find_segment64(ptr, num_segments, i);
-  float v[3], lo[3], hi[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    v[c] = c < d ? pts[(size_t)i * d + c] : 0.0f;
-    lo[c] = from_ordered_int(seg_box[seg * 6 + c]);
-    hi[c] = from_ordered_int(seg_box[seg * 6 + 3 + c]);
-  }
-  const uint32_t code = curve_place(v, lo, hi, d, axis_bits);
-  keys[i] = ((uint32_t)seg << (3 * axis_bits)) | code;
-  vals[i] = (uint32_t)i;
-}
-
 // Rows in curve order with their row numbers (plain and as the matrix-core
 // filter takes them), and the box of every tile of 32: half a wave per tile.
-__global__ __launch_bounds__(kBlock) void gather_tiles_kernel(
-    const float *__restrict__ x, const int64_t *__restrict__ ptr_x, int n,
-    int d, int num_segments, const int *__restrict__ tile_start,
-    const uint32_t *__restrict__ perm, float4 *__restrict__ rows,
-    uint4 *__restrict__ packed, Box *__restrict__ box) {
-  const int gt = (blockIdx.x * kBlock + threadIdx.x) / kBinTile;
+__device__ __forceinline__ void
+gather_tiles(int block, const float *__restrict__ x,
+             const int64_t *__restrict__ ptr_x, int n, int d, int num_segments,
+             const int *__restrict__ tile_start,
+             const uint32_t *__restrict__ perm, float4 *__restrict__ rows,
+             uint4 *__restrict__ packed, Box *__restrict__ box) {
+  const int gt = (block * kBlock + (int)threadIdx.x) / kBinTile;
   const int r = threadIdx.x & (kBinTile - 1);
   // behind the last row a tile of rows that never pass the filter (operand
   // w = NaN), so that a fetch of a whole tile stays inside the copy
-  if (blockIdx.x == 0 && threadIdx.x < kBinTile) {
+  if (block == 0 && threadIdx.x < kBinTile) {
     packed[(size_t)(n + r) * 2] = make_uint4(0u, 0x7fc00000u, 0u, 0u);
     packed[(size_t)(n + r) * 2 + 1] = make_uint4(0u, 0u, 0u, 0u);
   }
@@ -277,11 +260,11 @@ __global__ __launch_bounds__(kBlock) void gather_tiles_kernel(
 
 // Boxes of the groups of kBinGroup consecutive tiles of a segment: one wave
 // per group.
-__global__ __launch_bounds__(kBlock) void group_boxes_kernel(
-    int num_segments, const int *__restrict__ tile_start,
-    const int *__restrict__ group_start, const Box *__restrict__ box,
-    Box *__restrict__ group_box) {
-  const int gg = (blockIdx.x * kBlock + threadIdx.x) / kWave;
+__device__ __forceinline__ void
+group_boxes(int block, int num_segments, const int *__restrict__ tile_start,
+            const int *__restrict__ group_start, const Box *__restrict__ box,
+            Box *__restrict__ group_box) {
+  const int gg = (block * kBlock + (int)threadIdx.x) / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   if (gg >= group_start[num_segments])
     return;
@@ -312,6 +295,48 @@ __global__ __launch_bounds__(kBlock) void group_boxes_kernel(
     group_box[gg].min_row = min_row;
     group_box[gg].pad = 0u;
   }
+}
+
+// The rows' tiles and the queries' tasks do not need each other: one launch for
+// tiles and task classes, one for groups of tiles and task places (952,000
+// queries among 119,000 rows: 9 us a call less than four launches).  Workgroups
+// from tile_blocks / group_blocks on are the tasks'.
+struct BinsRows {
+  const float *x;
+  const int64_t *ptr_x;
+  int n, d, num_segments, tile_blocks, group_blocks;
+  const int *tile_start, *group_start;
+  const uint32_t *perm;
+  float4 *rows;
+  uint4 *packed;
+  Box *box, *group_box;
+};
+struct BinsTasks {
+  int groups, blocks, extra;
+  int *extra_used;
+  int2 *desc;
+  uint32_t *cls, *order;
+  int *hist;
+};
+__global__ __launch_bounds__(kBlock) void
+tiles_and_tasks_kernel(BinsRows r, BinnedParams p, BinsTasks t) {
+  const int block = blockIdx.x;
+  if (block < r.tile_blocks)
+    gather_tiles(block, r.x, r.ptr_x, r.n, r.d, r.num_segments, r.tile_start,
+                 r.perm, r.rows, r.packed, r.box);
+  else
+    task_spans(p, block - r.tile_blocks, t.blocks, t.extra, t.extra_used,
+               t.desc, t.cls, t.hist);
+}
+__global__ __launch_bounds__(kBlock) void
+groups_and_tasks_kernel(BinsRows r, BinsTasks t) {
+  const int block = blockIdx.x;
+  if (block < r.group_blocks)
+    group_boxes(block, r.num_segments, r.tile_start, r.group_start, r.box,
+                r.group_box);
+  else
+    task_places(block - r.group_blocks, t.groups, t.blocks, t.extra,
+                t.extra_used, t.cls, t.hist, t.order);
 }
 
 template <int K>
@@ -725,15 +750,14 @@ __global__ __launch_bounds__(kBlock) void radius_binned_kernel(
 }
 
 struct BinnedLayout {
-  size_t seg_box, keys_a, keys_b, keys_x, keys_y, vals_a, vals_b, perm_x,
-      perm_y, rows, packed, box, group_box, tile_start, group_start,
-      wave_start, half_start, task_keys, sort_temp, side_temp;
+  size_t seg_box, keys_x, keys_y, perm_x, perm_y, rows, packed, box, group_box,
+      tile_start, group_start, wave_start, half_start, task_keys, sort_x,
+      sort_y;
   int tiles_bound, groups_bound;
   size_t total() const {
-    return seg_box + keys_a + keys_b + keys_x + keys_y + vals_a + vals_b +
-           perm_x + perm_y + rows + packed + box + group_box + tile_start +
-           group_start + wave_start + half_start + task_keys + sort_temp +
-           side_temp;
+    return seg_box + keys_x + keys_y + perm_x + perm_y + rows + packed + box +
+           group_box + tile_start + group_start + wave_start + half_start +
+           task_keys + sort_x + sort_y;
   }
 };
 
@@ -747,37 +771,6 @@ int segment_bits(int num_segments) {
 }
 int axis_bits(int num_segments) {
   return std::min(10, (32 - segment_bits(num_segments)) / 3);
-}
-
-// rocPRIM's radix sort with this file's choices (measured on 1.03 M pairs
-// with 30-bit keys: the library's default - merge sort up to 2^20 items, 19
-// launches - 170 us; its one-sweep radix sort as configured by default
-// 140 us; the same with workgroups of 1,024 threads x 8 items and the
-// match-based ranking 109 us, and 98 us with 10 bits per pass, which saves
-// the fourth pass).  Below 200,000 items the merge sort is quicker (54 us
-// against 68 us at 131,072).
-template <unsigned int RadixBits>
-using SortConfig = rocprim::radix_sort_config<
-    rocprim::default_config, rocprim::default_config,
-    rocprim::radix_sort_onesweep_config<
-        rocprim::kernel_config<256, 12>, rocprim::kernel_config<1024, 8>,
-        RadixBits, rocprim::block_radix_rank_algorithm::match>,
-    200000>;
-
-hipError_t sort_pairs(void *temp, size_t &temp_bytes, const uint32_t *keys_in,
-                      uint32_t *keys_out, const uint32_t *vals_in,
-                      uint32_t *vals_out, int count, int num_segments,
-                      hipStream_t stream) {
-  const unsigned int bits = (unsigned int)std::max(
-      segment_bits(num_segments) + 3 * axis_bits(num_segments), 1);
-  // (10 bits per pass where that takes fewer passes than 8)
-  if ((bits + 9) / 10 < (bits + 7) / 8)
-    return rocprim::radix_sort_pairs<SortConfig<10>>(
-        temp, temp_bytes, keys_in, keys_out, vals_in, vals_out,
-        (unsigned int)count, 0u, bits, stream, false);
-  return rocprim::radix_sort_pairs<SortConfig<8>>(
-      temp, temp_bytes, keys_in, keys_out, vals_in, vals_out,
-      (unsigned int)count, 0u, bits, stream, false);
 }
 
 // Tasks in a row that one XCD takes, as a power of two: long runs keep what a
@@ -827,14 +820,8 @@ size_t task_buffer_words(int m, int num_segments) {
 BinnedLayout binned_layout(int n, int m, int num_segments) {
   BinnedLayout w;
   w.seg_box = align256(sizeof(int) * 6 * (size_t)num_segments);
-  // unsorted (key, row) of the rows (a) and of the queries (b): the two are
-  // sorted at the same time
-  w.keys_a = align256(sizeof(uint32_t) * (size_t)n);
-  w.keys_b = align256(sizeof(uint32_t) * (size_t)m);
   w.keys_x = align256(sizeof(uint32_t) * (size_t)n);
   w.keys_y = align256(sizeof(uint32_t) * (size_t)m);
-  w.vals_a = align256(sizeof(uint32_t) * (size_t)n);
-  w.vals_b = align256(sizeof(uint32_t) * (size_t)m);
   w.perm_x = align256(sizeof(uint32_t) * (size_t)n);
   w.perm_y = align256(sizeof(uint32_t) * (size_t)m);
   // (padded: the search reads rows four at a time)
@@ -851,34 +838,8 @@ BinnedLayout binned_layout(int n, int m, int num_segments) {
   // per task slot: descriptor (2 words), class, place in the starting order;
   // a histogram of the classes per kBlock blocks
   w.task_keys = align256(sizeof(uint32_t) * task_buffer_words(m, num_segments));
-  // (the sort's size queries are kept per thread for the sizes asked last:
-  // a call asks for the same layout three times -- workspace query, argument
-  // check, carving)
-  struct SortSizes {
-    int n = -1, m = -1, num_segments = -1;
-    size_t tx = 0, ty = 0;
-    bool sized = false;
-  };
-  thread_local SortSizes last;
-  if (last.n != n || last.m != m || last.num_segments != num_segments) {
-    last.n = n;
-    last.m = m;
-    last.num_segments = num_segments;
-    last.tx = last.ty = 0;
-    const hipError_t ex =
-        sort_pairs(nullptr, last.tx, nullptr, nullptr, nullptr, nullptr, n,
-                   num_segments, nullptr);
-    const hipError_t ey =
-        sort_pairs(nullptr, last.ty, nullptr, nullptr, nullptr, nullptr, m,
-                   num_segments, nullptr);
-    last.sized = ex == hipSuccess && ey == hipSuccess;
-  }
-  const size_t tx = last.tx, ty = last.ty;
-  // (a failed size query leaves a size no workspace can meet)
-  const bool sized = last.sized;
-  w.sort_temp = sized ? align256(tx) : ~(size_t)0 / 2;
-  // (the queries are sorted beside the rows' stream)
-  w.side_temp = sized ? align256(ty) : 0;
+  w.sort_x = curve_sort_bytes(n, num_segments);
+  w.sort_y = curve_sort_bytes(m, num_segments);
   return w;
 }
 
@@ -900,59 +861,6 @@ struct Bins {
   int code_bits;
 };
 
-// A second stream of the device: the queries are ordered there while the rows
-// are ordered on the caller's stream (both chains are short kernels that
-// leave most of the device idle).  The library keeps one such stream and two
-// events per device, made at the first call that needs them and held until
-// the process ends; fork / join are recorded and waited for within one call,
-// under g_lane_mutex (held only while that call queues its work).
-struct SideLane {
-  hipStream_t stream = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
-};
-constexpr int kMaxDevices = 64;
-constexpr int kSideLaneQueries = 131072; // fewer queries stay on one stream
-std::mutex g_lane_mutex;
-SideLane g_lanes[kMaxDevices];
-
-// The current device's lane, made at its first use (g_lane_mutex held).
-// PCA_BINNED_SIDE_STREAM=0 (diagnostic switch) keeps everything on the
-// caller's stream: `lane` stays null.
-hipError_t side_lane(SideLane *&lane) {
-  lane = nullptr;
-  const char *env = getenv("PCA_BINNED_SIDE_STREAM");
-  if (env != nullptr && env[0] == '0')
-    return hipSuccess;
-  int device = 0;
-  hipError_t err = hipGetDevice(&device);
-  if (err != hipSuccess)
-    return err;
-  if (device < 0 || device >= kMaxDevices)
-    return hipSuccess;
-  SideLane &mine = g_lanes[device];
-  if (mine.stream == nullptr) {
-    SideLane made;
-    if ((err = hipStreamCreateWithFlags(&made.stream, hipStreamNonBlocking)) !=
-        hipSuccess)
-      return err;
-    if ((err = hipEventCreateWithFlags(&made.fork, hipEventDisableTiming)) !=
-            hipSuccess ||
-        (err = hipEventCreateWithFlags(&made.join, hipEventDisableTiming)) !=
-            hipSuccess) {
-      // nothing half-made is kept
-      if (made.fork != nullptr)
-        (void)hipEventDestroy(made.fork);
-      (void)hipStreamDestroy(made.stream);
-      return err;
-    }
-    mine = made;
-  }
-  lane = &mine;
-  return hipSuccess;
-}
-
-// The tasks (blocks of 32 queries, long spans split) and their starting
-// order, from the sorted keys of the queries; results in `bins`.
 // The pieces of the task-slot buffer.
 struct TaskBuffers {
   int blocks, slots, groups; // groups: workgroups of kBlock blocks
@@ -972,35 +880,6 @@ TaskBuffers task_buffers(uint32_t *task_keys, int m, int num_segments) {
   t.order = t.cls + t.slots;
   t.hist = reinterpret_cast<int *>(t.order + t.slots);
   return t;
-}
-
-// The tasks (blocks of 32 queries, long spans split) and their starting
-// order, from the sorted keys of the queries; results in `bins`.  (The extra
-// slots were cleared by bins_setup_kernel.)
-hipError_t order_tasks(const SearchInput &in, Bins &bins, uint32_t *task_keys,
-                       hipStream_t stream) {
-  const TaskBuffers t = task_buffers(task_keys, in.m, in.num_segments);
-  const int extra = t.slots - t.blocks;
-  // (what task_span_kernel reads)
-  BinnedParams p;
-  memset(&p, 0, sizeof(p));
-  p.ptr_y = in.ptr_y;
-  p.m = in.m;
-  p.num_segments = in.num_segments;
-  p.wave_start = bins.half_start;
-  p.keys_y = bins.keys_y;
-  p.code_bits = 3 * axis_bits(in.num_segments);
-  hipLaunchKernelGGL(task_span_kernel, dim3(t.groups), dim3(kBlock), 0, stream,
-                     p, t.blocks, extra, t.extra_used, t.desc, t.cls, t.hist);
-  hipLaunchKernelGGL(task_order_kernel, dim3(t.groups), dim3(kBlock), 0,
-                     stream, t.blocks, extra, t.extra_used, t.cls, t.hist,
-                     t.order);
-  bins.task_desc = t.desc;
-  bins.task_order = t.order;
-  bins.task_slots = t.slots;
-  bins.task_grid = xcd_run_grid(t.slots);
-  bins.code_bits = p.code_bits;
-  return hipGetLastError();
 }
 
 // Workgroups per segment of seg_box_kernel: enough to fill the device when
@@ -1024,12 +903,8 @@ hipError_t prepare_bins(const SearchInput &in, void *scratch, bool with_tasks,
     return static_cast<void *>(piece);
   };
   int *seg_box = static_cast<int *>(take(lay.seg_box));
-  uint32_t *keys_a = static_cast<uint32_t *>(take(lay.keys_a));
-  uint32_t *keys_b = static_cast<uint32_t *>(take(lay.keys_b));
   uint32_t *keys_x = static_cast<uint32_t *>(take(lay.keys_x));
   uint32_t *keys_y = static_cast<uint32_t *>(take(lay.keys_y));
-  uint32_t *vals_a = static_cast<uint32_t *>(take(lay.vals_a));
-  uint32_t *vals_b = static_cast<uint32_t *>(take(lay.vals_b));
   uint32_t *perm_x = static_cast<uint32_t *>(take(lay.perm_x));
   uint32_t *perm_y = static_cast<uint32_t *>(take(lay.perm_y));
   float4 *rows = static_cast<float4 *>(take(lay.rows));
@@ -1041,8 +916,8 @@ hipError_t prepare_bins(const SearchInput &in, void *scratch, bool with_tasks,
   int *wave_start = static_cast<int *>(take(lay.wave_start));
   int *half_start = static_cast<int *>(take(lay.half_start));
   uint32_t *task_keys = static_cast<uint32_t *>(take(lay.task_keys));
-  void *sort_temp = take(lay.sort_temp);
-  void *side_temp = take(lay.side_temp);
+  void *sort_x = take(lay.sort_x);
+  void *sort_y = take(lay.sort_y);
 
   const float *x = static_cast<const float *>(in.x);
   const float *y = static_cast<const float *>(in.y);
@@ -1074,26 +949,23 @@ hipError_t prepare_bins(const SearchInput &in, void *scratch, bool with_tasks,
 
   hipError_t err;
   {
-    BinsSetup setup;
-    setup.ptr_x = in.ptr_x;
-    setup.ptr_y = in.ptr_y;
-    setup.n = in.n;
-    setup.m = in.m;
+    BinsSetup setup = {};
     setup.num_segments = nseg;
-    setup.tile_start = tile_start;
-    setup.group_start = group_start;
-    setup.wave_start = wave_start;
-    setup.half_start = half_start;
+    setup.add(in.ptr_x, in.n, kBinTile, tile_start);
+    setup.add(in.ptr_x, in.n, kBinTile * kBinGroup, group_start);
+    setup.add(in.ptr_y, in.m, kWave, wave_start);
+    setup.add(in.ptr_y, in.m, kWave / 2, half_start);
+    setup.add_sort(0, in.ptr_x, in.n, sort_x);
+    if (!self_search)
+      setup.add_sort(1, in.ptr_y, in.m, sort_y);
     setup.seg_box = seg_box;
     const TaskBuffers t = task_buffers(task_keys, in.m, nseg);
     setup.task_blocks = t.blocks;
     setup.task_extra = with_tasks ? t.slots - t.blocks : 0;
     setup.extra_used = with_tasks ? t.extra_used : nullptr;
     setup.task_desc = t.desc;
-    const int resets = std::max(6 * nseg, setup.task_extra);
-    hipLaunchKernelGGL(bins_setup_kernel,
-                       dim3(4 + (resets + kPlanThreads - 1) / kPlanThreads),
-                       dim3(kPlanThreads), 0, stream, setup);
+    if ((err = launch_bins_setup(setup, stream)) != hipSuccess)
+      return err;
   }
   {
     hipLaunchKernelGGL(seg_box_kernel,
@@ -1104,102 +976,46 @@ hipError_t prepare_bins(const SearchInput &in, void *scratch, bool with_tasks,
   if ((err = hipGetLastError()) != hipSuccess)
     return err;
 
-  // The queries' chain (keys, sort, tasks) runs beside the rows' chain: it
-  // forks off the caller's stream here and joins it again below - when it is
-  // long enough to pay for the two waits between streams (measured, with
-  // rocPRIM's default sort configuration: 0.82 -> 0.77 ms for 1.03 M rows and
-  // 258 k queries, 0.68 -> 0.59 ms for 500 k queries among 1 M rows; a loss
-  // of 0.02 ms at 65 k queries).  When the
-  // rows' order serves the queries too, only the tasks are left to order,
-  // which follows the rows' sort on the caller's stream.
-  const bool beside = !self_search && in.m >= kSideLaneQueries;
-  std::unique_lock<std::mutex> lane_lock(g_lane_mutex, std::defer_lock);
-  SideLane *lane = nullptr;
-  hipStream_t side = stream;
-  // Once the side stream has work of this call, the caller's stream waits for
-  // it on EVERY way out of this function -- also the failing ones: the
-  // workspace may be reused as soon as the caller's stream gets there.
-  struct Rejoin {
-    SideLane *&lane;
-    hipStream_t stream;
-    bool forked = false, joined = false;
-    hipError_t join() {
-      if (!forked || joined || lane == nullptr)
-        return hipSuccess;
-      joined = true;
-      hipError_t e = hipEventRecord(lane->join, lane->stream);
-      if (e == hipSuccess)
-        e = hipStreamWaitEvent(stream, lane->join, 0);
-      return e;
-    }
-    ~Rejoin() { (void)join(); }
-  } rejoin{lane, stream};
-  auto fork = [&]() -> hipError_t {
-    lane_lock.lock();
-    hipError_t e = side_lane(lane);
-    if (e != hipSuccess || lane == nullptr)
-      return e;
-    side = lane->stream;
-    e = hipEventRecord(lane->fork, stream);
-    if (e == hipSuccess)
-      e = hipStreamWaitEvent(side, lane->fork, 0);
-    rejoin.forked = e == hipSuccess;
-    return e;
-  };
-  auto queries_chain = [&]() -> hipError_t {
-    hipError_t e = hipSuccess;
-    if (!self_search) {
-      hipLaunchKernelGGL(curve_keys_kernel,
-                         dim3((in.m + kBlock - 1) / kBlock), dim3(kBlock), 0,
-                         side, y, in.ptr_y, in.m, in.d, nseg, seg_box,
-                         axis_bits(nseg), keys_b, vals_b, false);
-      if ((e = hipGetLastError()) != hipSuccess)
-        return e;
-      size_t bytes = lay.side_temp;
-      if ((e = sort_pairs(side_temp, bytes, keys_b, keys_y, vals_b, perm_y,
-                          in.m, nseg, side)) != hipSuccess)
-        return e;
-    }
-    if (with_tasks)
-      e = order_tasks(in, bins, task_keys, side);
-    return e;
-  };
-  // (the fork is where the segment boxes are done; the longer of the two
-  // chains is handed to the device first)
-  if (beside && (err = fork()) != hipSuccess)
+  const CurveSortSide sides[2] = {{x, in.ptr_x, in.n, sort_x, keys_x, perm_x},
+                                  {y, in.ptr_y, in.m, sort_y, keys_y, perm_y}};
+  if ((err = launch_curve_sort(sides, self_search ? 1 : 2, in.d, nseg,
+                               axis_bits(nseg), seg_box, stream)) != hipSuccess)
     return err;
-  const bool queries_first = beside && in.m > in.n;
-  if (queries_first && (err = queries_chain()) != hipSuccess)
-    return err;
-  hipLaunchKernelGGL(curve_keys_kernel, dim3((in.n + kBlock - 1) / kBlock),
-                     dim3(kBlock), 0, stream, x, in.ptr_x, in.n, in.d, nseg,
-                     seg_box, axis_bits(nseg), keys_a, vals_a, true);
-  if ((err = hipGetLastError()) != hipSuccess)
-    return err;
-  size_t sort_bytes = lay.sort_temp;
-  if ((err = sort_pairs(sort_temp, sort_bytes, keys_a, keys_x, vals_a, perm_x,
-                        in.n, nseg, stream)) != hipSuccess)
-    return err;
-  if (!queries_first && (!self_search || with_tasks) &&
-      (err = queries_chain()) != hipSuccess)
-    return err;
-  {
-    const int per_block = kBlock / kBinTile;
-    hipLaunchKernelGGL(gather_tiles_kernel,
-                       dim3((lay.tiles_bound + per_block - 1) / per_block),
-                       dim3(kBlock), 0, stream, x, in.ptr_x, in.n, in.d, nseg,
-                       tile_start, perm_x, plain_rows ? rows : nullptr, packed,
-                       box);
-    const int groups_per_block = kBlock / kWave;
-    hipLaunchKernelGGL(
-        group_boxes_kernel,
-        dim3((lay.groups_bound + groups_per_block - 1) / groups_per_block),
-        dim3(kBlock), 0, stream, nseg, tile_start, group_start, box,
-        group_box);
+  // the rows' tiles; the tasks (blocks of 32 queries, long spans split) and their
+  // starting order, from the sorted keys of the queries (the extra slots were
+  // cleared by bins_setup_kernel)
+  const TaskBuffers t = task_buffers(task_keys, in.m, nseg);
+  const BinsTasks tasks = {t.groups, t.blocks, t.slots - t.blocks,
+                           t.extra_used, t.desc, t.cls, t.order, t.hist};
+  const int per_block = kBlock / kBinTile, groups_per_block = kBlock / kWave;
+  const BinsRows r = {
+      x,        in.ptr_x,   in.n,
+      in.d,     nseg,       (lay.tiles_bound + per_block - 1) / per_block,
+      (lay.groups_bound + groups_per_block - 1) / groups_per_block,
+      tile_start, group_start, perm_x, plain_rows ? rows : nullptr, packed,
+      box,      group_box};
+  BinnedParams p; // (what task_spans reads)
+  memset(&p, 0, sizeof(p));
+  p.ptr_y = in.ptr_y;
+  p.m = in.m;
+  p.num_segments = nseg;
+  p.wave_start = half_start;
+  p.keys_y = keys_y;
+  p.code_bits = 3 * axis_bits(nseg);
+  const int task_blocks = with_tasks ? t.groups : 0;
+  hipLaunchKernelGGL(tiles_and_tasks_kernel, dim3(r.tile_blocks + task_blocks),
+                     dim3(kBlock), 0, stream, r, p, tasks);
+  hipLaunchKernelGGL(groups_and_tasks_kernel,
+                     dim3(r.group_blocks + task_blocks), dim3(kBlock), 0,
+                     stream, r, tasks);
+  if (with_tasks) {
+    bins.task_desc = t.desc;
+    bins.task_order = t.order;
+    bins.task_slots = t.slots;
+    bins.task_grid = xcd_run_grid(t.slots);
+    bins.code_bits = p.code_bits;
   }
-  if ((err = hipGetLastError()) != hipSuccess)
-    return err;
-  return rejoin.join();
+  return hipGetLastError();
 }
 
 void fill_params(BinnedParams &p, const SearchInput &in, const Bins &bins,
@@ -1238,28 +1054,15 @@ void fill_params(BinnedParams &p, const SearchInput &in, const Bins &bins,
 // that order only (fps): boxes, keys and the sort of prepare_bins.
 namespace {
 struct CurveLayout {
-  size_t seg_box, keys, keys_out, vals, perm, temp;
-  size_t total() const {
-    return seg_box + keys + keys_out + vals + perm + temp;
-  }
+  size_t seg_box, keys, perm, sort;
+  size_t total() const { return seg_box + keys + perm + sort; }
 };
 CurveLayout curve_layout(int n, int num_segments) {
   CurveLayout w;
   w.seg_box = align256(sizeof(int) * 6 * (size_t)num_segments);
-  w.keys = w.keys_out = w.vals = w.perm =
-      align256(sizeof(uint32_t) * (size_t)n);
-  size_t temp = 0;
-  const hipError_t err = sort_pairs(nullptr, temp, nullptr, nullptr, nullptr,
-                                    nullptr, n, num_segments, nullptr);
-  // (a failed size query leaves a size no workspace can meet)
-  w.temp = err == hipSuccess ? align256(temp) : ~(size_t)0 / 2;
+  w.keys = w.perm = align256(sizeof(uint32_t) * (size_t)n);
+  w.sort = curve_sort_bytes(n, num_segments);
   return w;
-}
-__global__ __launch_bounds__(kBlock) void seg_box_reset_kernel(
-    int num_segments, int *__restrict__ seg_box) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < 6 * num_segments)
-    seg_box[i] = (i % 6) < 3 ? INT_MAX : INT_MIN;
 }
 } // namespace
 
@@ -1279,28 +1082,26 @@ hipError_t launch_curve_order(const float *x, const int64_t *ptr, int n, int d,
   };
   int *seg_box = static_cast<int *>(take(lay.seg_box));
   uint32_t *keys = static_cast<uint32_t *>(take(lay.keys));
-  uint32_t *keys_out = static_cast<uint32_t *>(take(lay.keys_out));
-  uint32_t *vals = static_cast<uint32_t *>(take(lay.vals));
   uint32_t *order = static_cast<uint32_t *>(take(lay.perm));
-  void *temp = take(lay.temp);
-  hipLaunchKernelGGL(seg_box_reset_kernel,
-                     dim3((6 * num_segments + kBlock - 1) / kBlock),
-                     dim3(kBlock), 0, stream, num_segments, seg_box);
+  void *sort = take(lay.sort);
+  *perm = order;
+  BinsSetup setup = {};
+  setup.num_segments = num_segments;
+  setup.seg_box = seg_box;
+  setup.add_sort(0, ptr, n, sort);
+  hipError_t err = launch_bins_setup(setup, stream);
+  if (err != hipSuccess)
+    return err;
   hipLaunchKernelGGL(seg_box_kernel,
                      dim3(seg_box_parts(n, num_segments),
                           std::min(num_segments, 65535)),
                      dim3(kBlock), 0, stream, x, ptr, n, d, num_segments,
                      seg_box);
-  hipLaunchKernelGGL(curve_keys_kernel, dim3((n + kBlock - 1) / kBlock),
-                     dim3(kBlock), 0, stream, x, ptr, n, d, num_segments,
-                     seg_box, axis_bits(num_segments), keys, vals, true);
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess)
+  if ((err = hipGetLastError()) != hipSuccess)
     return err;
-  size_t bytes = lay.temp;
-  *perm = order;
-  return sort_pairs(temp, bytes, keys, keys_out, vals, order, n, num_segments,
-                    stream);
+  const CurveSortSide side = {x, ptr, n, sort, keys, order};
+  return launch_curve_sort(&side, 1, d, num_segments, axis_bits(num_segments),
+                           seg_box, stream);
 }
 
 bool knn_binned_supported(int d, int k, bool cosine) {

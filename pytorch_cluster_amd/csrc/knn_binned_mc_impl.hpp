@@ -288,8 +288,8 @@ __device__ __forceinline__ void bin_box_of_lane(const Box &held, int src,
 // classes, every class sweeps the whole cloud, and the search kernel of the
 // 1 M-point LiDAR-like workload fetched 594 MB instead of 258 MB.)  Unused
 // slots come last (their waves leave at once).  It is a counting sort in two
-// launches: task_span_kernel leaves every block's class and a histogram of
-// the classes per workgroup of kBlock blocks, task_order_kernel turns them
+// launches: task_spans leaves every block's class and a histogram of
+// the classes per workgroup of kBlock blocks, task_places turns them
 // into places.
 constexpr int kTaskClasses = 64; // classes 0..11, 33 = unused block, rest empty
 
@@ -298,15 +298,15 @@ __device__ __forceinline__ uint32_t bin_task_class(uint32_t span) {
 }
 
 // cls: [bound] class per block; hist: [workgroups][kTaskClasses].
-__global__ __launch_bounds__(kBlock) void task_span_kernel(
-    BinnedParams p, int bound, int extra, int *__restrict__ extra_used,
-    int2 *__restrict__ desc, uint32_t *__restrict__ cls,
-    int *__restrict__ hist) {
+__device__ __forceinline__ void
+task_spans(const BinnedParams &p, int group, int bound, int extra,
+           int *__restrict__ extra_used, int2 *__restrict__ desc,
+           uint32_t *__restrict__ cls, int *__restrict__ hist) {
   __shared__ int count_of[kTaskClasses];
   if (threadIdx.x < kTaskClasses)
     count_of[threadIdx.x] = 0;
   __syncthreads();
-  const int block = blockIdx.x * kBlock + threadIdx.x;
+  const int block = group * kBlock + (int)threadIdx.x;
   if (block < bound) {
     int2 mine = make_int2(0, 0);
     uint32_t mine_class = 33u;
@@ -337,14 +337,15 @@ __global__ __launch_bounds__(kBlock) void task_span_kernel(
   }
   __syncthreads();
   if (threadIdx.x < kTaskClasses)
-    hist[blockIdx.x * kTaskClasses + threadIdx.x] = count_of[threadIdx.x];
+    hist[group * kTaskClasses + threadIdx.x] = count_of[threadIdx.x];
 }
 
-// Same grid as task_span_kernel.  order: [bound + extra] slot numbers.
-__global__ __launch_bounds__(kBlock) void task_order_kernel(
-    int bound, int extra, const int *__restrict__ extra_used,
-    const uint32_t *__restrict__ cls, const int *__restrict__ hist,
-    uint32_t *__restrict__ order) {
+// The same `groups` workgroups.  order: [bound + extra] slot numbers.
+__device__ __forceinline__ void
+task_places(int group, int groups, int bound, int extra,
+            const int *__restrict__ extra_used,
+            const uint32_t *__restrict__ cls, const int *__restrict__ hist,
+            uint32_t *__restrict__ order) {
   constexpr int kParts = kBlock / kTaskClasses;
   constexpr int kWaves = kBlock / kWave;
   __shared__ int before_part[kParts][kTaskClasses];
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(kBlock) void task_order_kernel(
   const int used = min(*extra_used, extra);
 
   // the extra slots: used ones first, the others behind everything
-  for (int i = blockIdx.x * kBlock + tid; i < extra; i += gridDim.x * kBlock)
+  for (int i = group * kBlock + tid; i < extra; i += groups * kBlock)
     order[i < used ? i : bound + i] = (uint32_t)(bound + i);
 
   // blocks of every class in the workgroups before this one, and in all
@@ -365,10 +366,11 @@ __global__ __launch_bounds__(kBlock) void task_order_kernel(
     const int c = tid & (kTaskClasses - 1);
     const int part = tid / kTaskClasses;
     int before = 0, total = 0;
-    for (int g = part; g < (int)gridDim.x; g += kParts) {
+#pragma unroll 8
+    for (int g = part; g < groups; g += kParts) {
       const int v = hist[g * kTaskClasses + c];
       total += v;
-      before += g < (int)blockIdx.x ? v : 0;
+      before += g < group ? v : 0;
     }
     before_part[part][c] = before;
     total_part[part][c] = total;
@@ -376,20 +378,25 @@ __global__ __launch_bounds__(kBlock) void task_order_kernel(
   }
   static_assert(kParts == kWaves, "one zeroing pass covers wave_count");
   __syncthreads();
-  if (tid == 0) {
-    int run = used;
-    for (int c = 0; c < kTaskClasses; ++c) {
-      int before = 0, total = 0;
-      for (int part = 0; part < kParts; ++part) {
-        before += before_part[part][c];
-        total += total_part[part][c];
-      }
-      base[c] = run + before;
-      run += total;
+  // (a class per lane of the first wave)
+  if (tid < kTaskClasses) {
+    static_assert(kTaskClasses == kWave, "one wave scans the classes");
+    int before = 0, total = 0;
+#pragma unroll
+    for (int part = 0; part < kParts; ++part) {
+      before += before_part[part][tid];
+      total += total_part[part][tid];
     }
+    int run = total; // of the classes up to this one
+#pragma unroll
+    for (int sh = 1; sh < kWave; sh <<= 1) {
+      const int o = __shfl_up(run, sh);
+      run += lane >= sh ? o : 0;
+    }
+    base[tid] = used + run - total + before;
   }
   // place inside the wave among the blocks of the same class
-  const int block = blockIdx.x * kBlock + tid;
+  const int block = group * kBlock + tid;
   const bool valid = block < bound;
   const int mine = valid ? (int)cls[block] : -1;
   int rank = 0;
@@ -430,7 +437,7 @@ __device__ __forceinline__ int bin_xcd_run(int workgroup, int run_log2) {
 constexpr int kBinMcBlock = kWave;
 
 // p.wave_start counts blocks of 32 queries, p.task_desc / p.task_order are
-// task_span_kernel's.  NEAREST: the search of the
+// task_spans's.  NEAREST: the search of the
 // `nearest` operator - one neighbour, limit 1e38, the reference's order among
 // equal distances (device_utils.hpp) - whose result goes to p.out_nearest as
 // a row number (0 when nothing qualified).

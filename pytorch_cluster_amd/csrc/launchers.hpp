@@ -315,6 +315,33 @@ hipError_t launch_nearest_any(int dtype, const SearchInput &in,
                               const int *work_start, int grid_bound,
                               int64_t *out, hipStream_t stream);
 
+// --- curve_order.hip: the sort of rows along the curve ------------------------
+
+// What has to be there before the sort, for plan_segments and a clear: where
+// the segments' items start - buckets of `bucket_rows` rows; of the segments of
+// more rows than that also tiles of `tile_rows` and chunks of `chunk_rows` rows -
+// and zeros in the buckets' totals.
+struct CurveSortPlan {
+  int bucket_rows, tile_rows, chunk_rows;
+  int *bucket_start, *tile_start, *chunk_start; // [num_segments + 1]
+  uint32_t *total;                              // [buckets]
+  int buckets;
+};
+size_t curve_sort_bytes(int n, int num_segments);
+CurveSortPlan curve_sort_plan(void *scratch, int n, int num_segments);
+// keys, perm: [n], of the rows of segments in order; rows of no segment are left
+// out.  seg_box: the segments' boxes (seg_box_kernel).
+struct CurveSortSide {
+  const float *pts;
+  const int64_t *ptr; // NULL: one segment of n rows
+  int n;
+  void *scratch; // curve_sort_bytes
+  uint32_t *keys, *perm;
+};
+hipError_t launch_curve_sort(const CurveSortSide *sides, int num_sides, int d,
+                             int num_segments, int axis_bits,
+                             const int *seg_box, hipStream_t stream);
+
 // --- knn_binned.hip: rows in curve order ------------------------------------
 
 // perm: the rows of every segment along a space-filling curve inside the

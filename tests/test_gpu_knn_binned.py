@@ -183,6 +183,51 @@ def test_queries_ordered_beside_the_rows(monkeypatch):
         assert torch.equal(capi.nearest_rows(x, y, px, py, binned=True), want)
 
 
+@pytest.mark.parametrize("kind", ["uniform", "equal", "two_places", "in_order"])
+@pytest.mark.parametrize("d", [1, 3])
+def test_order_of_rows_in_segments_of_every_size(kind, d):
+    """The sort in front of the search: segments of one bucket of 768 rows, just
+    more than that, several tiles of 2,048 rows, empty ones; rows that share a
+    place on the curve, rows in order already."""
+    rng = np.random.default_rng(31 + d)
+    sizes = [1, 767, 768, 769, 0, 1536, 1537, 2048, 2049, 5000, 3, 40000]
+    ptr = np.cumsum([0] + sizes).astype(np.int64)
+    n = ptr[-1]
+    x = rng.random((n, d))
+    if kind == "equal":
+        x[:] = 0.25
+    elif kind == "two_places":
+        x = np.where(rng.random((n, 1)) < 0.5, 0.0, 1.0) + np.zeros((n, d))
+    elif kind == "in_order":
+        x = np.sort(x, axis=0)
+    x = x.astype(np.float32)
+    some = np.concatenate([np.arange(a, b, 37)
+                           for a, b in zip(ptr[:-1], ptr[1:])])
+    ptr_y = np.searchsorted(some, ptr).astype(np.int64)
+    args = (dev(x), dev(x[some]), dev(ptr, torch.long),
+            dev(ptr_y, torch.long), 5)
+    want, want_dist = capi.knn_edges(*args, want_dist=True)
+    got, got_dist = capi.knn_edges(*args, want_dist=True, binned=True)
+    assert torch.equal(got, want)
+    assert torch.equal(got_dist.view(torch.int32),
+                       want_dist.view(torch.int32))
+
+
+def test_order_of_rows_in_buckets_merged_in_memory():
+    """Nine million rows of one segment: buckets of more than the 4,096 rows a
+    workgroup sorts on the chip, tiles of several steps; a clump that shares
+    few places beside a uniform cloud."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.rand(9_000_000, 3, generator=g, device=DEV)
+    x[::3] *= 1e-3
+    y = x[:: 9_000_000 // 500].contiguous()
+    ptr = torch.tensor([0, 40, x.shape[0]], device=DEV)
+    ptr_y = torch.tensor([0, 1, y.shape[0]], device=DEV)
+    want = capi.knn_edges(x, y, ptr, ptr_y, 4)[0]
+    got = capi.knn_edges(x, y, ptr, ptr_y, 4, binned=True)[0]
+    assert torch.equal(got, want)
+
+
 def test_crowded_cells_and_many_segments():
     """What the ordering of the rows has to cope with: most rows in a handful of
     cells (duplicates, a dense clump beside a sparse cloud), more segments
