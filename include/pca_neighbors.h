@@ -434,10 +434,11 @@ int pca_nearest_host(const void *x, const void *y, const int64_t *ptr_x,
  *            segments of up to 16,384 rows are sampled on chip, larger ones
  *            of up to 3 dimensions from rows in curve order, everything else
  *            row by row), or 0 = unknown (row by row; also the faster choice
- *            for a handful of samples from larger segments).
+ *            for a handful of samples from larger segments; more than 16,384
+ *            is the faster one for hundreds of samples from segments of
+ *            more than 8,192 rows).
  * A stream that is being captured into a graph may be used: segments beyond
- * 16,384 rows are then sampled row by row (their sort clears its buffers with
- * memset nodes).
+ * 16,384 rows (by max_segment_rows) are then sampled row by row.
  *
  * Stands under the reference operator
  *   torch_cluster::fps(src, ptr, ratio, random_start)

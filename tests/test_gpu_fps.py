@@ -144,6 +144,26 @@ def test_several_samples_per_step_are_those_one_by_one(oracle, rows, d, kind):
     assert (got == want).all()
 
 
+# 8,192 / 16,384 rows, 340 samples: where the entry points change between the
+# kernels on the chip and rows in curve order
+@pytest.mark.parametrize("rows,samples", [(8192, 400), (8193, 330), (8193, 345),
+                                          (16384, 345), (16384, 100)])
+@pytest.mark.parametrize("d", [3, 4])
+def test_entry_points_where_the_kernels_change(oracle, rows, samples, d):
+    rng = np.random.default_rng(rows + samples)
+    ptr = np.array([0, rows, rows + 500, 2 * rows + 400], dtype=np.int64)
+    x = rng.random((ptr[-1], d)).astype(np.float32)
+    batch = np.repeat(np.arange(3), np.diff(ptr))
+    ratio = samples / rows
+    want = oracle.fps_op(x, ptr, np.float32(ratio))
+    got = pca.fps(dev(x), dev(batch, torch.long), ratio, random_start=False)
+    assert (got.cpu().numpy() == want).all()
+    got = torch.ops.torch_cluster.fps(
+        dev(x), dev(ptr, torch.long),
+        torch.tensor(ratio, dtype=torch.float32, device=DEV), False)
+    assert (got.cpu().numpy() == want).all()
+
+
 # whole buckets (64 or 128 consecutive rows along the curve) at an infinite
 # distance: rows without a finite coordinate on an axis, rows and first samples
 # at infinity, squared gaps beyond the fp32 range
