@@ -693,6 +693,34 @@ knn_binned_mc_kernel(BinnedParams p) {
       return __ballot(searching && !(box_gap2(lo, hi, yq, yq) >= thresh));
     };
 
+    // All boxes of `todo` (a lane each) at once, query by query: the lanes
+    // whose box some query reaches.  A query costs 18 instructions, a pair of
+    // boxes above a trip through the LDS crossbar and 30; waves where the points
+    // are sparse, whose bounds reach most boxes, were bound by the latter.
+    // kNN over LiDAR-like scans, calls: 36,000 rows, every fourth a query, k = 4 /
+    // 16 239 -> 209, 388 -> 359 us; 3 x 60,000, every eighth 226 -> 212, 333 ->
+    // 319; the 8 scans of up to 200,000 531 -> 516; uniform clouds the same.
+    const int many = task.y + task.y / 2;
+    auto reachable_of = [&](const Box &held, uint64_t todo) __attribute__((always_inline)) {
+      // (the two lanes of a query have a bound each)
+      const float mine = searching ? thresh : -__builtin_inff();
+      const auto bounds = __builtin_amdgcn_permlane32_swap(
+          __float_as_uint(mine), __float_as_uint(mine), false, false);
+      const float bound =
+          __builtin_fmaxf(mine, __uint_as_float(half ? bounds[0] : bounds[1]));
+      uint64_t pass = 0;
+      for (int c = 0; c < task.y; ++c) {
+        float at[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          at[i] = __uint_as_float((uint32_t)__builtin_amdgcn_readlane(
+              (int)__float_as_uint(yq[i]), c));
+        const float limit = __uint_as_float((uint32_t)__builtin_amdgcn_readlane(
+            (int)__float_as_uint(bound), c));
+        pass |= __ballot(!(box_gap2(held.lo, held.hi, at, at) >= limit));
+      }
+      return pass & todo;
+    };
     // Groups of tiles, 64 at a time (one box per lane), nearest to the seed
     // tiles first; a group, then a tile, is looked into if its box is within
     // the wave's largest bound of the box around the wave's queries, and then
@@ -713,6 +741,8 @@ knn_binned_mc_kernel(BinnedParams p) {
       uint64_t g_todo =
           __ballot(g_mine < num_groups &&
                    !(box_gap2(g_box.lo, g_box.hi, q_lo, q_hi) >= reach));
+      if (__builtin_popcountll(g_todo) >= many)
+        g_todo = reachable_of(g_box, g_todo);
       const int g_at = min(max(centre - round * kWave, 0), kWave - 1);
       while (g_todo != 0) {
         const int g_lane = nearest_bit(g_todo, g_at);
@@ -731,6 +761,10 @@ knn_binned_mc_kernel(BinnedParams p) {
         // the tiles of the group that some query can reach, by its bound of
         // now; their rows are fetched one tile ahead of the scan
         uint64_t t_pass = 0;
+        if (__builtin_popcountll(t_todo) >= many) {
+          t_pass = reachable_of(t_box, t_todo);
+          t_todo = 0;
+        }
         while (t_todo != 0) {
           // two boxes per step: the two halves of the wave hold the same 32
           // queries, so the lower half tests one box and the upper half the
