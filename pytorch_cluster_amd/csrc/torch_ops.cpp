@@ -372,40 +372,55 @@ std::string get_search_strategy() {
   return code == kBinned ? "binned" : code == kAuto ? "auto" : "scan";
 }
 
-// The estimates of "auto" per operator, fitted to whole calls on an MI355X
-// (`python bench.py --extras-only --case crossover` measures both strategies
-// over uniform clouds of 2,048 - 262,144 points in 1 and 8 examples and
-// reports where the pick loses).
+// The estimates of "auto" per operator, ms: fitted to whole calls of both searches on an
+// MI355X, 488 of kNN and 169 of nearest (uniform, clustered and LiDAR-like points
+// of 2 and 3 dimensions, 1 - 40 equal and ragged examples of 1,500 - 150,000
+// rows, every 1st - 16th a query, k = 1 - 64).  What the pick loses against the
+// faster search, on average: kNN 1.0 %, nearest 0.5 % (with one rate per operator,
+// whatever k, 4.5 and 4.8 %: 262,144 uniform points in 32 examples, k = 33, were
+// scanned in 1,308 us, 577 binned; 18,000 queries among 36,000 LiDAR-like rows,
+// k = 16, binned in 398, scanned in 216).  What it cannot see is the density: the
+// largest loss left is 1.7-fold, kNN of 19,873 among 79,492 points in the plane.
 struct SearchCost {
-  double scan_rate;   // pairs per ms the scan looks at
-  double query_us;    // binned search: us per searching row
-  double binned_base; // binned search: ms before the first row counts
+  double scan_base, scan_pair; // the scan: a call, a pair it looks at
+  double scan_list;            // ... a list place's share in the insertions
+  double scan_wide;            // ... all of them beyond 32 places
+  double bin_base, bin_place;  // the binned search: a call, a list place
+  double bin_row, bin_query;   // ... a row that gets binned, a query
+  double bin_query_place;      // ... a list place of a query
 };
-// kNN ~3 G pairs/ms (between its small-cloud and large-cloud rates); radius and
-// nearest ~10 G (the radius scan stops at max_num_neighbors, nearest keeps one
-// neighbour); a binned radius call starts sooner than a binned kNN call (no
-// tasks to order).
-constexpr SearchCost kKnnCost{3e9, 2e-3, 0.2};
-constexpr SearchCost kRadiusCost{1e10, 0.5e-3, 0.13};
-constexpr SearchCost kNearestCost{1e10, 0.5e-3, 0.2};
+constexpr SearchCost kKnnCost{4.77e-2, 1.68e-10, 7.68e-9, 2.69,    2.05e-1,
+                              3.06e-4, 2.47e-7,  1.79e-7, 4.05e-8};
+// (a radius scan stops at max_num_neighbors)
+constexpr SearchCost kRadiusCost{0.1, 1e-10, 0, 1, 0.13, 0, 1e-6, 5e-7, 0};
+constexpr SearchCost kNearestCost{5.95e-2, 2.417e-10, 0,     1, 3.491e-1,
+                                  0,       1.126e-7,  8.9e-8, 0};
 
 // searched: rows that get binned (x of knn / radius, y of nearest);
-// searching: the rows that look for neighbours.  "auto" compares two rough
-// estimates in ms: the scan looks at every pair of a segment (segments taken
-// as equal) at scan_rate pairs per ms, binning costs a sort of both sides and
-// a search that grows with their sizes.  It picks the scan for clouds of a few
-// thousand points and for a handful of queries against many rows, bins from
-// some ten thousand rows per segment on.
+// searching: the rows that look for k neighbours.  "auto" compares two rough
+// estimates: the scan looks at every pair of a segment (segments taken as
+// equal) and keeps lists, a place of which changes with the logarithm of the rows
+// it has seen; binning costs a sort of both sides and a search that grows with
+// their sizes and the lists.  It picks the scan for clouds of a few thousand points
+// and for a handful of queries against many rows, bins from some ten thousand
+// rows per segment on.
 bool bins_wanted(int64_t searched, int64_t searching, int64_t num_segments,
-                 const SearchCost &cost) {
+                 int64_t k, const SearchCost &cost) {
   const int code = g_strategy.load();
   if (code != kAuto)
     return code == kBinned;
-  const double pairs = (double)searched * (double)searching /
-                       (double)std::max<int64_t>(num_segments, 1);
-  const double scan_ms = 0.1 + pairs / cost.scan_rate;
-  const double binned_ms = cost.binned_base + 1e-6 * (double)searched +
-                           1e-3 * cost.query_us * (double)searching;
+  const double rows = (double)searched, queries = (double)searching;
+  const double segment =
+      rows / (double)std::max<int64_t>(num_segments, 1);
+  const double places = (double)((k + 7) / 8 * 8); // of a list
+  const double scan_ms =
+      cost.scan_base +
+      (k > 32 ? cost.scan_wide : 1.0) *
+          (segment * queries * cost.scan_pair +
+           queries * places * std::log1p(segment / places) * cost.scan_list);
+  const double binned_ms =
+      cost.bin_base + (double)k * cost.bin_place + rows * cost.bin_row +
+      queries * (cost.bin_query + places * cost.bin_query_place);
   return scan_ms > binned_ms;
 }
 
@@ -420,7 +435,7 @@ bool being_captured(hipStream_t stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
-// What the current strategy picks for an operator ("knn", "radius",
+// What the current strategy picks for an operator ("knn" with k = 16, "radius",
 // "nearest") and these sizes, when the points qualify for binning at all
 // (fp32, up to 3 dimensions, Euclidean): "scan" or "binned".
 std::string strategy_for(std::string op, int64_t searched, int64_t searching,
@@ -431,7 +446,7 @@ std::string strategy_for(std::string op, int64_t searched, int64_t searching,
                                              : nullptr;
   TORCH_CHECK(cost != nullptr, "operator is 'knn', 'radius' or 'nearest', got '",
               op, "'");
-  return bins_wanted(searched, searching, num_segments, *cost)
+  return bins_wanted(searched, searching, num_segments, 16, *cost)
              ? "binned"
              : "scan";
 }
@@ -475,7 +490,7 @@ at::Tensor knn_search(at::Tensor x, at::Tensor y,
   refuse_capture(c10::hip::getCurrentHIPStream(x.get_device()).stream(),
                  "knn");
   const int dtype = dtype_code(x);
-  const bool binned = bins_wanted(n, m, seg.count, kKnnCost) &&
+  const bool binned = bins_wanted(n, m, seg.count, k, kKnnCost) &&
                       dtype == PCA_F32 && !cosine && d <= 3 && k <= 64;
   const size_t ws_bytes =
       binned ? pca_knn_binned_workspace_bytes(n, m, d, seg.count, k)
@@ -642,7 +657,7 @@ at::Tensor radius_search(at::Tensor x, at::Tensor y,
                  "radius");
   const int dtype = dtype_code(x);
   const int64_t slots = pca_radius_slots(n, max_num_neighbors);
-  const bool binned = bins_wanted(n, m, seg.count, kRadiusCost) &&
+  const bool binned = bins_wanted(n, m, seg.count, 1, kRadiusCost) &&
                       dtype == PCA_F32 && d <= 3 && slots <= 64;
   const size_t ws_bytes =
       binned ? pca_radius_binned_workspace_bytes(n, m, d, seg.count,
@@ -761,7 +776,7 @@ void nearest_search(const at::Tensor &x, const at::Tensor &y,
   TORCH_CHECK(dtype != PCA_BF16,
               "nearest is not implemented for 'BFloat16'");
   // (the searched rows, y, are the ones a binned search orders)
-  const bool binned = bins_wanted(m, n, segments, kNearestCost) &&
+  const bool binned = bins_wanted(m, n, segments, 1, kNearestCost) &&
                       dtype == PCA_F32 && d <= 3 && m > 0 &&
                       !being_captured(stream);
   const size_t ws_bytes =
