@@ -60,3 +60,23 @@ def test_clustered_graph(oracle):
     x[7], x[1200, 1], x[6000] = np.nan, np.inf, 3e38
     for r, limit in ((0.05, 32), (0.02, 8), (0.1, 64), (np.inf, 16)):
         check(oracle, x, x, ptr, ptr, r, limit, ignore_same=True)
+
+
+@pytest.mark.parametrize("d", [2, 3, 4, 8])
+@pytest.mark.parametrize("share", [0.002, 0.03, 0.06, 0.3, 1.0])
+def test_open_queries_by_share_of_rows_in_reach(oracle, d, share):
+    """Few neighbours (rows shared by the waves), many (query by query), and
+    the one after the other, at ends of a wave's rows and of a round."""
+    rng = np.random.default_rng(int(share * 1000) + d)
+    for n, m in ((31, 5), (513, 32), (2047, 17), (2049, 4), (6500, 29)):
+        x = rng.random((n, d)).astype(np.float32)
+        near = rng.random(n) < np.where(np.arange(n) < n // 2, share / 8, share)
+        x[~near] += 5
+        y = rng.random((m, d)).astype(np.float32)
+        y[::7] += 5
+        y[m // 2, d - 1] = np.nan
+        k = min(n, m)
+        x[:k:3] = y[:k:3]
+        for limit in (7, 100, 3000):
+            check(oracle, x, y, [0, n], [0, m], 0.5 * d ** 0.5, limit,
+                  ignore_same=limit == 100)
