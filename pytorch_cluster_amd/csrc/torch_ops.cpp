@@ -373,24 +373,26 @@ std::string get_search_strategy() {
 }
 
 // The estimates of "auto" per operator, ms: fitted to whole calls of both searches on an
-// MI355X, 488 of kNN and 169 of nearest (uniform, clustered and LiDAR-like points
+// MI355X, 524 of kNN and 169 of nearest (uniform, clustered and LiDAR-like points
 // of 2 and 3 dimensions, 1 - 40 equal and ragged examples of 1,500 - 150,000
 // rows, every 1st - 16th a query, k = 1 - 64).  What the pick loses against the
 // faster search, on average: kNN 1.0 %, nearest 0.5 % (with one rate per operator,
 // whatever k, 4.5 and 4.8 %: 262,144 uniform points in 32 examples, k = 33, were
 // scanned in 1,308 us, 577 binned; 18,000 queries among 36,000 LiDAR-like rows,
 // k = 16, binned in 398, scanned in 216).  What it cannot see is the density: the
-// largest loss left is 1.7-fold, kNN of 19,873 among 79,492 points in the plane.
+// graph of 29,390 uniform points, k = 9, takes 182 us scanned, 153 binned, that of
+// 36,000 LiDAR-like ones, k = 16, 298 and 446; both are binned.  The largest loss
+// left is 1.8-fold, kNN of 58,809 among 235,236 points in the plane, k = 32.
 struct SearchCost {
   double scan_base, scan_pair; // the scan: a call, a pair it looks at
   double scan_list;            // ... a list place's share in the insertions
   double scan_wide;            // ... all of them beyond 32 places
-  double bin_base, bin_place;  // the binned search: a call, a list place
+  double bin_base, bin_spread; // the binned search: a call, the spread of a tile
   double bin_row, bin_query;   // ... a row that gets binned, a query
   double bin_query_place;      // ... a list place of a query
 };
-constexpr SearchCost kKnnCost{4.77e-2, 1.68e-10, 7.68e-9, 2.69,    2.05e-1,
-                              3.06e-4, 2.47e-7,  1.79e-7, 4.05e-8};
+constexpr SearchCost kKnnCost{1.6e-2,  1.7e-10, 1.53e-10, 2.98,   1.45e-1,
+                              2.42e-2, 1.55e-8, 8.1e-8,   1.03e-9};
 // (a radius scan stops at max_num_neighbors)
 constexpr SearchCost kRadiusCost{0.1, 1e-10, 0, 1, 0.13, 0, 1e-6, 5e-7, 0};
 constexpr SearchCost kNearestCost{5.95e-2, 2.417e-10, 0,     1, 3.491e-1,
@@ -401,7 +403,8 @@ constexpr SearchCost kNearestCost{5.95e-2, 2.417e-10, 0,     1, 3.491e-1,
 // estimates: the scan looks at every pair of a segment (segments taken as
 // equal) and keeps lists, a place of which changes with the logarithm of the rows
 // it has seen; binning costs a sort of both sides and a search that grows with
-// their sizes and the lists.  It picks the scan for clouds of a few thousand points
+// their sizes, the lists and the space between the queries of a tile (the fewer
+// there are to the rows, the more boxes are in reach of one).  It picks the scan for clouds of a few thousand points
 // and for a handful of queries against many rows, bins from some ten thousand
 // rows per segment on.
 bool bins_wanted(int64_t searched, int64_t searching, int64_t num_segments,
@@ -419,7 +422,9 @@ bool bins_wanted(int64_t searched, int64_t searching, int64_t num_segments,
           (segment * queries * cost.scan_pair +
            queries * places * std::log1p(segment / places) * cost.scan_list);
   const double binned_ms =
-      cost.bin_base + (double)k * cost.bin_place + rows * cost.bin_row +
+      cost.bin_base +
+      cost.bin_spread * std::log(std::max(1.0, rows / queries)) +
+      rows * cost.bin_row +
       queries * (cost.bin_query + places * cost.bin_query_place);
   return scan_ms > binned_ms;
 }
