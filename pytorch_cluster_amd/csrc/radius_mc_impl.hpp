@@ -249,6 +249,7 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
   for (int c = 0; c < DIM; ++c)
     done = done || !(__builtin_fabsf(yq[c]) <= 3.402823466e+38f);
   const bool ignore_same = p.ignore_same_index != 0;
+  const int self = ignore_same ? q : -1; // the row that is left out
   int *const slot_row = p.out_idx + (size_t)(valid ? q : y_begin) * slots;
 
   // ---- tile staging -------------------------------------------------------
@@ -309,7 +310,7 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
       float row[XF];
 #pragma unroll
       for (int e = 0; e < XF; e += 4) {
-        const uint4 q4 = rows_lds[NI + e / 4][min(j, TX - 1)];
+        const uint4 q4 = rows_lds[NI + e / 4][j];
         row[e] = __uint_as_float(q4.x);
         row[e + 1] = __uint_as_float(q4.y);
         row[e + 2] = __uint_as_float(q4.z);
@@ -324,7 +325,7 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
       }
       const int g = g_base + j;
       // (j < rows: no padding rows)
-      if (has && dist < r2 && j < rows && !(ignore_same && g == q)) {
+      if (has && dist < r2 && j < rows && g != self) {
         slot_row[count] = g;
         ++count;
         if (count >= slots) {
@@ -417,6 +418,7 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const int e = min(col, few - 1);
     const int qe = (int)table[e];
+    const int self_e = ignore_same ? qe : -1;
     int filled = (int)table[kRadiusFew + e];
     float at[DIM];
 #pragma unroll
@@ -500,7 +502,7 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
           dist = __builtin_fmaf(dc, dc, dist);
         }
         const bool hit = dist < r2 && j < c_count &&
-                         !(ignore_same && x_begin + j == qe);
+                         x_begin + j != self_e;
         mine += has && hit ? 1 : 0;
         if (has && !hit)
           queue[step][pair] &= ~bit;
