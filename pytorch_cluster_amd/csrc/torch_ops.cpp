@@ -974,19 +974,19 @@ at::Tensor fps_host(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
   return out;
 }
 
-// The bound on the rows of an example that pca_fps is given: it selects the kernel.
-// Beyond 16,384 rows the rows are sorted, 60 us and more, for steps of 2 - 12 us;
-// with the bound 0 every row is looked at in every step, 0.6 us per 1,000 rows.  All
-// rows / sorted, us, for `samples` at most per example: 4 x 17,000 rows, 4 samples
-// 35 / 69, 8 79 / 89, 16 167 / 108; 2 x 60,000, 2 samples 38 / 75, 4 107 / 97.
-// Between 8,192 and 16,384 rows of up to 3 dimensions examples of many samples
-// (`each` of them) are better off sorted as well, several samples to a step: on
-// the chip / sorted 16 x 8,300 rows, 200 samples 263 / 276, 300 390 / 327, 500 512 /
-// 424; 8 x 16,384, 200 262 / 309, 300 389 / 371; 200 x 9,000, 300 413 / 431.
-int64_t fps_bound(int64_t longest, int64_t samples, int64_t each, int64_t d) {
+// The bound on the rows of an example that pca_fps is given: it selects the kernel,
+// by the longest example and the most samples of one.  Beyond 16,384 rows the rows are
+// sorted, 60 us and more, for steps of 2 - 12 us; with the bound 0 every row is looked
+// at in every step, 0.6 us per 1,000 rows.  All rows / sorted, us: 4 x 17,000 rows, 4
+// samples each 35 / 69, 8 79 / 89, 16 167 / 108; 2 x 60,000, 2 samples 38 / 75, 4 107 /
+// 97.  Between 8,192 and 16,384 rows of up to 3 dimensions examples of many samples
+// are better off sorted as well, several samples to a step: on the chip / sorted
+// 16 x 8,300 rows, 200 samples 263 / 276, 300 390 / 327, 500 512 / 424; 8 x 16,384,
+// 200 262 / 309, 300 389 / 371; 200 x 9,000, 300 413 / 431.
+int64_t fps_bound(int64_t longest, int64_t samples, int64_t d) {
   if (longest > 16384)
     return (samples - 1) * longest <= 130000 ? 0 : longest;
-  return longest > 8192 && each >= 340 && d <= 3 ? 16385 : longest;
+  return longest > 8192 && samples >= 340 && d <= 3 ? 16385 : longest;
 }
 
 at::Tensor fps(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
@@ -1005,9 +1005,11 @@ at::Tensor fps(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
   const int64_t batch_size = ptr.numel() - 1;
 
   auto deg = ptr.narrow(0, 1, batch_size) - ptr.narrow(0, 0, batch_size);
-  auto out_ptr = deg.toType(ratio.scalar_type()) * ratio;
-  out_ptr = out_ptr.ceil().toType(at::kLong).cumsum(0);
-  out_ptr = at::cat({at::zeros({1}, ptr.options()), out_ptr}, 0).contiguous();
+  const auto samples =
+      (deg.toType(ratio.scalar_type()) * ratio).ceil().toType(at::kLong);
+  auto out_ptr = at::zeros({batch_size + 1}, ptr.options());
+  auto ends = out_ptr.narrow(0, 1, batch_size);
+  at::cumsum_out(ends, samples, 0);
 
   at::Tensor start;
   if (random_start) {
@@ -1016,16 +1018,16 @@ at::Tensor fps(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
     start = start.contiguous();
   }
 
-  // [number of samples, largest example] in one read
-  auto sizes = at::stack({out_ptr[-1], deg.max()}).cpu();
+  // [number of samples, most of an example, largest example] in one read
+  auto sizes = at::stack({out_ptr[-1], samples.max(), deg.max()}).cpu();
   const int64_t out_size = sizes[0].item<int64_t>();
   auto out = at::empty({out_size}, ptr.options());
   const int64_t n = src.size(0);
   if (n == 0 || out_size == 0)
     return out;
   const int64_t d = src.size(1);
-  const int64_t max_rows = fps_bound(sizes[1].item<int64_t>(), out_size,
-                                     out_size / batch_size, d);
+  const int64_t max_rows =
+      fps_bound(sizes[2].item<int64_t>(), sizes[1].item<int64_t>(), d);
   const int dtype = dtype_code(src);
   TORCH_CHECK(dtype != PCA_BF16, "fps is not implemented for 'BFloat16'");
   const size_t ws_bytes =
@@ -1115,7 +1117,7 @@ at::Tensor fps_batched(at::Tensor src, std::optional<at::Tensor> batch,
   if (samples == 0)
     return out;
   const int64_t most = (int64_t)std::ceil((float)longest * (float)ratio);
-  longest = fps_bound(longest, most, most, d);
+  longest = fps_bound(longest, most, d);
   const size_t ws_bytes =
       pca_fps_workspace_bytes(n, d, examples, longest, PCA_F32);
   TORCH_CHECK(ws_bytes > 0, "problem size not supported");

@@ -245,6 +245,38 @@ def test_a_handful_of_samples_from_large_examples(oracle, rows, samples):
     assert (one.cpu().numpy() == want[:samples]).all()
 
 
+@pytest.mark.parametrize("sizes,samples", [
+    ([17000] * 64, 4), ([16384, 17000, 40], 8), ([16000] + [500] * 31, 800),
+    ([9000] * 8, 450)])
+def test_both_entry_points_take_the_same_kernel(sizes, samples):
+    """The kernel follows the largest example and its samples, whatever the number
+    of examples and whoever asks: seen by the workspace it takes (none on the
+    chip, 8 bytes a row with every row looked at, more than 24 in curve order)."""
+    n, longest = sum(sizes), max(sizes)
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = torch.rand(n, 3, generator=g, device=DEV)
+    batch = torch.arange(len(sizes)).repeat_interleave(torch.tensor(sizes))
+    batch = batch.to(DEV)
+    ptr = torch.tensor(np.cumsum([0] + sizes), device=DEV)
+    ratio = (samples - 0.5) / longest
+    ratios = torch.full((len(sizes),), ratio, device=DEV)
+    taken, rows = [], []
+    for call in (lambda: pca.fps(x, batch, ratio, random_start=False),
+                 lambda: torch.ops.torch_cluster.fps(x, ptr, ratios, False)):
+        call()
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        rows.append(call())
+        taken.append((torch.cuda.max_memory_allocated() - before) / n)
+    assert torch.equal(rows[0], rows[1])
+    bound = 0 if longest <= 8192 or longest <= 16384 and samples < 340 else \
+        24 if (samples - 1) * longest > 130000 else 8
+    for bytes_per_row in taken:
+        assert bytes_per_row > bound if bound == 24 else \
+            bytes_per_row < bound + 4
+
+
 def test_captured_into_a_graph(oracle):
     """While its stream is being captured the search does without the sort of
     the large examples; every replay samples the same rows."""
