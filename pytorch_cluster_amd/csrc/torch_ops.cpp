@@ -372,41 +372,51 @@ std::string get_search_strategy() {
   return code == kBinned ? "binned" : code == kAuto ? "auto" : "scan";
 }
 
-// The estimates of "auto" per operator, ms: fitted to whole calls of both searches on an
-// MI355X, 524 of kNN and 169 of nearest (uniform, clustered and LiDAR-like points
-// of 2 and 3 dimensions, 1 - 40 equal and ragged examples of 1,500 - 150,000
-// rows, every 1st - 16th a query, k = 1 - 64).  What the pick loses against the
-// faster search, on average: kNN 1.0 %, nearest 0.5 % (with one rate per operator,
-// whatever k, 4.5 and 4.8 %: 262,144 uniform points in 32 examples, k = 33, were
-// scanned in 1,308 us, 577 binned; 18,000 queries among 36,000 LiDAR-like rows,
-// k = 16, binned in 398, scanned in 216).  What it cannot see is the density: the
-// graph of 29,390 uniform points, k = 9, takes 182 us scanned, 153 binned, that of
-// 36,000 LiDAR-like ones, k = 16, 298 and 446; both are binned.  The largest loss
-// left is 1.8-fold, kNN of 58,809 among 235,236 points in the plane, k = 32.
+// The estimates of "auto" per operator, us.  Only the pick matters: for kNN both
+// sides start from whole calls of uniform clouds where the searches are within a
+// factor of two of each other (rms 8 - 13 %) and were then moved for what the picks lose
+// over 4,512 calls on an MI355X (uniform, clustered and LiDAR-like points of 2 and 3
+// dimensions, 1 - 64 equal and ragged examples of 1,500 - 3,000,000 rows, every 1st -
+// 1,024th a query, k = 1 - 64); beyond the sizes where the two meet they are no times.
+// A pick loses 1.0 % of the calls of uniform points on average, 1.6 % of all.  What it
+// cannot see is the density: one uniform cloud of 23,000 rows, k = 17, takes 209 us
+// scanned and 167 binned, a LiDAR-like one 211 and 314, both are binned; the largest loss
+// is 2.2-fold (29,000 LiDAR-like rows, k = 16, 222 scanned, 493 binned).  Scanned / binned:
+// one uniform cloud of 23,000 rows, k = 4 109 / 123, 25 257 / 195; 27,000 rows, k = 4
+// 141 / 125, 17 252 / 171, 25 319 / 200; 1,954 queries among 1,000,000 rows, k = 4 384 /
+// 1,122, 32 670 / 2,210; 7,813 queries, k = 16, 786 / 898.
 struct SearchCost {
-  double scan_base, scan_pair; // the scan: a call, a pair it looks at
-  double scan_list;            // ... a list place's share in the insertions
-  double scan_wide;            // ... all of them beyond 32 places
-  double bin_base, bin_spread; // the binned search: a call, the spread of a tile
-  double bin_row, bin_query;   // ... a row that gets binned, a query
-  double bin_query_place;      // ... a list place of a query
+  double scan_base, scan_pair, scan_query; // a call, a pair looked at, a query
+  double scan_place;                       // ... all of them, per place of a list
+  double bin_base;                         // a call
+  // the space between the queries of a tile, by the root of the rows per query,
+  // and for a place of a list
+  double bin_spread, bin_spread_place;
+  double bin_row, bin_query; // a row that gets binned, a query
+  double bin_query_place;    // a place of a query's list
+  double bin_place;          // a place of the longest chain of insertions
 };
-constexpr SearchCost kKnnCost{1.6e-2,  1.7e-10, 1.53e-10, 2.98,   1.45e-1,
-                              2.42e-2, 1.55e-8, 8.1e-8,   1.03e-9};
+// (lists of up to 32 places are in registers throughout; a scan of longer ones
+// takes twice the time and more beyond 20,000 rows: 258 / 383 us at 19,000, 282 / 632
+// at 22,000 for 32 and 33 places)
+constexpr SearchCost kKnnCost{16.3, 8.90e-8, 9.95e-7,  5.92e-2,  89.8, 26.8,
+                              2.77, 1.058e-4, 1.402e-4, 2.863e-5, 0.984};
+constexpr SearchCost kKnnWideCost{13.3, 1.015e-6, 1.037e-3, 1.199e-2, 268, 18.7,
+                                  0.95, 8.17e-5,  1.392e-4, 9.99e-6,  4.70};
 // (a radius scan stops at max_num_neighbors)
-constexpr SearchCost kRadiusCost{0.1, 1e-10, 0, 1, 0.13, 0, 1e-6, 5e-7, 0};
-constexpr SearchCost kNearestCost{5.95e-2, 2.417e-10, 0,     1, 3.491e-1,
-                                  0,       1.126e-7,  8.9e-8, 0};
+constexpr SearchCost kRadiusCost{100, 1e-7, 0, 0, 130, 0, 0, 1e-3, 5e-4, 0, 0};
+constexpr SearchCost kNearestCost{59.5, 2.417e-7, 0,        0,      349.1, 0,
+                                  0,    1.126e-4, 8.9e-5, 0, 0};
 
 // searched: rows that get binned (x of knn / radius, y of nearest);
 // searching: the rows that look for k neighbours.  "auto" compares two rough
 // estimates: the scan looks at every pair of a segment (segments taken as
-// equal) and keeps lists, a place of which changes with the logarithm of the rows
-// it has seen; binning costs a sort of both sides and a search that grows with
-// their sizes, the lists and the space between the queries of a tile (the fewer
-// there are to the rows, the more boxes are in reach of one).  It picks the scan for clouds of a few thousand points
-// and for a handful of queries against many rows, bins from some ten thousand
-// rows per segment on.
+// equal) and is slower the longer the lists are; binning costs a sort of both sides
+// and a search that grows with their sizes, the lists and the space between the
+// queries of a tile (the fewer there are to the rows, the more boxes are in reach of
+// one).  It picks the scan for clouds of a few thousand points and for a handful of
+// queries against many rows; one cloud is binned from 27,600 rows on for k = 4, 22,800
+// for 16, 19,400 for 32, eight from 11,000, 9,600 and 8,700 each.
 bool bins_wanted(int64_t searched, int64_t searching, int64_t num_segments,
                  int64_t k, const SearchCost &cost) {
   const int code = g_strategy.load();
@@ -415,18 +425,20 @@ bool bins_wanted(int64_t searched, int64_t searching, int64_t num_segments,
   const double rows = (double)searched, queries = (double)searching;
   const double segment =
       rows / (double)std::max<int64_t>(num_segments, 1);
-  const double places = (double)((k + 7) / 8 * 8); // of a list
-  const double scan_ms =
-      cost.scan_base +
-      (k > 32 ? cost.scan_wide : 1.0) *
-          (segment * queries * cost.scan_pair +
-           queries * places * std::log1p(segment / places) * cost.scan_list);
-  const double binned_ms =
-      cost.bin_base +
-      cost.bin_spread * std::log(std::max(1.0, rows / queries)) +
+  const double places = (double)k;
+  const double apart = std::sqrt(std::max(1.0, rows / queries)) - 1.0;
+  const double scan_us = (cost.scan_base + segment * queries * cost.scan_pair +
+                          queries * cost.scan_query) *
+                         (1.0 + places * cost.scan_place);
+  const double binned_us =
+      cost.bin_base + (cost.bin_spread + places * cost.bin_spread_place) * apart +
       rows * cost.bin_row +
-      queries * (cost.bin_query + places * cost.bin_query_place);
-  return scan_ms > binned_ms;
+      queries * (cost.bin_query + places * cost.bin_query_place) +
+      places * cost.bin_place;
+  return scan_us > binned_us;
+}
+bool knn_bins_wanted(int64_t n, int64_t m, int64_t num_segments, int64_t k) {
+  return bins_wanted(n, m, num_segments, k, k > 32 ? kKnnWideCost : kKnnCost);
 }
 
 // A stream that is being captured into a graph takes the scanning kernels:
@@ -440,20 +452,19 @@ bool being_captured(hipStream_t stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
-// What the current strategy picks for an operator ("knn" with k = 16, "radius",
-// "nearest") and these sizes, when the points qualify for binning at all
+// What the current strategy picks for an operator ("knn" with lists of k places,
+// "radius", "nearest") and these sizes, when the points qualify for binning at all
 // (fp32, up to 3 dimensions, Euclidean): "scan" or "binned".
 std::string strategy_for(std::string op, int64_t searched, int64_t searching,
-                         int64_t num_segments) {
-  const SearchCost *cost = op == "knn"       ? &kKnnCost
-                           : op == "radius"  ? &kRadiusCost
-                           : op == "nearest" ? &kNearestCost
-                                             : nullptr;
-  TORCH_CHECK(cost != nullptr, "operator is 'knn', 'radius' or 'nearest', got '",
-              op, "'");
-  return bins_wanted(searched, searching, num_segments, 16, *cost)
-             ? "binned"
-             : "scan";
+                         int64_t num_segments, int64_t k) {
+  TORCH_CHECK(op == "knn" || op == "radius" || op == "nearest",
+              "operator is 'knn', 'radius' or 'nearest', got '", op, "'");
+  const bool binned =
+      op == "knn"
+          ? knn_bins_wanted(searched, searching, num_segments, k)
+          : bins_wanted(searched, searching, num_segments, 1,
+                        op == "radius" ? kRadiusCost : kNearestCost);
+  return binned ? "binned" : "scan";
 }
 
 at::Tensor knn_search(at::Tensor x, at::Tensor y,
@@ -495,7 +506,7 @@ at::Tensor knn_search(at::Tensor x, at::Tensor y,
   refuse_capture(c10::hip::getCurrentHIPStream(x.get_device()).stream(),
                  "knn");
   const int dtype = dtype_code(x);
-  const bool binned = bins_wanted(n, m, seg.count, k, kKnnCost) &&
+  const bool binned = knn_bins_wanted(n, m, seg.count, k) &&
                       dtype == PCA_F32 && !cosine && d <= 3 && k <= 64;
   const size_t ws_bytes =
       binned ? pca_knn_binned_workspace_bytes(n, m, d, seg.count, k)
@@ -1180,7 +1191,7 @@ TORCH_LIBRARY(pytorch_cluster_amd, m) {
   m.def("host_waits() -> int", &host_waits);
   m.def("set_search_strategy(str name) -> ()", &set_search_strategy);
   m.def("get_search_strategy() -> str", &get_search_strategy);
-  m.def("strategy_for(str op, int searched, int searching, int num_segments) "
-        "-> str",
+  m.def("strategy_for(str op, int searched, int searching, int num_segments, "
+        "int k=16) -> str",
         &strategy_for);
 }
