@@ -35,16 +35,23 @@
 // and the waves share the rows: 16 steps each, operands straight from memory,
 // the exact distances of even and odd steps by the two lanes of a pair; the
 // waves tell each other how many hits they have and each writes its own behind
-// those of the waves before it.  One barrier per 2,048 rows, no tiles.  An
-// exact scan per query costs a wave 8 instructions per 64 rows whatever they
-// hold, the filter 30 per 32 rows x 32 queries and then some 60 for a row that
-// passes: where more than few + 8 of a lane's 256 rows pass, or up to four
+// those of the waves before it.  One barrier per 2,048 rows (1,024 for d > 4), no
+// tiles.  An exact scan per query costs a wave 8 instructions per 64 rows whatever
+// they hold, the filter 30 per 32 rows x 32 queries and then some 60 for a row that
+// passes: where more than few + 8 of a lane's 256 rows (128) pass, or up to four
 // queries are open, the rest is scanned query by query.  (32 queries each in
 // 64 clouds of 16,384 points, by neighbours per query: 20 / 70 / 230 / 1,000 /
 // 4,400: 72 / 77 / 118 / 182 / 239 us, all by query 116 / 156 / 234 / 270 /
 // 249 us; a threshold without the 8: 234 us for the fourth, with 2 few: 253 us
-// for the last.  Tens of queries per 4,096 rows of which 6 % and more are in
-// reach: up to 8 % more time for the round that finds it out.)
+// for the last.)  So are the rows of less than a wave at the end, which would leave
+// three waves idle (32 queries each in 128 clouds of 2,500 rows, 0.05 / 0.5 / 4 % in
+// reach: 56 / 62 / 59 -> 48 / 53 / 50 us), and all of them where no tile was scanned
+// yet and after four steps most lists look full soon (64 clouds of 4,096 rows, lists
+// of 32, 20 / 40 % in reach: 8 queries each 41 / 40 -> 39 / 38 us, 16 42 / 41 -> 41 /
+// 39, 32 45 / 42 -> 44 / 40; all by query 40 / 39, 42 / 40, 44 / 41).  Between that and the
+// few hits that the filter is for, at 4 - 12 % in reach, short lists take up to 10 %
+// more time than all by query (32 queries, 12 %: 58 us instead of 48): four steps
+// cannot tell, and asking 256 rows query by query first costs the others 4 us.
 //
 // 8 clouds of 16,384 clustered points, r = 0.05, 32 neighbours: kernel 132 ->
 // 100 us (the shared rows alone 117 us), r = 0.02: the call 277 -> 225 us.
@@ -60,6 +67,9 @@
 namespace pca {
 
 constexpr int kRadiusFew = 32; // open queries a workgroup deals to its waves
+// Rows times open queries that take as long query by query as a round of the filter
+// and its walks.
+constexpr float kRadiusSoon = 8192.0f;
 
 struct RadiusMcParams {
   const float *x;
@@ -212,15 +222,15 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
       mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(acc[v]), 31);
     return mask;
   };
-  // STEPS steps of the filter into the queue: the steps with a row that passed
-  // as a set, and how many rows of the lane's steps passed.  A swap gives the
+  // Steps [from, to) of the filter into the queue: those with a row that passed
+  // as a set, the rows of the lane's steps that passed added to `ones`.  A swap gives the
   // lower lane of a pair both masks of the first of two steps, the upper lane
   // those of the second; their nibbles alternate in the rows' order.
-  auto filter = [&](auto rows_of_step, const mc_bf16x8_t(&qb)[NI], int &ones) {
+  auto filter = [&](auto from, auto to, auto rows_of_step,
+                    const mc_bf16x8_t(&qb)[NI], int &ones) {
     uint32_t some = 0;
-    ones = 0;
 #pragma unroll
-    for (int s = 0; s < STEPS; s += 2) {
+    for (int s = from; s < to; s += 2) {
       uint4 rows[NI];
       rows_of_step(s, rows);
       const uint32_t first = passing(rows, qb);
@@ -345,6 +355,8 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
 
   if (num_tiles > 0)
     load_tile(0);
+  constexpr std::integral_constant<int, 0> no_steps{};
+  constexpr std::integral_constant<int, STEPS> all_steps{};
   bool wave_done = false;
   int few = 0, few_before = 0; // open queries, those of the waves before
   int t = 0;
@@ -377,8 +389,9 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
     const int g_base = x_begin + t * TX;
     const int rows = min(TX, c_count - t * TX);
     for (int start = 0; start < rows; start += STEPS * 32) {
-      int ones;
+      int ones = 0;
       const uint32_t some = filter(
+          no_steps, all_steps,
           [&](int s, uint4(&a)[NI]) {
 #pragma unroll
             for (int i = 0; i < NI; ++i)
@@ -400,6 +413,7 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
     constexpr int ROUND = W * STEPS * 32;
     constexpr int AHEAD = NI == 1 ? 8 : NI == 2 ? 4 : 2;
     constexpr uint32_t kMany = 0xffffffffu;
+    constexpr int LOOK = 4; // steps after which a wave may know better
     static_assert((2 + DIM + 2 * W) * kRadiusFew <= 4 * TX, "the tile's LDS");
     uint32_t *const table = reinterpret_cast<uint32_t *>(&rows_lds[0][0]);
     uint32_t *const hits_of = table + (2 + DIM) * kRadiusFew;
@@ -445,24 +459,52 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
       for (int s = 0; s < AHEAD; ++s)
         load_step(first + s * 32, ahead[s]);
     }
-    // where the scan goes on query by query
-    int rest = filtered ? c_count : t * TX;
-    for (int round = 0; filtered && t * TX + round * ROUND < c_count; ++round) {
-      int ones;
-      uint32_t some = filter(
-          [&](int s, uint4(&a)[NI]) {
+    int rest = t * TX; // the first row that no query was compared to
+    // (the rows of less than a wave would leave the others idle)
+    for (int round = 0; filtered && c_count - rest > STEPS * 32; ++round) {
+      auto rows_ahead = [&](int s, uint4(&a)[NI]) {
 #pragma unroll
-            for (int i = 0; i < NI; ++i)
-              a[i] = ahead[s % AHEAD][i];
-            const int next = s + AHEAD;
-            load_step(first + (next < STEPS ? next * 32
-                                            : ROUND + (next - STEPS) * 32),
-                      ahead[s % AHEAD]);
-          },
-          yb, ones);
-      const int steps = max(0, min(STEPS, (c_count - first + 31) / 32));
-      some = full ? 0u : some & ((1u << steps) - 1u);
-      const bool many = __any(!full && ones > few + 8);
+        for (int i = 0; i < NI; ++i)
+          a[i] = ahead[s % AHEAD][i];
+        const int next = s + AHEAD;
+        load_step(first + (next < STEPS ? next * 32
+                                        : ROUND + (next - STEPS) * 32),
+                  ahead[s % AHEAD]);
+      };
+      constexpr std::integral_constant<int, LOOK> look{};
+      const int there = c_count - first; // rows of the wave
+      int ones = 0;
+      uint32_t some = 0;
+      bool many = false; // too many pass, or most lists are full soon
+      if (there > 0) {
+        some = filter(no_steps, look, rows_ahead, yb, ones);
+        if (t == 0 && round == 0 && there >= STEPS * 32) {
+          const auto both = __builtin_amdgcn_permlane32_swap(
+              (unsigned)ones, (unsigned)ones, false, false);
+          const float met = (float)(both[0] + both[1]); // of LOOK x 32 rows
+          const uint64_t soon =
+              __ballot(!full && met * (kRadiusSoon / (LOOK * 32)) >=
+                                    (float)(slots - filled) * (float)few);
+          many = 4 * __builtin_popcountll(soon) >=
+                 3 * __builtin_popcountll(__ballot(!full));
+        }
+      }
+      if (there > 0 && !many) {
+        some |= filter(look, all_steps, rows_ahead, yb, ones);
+        if (there < STEPS * 32) {
+          // (beyond the last row it was that row again)
+          const int last = there / 32; // the first step that is not whole
+          some &= (2u << last) - 1u;
+          const uint32_t rest_of = ~(uint32_t)(0xffffffffull >> (there & 31));
+          if ((last & 1) == half)
+            queue[last][pair] &= rest_of;
+          ones = 0;
+          for (int s = half; s <= last; s += 2)
+            ones += __builtin_popcount(queue[s][pair]);
+        }
+        many = __any(!full && ones > few + 8);
+      }
+      some = full ? 0u : some;
       // the lower lane of a pair takes the even steps, the upper lane the odd
       // ones; what is left of a mask are the hits
       uint32_t left = many ? 0u : some & (half ? 0xaaaaaaaau : 0x55555555u);
@@ -501,8 +543,7 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
           const float dc = row[c] - at[c];
           dist = __builtin_fmaf(dc, dc, dist);
         }
-        const bool hit = dist < r2 && j < c_count &&
-                         x_begin + j != self_e;
+        const bool hit = dist < r2 && x_begin + j != self_e;
         mine += has && hit ? 1 : 0;
         if (has && !hit)
           queue[step][pair] &= ~bit;
@@ -525,10 +566,9 @@ __global__ __launch_bounds__(kBlock) void radius_mc_kernel(RadiusMcParams p) {
         after += (int)h;
       }
       // (the same in every wave)
-      if (__any(stop)) {
-        rest = t * TX + round * ROUND;
+      if (__any(stop))
         break;
-      }
+      rest += ROUND;
       left = half == 0 && slot < slots ? some : 0u;
       for (;;) {
         const bool refill = pending == 0 && left != 0;

@@ -80,3 +80,21 @@ def test_open_queries_by_share_of_rows_in_reach(oracle, d, share):
         for limit in (7, 100, 3000):
             check(oracle, x, y, [0, n], [0, m], 0.5 * d ** 0.5, limit,
                   ignore_same=limit == 100)
+
+
+@pytest.mark.parametrize("rows", [1, 31, 33, 511, 512, 513, 1025, 1999, 2047])
+@pytest.mark.parametrize("d", [3, 6])
+def test_last_rows_of_the_open_queries(oracle, rows, d):
+    """Rounds that end inside a wave's rows or leave less than a wave's: the last
+    row in reach of one query, of all, of none; lists that are full early."""
+    rng = np.random.default_rng(rows + d)
+    for round_rows in (2048, 4096):
+        n = round_rows + rows
+        for m in (5, 32):
+            x = (0.2 * rng.random((n, d)) + 3).astype(np.float32)
+            y = rng.random((m, d)).astype(np.float32)
+            x[rng.integers(0, n, 40)] = y[rng.integers(0, m, 40)]
+            for last in (y[m - 1], y.mean(0), np.full(d, 9)):
+                x[-1] = last
+                for r, limit in ((0.01, 32), (1.0, 4), (1.0, 32), (9.0, 60)):
+                    check(oracle, x, y, [0, n], [0, m], r, limit)
