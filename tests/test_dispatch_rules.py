@@ -60,6 +60,24 @@ FEW_QUERIES = [
     (3000000, 11719, 8, 16, 545, 1246), (3000000, 2930, 1, 16, 1269, 2466)]
 
 
+@pytest.mark.parametrize("queries,rows,clouds,scan,binned", [
+    (3000, 1000000, 1, 358, 683),
+    (1000, 100000, 1, 61, 352), (300000, 30000, 1, 580, 135),
+    (100000, 300000, 1, 1711, 137), (1000000, 100000, 8, 871, 239)])
+def test_auto_of_nearest_scans_for_few_queries(queries, rows, clouds, scan,
+                                               binned):
+    import torch
+    import pytorch_cluster_amd as pca
+    before = pca.get_search_strategy()
+    pca.set_search_strategy("auto")
+    try:
+        assert torch.ops.pytorch_cluster_amd.strategy_for(
+            "nearest", rows, queries, clouds) == \
+            ("binned" if binned < scan else "scan")
+    finally:
+        pca.set_search_strategy(before)
+
+
 @pytest.mark.parametrize("rows,queries,clouds,k,scan,binned", FEW_QUERIES)
 def test_auto_scans_for_few_queries_among_many_rows(rows, queries, clouds, k,
                                                     scan, binned):
