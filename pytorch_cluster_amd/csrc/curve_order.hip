@@ -1,9 +1,9 @@
 // Rows in the order of a space-filling curve, segment by segment: the sort in
 // front of the binned searches and of fps over large examples.
 //
-// A sample sort in four launches, both sides of a search in each of them.  The
-// keys (the segment above the 30-bit place on the Hilbert curve through its box)
-// are made unique by the row number below them, so that buckets cut between
+// Up to four million rows it is a sample sort in four launches, both sides of a
+// search in each of them.  The keys (the segment above the 30-bit place on the Hilbert
+// curve through its box) are made unique by the row number below them, so that buckets cut between
 // sampled keys are of similar size whatever the points are -- half of a LiDAR
 // scan's rows share a few cells, and equal places part by their row numbers --
 // and the result is that of a stable sort:
@@ -17,17 +17,29 @@
 //   buckets  a workgroup per bucket of 768 rows on average, a bitonic network in
 //            registers; segments of a single bucket come straight from the points.
 //            A bucket of more than 4,096 rows (eight samples to a bucket leave one
-//            with a probability of about 1e-10; inputs of several million rows
-//            have 2,048 larger buckets) is merged in memory.
+//            with a probability of about 1e-10 where buckets have 768 rows, 1 %
+//            where they have 2,000) is merged in memory.
+// Larger calls and long segments are sorted by the keys' digits of eight bits, the
+// lowest first, three launches each: the tiles' rows by digit are counted, the counts
+// summed over the tiles, the rows put in their places (DigitPass).
 // No workgroup waits for another one and nothing is cleared by memset.
 //
 // 952,000 LiDAR-like rows in eight segments and 119,000 of them as the other side:
 // 13 + 20 + 11 + 24 us (rocPRIM's one-sweep radix sort, which was here before, of
 // both sides on two streams: 22 launches, 171 us of kernels and clears); nearest of
-// the 952,000 among the 119,000 334 -> 263 us a call, kNN of every fourth row of
-// them 696 -> 631.  Bound by latency: hash places and their keys in `sample`, the
+// the 952,000 among the 119,000 334 -> 262 us a call, kNN of every fourth row of
+// them 696 -> 621.  Bound by latency: hash places and their keys in `sample`, the
 // Hilbert steps and the search among splitters in `count`, the network's exchanges
 // in `buckets` (LDS instead of registers 65 us; 256 threads of up to 16 rows 25).
+//
+// The digits' kernels pass over the rows twice per digit, 100 bytes a row; samples cost
+// more per row the more of them a segment has (every workgroup looks at all of them) and
+// larger buckets take more steps of the network.  Calls, us, radix sort as above /
+// samples / digits, nearest of uniform rows to every 16th of them: 1 x 500,000 244 /
+// 195 / 203, 1 x 1 M 324 / 308 / 288, 1 x 2 M 499 / 523 / 434, 20 x 100,000 470 / 390 /
+// 406, 40 x 100,000 756 / 683 / 674, 200 x 100,000 3,537 / 3,652 / 3,085, 1 x 8 M
+// 1,615 / 1,786 / 1,473, 1 x 20 M 4,567 / 5,367 / 4,191; LiDAR-like 1 x 1 M 354 / 343 /
+// 331, 40 x 100,000 904 / 837 / 849, 1 x 8 M 2,069 / 2,248 / 1,973.
 #include "device_utils.hpp"
 #include "launchers.hpp"
 
@@ -38,23 +50,27 @@ namespace pca {
 namespace {
 
 constexpr int kSortThreads = 512;   // of a workgroup that counts
-constexpr int kSortStep = 2048;     // rows it has at a time
+constexpr int kSortTile = 2048;     // rows of a tile
 constexpr int kBucketThreads = 512; // of a workgroup that sorts a bucket
 constexpr int kSortCap = 8 * kBucketThreads; // rows it sorts on the chip
 constexpr int kSortPer = 8;         // samples per bucket
 constexpr int kSortRanked = 64;     // samples a workgroup ranks
 constexpr int kMaxBuckets = 2048;   // of a segment
 
-// Rows of a bucket on average, of a tile (a row's rank in it has 16 bits) and of
-// the buckets whose samples a workgroup ranks, by the number of all rows.
+// The most rows of a side, and of its segments on average, that are sorted by samples
+// (calls on both sides of the lines: above).
+constexpr int kSampledRows = 4000000, kSampledSegment = 750000;
+bool sorted_by_digits(int n, int num_segments) {
+  return n > kSampledRows || n / num_segments > kSampledSegment;
+}
+constexpr int kDigitBits = 8, kDigits = 1 << kDigitBits;
+constexpr int kDigitPer = 8;                         // rows of a thread
+constexpr int kDigitTile = kDigitPer * kSortThreads; // ... of a workgroup
+
+// Rows of a bucket on average (one segment may have almost all rows) and of the
+// buckets whose samples a workgroup ranks, by the number of all rows.
 int bucket_rows(int n) {
   return std::max(768, (int)(((int64_t)n + kMaxBuckets - 1) / kMaxBuckets));
-}
-int tile_rows(int n) {
-  int rows = kSortStep;
-  while (rows < 65536 && n / rows > 2048)
-    rows *= 2;
-  return rows;
 }
 int chunk_rows(int n) { return bucket_rows(n) * (kSortRanked / kSortPer); }
 
@@ -68,8 +84,11 @@ struct SortSide {
   CurveSortPlan plan;
   uint64_t *splitters;  // [buckets]
   uint32_t *base;       // [buckets]
-  uint32_t *tile_off;   // [tiles][stride]
-  int stride;           // largest number of buckets of a segment
+  union {
+    uint32_t *tile_off; // [tiles][stride]
+    uint32_t *digits;   // [kDigits][stride], then [kDigits] totals
+  };
+  int stride;           // largest number of buckets of a segment; digits: tiles
   uint64_t *pairs;      // [n] (key, row), by bucket
   uint64_t *spare;      // [n]; until the scatter: keys, then places
   uint32_t *keys, *perm;
@@ -182,8 +201,8 @@ __global__ __launch_bounds__(kSortThreads) void curve_count_kernel(SortSides p) 
   const int seg = find_segment(tile_start, p.num_segments, block);
   const SortSegment r = sort_segment(s, seg);
   const SortBox box = sort_box(p, seg);
-  const int first = (block - tile_start[seg]) * s.plan.tile_rows;
-  const int some = min(s.plan.tile_rows, r.rows - first);
+  const int first = (block - tile_start[seg]) * kSortTile;
+  const int some = min(kSortTile, r.rows - first);
   const int begin = r.begin + first;
   const int bucket0 = s.plan.bucket_start[seg];
   const int buckets = min(r.buckets, kMaxBuckets);
@@ -199,34 +218,31 @@ __global__ __launch_bounds__(kSortThreads) void curve_count_kernel(SortSides p) 
   uint32_t *keys = reinterpret_cast<uint32_t *>(s.spare);
   uint32_t *places = keys + s.n;
   // (a thread's rows together: their reads and searches overlap)
-  constexpr int PER = kSortStep / kSortThreads;
-  for (int done = 0; done < some; done += kSortStep) {
-    uint64_t v[PER];
-    int at[PER];
+  constexpr int PER = kSortTile / kSortThreads;
+  uint64_t v[PER];
+  int at[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int row = begin + min(i * kSortThreads + (int)threadIdx.x, some - 1);
+    v[i] = (uint64_t)sort_key(p, s, box, seg, row) << 32 | (uint32_t)row;
+    at[i] = 0;
+  }
+  // number of splitters that are not above a row
+  for (int step = top >> 1; step > 0; step >>= 1) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int row =
-          begin + min(done + i * kSortThreads + (int)threadIdx.x, some - 1);
-      v[i] = (uint64_t)sort_key(p, s, box, seg, row) << 32 | (uint32_t)row;
-      at[i] = 0;
+      const int probe = at[i] + step;
+      const bool is = probe <= buckets - 1;
+      at[i] = splitter[is ? probe - 1 : 0] <= v[i] && is ? probe : at[i];
     }
-    // number of splitters that are not above a row
-    for (int step = top >> 1; step > 0; step >>= 1) {
+  }
 #pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int probe = at[i] + step;
-        const bool is = probe <= buckets - 1;
-        at[i] = splitter[is ? probe - 1 : 0] <= v[i] && is ? probe : at[i];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int row = done + i * kSortThreads + (int)threadIdx.x;
-      if (row < some) {
-        const uint32_t rank = atomicAdd(&count[at[i]], 1u);
-        keys[begin + row] = (uint32_t)(v[i] >> 32);
-        places[begin + row] = (uint32_t)at[i] << 16 | rank;
-      }
+  for (int i = 0; i < PER; ++i) {
+    const int row = i * kSortThreads + (int)threadIdx.x;
+    if (row < some) {
+      const uint32_t rank = atomicAdd(&count[at[i]], 1u);
+      keys[begin + row] = (uint32_t)(v[i] >> 32);
+      places[begin + row] = (uint32_t)at[i] << 16 | rank;
     }
   }
   __syncthreads();
@@ -250,8 +266,8 @@ curve_scatter_kernel(SortSides p) {
   const SortSegment r = sort_segment(s, seg);
   const int buckets = min(r.buckets, kMaxBuckets);
   const int tile = block - tile_start[seg];
-  const int first = tile * s.plan.tile_rows;
-  const int some = min(s.plan.tile_rows, r.rows - first);
+  const int first = tile * kSortTile;
+  const int some = min(kSortTile, r.rows - first);
   const int begin = r.begin + first;
   const int bucket0 = s.plan.bucket_start[seg];
   // rows of the buckets before each
@@ -459,12 +475,251 @@ __global__ __launch_bounds__(kBucketThreads) void curve_bucket_kernel(SortSides 
     put(i, from[i]);
 }
 
+// A pass of the sort by digits, the one from bit `shift` on.  The first one reads the
+// points and leaves their keys in `spare`, then the rows go from one buffer of pairs to
+// the other; the last pass writes keys and rows.  Rows of equal digits stay in their
+// order, so the result is a stable sort's whatever the points are.
+struct DigitPass {
+  int shift, number;
+  bool last;
+};
+struct DigitRows {
+  int begin, rows, first, some; // of all segments; of the tile
+};
+__device__ __forceinline__ DigitRows digit_rows(const SortSides &p,
+                                                const SortSide &s, int tile) {
+  const int64_t lo = s.ptr ? s.ptr[0] : 0;
+  const int64_t hi = s.ptr ? s.ptr[p.num_segments] : s.n;
+  DigitRows r;
+  r.begin = (int)min(max(lo, (int64_t)0), (int64_t)s.n);
+  r.rows = (int)max(min(hi, (int64_t)s.n) - r.begin, (int64_t)0);
+  r.first = tile * kDigitTile;
+  r.some = min(kDigitTile, r.rows - r.first);
+  return r;
+}
+
+// Rows of a tile by digit.  Bound by its reads: 8.5 M rows 16 us a pass (4.3 TB/s), 72
+// with the Hilbert steps of the first one.
+__global__ __launch_bounds__(kSortThreads) void
+digit_count_kernel(SortSides p, DigitPass pass) {
+  __shared__ uint32_t count[kDigits];
+  int tile;
+  const SortSide &s = p.side[sort_block(p, tile)];
+  const DigitRows r = digit_rows(p, s, tile);
+  if (r.some <= 0)
+    return; // (the whole workgroup)
+  const int tid = threadIdx.x;
+  if (tid < kDigits)
+    count[tid] = 0u;
+  __syncthreads();
+  const int begin = r.begin + r.first;
+  uint32_t key[kDigitPer];
+  if (pass.number == 0) {
+    uint32_t *keys = reinterpret_cast<uint32_t *>(s.spare);
+    const int seg0 = find_segment64(s.ptr, p.num_segments, begin);
+    const int64_t end0 = s.ptr ? s.ptr[seg0 + 1] : s.n;
+    const SortBox box0 = sort_box(p, seg0);
+#pragma unroll
+    for (int i = 0; i < kDigitPer; ++i) {
+      const int row = begin + min(i * kSortThreads + tid, r.some - 1);
+      if (row < end0) {
+        key[i] = sort_key(p, s, box0, seg0, row);
+      } else {
+        const int seg = find_segment64(s.ptr, p.num_segments, row);
+        key[i] = sort_key(p, s, sort_box(p, seg), seg, row);
+      }
+      if (i * kSortThreads + tid < r.some)
+        keys[row] = key[i];
+    }
+  } else {
+    const uint64_t *from = (pass.number & 1 ? s.pairs : s.spare) + begin;
+#pragma unroll
+    for (int i = 0; i < kDigitPer; ++i)
+      key[i] =
+          (uint32_t)(from[min(i * kSortThreads + tid, r.some - 1)] >> 32);
+  }
+#pragma unroll
+  for (int i = 0; i < kDigitPer; ++i)
+    if (i * kSortThreads + tid < r.some)
+      atomicAdd(&count[key[i] >> pass.shift & (kDigits - 1)], 1u);
+  __syncthreads();
+  if (tid < kDigits)
+    s.digits[(size_t)tid * s.stride + tile] = count[tid];
+}
+
+// Exclusive prefix of one value per thread of a workgroup; part: a word per wave.
+__device__ __forceinline__ uint32_t digit_prefix(uint32_t v, uint32_t *part,
+                                                 uint32_t &total) {
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  uint32_t up = v;
+#pragma unroll
+  for (int sh = 1; sh < kWave; sh <<= 1) {
+    const uint32_t o = (uint32_t)__shfl_up((int)up, sh);
+    up += lane >= sh ? o : 0u;
+  }
+  __syncthreads(); // (part may be in use)
+  if (lane == kWave - 1)
+    part[wave] = up;
+  __syncthreads();
+  uint32_t before = 0;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < kSortThreads / kWave; ++w) {
+    before += w < wave ? part[w] : 0u;
+    total += part[w];
+  }
+  return before + up - v;
+}
+
+// A workgroup per digit: rows of the digit in the tiles before each.
+__global__ __launch_bounds__(kSortThreads) void digit_scan_kernel(SortSides p) {
+  __shared__ uint32_t part[kSortThreads / kWave];
+  const int digit = (int)blockIdx.x % kDigits;
+  const SortSide &s = p.side[(int)blockIdx.x / kDigits];
+  const int rows = digit_rows(p, s, 0).rows;
+  const int tiles = (rows + kDigitTile - 1) / kDigitTile;
+  uint32_t *column = s.digits + (size_t)digit * s.stride;
+  uint32_t before = 0;
+  for (int first = 0; first < tiles; first += kSortThreads * kDigitPer) {
+    const int at = first + (int)threadIdx.x * kDigitPer;
+    uint32_t v[kDigitPer], sum = 0, total;
+#pragma unroll
+    for (int i = 0; i < kDigitPer; ++i) {
+      v[i] = at + i < tiles ? column[at + i] : 0u;
+      sum += v[i];
+    }
+    uint32_t run = before + digit_prefix(sum, part, total);
+#pragma unroll
+    for (int i = 0; i < kDigitPer; ++i) {
+      if (at + i < tiles)
+        column[at + i] = run;
+      run += v[i];
+    }
+    before += total;
+  }
+  if (threadIdx.x == 0)
+    s.digits[(size_t)kDigits * s.stride + digit] = before;
+}
+
+// A tile's rows by digit, rows of a digit in the order they came in: a wave ranks its
+// rows among their like by ballots, sixty-four at a time; in LDS the rows are put
+// together digit by digit, so that neighbouring threads write neighbouring places.
+// 8.5 M rows 40 us a pass (3.4 TB/s).
+__global__ __launch_bounds__(kSortThreads) void
+digit_scatter_kernel(SortSides p, DigitPass pass) {
+  constexpr int WAVES = kSortThreads / kWave;
+  __shared__ uint64_t lds[kDigitTile];
+  __shared__ uint32_t place[WAVES][kDigits]; // 40 KB in all: four to a CU
+  int tile;
+  const SortSide &s = p.side[sort_block(p, tile)];
+  const DigitRows r = digit_rows(p, s, tile);
+  if (r.some <= 0)
+    return; // (the whole workgroup)
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  const int begin = r.begin + r.first;
+  const int mine = wave * (kDigitTile / WAVES) + lane;
+  uint64_t v[kDigitPer];
+  if (pass.number == 0) {
+    const uint32_t *keys = reinterpret_cast<const uint32_t *>(s.spare);
+#pragma unroll
+    for (int i = 0; i < kDigitPer; ++i) {
+      const int row = begin + min(mine + i * kWave, r.some - 1);
+      v[i] = (uint64_t)keys[row] << 32 | (uint32_t)row;
+    }
+  } else {
+    const uint64_t *from = (pass.number & 1 ? s.pairs : s.spare) + begin;
+#pragma unroll
+    for (int i = 0; i < kDigitPer; ++i)
+      v[i] = from[min(mine + i * kWave, r.some - 1)];
+  }
+  // what is before the digit's rows: of smaller digits, in the tiles before
+  uint32_t offset = 0, all = 0;
+  if (tid < kDigits) {
+    offset = s.digits[(size_t)tid * s.stride + tile];
+    all = s.digits[(size_t)kDigits * s.stride + tid];
+  }
+  for (int i = tid; i < WAVES * kDigits; i += kSortThreads)
+    (&place[0][0])[i] = 0u;
+  __syncthreads();
+  const int shift = 32 + pass.shift;
+  uint32_t rank[kDigitPer];
+#pragma unroll
+  for (int i = 0; i < kDigitPer; ++i) {
+    const uint32_t digit = (uint32_t)(v[i] >> shift) & (kDigits - 1);
+    const bool is = mine + i * kWave < r.some;
+    uint64_t same = __ballot(is);
+#pragma unroll
+    for (int b = 0; b < kDigitBits; ++b) {
+      const bool set = (digit >> b & 1u) != 0u;
+      const uint64_t lanes = __ballot(set);
+      same &= set ? lanes : ~lanes;
+    }
+    // (the first of them counts for all; a wave's atomics come in order)
+    const int leader = same != 0 ? __ffsll((unsigned long long)same) - 1 : lane;
+    uint32_t before = 0;
+    if (is && lane == leader)
+      before = atomicAdd(&place[wave][digit], (uint32_t)__popcll(same));
+    before = (uint32_t)__shfl((int)before, leader);
+    rank[i] =
+        before + (uint32_t)__popcll(same & (((uint64_t)1 << lane) - 1));
+  }
+  __syncthreads();
+  uint32_t *part = reinterpret_cast<uint32_t *>(lds);
+  uint32_t count = 0, total;
+  if (tid < kDigits)
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+      count += place[w][tid];
+  offset += digit_prefix(all, part, total);
+  const uint32_t local = digit_prefix(count, part, total);
+  if (tid < kDigits) {
+    uint32_t run = local;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const uint32_t c = place[w][tid];
+      place[w][tid] = run;
+      run += c;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kDigitPer; ++i) {
+    const uint32_t digit = (uint32_t)(v[i] >> shift) & (kDigits - 1);
+    if (mine + i * kWave < r.some)
+      lds[place[wave][digit] + rank[i]] = v[i];
+  }
+  __syncthreads();
+  if (tid < kDigits)
+    place[0][tid] = offset - local; // (modulo 2^32)
+  __syncthreads();
+  uint64_t *out = (pass.number & 1 ? s.spare : s.pairs) + r.begin;
+#pragma unroll
+  for (int i = 0; i < kDigitPer; ++i) {
+    const int at = i * kSortThreads + tid;
+    if (at < r.some) {
+      const uint64_t pair = lds[at];
+      const uint32_t to =
+          place[0][(uint32_t)(pair >> shift) & (kDigits - 1)] + (uint32_t)at;
+      if (to < (uint32_t)r.rows) {
+        if (pass.last) {
+          s.keys[r.begin + to] = (uint32_t)(pair >> 32);
+          s.perm[r.begin + to] = (uint32_t)pair;
+        } else {
+          out[to] = pair;
+        }
+      }
+    }
+  }
+}
+
+int digit_tiles(int n, int) { return n / kDigitTile + 1; }
+
 // Segments of more than one bucket, at most; their items of so many rows.
 int sort_items(int n, int num_segments, int rows) {
   return n / rows + std::min(num_segments, n / bucket_rows(n)) + 1;
 }
 int sort_tiles(int n, int num_segments) {
-  return sort_items(n, num_segments, tile_rows(n));
+  return sort_items(n, num_segments, kSortTile);
 }
 int sort_chunks(int n, int num_segments) {
   return sort_items(n, num_segments, chunk_rows(n));
@@ -484,12 +739,20 @@ struct SortCarve {
 SortSide carve_side(char *&cursor, int n, int num_segments) {
   SortSide s = {};
   SortCarve c{cursor};
-  const size_t segs = (size_t)num_segments + 1;
-  const size_t buckets = (size_t)sort_buckets(n, num_segments);
   s.n = n;
+  const size_t digits = (size_t)kDigits * (digit_tiles(n, num_segments) + 1);
+  if (sorted_by_digits(n, num_segments)) {
+    s.digits = c.take<uint32_t>(digits);
+    s.pairs = c.take<uint64_t>((size_t)n);
+    s.spare = c.take<uint64_t>((size_t)n);
+    cursor = c.cursor;
+    return s;
+  }
+  const size_t segs = (size_t)num_segments + 1;
   s.stride = (n + bucket_rows(n) - 1) / bucket_rows(n);
+  const size_t buckets = (size_t)sort_buckets(n, num_segments);
   s.plan.bucket_rows = bucket_rows(n);
-  s.plan.tile_rows = tile_rows(n);
+  s.plan.tile_rows = kSortTile;
   s.plan.chunk_rows = chunk_rows(n);
   s.plan.buckets = (int)buckets;
   s.plan.bucket_start = c.take<int>(segs);
@@ -498,8 +761,9 @@ SortSide carve_side(char *&cursor, int n, int num_segments) {
   s.plan.total = c.take<uint32_t>(buckets);
   s.base = c.take<uint32_t>(buckets);
   s.splitters = c.take<uint64_t>(buckets);
-  s.tile_off =
-      c.take<uint32_t>((size_t)sort_tiles(n, num_segments) * s.stride);
+  // (by digits beside a larger side)
+  s.tile_off = c.take<uint32_t>(std::max(
+      (size_t)sort_tiles(n, num_segments) * s.stride, digits));
   s.pairs = c.take<uint64_t>((size_t)n);
   s.spare = c.take<uint64_t>((size_t)n);
   cursor = c.cursor;
@@ -543,6 +807,28 @@ hipError_t launch_curve_sort(const CurveSortSide *sides, int num_sides, int d,
     }
     return dim3(all);
   };
+  bool by_digits = false; // (both sides, if one of them is better off)
+  for (int i = 0; i < num_sides; ++i)
+    by_digits = by_digits || sorted_by_digits(sides[i].n, num_segments);
+  if (by_digits) {
+    for (int i = 0; i < num_sides; ++i)
+      p.side[i].stride = digit_tiles(p.side[i].n, num_segments);
+    int bits = 3 * axis_bits; // of the keys
+    while (((int64_t)1 << (bits - 3 * axis_bits)) < num_segments)
+      ++bits;
+    const dim3 tiles = grid(digit_tiles);
+    for (DigitPass pass = {0, 0, false}; !pass.last; ++pass.number) {
+      pass.shift = pass.number * kDigitBits;
+      pass.last = pass.shift + kDigitBits >= bits;
+      hipLaunchKernelGGL(digit_count_kernel, tiles, dim3(kSortThreads), 0,
+                         stream, p, pass);
+      hipLaunchKernelGGL(digit_scan_kernel, dim3(num_sides * kDigits),
+                         dim3(kSortThreads), 0, stream, p);
+      hipLaunchKernelGGL(digit_scatter_kernel, tiles, dim3(kSortThreads), 0,
+                         stream, p, pass);
+    }
+    return hipGetLastError();
+  }
   dim3 blocks = grid(sort_chunks);
   hipLaunchKernelGGL(curve_sample_kernel, blocks, dim3(1024), 0, stream, p);
   blocks = grid(sort_tiles);

@@ -89,6 +89,8 @@ struct BinsSetup {
   }
   void add_sort(int side, const int64_t *ptr, int rows, void *scratch) {
     const CurveSortPlan s = curve_sort_plan(scratch, rows, num_segments);
+    if (s.buckets == 0)
+      return;
     add(ptr, rows, s.bucket_rows, s.bucket_start);
     add(ptr, rows, s.tile_rows, s.tile_start, s.bucket_rows);
     add(ptr, rows, s.chunk_rows, s.chunk_start, s.bucket_rows);

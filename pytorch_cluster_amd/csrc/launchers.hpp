@@ -320,7 +320,8 @@ hipError_t launch_nearest_any(int dtype, const SearchInput &in,
 // What has to be there before the sort, for plan_segments and a clear: where
 // the segments' items start - buckets of `bucket_rows` rows; of the segments of
 // more rows than that also tiles of `tile_rows` and chunks of `chunk_rows` rows -
-// and zeros in the buckets' totals.
+// and zeros in the buckets' totals.  Nothing (buckets 0) for rows that are sorted by
+// digits.
 struct CurveSortPlan {
   int bucket_rows, tile_rows, chunk_rows;
   int *bucket_start, *tile_start, *chunk_start; // [num_segments + 1]
