@@ -148,18 +148,18 @@ def test_full_size_against_the_scanning_kernels():
     assert torch.equal(da.view(torch.int32), db.view(torch.int32))
 
 
-def test_queries_ordered_beside_the_rows(monkeypatch):
-    """From 131,072 queries on, the queries are ordered on a second stream
-    while the rows are ordered on the caller's: same edges with and without
-    it, call after call, on the default stream and on another one."""
+def test_large_calls_on_several_streams():
+    """The binned searches at full size between other work of the caller's
+    stream, call after call, on the default stream and on another one: the
+    edges, distances and nearest rows of the scanning kernels."""
     c = testing.lidar_scans(0)
     x, y = c["x"].to(DEV), c["y"].to(DEV)
     px = testing.pointers(c["batch_x"], c["batch_size"]).to(DEV)
     py = testing.pointers(c["batch_y"], c["batch_size"]).to(DEV)
-    monkeypatch.setenv("PCA_BINNED_SIDE_STREAM", "0")
     want, want_dist = capi.knn_edges(x, y, px, py, 16, want_dist=True,
-                                     binned=True)
-    monkeypatch.delenv("PCA_BINNED_SIDE_STREAM")
+                                     binned=False)
+    # the nearest search: 1M searching rows
+    want_rows = capi.nearest_rows(x, y, px, py, binned=False)
     other = torch.cuda.Stream()
     for stream in (torch.cuda.current_stream(), other, other):
         stream.wait_stream(torch.cuda.current_stream())
@@ -168,27 +168,24 @@ def test_queries_ordered_beside_the_rows(monkeypatch):
             noise = torch.rand(1 << 20, device=DEV).sort().values
             got, got_dist = capi.knn_edges(x, y, px, py, 16, want_dist=True,
                                            binned=True)
+            got_rows = capi.nearest_rows(x, y, px, py, binned=True)
             total = got.sum() + noise.numel()
         torch.cuda.current_stream().wait_stream(stream)
         torch.cuda.synchronize()
         assert torch.equal(got, want)
         assert torch.equal(got_dist.view(torch.int32),
                            want_dist.view(torch.int32))
+        assert torch.equal(got_rows, want_rows)
         assert int(total) == int(want.sum()) + (1 << 20)
-    # the nearest search: 1M searching rows
-    monkeypatch.setenv("PCA_BINNED_SIDE_STREAM", "0")
-    want = capi.nearest_rows(x, y, px, py, binned=True)
-    monkeypatch.delenv("PCA_BINNED_SIDE_STREAM")
-    for _ in range(2):
-        assert torch.equal(capi.nearest_rows(x, y, px, py, binned=True), want)
 
 
 @pytest.mark.parametrize("kind", ["uniform", "equal", "two_places", "in_order"])
 @pytest.mark.parametrize("d", [1, 3])
-def test_order_of_rows_in_segments_of_every_size(kind, d):
-    """The sort in front of the search: segments of one bucket of 768 rows, just
-    more than that, several tiles of 2,048 rows, empty ones; rows that share a
-    place on the curve, rows in order already."""
+def test_segments_of_every_size(kind, d):
+    """Segments of one bucket of the sort (768 rows), just more than that,
+    several tiles of 2,048 rows, empty ones; rows that share a place on the
+    curve, rows in order already: no row is lost or met twice (any order would
+    give these edges; the order itself: test_gpu_curve_order.py)."""
     rng = np.random.default_rng(31 + d)
     sizes = [1, 767, 768, 769, 0, 1536, 1537, 2048, 2049, 5000, 3, 40000]
     ptr = np.cumsum([0] + sizes).astype(np.int64)
@@ -213,10 +210,10 @@ def test_order_of_rows_in_segments_of_every_size(kind, d):
                        want_dist.view(torch.int32))
 
 
-def test_order_of_rows_in_buckets_merged_in_memory():
-    """Nine million rows of one segment: buckets of more than the 4,096 rows a
-    workgroup sorts on the chip, tiles of several steps; a clump that shares
-    few places beside a uniform cloud."""
+def test_nine_million_rows():
+    """Nine million rows, nearly all in one segment: sorted by digits, beside few
+    queries, which are sorted by samples; a clump that shares few places beside
+    a uniform cloud."""
     g = torch.Generator(device=DEV).manual_seed(3)
     x = torch.rand(9_000_000, 3, generator=g, device=DEV)
     x[::3] *= 1e-3
@@ -260,9 +257,9 @@ def test_crowded_cells_and_many_segments():
                                196608, 196640])
 def test_task_counts_at_the_edges(m):
     """Blocks of 32 queries: one, one and a bit, a whole workgroup of the
-    ordering kernels (256 blocks) and one more, the first size ordered on a
-    second stream (131,072 queries), the last size whose long blocks are
-    split (6,144 blocks) and the first that is not.  Clustered queries (long
+    ordering kernels (256 blocks) and one more, 4,096 blocks and one query
+    less, the last size whose long blocks are split (6,144 blocks) and the
+    first that is not.  Clustered queries (long
     and short spans) in two segments, against the scanning kernels."""
     g = torch.Generator().manual_seed(m)
     x = torch.rand(40000, 3, generator=g)

@@ -106,9 +106,9 @@ def test_more_than_three_dimensions_are_refused():
 
 
 def test_graph_capture_takes_the_scanning_kernel():
-    """A stream that is being captured never gets the binned search (its
-    sorts would record memset nodes): the operator scans instead, the C entry
-    point says so.  Replays give the eager result every time."""
+    """A stream that is being captured never gets the binned search, which its
+    entry points refuse there: the operator scans instead, the C entry point
+    says so.  Replays give the eager result every time."""
     import pytorch_cluster_amd as pca
     from pytorch_cluster_amd import capi
     from pytorch_cluster_amd._native import capi as lib
