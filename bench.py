@@ -420,22 +420,25 @@ class Cases:
             ms, out = _median_ms(
                 t, lambda: t.ops.torch_cluster.fps(pts, ptr, ratio, False),
                 reps or 5)
-            # A sample step depends on the one before it, and a cloud is
-            # one workgroup's, so the floor is latency, not bandwidth or
-            # rows (most rows are left alone in a step): about 100 vector
+            # A step depends on the one before it, and a cloud is one
+            # workgroup's, so the floor is latency, not bandwidth or rows
+            # (most rows are left alone in a step): about 100 vector
             # instructions that wait for each other, 4 cycles each, and
-            # three trips to the LDS of 64 cycles, at 2.4 GHz.
-            step_us = ms * 1e3 / (points // 4)
-            floor_us = (100 * 4 + 3 * 64) / 2400.0
+            # three trips to the LDS of 64 cycles, at 2.4 GHz.  A step finds
+            # at most eight samples (about five in these clouds), so no
+            # sample takes less than an eighth of that.
+            sample_us = ms * 1e3 / (points // 4)
+            floor_us = (100 * 4 + 3 * 64) / 2400.0 / 8
             report["fps %dx%d ratio 0.25" % (clouds, points)] = {
                 "ms": ms, "samples": int(out.numel()),
-                "us_per_sample_step": step_us,
+                "us_per_sample": sample_us,
                 "roofline": {
-                    "bound": "latency", "unit": "us/step",
-                    "floor": floor_us, "achieved": step_us,
-                    "frac": floor_us / step_us,
-                    "note": "dependent instructions and LDS trips of a "
-                            "sample step that looks at one bucket of rows; "
+                    "bound": "latency", "unit": "us/sample",
+                    "floor": floor_us, "achieved": sample_us,
+                    "frac": floor_us / sample_us,
+                    "note": "dependent instructions and LDS trips of a step "
+                            "that looks at one bucket of rows and finds the "
+                            "most samples it can, eight; "
                             "clouds run side by side, %d of the chip's "
                             "256 units busy" % clouds}}
         return report
