@@ -820,10 +820,10 @@ __device__ __forceinline__ void fps_few_samples(
 // groups of the samples' table.  A step: wave i tests all boxes against sample i,
 // the waves share the buckets that some sample is near to, the entries are ranked.
 //
-// 16 uniform clouds, a quarter sampled, calls (before: one sample per step): 2,048
-// rows 274 -> 231 us, 4,096 552 -> 365, 8,192 1,175 -> 687; 4,096 rows of 4
-// dimensions 646 -> 458; on 33^3 places (ties) 4,096 rows 727 -> 499, 8,192 1,588 ->
-// 960.  Of the 365 us 50 are the order of the rows; the rest are some 200 steps of
+// 16 uniform clouds, a quarter sampled, kernel (before: one sample per step): 2,048
+// rows 274 -> 231 us, 4,096 552 -> 365 (the call 575 -> 389), 8,192 1,175 -> 687;
+// 4,096 rows of 4 dimensions 646 -> 458; on 33^3 places (ties) 4,096 rows 727 -> 499,
+// 8,192 1,588 -> 960.  Of the 365 us 50 are the order of the rows; the rest are some 200 steps of
 // about 3,700 cycles, a chain of three barriers with five LDS trips between them.
 // 16 waves measured faster than 8 (452 us): two or more of the 20 buckets of a step
 // then fall to one wave.
@@ -1093,7 +1093,9 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
 // Examples of up to 64 W P rows: bucket i of wave w is in the registers of
 // that wave (row of a lane in px[.][i], pm[i]), its box and best in lane i.
 // The buckets of 16,384 rows (and those of 4 dimensions beyond 4,096) do not
-// fit the LDS.  8 x 16,384 uniform rows, a quarter sampled: 1.27 -> 0.86 us
+// fit the LDS.  With up to 3 dimensions it is for callers that give pca_fps a bound
+// of 8,193 - 16,384 rows, the only way to sample such examples in buckets on a stream
+// that is being captured; fps_stream_kernel is faster elsewhere.  8 x 16,384 uniform rows, a quarter sampled: 1.27 -> 0.86 us
 // per step (before: every row, from the same registers).
 template <int DIM, int W, int P>
 __global__ __launch_bounds__(W *kWave) void fps_bucket_kernel(
