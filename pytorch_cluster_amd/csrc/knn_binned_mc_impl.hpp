@@ -699,7 +699,7 @@ knn_binned_mc_kernel(BinnedParams p) {
     // are sparse, whose bounds reach most boxes, were bound by the latter.
     // kNN over LiDAR-like scans, calls: 36,000 rows, every fourth a query, k = 4 /
     // 16 239 -> 209, 388 -> 359 us; 3 x 60,000, every eighth 226 -> 212, 333 ->
-    // 319; the 8 scans of up to 200,000 531 -> 516; uniform clouds the same.
+    // 319; the 8 scans of up to 200,000 3 % less; uniform clouds the same.
     const int many = task.y + task.y / 2;
     auto reachable_of = [&](const Box &held, uint64_t todo) __attribute__((always_inline)) {
       // (the two lanes of a query have a bound each)
