@@ -20,13 +20,14 @@
 // The sampling is a chain of dependent steps, each an arg-max over the
 // example's rows, so the time per sample is what counts, and an example is one
 // workgroup's (a step that several workgroups share costs two trips through
-// the L2).  fps_stream_kernel has several samples per step (see "several samples
-// per step").  Up to 1,024 rows of up to 4 dimensions fps_reg_kernel looks at
+// the L2).  fps_own_kernel and fps_stream_kernel have several samples per step
+// ("a wave's own stretch of the curve", "several samples per step").  Up to 1,024
+// rows of up to 4 dimensions fps_reg_kernel looks at
 // every row in every step, from registers.  Beyond that most rows are left
 // alone (see "rows in buckets" below) where more than a few hundred samples
-// repay the sort: fps_lds_kernel keeps up to 8,192 rows in LDS,
-// fps_bucket_kernel up to 16,384 in registers, fps_stream_kernel any number in
-// memory (up to 3 dimensions).  fps_any_kernel (any size, dimension
+// repay the sort: fps_own_kernel up to 8,192 rows and fps_bucket_kernel up to
+// 16,384, from registers, fps_stream_kernel any number in memory (up to 3
+// dimensions).  fps_any_kernel (any size, dimension
 // and element type) streams the rows and a `dist` array from memory.
 #include "device_utils.hpp"
 #include "launchers.hpp"
@@ -578,13 +579,13 @@ __device__ __forceinline__ float fps_lower(const float (&q)[DIM],
 // order, as one by one.  (A sample that does not lower its own minimum -- a row
 // without a finite distance to itself, or a minimum of 0 -- is the next sample
 // again: the run ends with it.)
-constexpr int kFpsBatch = 8; // at most; 8 x 8 pairs are a wave's lanes
+constexpr int kFpsRun = 8; // at most; 8 x 8 pairs are a wave's lanes
 
 struct FpsTable {
   float4 head[kWave];      // value, row, first two coordinates
   float4 tail[kWave];      // the other coordinates, rest, its tie
-  float4 first[kFpsBatch]; // of rank i: value, coordinates
-  float4 more[kFpsBatch];  // fourth coordinate, rest, row, tie of rest
+  float4 first[kFpsRun]; // of rank i: value, coordinates
+  float4 more[kFpsRun];  // fourth coordinate, rest, row, tie of rest
 };
 // Among rows of the value `rest` of a group the complement of the smallest tie;
 // where nobody looked for it, a number that is before all others.
@@ -642,12 +643,12 @@ __device__ __forceinline__ int fps_rank(FpsTable &t, int wave, Rel rel,
 #pragma unroll
   for (int e = 1; e < OWN; ++e)
     rank = (lane & (OWN - 1)) == e ? before[e] : rank;
-  if (lane < OWN && rank < kFpsBatch) {
+  if (lane < OWN && rank < kFpsRun) {
     t.first[rank] = make_float4(h.x, h.z, h.w, g.x);
     t.more[rank] = make_float4(g.y, g.z, h.y, g.w);
   }
   fps_meet();
-  const int a = lane & (kFpsBatch - 1), b = lane / kFpsBatch;
+  const int a = lane & (kFpsRun - 1), b = lane / kFpsRun;
   const float4 ra = t.first[a], rb = t.first[b];
   const float4 ma = t.more[a];
   const float xa[4] = {ra.y, ra.z, ra.w, ma.x};
@@ -671,7 +672,7 @@ __device__ __forceinline__ int fps_rank(FpsTable &t, int wave, Rel rel,
     apart = apart && (!equal_rest || __float_as_uint(ma.w) < tie);
   }
   const uint64_t ends = __ballot(a < b && !apart);
-  return ends != 0 ? (int)__builtin_ctzll(ends) / kFpsBatch : kFpsBatch;
+  return ends != 0 ? (int)__builtin_ctzll(ends) / kFpsRun : kFpsRun;
 }
 
 // The rows of an example in curve order, by one workgroup: afterwards keys[i],
@@ -816,39 +817,295 @@ __device__ __forceinline__ void fps_few_samples(
   }
 }
 
-// Examples of up to 4,096 R rows in LDS: 64 buckets of 64 R rows, which are the
-// groups of the samples' table.  A step: wave i tests all boxes against sample i,
-// the waves share the buckets that some sample is near to, the entries are ranked.
+// ---- fp32, up to 8,192 rows: a wave's own stretch of the curve ------------------
 //
-// 16 uniform clouds, a quarter sampled, kernel (before: one sample per step): 2,048
-// rows 274 -> 231 us, 4,096 552 -> 365 (the call 575 -> 389), 8,192 1,175 -> 687;
-// 4,096 rows of 4 dimensions 646 -> 458; on 33^3 places (ties) 4,096 rows 727 -> 499,
-// 8,192 1,588 -> 960.  Of the 365 us 50 are the order of the rows; the rest are some 200 steps of
-// about 3,700 cycles, a chain of three barriers with five LDS trips between them.
-// 16 waves measured faster than 8 (452 us): two or more of the 20 buckets of a step
-// then fall to one wave.
-template <int DIM, int W, int R>
-__global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
-    const float *__restrict__ src, const int64_t *__restrict__ ptr,
-    const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
-    int d, int64_t *__restrict__ out) {
-  constexpr int T = W * kWave;
-  constexpr int CAP = 64 * kWave * R;
-  constexpr int REL_BITS = R == 1 ? 12 : 13;
-  static_assert(R == 1 || R == 2, "row numbers of 13 bits");
-  constexpr int PER = CAP / T;
-  constexpr int STRIDE = DIM <= 3 ? 4 : 5; // words of a row
-  constexpr int AT_M = STRIDE - 1;
-  __shared__ __align__(16) float rows_lds[CAP * STRIDE];
-  __shared__ uint16_t perm[CAP + 2];
-  __shared__ float part[2 * 3][W];
-  __shared__ FpsTable table;
-  __shared__ uint32_t hits_of[2][kWave]; // bit i: sample i is near to the bucket
-  __shared__ uint16_t sampled[2 * kWave];
+// The rows of an example in curve order are dealt to the 16 waves of a workgroup,
+// a stretch each, and stay in registers: row r of a lane is the lane's of the r-th
+// 64 rows of the stretch, a "piece" with a box.  A step has several samples (up to
+// 16), found as follows.
+//
+// Every wave has D entries: the row with the largest running minimum of the
+// stretch, the one that would have it if that row were sampled too, and so on, each
+// with the value it would then have; and `rest`, the first of what would be left
+// after all D.  Values with the reference's tie rule below them make one 64-bit
+// number (the key), larger ones first, so equal values need no special case.  The
+// entries of all waves are ranked.  A sample lowers minima only: while an entry's
+// row is at least its value away from all entries ranked before it, those leave its
+// value as it is, and while it comes before the `rest` of the waves whose last entry
+// is ranked before it, no row without an entry can be ahead of it.  So the samples
+// of a step are the longest run of first entries of which that holds for every pair
+// -- the same samples, in the same order, as one by one.  (The first of all always
+// holds.  A row that does not lower its own minimum -- no finite distance to itself,
+// or a minimum of 0 -- is its wave's next entry again, and the `rest` ends the run.)
+//
+// A wave then tests the boxes of its pieces against all samples at once (16 samples
+// x 4 boxes are its lanes) and goes through the pieces that a sample is near to.
+//
+// Bound by the chain of a step: three meetings with an LDS trip each, and the
+// instructions between them, of which the four waves of a SIMD execute their own.
+// 16 uniform clouds, calls, before (64 buckets in LDS, one entry each, the waves
+// sharing the buckets of a step) and now: 2,048 rows, 512 samples 258 -> 164 us;
+// 4,096 rows, a quarter 387 -> 304, half 610 -> 482, of 4 dimensions 479 -> 383,
+// on 33^3 places (ties) 522 -> 314; 8,192 rows, a quarter 701 -> 659, on 33^3
+// places 981 -> 680.  Samples per step (simulated, 4,096 rows, 1,024 samples): 64
+// buckets of one entry 5.3; 16 stretches of one entry 4.4, two 9.1, three 10.5 --
+// the third costs every changed stretch another pass over its rows (310 us).
+constexpr int kFpsBatch = 16; // samples per step at most
+template <int D> struct FpsRanks {
+  uint64_t key[D * kFpsWaves]; // entry by entry, wave by wave
+  // of rank i: coordinates; value, code, rest (0: not the wave's last entry)
+  float4 place[kFpsBatch];
+  uint4 what[kFpsBatch];
+  int end[2]; // the first rank that is no sample of the step (by turns)
+};
 
+// The low word of a key: the complement of the tie rule's number of a row of up to
+// 16,384, then the piece that it is in.  Never 0 (no row).
+__device__ __forceinline__ uint32_t fps_code(uint32_t rel, int piece) {
+  const uint32_t tie = (rel & 255u) << 6 | rel >> 8;
+  return (~tie & 0x3fffu) << 4 | (uint32_t)piece;
+}
+__device__ __forceinline__ uint32_t fps_row_of(uint32_t code) {
+  const uint32_t tie = ~(code >> 4) & 0x3fffu;
+  return (tie & 63u) << 8 | tie >> 6;
+}
+// Largest number of a wave, of numbers that are not NaN.
+__device__ __forceinline__ float wave_fmax(float v) {
+  const uint32_t u = __float_as_uint(v);
+  const uint32_t top =
+      wave_umax((int)u < 0 ? ~u : u | 0x80000000u); // (ordered like v)
+  return __uint_as_float((int)top < 0 ? top & 0x7fffffffu : ~top);
+}
+
+template <int DIM, int R, int D>
+__device__ __forceinline__ void
+fps_own_rows(const float *__restrict__ rows, int count, int d,
+             const uint32_t *keys, uint32_t row_mask, FpsRanks<D> &t,
+             uint16_t *sampled, const float (&begin_at)[DIM], int steps,
+             int64_t start_idx, int64_t *__restrict__ out) {
+  constexpr int W = kFpsWaves;
+  constexpr int CHUNKS = (R + 3) / 4; // of four boxes
+  static_assert(D * W <= kWave, "a lane per entry");
+  static_assert(R <= 16, "pieces of 4 bits in a code");
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int from = wave * count / W, to = (wave + 1) * count / W;
+
+  float x[R][DIM], low[R];
+  uint32_t code[R];
+  float blo[CHUNKS][DIM], bhi[CHUNKS][DIM]; // box 4 i + lane / 16
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int at = from + r * kWave + lane;
+    const bool ok = at < to;
+    const uint32_t rel = ok ? keys[at] & row_mask : 0u;
+    code[r] = ok ? fps_code(rel, r) : 0u;
+    low[r] = ok ? 5e4f : 0.0f;
+#pragma unroll
+    for (int c = 0; c < DIM; ++c)
+      x[r][c] = ok && c < d ? rows[(size_t)rel * d + c] : 0.0f;
+  }
+#pragma unroll
+  for (int i = 0; i < CHUNKS; ++i)
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) {
+      blo[i][c] = __builtin_inff();
+      bhi[i][c] = -__builtin_inff();
+    }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const bool ok = code[r] != 0u;
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) {
+      // (a NaN is left out: such a row's minimum never changes)
+      const float v = x[r][c];
+      const bool in = ok && v == v;
+      const float hi = wave_fmax(in ? v : -__builtin_inff());
+      const float lo = -wave_fmax(in ? -v : -__builtin_inff());
+      if (lane / 16 == (r & 3)) {
+        blo[r / 4][c] = lo;
+        bhi[r / 4][c] = hi;
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    low[r] = fps_lower<DIM>(begin_at, x[r], low[r]);
+
+  // the wave's entries (uniform), and what is left after them
+  uint32_t value[D], value_code[D], rest = 0u, rest_code = 0u;
+  float q[D][DIM];
+  auto best_of = [&](const float (&m)[R], uint32_t &most, uint32_t &its_code) {
+    double key = __hiloint2double(__float_as_int(m[0]), (int)code[0]);
+#pragma unroll
+    for (int r = 1; r < R; ++r)
+      asm("v_max_f64 %0, %1, %2"
+          : "=v"(key)
+          : "v"(key),
+            "v"(__hiloint2double(__float_as_int(m[r]), (int)code[r])));
+    const uint32_t high = (uint32_t)__double2hiint(key);
+    const uint32_t word = (uint32_t)__double2loint(key);
+    most = wave_umax(high);
+    const uint64_t who = __ballot(high == most);
+    int at = (int)__builtin_ctzll(who);
+    if (__builtin_expect((who & (who - 1)) != 0, 0)) {
+      const uint32_t mine = high == most ? word : 0u;
+      const uint32_t top = wave_umax(mine);
+      at = (int)__builtin_ctzll(__ballot(mine == top));
+    }
+    its_code = lane_value(word, at);
+    return at;
+  };
+  auto find_entries = [&]() {
+    float m[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      m[r] = low[r];
+#pragma unroll
+    for (int l = 0; l < D; ++l) {
+      const int at = best_of(m, value[l], value_code[l]);
+      const int piece = (int)(value_code[l] & 15u);
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (R == 1 || piece == r) {
+#pragma unroll
+          for (int c = 0; c < DIM; ++c)
+            q[l][c] = lane_value(x[r][c], at);
+        }
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        m[r] = fps_lower<DIM>(q[l], x[r], m[r]);
+    }
+    best_of(m, rest, rest_code);
+  };
+  if (tid < 2)
+    t.end[tid] = kFpsBatch;
+
+  int m = 1, par = 0;
+  bool changed = true;
+  while (true) {
+    if (changed) {
+      find_entries();
+      if (lane == 0) {
+#pragma unroll
+        for (int l = 0; l < D; ++l)
+          t.key[l * W + wave] = (uint64_t)value[l] << 32 | value_code[l];
+      }
+    }
+    fps_meet();
+    // how many entries come before the wave's
+    const uint64_t key = lane < D * W ? t.key[lane] : 0u;
+    int rank = 0;
+#pragma unroll
+    for (int l = 0; l < D; ++l) {
+      const uint64_t mine = (uint64_t)value[l] << 32 | value_code[l];
+      // (a row that would be sampled again)
+      const bool again = l > 0 && value[l] == value[l > 0 ? l - 1 : 0] &&
+                         value_code[l] == value_code[l > 0 ? l - 1 : 0];
+      rank = again ? rank + 1 : __builtin_popcountll(__ballot(key > mine));
+      if (rank < kFpsBatch && lane == 0) {
+        t.place[rank] = make_float4(q[l][0], DIM > 1 ? q[l][DIM > 1 ? 1 : 0] : 0.0f,
+                                    DIM > 2 ? q[l][DIM > 2 ? 2 : 0] : 0.0f,
+                                    DIM > 3 ? q[l][DIM > 3 ? 3 : 0] : 0.0f);
+        t.what[rank] = make_uint4(value[l], value_code[l],
+                                  l == D - 1 ? rest : 0u,
+                                  l == D - 1 ? rest_code : 0u);
+      }
+    }
+    fps_meet();
+    // lane i % 16: the entry of rank i
+    const int a = lane & (kFpsBatch - 1);
+    const float4 at = t.place[a];
+    const uint4 of = t.what[a];
+    const float xs[4] = {at.x, at.y, at.z, at.w};
+    float sx[DIM];
+#pragma unroll
+    for (int c = 0; c < DIM; ++c)
+      sx[c] = xs[c];
+    if (wave < kFpsBatch / 4) {
+      // sixteen entries against four that may follow them
+      const int b = lane / 16 * 4 + wave;
+      const float4 at_b = t.place[b];
+      const uint4 of_b = t.what[b];
+      const float xb[4] = {at_b.x, at_b.y, at_b.z, at_b.w};
+      float dd = 0.0f;
+#pragma unroll
+      for (int c = 0; c < DIM; ++c) {
+        const float df = sx[c] - xb[c];
+        dd = c == 0 ? df * df : __builtin_fmaf(df, df, dd);
+      }
+      const uint64_t left = (uint64_t)of.z << 32 | of.w;
+      const uint64_t key_b = (uint64_t)of_b.x << 32 | of_b.y;
+      // (a distance that is NaN ends the run)
+      const bool apart =
+          (dd >= __uint_as_float(of_b.x)) & (left < key_b);
+      const uint64_t ends = __ballot((a < b) & !apart);
+      if (ends != 0 && lane == 0)
+        atomicMin(&t.end[par], (int)__builtin_ctzll(ends) / 16 * 4 + wave);
+    }
+    // the pieces that a sample is near to, by samples
+    uint64_t near[CHUNKS];
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i)
+      near[i] = __ballot(!(fps_box_distance<DIM>(sx, blo[i], bhi[i]) >=
+                           __uint_as_float(value[0])));
+    fps_meet();
+    const int end = t.end[par];
+    const int got = min(__builtin_amdgcn_readfirstlane(end), steps - m);
+    par ^= 1;
+    if (wave == W - 1) {
+      if (lane == 0)
+        t.end[par] = kFpsBatch;
+      // (64 samples are written out at a time: the store's way to memory is
+      // then no part of a step)
+      if (lane < got)
+        sampled[(m + lane) & (2 * kWave - 1)] = (uint16_t)fps_row_of(of.y);
+      const int first = m & ~(kWave - 1), last = m + got;
+      if (last >= first + kWave || last == steps) {
+        // (the last step may end one block of samples and begin another)
+        for (int k = first + lane; k < last; k += kWave)
+          if (k > 0 && (k < first + kWave || last == steps))
+            out[k] = start_idx + sampled[k & (2 * kWave - 1)];
+      }
+    }
+    m += got;
+    if (m >= steps)
+      break;
+    bool lower = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      uint32_t some = (uint32_t)(near[r / 4] >> (r & 3) * 16) &
+                      ((1u << got) - 1);
+      if (some != 0) {
+        const float was = low[r];
+        do {
+          float s[DIM];
+#pragma unroll
+          for (int c = 0; c < DIM; ++c)
+            s[c] = lane_value(sx[c], __builtin_ctz(some));
+          some &= some - 1;
+          low[r] = fps_lower<DIM>(s, x[r], low[r]);
+        } while (some != 0);
+        lower |= low[r] < was;
+      }
+    }
+    changed = __ballot(lower) != 0;
+  }
+}
+
+template <int DIM, int CAP>
+__global__ __launch_bounds__(kFpsThreads) void fps_own_kernel(
+    const float *__restrict__ src, const int64_t *__restrict__ ptr,
+    const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
+    int d, int64_t *__restrict__ out) {
+  constexpr int REL_BITS = CAP <= 4096 ? 12 : 13;
+  constexpr int D = 2;
+  static_assert(CAP <= 8192, "row numbers of 13 bits");
+  __shared__ uint32_t keys[CAP];
+  __shared__ float part[2 * 3][kFpsWaves];
+  __shared__ __align__(16) FpsRanks<D> ranks;
+  __shared__ uint16_t sampled[2 * kWave];
   const int b = blockIdx.x;
   const int64_t start_idx = ptr[b];
   // (CAP: the caller's bound on the rows of an example)
@@ -857,237 +1114,33 @@ __global__ __launch_bounds__(W *kWave) void fps_lds_kernel(
   const int64_t o_end = out_ptr[b + 1];
   if (o_begin >= o_end)
     return;
-  if (o_end - o_begin < fps_few(DIM, true) || count <= 0) {
-    fps_few_samples<DIM, CAP, T>(src, ptr, out_ptr, start, d, out, count,
-                                 (int)(o_end - o_begin));
+  if (o_end - o_begin < fps_few(DIM, true) || count < kFpsThreads / 4) {
+    fps_few_samples<DIM, CAP, kFpsThreads>(src, ptr, out_ptr, start, d, out,
+                                           count, (int)(o_end - o_begin));
     return;
   }
   const float *rows = src + (size_t)start_idx * d;
-  const int buckets = (count + kWave * R - 1) / (kWave * R);
-
-  uint32_t *keys = reinterpret_cast<uint32_t *>(rows_lds);
-  fps_curve_order<W, DIM, REL_BITS>(rows, count, d, keys, part);
-  // (the keys give way to the rows)
-  uint16_t rel[PER];
+  fps_curve_order<kFpsWaves, DIM, REL_BITS>(rows, count, d, keys, part);
+  const int64_t first = start_idx + (start ? start[b] : 0);
+  if (threadIdx.x == 0)
+    out[o_begin] = first;
+  float at[DIM];
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int at = i * T + tid;
-    rel[i] = at < count ? (uint16_t)(keys[at] & ((1u << REL_BITS) - 1))
-                        : (uint16_t)0xffffu;
-  }
-  __syncthreads();
-#pragma unroll 4
-  for (int i = 0; i < PER; ++i) {
-    const int at = i * T + tid;
-    if (at >= buckets * kWave * R)
-      break;
-    const bool ok = rel[i] != 0xffffu;
-    perm[at] = rel[i];
-#pragma unroll
-    for (int c = 0; c < (DIM <= 3 ? 3 : DIM); ++c)
-      rows_lds[at * STRIDE + c] =
-          ok && c < d ? rows[(size_t)rel[i] * d + c] : 0.0f;
-    // (places without a row: minimum 0 and the last of all ties)
-    rows_lds[at * STRIDE + AT_M] = ok ? 5e4f : 0.0f;
-  }
-  if (tid == 0)
-    perm[CAP] = 0xffffu;
-  __syncthreads();
-
-  // lane = bucket: its box, and the best of its rows
-  float blo[DIM], bhi[DIM];
-#pragma unroll
-  for (int c = 0; c < DIM; ++c) {
-    blo[c] = __builtin_inff();
-    bhi[c] = -__builtin_inff();
-  }
-  {
-    float *low_of = &table.head[0].x, *high_of = &table.tail[0].x;
-    // (a wave goes through its share of the buckets, a row per lane; the
-    // boxes then travel through the table)
-    for (int i = wave; i < buckets; i += W) {
-      float l[DIM], h[DIM];
-#pragma unroll
-      for (int c = 0; c < DIM; ++c) {
-        l[c] = __builtin_inff();
-        h[c] = -__builtin_inff();
-      }
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int at = (i * R + r) * kWave + lane;
-        const bool ok = at < count;
-#pragma unroll
-        for (int c = 0; c < DIM; ++c) {
-          // (fminf / fmaxf drop a NaN; such a row's minimum never changes)
-          const float v = rows_lds[at * STRIDE + c];
-          l[c] = __builtin_fminf(l[c], ok ? v : __builtin_inff());
-          h[c] = __builtin_fmaxf(h[c], ok ? v : -__builtin_inff());
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < DIM; ++c) {
-#pragma unroll
-        for (int sh = 1; sh < kWave; sh <<= 1) {
-          l[c] = __builtin_fminf(l[c], __shfl_xor(l[c], sh));
-          h[c] = __builtin_fmaxf(h[c], __shfl_xor(h[c], sh));
-        }
-        if (lane == 0) {
-          low_of[i * 4 + c] = l[c];
-          high_of[i * 4 + c] = h[c];
-        }
-      }
-    }
-    __syncthreads();
-    if (lane < buckets) {
-#pragma unroll
-      for (int c = 0; c < DIM; ++c) {
-        blo[c] = low_of[lane * 4 + c];
-        bhi[c] = high_of[lane * 4 + c];
-      }
-    }
-    __syncthreads();
-  }
-  // lane i: sample i of the step
-  float sx[DIM];
-  int got = 1;
-  {
-    const int64_t first = start_idx + (start ? start[b] : 0);
-    if (tid == 0)
-      out[o_begin] = first;
-#pragma unroll
-    for (int c = 0; c < DIM; ++c)
-      sx[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
-  }
-  if (wave == 0) {
-    const float none[DIM] = {};
-    fps_enter<DIM>(table, lane, lane < buckets ? kFpsUnseen : 0u, CAP, none, 0u,
-                   kFpsAnyTie);
-    hits_of[0][lane] = 0u;
-    hits_of[1][lane] = 0u;
-  }
-  __syncthreads();
-
-  const int steps = (int)(o_end - o_begin);
-  int m = 1, par = 0;
-  while (m < steps) {
-    // sample i against the boxes by wave i
-    static_assert(W >= kFpsBatch, "a wave per sample");
-    if (wave < got) {
-      float q[DIM];
-#pragma unroll
-      for (int c = 0; c < DIM; ++c)
-        q[c] = lane_value(sx[c], wave);
-      if (!(fps_box_distance<DIM>(q, blo, bhi) >= table.head[lane].x))
-        atomicOr(&hits_of[par][lane], 1u << wave);
-    }
-    fps_meet();
-    const uint32_t hits = hits_of[par][lane];
-    par ^= 1;
-    if (wave == 0)
-      hits_of[par][lane] = 0u;
-    const uint64_t pass = __ballot(hits != 0);
-    const int passing = __builtin_popcountll(pass);
-    // (how many passing buckets come before this lane's)
-    const int before = __builtin_amdgcn_mbcnt_hi(
-        (uint32_t)(pass >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)pass, 0u));
-    const int item = hits != 0 ? before : -1;
-    for (int j = wave; j < passing; j += W) {
-      const int bucket = (int)__builtin_ctzll(__ballot(item == j));
-      float x[R][DIM], low[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const float *row = rows_lds + ((bucket * R + r) * kWave + lane) * STRIDE;
-        if (DIM <= 3) {
-          const float4 v = *reinterpret_cast<const float4 *>(row);
-          x[r][0] = v.x;
-          if (DIM > 1)
-            x[r][DIM > 1 ? 1 : 0] = v.y;
-          if (DIM > 2)
-            x[r][DIM > 2 ? 2 : 0] = v.z;
-          low[r] = v.w;
-        } else {
-#pragma unroll
-          for (int c = 0; c < DIM; ++c)
-            x[r][c] = row[c];
-          low[r] = row[AT_M];
-        }
-      }
-      uint32_t some = lane_value(hits, bucket);
-      do {
-        float q[DIM];
-#pragma unroll
-        for (int c = 0; c < DIM; ++c)
-          q[c] = lane_value(sx[c], __builtin_ctz(some));
-        some &= some - 1;
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-          low[r] = fps_lower<DIM>(q, x[r], low[r]);
-      } while (some != 0);
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        rows_lds[((bucket * R + r) * kWave + lane) * STRIDE + AT_M] = low[r];
-      // a lane's largest minimum and the other one
-      uint32_t most = __float_as_uint(low[0]), less = 0u;
-      int at_r = 0;
-      if (R == 2) {
-        const uint32_t other = __float_as_uint(low[R - 1]);
-        at_r = other > most ? 1 : 0;
-        less = min(most, other);
-        most = max(most, other);
-      }
-      const uint32_t top = wave_umax(most);
-      const bool is = most == top;
-      const uint64_t who = __ballot(is);
-      uint32_t next = wave_umax(is ? less : most);
-      uint32_t next_tie = kFpsAnyTie;
-      int at = (int)__builtin_ctzll(who);
-      if (__builtin_expect((who & (who - 1)) != 0 || next == top, 0)) {
-        // rows of equal value: the one that comes first in the reference's order
-        next = top;
-        uint32_t first = 0u, second = 0u; // (complements of the smallest ties)
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const bool equal = __float_as_uint(low[r]) == top;
-          const uint32_t t =
-              equal ? ~fps_tie(perm[(bucket * R + r) * kWave + lane]) : 0u;
-          at_r = t > first ? r : at_r;
-          second = max(second, min(first, t));
-          first = max(first, t);
-        }
-        const uint32_t t_top = wave_umax(first);
-        at = (int)__builtin_ctzll(__ballot(first == t_top));
-        next_tie = wave_umax(lane == at ? second : first);
-      }
-      if (lane == at) {
-        float best[DIM];
-#pragma unroll
-        for (int c = 0; c < DIM; ++c)
-          best[c] = R == 2 && at_r ? x[R - 1][c] : x[0][c];
-        fps_enter<DIM>(table, bucket, top,
-                       (uint32_t)((bucket * R + at_r) * kWave + lane), best,
-                       next, next_tie);
-      }
-    }
-    uint32_t chosen;
-    got = fps_rank<kWave / W, DIM>(
-        table, wave, [&](uint32_t place) { return (uint32_t)perm[place]; }, sx,
-        chosen);
-    got = min(got, steps - m);
-    if (wave == 0) {
-      // (64 samples are written out at a time: the store's way to memory is
-      // then no part of a step)
-      if (lane < got)
-        sampled[(m + lane) & (2 * kWave - 1)] = (uint16_t)chosen;
-      const int from = m & ~(kWave - 1), to = m + got;
-      if (to >= from + kWave || to == steps) {
-        // (the last step may end one block of samples and begin another)
-        for (int k = from + lane; k < to; k += kWave)
-          if (k > 0 && (k < from + kWave || to == steps))
-            out[o_begin + k] = start_idx + perm[sampled[k & (2 * kWave - 1)]];
-      }
-    }
-    m += got;
-  }
+  for (int c = 0; c < DIM; ++c)
+    at[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
+  auto run = [&](auto pieces) {
+    fps_own_rows<DIM, decltype(pieces)::value, D>(
+        rows, count, d, keys, (1u << REL_BITS) - 1, ranks, sampled, at,
+        (int)(o_end - o_begin), start_idx, out + o_begin);
+  };
+  if (CAP == 8192 && count > 4096)
+    run(std::integral_constant<int, CAP / kFpsThreads>{});
+  else if (count > 2048)
+    run(std::integral_constant<int, 4>{});
+  else if (count > 1024)
+    run(std::integral_constant<int, 2>{});
+  else
+    run(std::integral_constant<int, 1>{});
 }
 
 // Examples of up to 64 W P rows: bucket i of wave w is in the registers of
@@ -1686,9 +1739,9 @@ hipError_t launch_fps_on_chip(const float *src, const int64_t *ptr,
   else if (max_rows <= 1024)
     PCA_FPS_LAUNCH((fps_reg_kernel<DIM, 2, 512>), 512);
   else if (max_rows <= 4096)
-    PCA_FPS_LAUNCH((fps_lds_kernel<DIM, 16, 1>), 1024);
+    PCA_FPS_LAUNCH((fps_own_kernel<DIM, 4096>), 1024);
   else if (DIM <= 3 && max_rows <= 8192)
-    PCA_FPS_LAUNCH((fps_lds_kernel<DIM <= 3 ? DIM : 3, 16, 2>), 1024);
+    PCA_FPS_LAUNCH((fps_own_kernel<DIM <= 3 ? DIM : 3, 8192>), 1024);
   else
     PCA_FPS_LAUNCH((fps_bucket_kernel<DIM, 16, 16>), 1024);
 #undef PCA_FPS_LAUNCH

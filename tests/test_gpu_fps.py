@@ -115,7 +115,7 @@ def test_skipped_rows_change_nothing(oracle, rows, d, kind):
     assert (got == want).all()
 
 
-# 1,025 / 4,097: buckets of 64 and 128 rows in LDS; 32,768 / 65,536 / 262,144:
+# 1,025 / 2,048 / 4,097: rows per lane of a wave's stretch; 32,768 / 65,536 / 262,144:
 # of one, two, four pieces of 64 rows in memory and of several times four; hundreds
 # of samples, most of them several to a step
 @pytest.mark.parametrize("kind", ["uniform", "grid", "copies", "clusters"])
@@ -142,6 +142,26 @@ def test_several_samples_per_step_are_those_one_by_one(oracle, rows, d, kind):
     got = gpu_fps(oracle, x, ptr, share, start)
     want = oracle.fps_op(x, ptr, share, start)
     assert (got == want).all()
+
+
+# 255 / 256 rows: fewest of which the waves have stretches; 1,024 to 8,192: rows per
+# lane; stretches of equal and of unequal length, all examples in one call
+@pytest.mark.parametrize("kind", ["uniform", "grid"])
+@pytest.mark.parametrize("sizes,d", [
+    ([255, 256, 271, 1024, 1025, 2048, 4096], 3), ([2049, 300, 3000], 2),
+    ([4096, 1023, 2047], 4), ([8192, 4097, 4096, 1024, 260], 3),
+    ([8191, 5000], 1)])
+def test_stretches_of_every_length(oracle, sizes, d, kind):
+    rng = np.random.default_rng(sum(sizes) + d)
+    ptr = np.cumsum([0] + sizes).astype(np.int64)
+    x = rng.random((ptr[-1], d)) if kind == "uniform" else \
+        rng.integers(0, 13, (ptr[-1], d))
+    x = x.astype(np.float32)
+    # (more samples than rows: the smallest tie among minima of 0, again and again)
+    share = np.array([520.0 / n for n in sizes])
+    start = np.array([n // 2 for n in sizes], dtype=np.int64)
+    got = gpu_fps(oracle, x, ptr, share, start)
+    assert (got == oracle.fps_op(x, ptr, share, start)).all()
 
 
 # 8,192 / 16,384 rows, 340 samples: where the entry points change between the
