@@ -425,10 +425,10 @@ class Cases:
             # (most rows are left alone in a step): about 100 vector
             # instructions that wait for each other, 4 cycles each, and
             # three trips to the LDS of 64 cycles, at 2.4 GHz.  A step finds
-            # at most eight samples (about five in these clouds), so no
-            # sample takes less than an eighth of that.
+            # at most sixteen samples (about nine in these clouds), so no
+            # sample takes less than a sixteenth of that.
             sample_us = ms * 1e3 / (points // 4)
-            floor_us = (100 * 4 + 3 * 64) / 2400.0 / 8
+            floor_us = (100 * 4 + 3 * 64) / 2400.0 / 16
             report["fps %dx%d ratio 0.25" % (clouds, points)] = {
                 "ms": ms, "samples": int(out.numel()),
                 "us_per_sample": sample_us,
@@ -437,8 +437,8 @@ class Cases:
                     "floor": floor_us, "achieved": sample_us,
                     "frac": floor_us / sample_us,
                     "note": "dependent instructions and LDS trips of a step "
-                            "that looks at one bucket of rows and finds the "
-                            "most samples it can, eight; "
+                            "that looks at one piece of rows and finds the "
+                            "most samples it can, sixteen; "
                             "clouds run side by side, %d of the chip's "
                             "256 units busy" % clouds}}
         return report

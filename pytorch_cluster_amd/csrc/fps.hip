@@ -21,10 +21,11 @@
 // example's rows, so the time per sample is what counts, and an example is one
 // workgroup's (a step that several workgroups share costs two trips through
 // the L2).  fps_own_kernel and fps_stream_kernel have several samples per step
-// ("a wave's own stretch of the curve", "several samples per step").  Up to 1,024
-// rows of up to 4 dimensions fps_reg_kernel looks at
+// ("a wave's own stretch of the curve", "several samples per step").  Up to 256
+// rows of up to 4 dimensions, and up to 1,024 in calls of more examples than there
+// are compute units, fps_reg_kernel looks at
 // every row in every step, from registers.  Beyond that most rows are left
-// alone (see "rows in buckets" below) where more than a few hundred samples
+// alone (see "rows in buckets" below) where more than a hundred or so samples
 // repay the sort: fps_own_kernel up to 8,192 rows and fps_bucket_kernel up to
 // 16,384, from registers, fps_stream_kernel any number in memory (up to 3
 // dimensions).  fps_any_kernel (any size, dimension
@@ -110,6 +111,13 @@ template <int U> __device__ __forceinline__ void wave_umax_of(uint32_t (&v)[U]) 
     v[u] = (uint32_t)__builtin_amdgcn_readlane((int)v[u], 63);
 }
 #undef PCA_DPP_UMAX
+// Largest number of a wave, of numbers that are not NaN.
+__device__ __forceinline__ float wave_fmax(float v) {
+  const uint32_t u = __float_as_uint(v);
+  const uint32_t top =
+      wave_umax((int)u < 0 ? ~u : u | 0x80000000u); // (ordered like v)
+  return __uint_as_float((int)top < 0 ? top & 0x7fffffffu : ~top);
+}
 
 // ---- element types ----------------------------------------------------------
 
@@ -675,123 +683,161 @@ __device__ __forceinline__ int fps_rank(FpsTable &t, int wave, Rel rel,
   return ends != 0 ? (int)__builtin_ctzll(ends) / kFpsRun : kFpsRun;
 }
 
-// The rows of an example in curve order, by one workgroup: afterwards keys[i],
-// i < count, holds the i-th row's number (relative to the example) in its
-// REL_BITS low bits, above them its cell of the example's box.  `part`: 6 W
-// floats of LDS.
-template <int W, int DIM, int REL_BITS>
+// The rows of an example in curve order, by a workgroup of 16 waves: afterwards
+// keys[i], i < count, holds the i-th row's number (relative to the example) in its
+// REL_BITS low bits, above them its cell of the example's box (6 bits per axis).
+//
+// Two passes of 9 bits, the keys in registers between them.  A pass counts every
+// wave's digits in LDS (two waves to a word: 16 bits each, of at most 16,384 rows),
+// turns the counts into places, digit by digit and wave by wave, and writes the keys
+// there.  A wave owns a run of places, so a pass keeps the order of the one
+// before as far as the counters hand out places lane by lane; where they do not,
+// rows of one cell of the curve's upper 9 bits lie in another order, which no
+// sample depends on.  4,096 rows, until the first step: 41 us with a bitonic sort of
+// the LDS, 16 now, most of it the cells of the rows and their way from memory.
+constexpr int kFpsDigits = 512;
+struct FpsSort {
+  uint32_t count[kFpsWaves / 2][kFpsDigits];
+  float part[2 * 3][kFpsWaves];
+  uint32_t total[kFpsWaves];
+};
+template <int DIM, int REL_BITS, int CAP>
 __device__ __forceinline__ void
 fps_curve_order(const float *__restrict__ rows, int count, int d,
-                uint32_t *keys, float (*part)[W]) {
-  constexpr int T = W * kWave;
-  constexpr int AXIS_BITS = (32 - REL_BITS) / 3;
+                uint32_t *keys, FpsSort &t) {
+  constexpr int W = kFpsWaves;
+  constexpr int PER = CAP / kFpsThreads;
+  constexpr int AXIS_BITS = 6;
+  static_assert(3 * AXIS_BITS + REL_BITS <= 32 && (1 << REL_BITS) >= CAP,
+                "row and place in a word");
+  static_assert((1 << 3 * AXIS_BITS) == kFpsDigits * kFpsDigits, "two digits");
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
-  const int wave = tid / kWave;
-  float lo[3], hi[3];
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  // (a wave's rows follow each other)
+  const int first = wave * (kWave * PER) + lane;
+  float v[PER][3], lo[3], hi[3];
+#pragma unroll
+  for (int i = 0; i < PER; ++i)
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      v[i][c] = first + i * kWave < count && c < DIM && c < d
+                    ? rows[(size_t)(first + i * kWave) * d + c]
+                    : 0.0f;
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    lo[c] = __builtin_inff();
-    hi[c] = -__builtin_inff();
-  }
-  for (int i = tid; i < count; i += T) {
+    lo[c] = hi[c] = 0.0f;
+    if (c < DIM) {
+      lo[c] = __builtin_inff();
+      hi[c] = -__builtin_inff();
 #pragma unroll
-    for (int c = 0; c < (DIM < 3 ? DIM : 3); ++c)
-      if (c < d) {
-        const float v = rows[(size_t)i * d + c];
-        if (__builtin_fabsf(v) < __builtin_inff()) {
-          lo[c] = __builtin_fminf(lo[c], v);
-          hi[c] = __builtin_fmaxf(hi[c], v);
+      for (int i = 0; i < PER; ++i)
+        if (first + i * kWave < count &&
+            __builtin_fabsf(v[i][c]) < __builtin_inff()) {
+          lo[c] = __builtin_fminf(lo[c], v[i][c]);
+          hi[c] = __builtin_fmaxf(hi[c], v[i][c]);
         }
+      lo[c] = -wave_fmax(-lo[c]);
+      hi[c] = wave_fmax(hi[c]);
+      if (lane == 0) {
+        t.part[c][wave] = lo[c];
+        t.part[3 + c][wave] = hi[c];
       }
-  }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-#pragma unroll
-    for (int sh = 1; sh < kWave; sh <<= 1) {
-      lo[c] = __builtin_fminf(lo[c], __shfl_xor(lo[c], sh));
-      hi[c] = __builtin_fmaxf(hi[c], __shfl_xor(hi[c], sh));
-    }
-    if (lane == 0) {
-      part[c][wave] = lo[c];
-      part[3 + c][wave] = hi[c];
     }
   }
+  auto clear = [&]() {
+    for (int i = tid; i < W / 2 * kFpsDigits; i += kFpsThreads)
+      (&t.count[0][0])[i] = 0u;
+  };
+  clear();
   __syncthreads();
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      lo[c] = __builtin_fminf(lo[c], part[c][w]);
-      hi[c] = __builtin_fmaxf(hi[c], part[3 + c][w]);
-    }
+  for (int c = 0; c < DIM && c < 3; ++c) {
+    lo[c] = -wave_fmax(-t.part[c][lane & (W - 1)]);
+    hi[c] = wave_fmax(t.part[3 + c][lane & (W - 1)]);
   }
-  int n2 = kWave;
-  while (n2 < count)
-    n2 <<= 1;
-  for (int i = tid; i < n2; i += T) {
-    uint32_t key = 0xffffffffu;
-    if (i < count) {
-      float v[3] = {0.0f, 0.0f, 0.0f};
+  uint32_t key[PER];
 #pragma unroll
-      for (int c = 0; c < (DIM < 3 ? DIM : 3); ++c)
-        if (c < d)
-          v[c] = rows[(size_t)i * d + c];
-      const uint32_t code =
-          curve_place(v, lo, hi, d < DIM ? d : DIM, AXIS_BITS);
-      key = (code << REL_BITS) | (uint32_t)i;
-    }
-    keys[i] = key;
-  }
-  __syncthreads();
-  // bitonic sort; exchanges over fewer than 64 places inside the waves
-  for (int k = kWave; k <= n2; k <<= 1) {
-    for (int j = k >> 1; j >= kWave; j >>= 1) {
-      for (int i = tid; i < n2 / 2; i += T) {
-        const int a = ((i & ~(j - 1)) << 1) | (i & (j - 1));
-        const uint32_t u = keys[a], v = keys[a | j];
-        if ((u > v) == ((a & k) == 0)) {
-          keys[a] = v;
-          keys[a | j] = u;
-        }
-      }
-      __syncthreads();
-    }
-    for (int i = tid; i < n2; i += T) {
-      uint32_t u = keys[i];
-      auto exchange = [&](int j, bool up) {
-        const uint32_t v = (uint32_t)__shfl_xor((int)u, j);
-        u = ((lane & j) == 0) == up ? min(u, v) : max(u, v);
-      };
-      if (k == kWave) {
+  for (int i = 0; i < PER; ++i)
+    key[i] = curve_place(v[i], lo, hi, d < DIM ? d : DIM, AXIS_BITS)
+                 << REL_BITS |
+             (uint32_t)(first + i * kWave);
+  const int shift = (wave & 1) * 16;
+  uint32_t *const mine = t.count[wave / 2];
 #pragma unroll
-        for (int kk = 2; kk < kWave; kk <<= 1)
+  for (int pass = 0; pass < 2; ++pass) {
+    uint32_t digit[PER], at[PER];
 #pragma unroll
-          for (int j = kk >> 1; j > 0; j >>= 1)
-            exchange(j, (lane & kk) == 0);
-      }
-#pragma unroll
-      for (int j = kWave / 2; j > 0; j >>= 1)
-        exchange(j, (i & k) == 0);
-      keys[i] = u;
+    for (int i = 0; i < PER; ++i) {
+      digit[i] = key[i] >> (REL_BITS + 9 * pass) & (kFpsDigits - 1);
+      at[i] = first + i * kWave < count
+                  ? atomicAdd(&mine[digit[i]], 1u << shift) >> shift & 0xffffu
+                  : 0u;
     }
     __syncthreads();
+    // a thread: eight waves' counts of one digit, two threads a digit
+    uint32_t of[4], sum = 0u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      of[i] = t.count[(tid & 1) * 4 + i][tid / 2];
+      sum += (of[i] & 0xffffu) + (of[i] >> 16);
+    }
+    uint32_t before = sum;
+#pragma unroll
+    for (int sh = 1; sh < kWave; sh <<= 1) {
+      const uint32_t other = __shfl_up(before, sh);
+      before += lane >= sh ? other : 0u;
+    }
+    if (lane == kWave - 1)
+      t.total[wave] = before;
+    before -= sum;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+      before += w < wave ? t.total[w] : 0u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t low = before;
+      before += of[i] & 0xffffu;
+      t.count[(tid & 1) * 4 + i][tid / 2] = before << 16 | low;
+      before += of[i] >> 16;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (first + i * kWave < count)
+        keys[(mine[digit[i]] >> shift & 0xffffu) + at[i]] = key[i];
+    __syncthreads();
+    if (pass == 0) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        key[i] = first + i * kWave < count ? keys[first + i * kWave] : 0u;
+      clear();
+      __syncthreads();
+    }
   }
 }
 
-// Putting the rows in buckets has to pay: with fewer samples than this every
-// row is looked at instead.  Kernel, us, all rows / buckets, 16 examples of 100,
-// 220, 300 samples each, from LDS: 1,100 rows 59 / 93, 126 / 137, 171 / 163; 2,048
-// rows 59 / 101, 127 / 144, 171 / 170; 4,096 69 / 118, 149 / 163, 202 / 185; 8,192
-// 85 / 168, 182 / 219, 247 / 247; 4,096 of 4 dimensions 76 / 142, 160 / 195, 218 /
-// 229.  From registers (fps_bucket_kernel), 256 and 512 samples: 8 x 16,384 342 /
-// 398, 669 / 584; 16 x 4,096 of 4 dimensions 196 / 240, 384 / 386.
-constexpr int fps_few(int dim, bool lds) {
-  return lds ? (dim > 3 ? 340 : 280) : (dim > 3 ? 480 : 340);
+// The order along the curve has to pay: with fewer samples than this every row is
+// looked at instead.  Calls, us, all rows / stretches, 16 examples: 400 rows, 100
+// samples 63 / 64, 150 83 / 71; 1,024, 60 56 / 61, 100 76 / 68; 2,048, 110 86 / 91, 140
+// 104 / 97; 4,096, 110 98 / 106, 140 118 / 113; 8,192, 140 140 / 155, 180 173 / 168;
+// of 4 dimensions 2,048, 110 93 / 102, 140 111 / 109; 4,096, 140 129 / 135, 170 152 /
+// 148.  Beyond that fps_bucket_kernel, 256 and 512 samples of 8 x 16,384 rows: 342 /
+// 398, 669 / 584.
+__device__ __forceinline__ int fps_few(int dim, int count) {
+  if (dim <= 3)
+    return count <= 512    ? 120
+           : count <= 1024 ? 90
+           : count <= 4096 ? 130
+           : count <= 8192 ? 170
+                           : 340;
+  return count <= 2048 ? 140 : count <= 8192 ? 170 : 480;
 }
 
-// Such an example by a workgroup of 1,024 threads.  Up to 8,192 rows half of
-// them hold the rows, which leaves fewer results to hand over per step; the
+// Such an example by a workgroup of 1,024 threads.  Up to 512 rows one wave has
+// them all; up to 8,192 half of the threads hold the rows, which leaves fewer
+// results to hand over per step; the
 // others only come to the barriers of fps_every_row (one before the first step
 // and one per step; 16 x 2,048 rows, 128 samples: 85 us, by all threads 111).
 template <int DIM, int CAP, int T>
@@ -799,11 +845,15 @@ __device__ __forceinline__ void fps_few_samples(
     const float *__restrict__ src, const int64_t *__restrict__ ptr,
     const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
     int d, int64_t *__restrict__ out, int count, int samples) {
-  static_assert(T == 1024 && (CAP == 4096 || CAP == 8192 || CAP == 16384),
-                "rows per thread");
+  static_assert(T == 1024 && CAP % T == 0 && CAP <= 16 * T, "rows per thread");
   if constexpr (CAP == 16384) {
     fps_every_row<DIM, 16, T>(src, ptr, out_ptr, start, d, out);
   } else {
+    if (CAP == 1024 && count <= 512) {
+      if (threadIdx.x < kWave)
+        fps_every_row<DIM, 8, kWave>(src, ptr, out_ptr, start, d, out);
+      return;
+    }
     if (threadIdx.x >= T / 2) {
       for (int m = 0; m < samples; ++m)
         __syncthreads();
@@ -818,6 +868,7 @@ __device__ __forceinline__ void fps_few_samples(
 }
 
 // ---- fp32, up to 8,192 rows: a wave's own stretch of the curve ------------------
+// (up to 16,384 of sorted rows of up to 3 dimensions, by fps_stream_kernel)
 //
 // The rows of an example in curve order are dealt to the 16 waves of a workgroup,
 // a stretch each, and stay in registers: row r of a lane is the lane's of the r-th
@@ -841,16 +892,21 @@ __device__ __forceinline__ void fps_few_samples(
 // A wave then tests the boxes of its pieces against all samples at once (16 samples
 // x 4 boxes are its lanes) and goes through the pieces that a sample is near to.
 //
-// Bound by the chain of a step: three meetings with an LDS trip each, and the
-// instructions between them, of which the four waves of a SIMD execute their own.
+// Bound by the chain of a step, about 5,000 cycles for nine samples of 4,096 rows:
+// three meetings with an LDS trip each, and the
+// instructions between them, of which the four waves of a SIMD execute their own
+// (1,500 for the entries of a wave whose rows changed, ten of sixteen do, 750 for the
+// rows themselves, 500 for ranks, 400 for pairs and boxes).
 // 16 uniform clouds, calls, before (64 buckets in LDS, one entry each, the waves
-// sharing the buckets of a step) and now: 2,048 rows, 512 samples 258 -> 164 us;
-// 4,096 rows, a quarter 387 -> 304, half 610 -> 482, of 4 dimensions 479 -> 383,
-// on 33^3 places (ties) 522 -> 314; 8,192 rows, a quarter 701 -> 659, on 33^3
-// places 981 -> 680.  Samples per step (simulated, 4,096 rows, 1,024 samples): 64
+// sharing the buckets of a step; up to 1,024 rows every row in every step) and now:
+// 1,024 rows, 300 samples 180 -> 100 us; 2,048, 512 258 -> 158;
+// 4,096 rows, a quarter 386 -> 283, half 609 -> 458, of 4 dimensions 477 -> 365,
+// on 33^3 places (ties) 522 -> 294; 8,192 rows, a quarter 702 -> 601, on 33^3
+// places 982 -> 621; 1,000 of 4 dimensions, 8 clouds, 1,043 -> 533.  Samples per step (simulated, 4,096 rows, 1,024 samples): 64
 // buckets of one entry 5.3; 16 stretches of one entry 4.4, two 9.1, three 10.5 --
 // the third costs every changed stretch another pass over its rows (310 us).
 constexpr int kFpsBatch = 16; // samples per step at most
+constexpr int kFpsOwnLeast = 256; // rows of an example (every wave has some)
 template <int D> struct FpsRanks {
   uint64_t key[D * kFpsWaves]; // entry by entry, wave by wave
   // of rank i: coordinates; value, code, rest (0: not the wave's last entry)
@@ -860,29 +916,28 @@ template <int D> struct FpsRanks {
 };
 
 // The low word of a key: the complement of the tie rule's number of a row of up to
-// 16,384, then the piece that it is in.  Never 0 (no row).
+// 16,384 (15 bits of it: never 0, which is no row), then the piece that it is in.
 __device__ __forceinline__ uint32_t fps_code(uint32_t rel, int piece) {
   const uint32_t tie = (rel & 255u) << 6 | rel >> 8;
-  return (~tie & 0x3fffu) << 4 | (uint32_t)piece;
+  return (~tie & 0x7fffu) << 4 | (uint32_t)piece;
 }
 __device__ __forceinline__ uint32_t fps_row_of(uint32_t code) {
   const uint32_t tie = ~(code >> 4) & 0x3fffu;
   return (tie & 63u) << 8 | tie >> 6;
 }
-// Largest number of a wave, of numbers that are not NaN.
-__device__ __forceinline__ float wave_fmax(float v) {
-  const uint32_t u = __float_as_uint(v);
-  const uint32_t top =
-      wave_umax((int)u < 0 ? ~u : u | 0x80000000u); // (ordered like v)
-  return __uint_as_float((int)top < 0 ? top & 0x7fffffffu : ~top);
+template <int N, typename F> __device__ __forceinline__ void for_each_of(F f) {
+  if constexpr (N > 0) {
+    for_each_of<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
 }
 
-template <int DIM, int R, int D>
+// `row_at`(i, x): number and coordinates of the i-th row along the curve.
+template <int DIM, int R, int D, typename Rows>
 __device__ __forceinline__ void
-fps_own_rows(const float *__restrict__ rows, int count, int d,
-             const uint32_t *keys, uint32_t row_mask, FpsRanks<D> &t,
-             uint16_t *sampled, const float (&begin_at)[DIM], int steps,
-             int64_t start_idx, int64_t *__restrict__ out) {
+fps_own_rows(const Rows &row_at, int count, FpsRanks<D> &t,
+             const float (&begin_at)[DIM], int steps, int64_t start_idx,
+             int64_t *__restrict__ out) {
   constexpr int W = kFpsWaves;
   constexpr int CHUNKS = (R + 3) / 4; // of four boxes
   static_assert(D * W <= kWave, "a lane per entry");
@@ -892,19 +947,23 @@ fps_own_rows(const float *__restrict__ rows, int count, int d,
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int from = wave * count / W, to = (wave + 1) * count / W;
 
-  float x[R][DIM], low[R];
-  uint32_t code[R];
+  // a row's key: running minimum above, code below (minima are in [0, 5e4]: read
+  // as doubles the keys order as they should, and none is a NaN); `left`: with the
+  // entries found so far sampled
+  float x[R][DIM];
+  constexpr bool KEEP = R <= 8; // (16 rows: not the registers; formed again)
+  double low[R], left[KEEP ? R : 1];
   float blo[CHUNKS][DIM], bhi[CHUNKS][DIM]; // box 4 i + lane / 16
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int at = from + r * kWave + lane;
     const bool ok = at < to;
-    const uint32_t rel = ok ? keys[at] & row_mask : 0u;
-    code[r] = ok ? fps_code(rel, r) : 0u;
-    low[r] = ok ? 5e4f : 0.0f;
-#pragma unroll
-    for (int c = 0; c < DIM; ++c)
-      x[r][c] = ok && c < d ? rows[(size_t)rel * d + c] : 0.0f;
+    // (where there is none, the last one again)
+    const uint32_t rel = row_at(min(at, to - 1), x[r]);
+    low[r] = __hiloint2double(__float_as_int(ok ? 5e4f : 0.0f),
+                              (int)(ok ? fps_code(rel, r) : 0u));
+    if (KEEP)
+      left[KEEP ? r : 0] = low[r];
   }
 #pragma unroll
   for (int i = 0; i < CHUNKS; ++i)
@@ -915,7 +974,7 @@ fps_own_rows(const float *__restrict__ rows, int count, int d,
     }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const bool ok = code[r] != 0u;
+    const bool ok = __double2loint(low[r]) != 0;
 #pragma unroll
     for (int c = 0; c < DIM; ++c) {
       // (a NaN is left out: such a row's minimum never changes)
@@ -929,21 +988,42 @@ fps_own_rows(const float *__restrict__ rows, int count, int d,
       }
     }
   }
+  auto minimum = [](double key) {
+    return __int_as_float(__double2hiint(key));
+  };
+  auto with_minimum = [](double key, float m) {
+    return __hiloint2double(__float_as_int(m), __double2loint(key));
+  };
 #pragma unroll
   for (int r = 0; r < R; ++r)
-    low[r] = fps_lower<DIM>(begin_at, x[r], low[r]);
+    low[r] = with_minimum(low[r],
+                          fps_lower<DIM>(begin_at, x[r], minimum(low[r])));
 
   // the wave's entries (uniform), and what is left after them
   uint32_t value[D], value_code[D], rest = 0u, rest_code = 0u;
   float q[D][DIM];
-  auto best_of = [&](const float (&m)[R], uint32_t &most, uint32_t &its_code) {
-    double key = __hiloint2double(__float_as_int(m[0]), (int)code[0]);
+  // the first of the rows with the entries found before sampled
+  auto best_of = [&](auto found, uint32_t &most, uint32_t &its_code) {
+    constexpr int l = decltype(found)::value;
+    double key = 0.0;
 #pragma unroll
-    for (int r = 1; r < R; ++r)
-      asm("v_max_f64 %0, %1, %2"
-          : "=v"(key)
-          : "v"(key),
-            "v"(__hiloint2double(__float_as_int(m[r]), (int)code[r])));
+    for (int r = 0; r < R; ++r) {
+      double with = low[r];
+      if constexpr (KEEP && l > 0) {
+        left[r] = with_minimum(
+            left[r], fps_lower<DIM>(q[l - 1], x[r],
+                                    minimum(l == 1 ? low[r] : left[r])));
+        with = left[r];
+      } else {
+#pragma unroll
+        for (int j = 0; j < l; ++j)
+          with = with_minimum(with, fps_lower<DIM>(q[j], x[r], minimum(with)));
+      }
+      if (r == 0)
+        key = with;
+      else
+        asm("v_max_f64 %0, %1, %2" : "=v"(key) : "v"(key), "v"(with));
+    }
     const uint32_t high = (uint32_t)__double2hiint(key);
     const uint32_t word = (uint32_t)__double2loint(key);
     most = wave_umax(high);
@@ -958,13 +1038,9 @@ fps_own_rows(const float *__restrict__ rows, int count, int d,
     return at;
   };
   auto find_entries = [&]() {
-    float m[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      m[r] = low[r];
-#pragma unroll
-    for (int l = 0; l < D; ++l) {
-      const int at = best_of(m, value[l], value_code[l]);
+    for_each_of<D>([&](auto which) {
+      constexpr int l = decltype(which)::value;
+      const int at = best_of(which, value[l], value_code[l]);
       const int piece = (int)(value_code[l] & 15u);
 #pragma unroll
       for (int r = 0; r < R; ++r)
@@ -973,11 +1049,8 @@ fps_own_rows(const float *__restrict__ rows, int count, int d,
           for (int c = 0; c < DIM; ++c)
             q[l][c] = lane_value(x[r][c], at);
         }
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        m[r] = fps_lower<DIM>(q[l], x[r], m[r]);
-    }
-    best_of(m, rest, rest_code);
+    });
+    best_of(std::integral_constant<int, D>{}, rest, rest_code);
   };
   if (tid < 2)
     t.end[tid] = kFpsBatch;
@@ -1054,20 +1127,11 @@ fps_own_rows(const float *__restrict__ rows, int count, int d,
     const int end = t.end[par];
     const int got = min(__builtin_amdgcn_readfirstlane(end), steps - m);
     par ^= 1;
-    if (wave == W - 1) {
+    if (wave == W - 1 && lane < got) {
+      // (nobody waits for the stores)
+      out[m + lane] = start_idx + fps_row_of(of.y);
       if (lane == 0)
         t.end[par] = kFpsBatch;
-      // (64 samples are written out at a time: the store's way to memory is
-      // then no part of a step)
-      if (lane < got)
-        sampled[(m + lane) & (2 * kWave - 1)] = (uint16_t)fps_row_of(of.y);
-      const int first = m & ~(kWave - 1), last = m + got;
-      if (last >= first + kWave || last == steps) {
-        // (the last step may end one block of samples and begin another)
-        for (int k = first + lane; k < last; k += kWave)
-          if (k > 0 && (k < first + kWave || last == steps))
-            out[k] = start_idx + sampled[k & (2 * kWave - 1)];
-      }
     }
     m += got;
     if (m >= steps)
@@ -1078,16 +1142,18 @@ fps_own_rows(const float *__restrict__ rows, int count, int d,
       uint32_t some = (uint32_t)(near[r / 4] >> (r & 3) * 16) &
                       ((1u << got) - 1);
       if (some != 0) {
-        const float was = low[r];
+        const float was = minimum(low[r]);
+        float now = was;
         do {
           float s[DIM];
 #pragma unroll
           for (int c = 0; c < DIM; ++c)
             s[c] = lane_value(sx[c], __builtin_ctz(some));
           some &= some - 1;
-          low[r] = fps_lower<DIM>(s, x[r], low[r]);
+          now = fps_lower<DIM>(s, x[r], now);
         } while (some != 0);
-        lower |= low[r] < was;
+        lower |= now < was;
+        low[r] = with_minimum(low[r], now);
       }
     }
     changed = __ballot(lower) != 0;
@@ -1095,17 +1161,51 @@ fps_own_rows(const float *__restrict__ rows, int count, int d,
 }
 
 template <int DIM, int CAP>
+__device__ __forceinline__ void
+fps_own_example(const float *__restrict__ src, int64_t start_idx, int count,
+                int64_t first, int d, int steps, int64_t *__restrict__ out) {
+  constexpr int REL_BITS = 13;
+  constexpr int D = 2;
+  static_assert(CAP <= 8192, "row numbers of 13 bits");
+  __shared__ uint32_t keys[CAP];
+  __shared__ FpsSort sort;
+  __shared__ __align__(16) FpsRanks<D> ranks;
+  const float *rows = src + (size_t)start_idx * d;
+  fps_curve_order<DIM, REL_BITS, CAP>(rows, count, d, keys, sort);
+  if (threadIdx.x == 0)
+    out[0] = first;
+  float at[DIM];
+#pragma unroll
+  for (int c = 0; c < DIM; ++c)
+    at[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
+  auto run = [&](auto pieces) {
+    fps_own_rows<DIM, decltype(pieces)::value>(
+        [&](int i, float (&x)[DIM]) {
+          const uint32_t rel = keys[i] & ((1u << REL_BITS) - 1);
+#pragma unroll
+          for (int c = 0; c < DIM; ++c)
+            x[c] = c < d ? rows[(size_t)rel * d + c] : 0.0f;
+          return rel;
+        },
+        count, ranks, at, steps, start_idx, out);
+  };
+  // (rows of a lane: what the example takes, at most what the launch allows for)
+  constexpr int MOST = CAP / kFpsThreads;
+  if (MOST > 4 && count > 4 * kFpsThreads)
+    run(std::integral_constant<int, MOST>{});
+  else if (MOST > 2 && count > 2 * kFpsThreads)
+    run(std::integral_constant<int, MOST < 4 ? MOST : 4>{});
+  else if (MOST > 1 && count > kFpsThreads)
+    run(std::integral_constant<int, MOST < 2 ? MOST : 2>{});
+  else
+    run(std::integral_constant<int, 1>{});
+}
+
+template <int DIM, int CAP>
 __global__ __launch_bounds__(kFpsThreads) void fps_own_kernel(
     const float *__restrict__ src, const int64_t *__restrict__ ptr,
     const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
     int d, int64_t *__restrict__ out) {
-  constexpr int REL_BITS = CAP <= 4096 ? 12 : 13;
-  constexpr int D = 2;
-  static_assert(CAP <= 8192, "row numbers of 13 bits");
-  __shared__ uint32_t keys[CAP];
-  __shared__ float part[2 * 3][kFpsWaves];
-  __shared__ __align__(16) FpsRanks<D> ranks;
-  __shared__ uint16_t sampled[2 * kWave];
   const int b = blockIdx.x;
   const int64_t start_idx = ptr[b];
   // (CAP: the caller's bound on the rows of an example)
@@ -1114,41 +1214,24 @@ __global__ __launch_bounds__(kFpsThreads) void fps_own_kernel(
   const int64_t o_end = out_ptr[b + 1];
   if (o_begin >= o_end)
     return;
-  if (o_end - o_begin < fps_few(DIM, true) || count < kFpsThreads / 4) {
+  const int steps = (int)(o_end - o_begin);
+  if (steps < fps_few(DIM, count) || count < kFpsOwnLeast) {
     fps_few_samples<DIM, CAP, kFpsThreads>(src, ptr, out_ptr, start, d, out,
-                                           count, (int)(o_end - o_begin));
+                                           count, steps);
     return;
   }
-  const float *rows = src + (size_t)start_idx * d;
-  fps_curve_order<kFpsWaves, DIM, REL_BITS>(rows, count, d, keys, part);
   const int64_t first = start_idx + (start ? start[b] : 0);
-  if (threadIdx.x == 0)
-    out[o_begin] = first;
-  float at[DIM];
-#pragma unroll
-  for (int c = 0; c < DIM; ++c)
-    at[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
-  auto run = [&](auto pieces) {
-    fps_own_rows<DIM, decltype(pieces)::value, D>(
-        rows, count, d, keys, (1u << REL_BITS) - 1, ranks, sampled, at,
-        (int)(o_end - o_begin), start_idx, out + o_begin);
-  };
-  if (CAP == 8192 && count > 4096)
-    run(std::integral_constant<int, CAP / kFpsThreads>{});
-  else if (count > 2048)
-    run(std::integral_constant<int, 4>{});
-  else if (count > 1024)
-    run(std::integral_constant<int, 2>{});
-  else
-    run(std::integral_constant<int, 1>{});
+  fps_own_example<DIM, CAP>(src, start_idx, count, first, d, steps,
+                            out + o_begin);
 }
 
 // Examples of up to 64 W P rows: bucket i of wave w is in the registers of
 // that wave (row of a lane in px[.][i], pm[i]), its box and best in lane i.
-// The buckets of 16,384 rows (and those of 4 dimensions beyond 4,096) do not
-// fit the LDS.  With up to 3 dimensions it is for callers that give pca_fps a bound
-// of 8,193 - 16,384 rows, the only way to sample such examples in buckets on a stream
-// that is being captured; fps_stream_kernel is faster elsewhere.  8 x 16,384 uniform rows, a quarter sampled: 1.27 -> 0.86 us
+// For 8,193 - 16,384 rows.  With up to 3 dimensions it is for callers that give
+// pca_fps such a bound, the only way to sample such examples in buckets on a stream
+// that is being captured; of hundreds of samples the sorted path is faster.  (The
+// stretches with 16 rows per lane in its place: 200 - 300 samples 1.03 - 1.4 times as
+// fast, but fewer, which look at every row, 2 - 12 % slower beside them.)  8 x 16,384 uniform rows, a quarter sampled: 1.27 -> 0.86 us
 // per step (before: every row, from the same registers).
 template <int DIM, int W, int P>
 __global__ __launch_bounds__(W *kWave) void fps_bucket_kernel(
@@ -1160,7 +1243,7 @@ __global__ __launch_bounds__(W *kWave) void fps_bucket_kernel(
   constexpr int REL_BITS = 14;
   static_assert(CAP <= 16384 && P <= 16 && W <= 16, "row numbers in the keys");
   __shared__ uint32_t keys[CAP];
-  __shared__ float part[2 * 3][W];
+  __shared__ FpsSort sort;
   __shared__ FpsBest<DIM> table[2][W];
 
   const int tid = threadIdx.x;
@@ -1174,14 +1257,14 @@ __global__ __launch_bounds__(W *kWave) void fps_bucket_kernel(
   const int64_t o_end = out_ptr[b + 1];
   if (o_begin >= o_end)
     return;
-  if (o_end - o_begin < fps_few(DIM, false) || count <= 0) {
+  if (o_end - o_begin < fps_few(DIM, count) || count <= 0) {
     fps_few_samples<DIM, CAP, T>(src, ptr, out_ptr, start, d, out, count,
                                  (int)(o_end - o_begin));
     return;
   }
   const float *rows = src + (size_t)start_idx * d;
 
-  fps_curve_order<W, DIM, REL_BITS>(rows, count, d, keys, part);
+  fps_curve_order<DIM, REL_BITS, CAP>(rows, count, d, keys, sort);
 
   // -- the buckets of this wave -----------------------------------------------
   float px[DIM][P];
@@ -1373,7 +1456,7 @@ __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
 // it waits for the wave with the most; minima stored where nothing changed 3.4;
 // up to four samples per step 3.7; buckets of 128 rows 2.9 (16-lane groups of
 // 64 rows could not hold 200,000).
-template <int W, int R, bool MANY>
+template <int W, int R, bool MANY, bool OWN>
 __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
     const float *__restrict__ src, const int64_t *__restrict__ ptr,
     const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
@@ -1389,6 +1472,7 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
   __shared__ float4 found_tail[kWave * W]; // z, rest, its tie, -
   __shared__ int items[2];
   __shared__ uint32_t sampled[2 * kWave];
+  __shared__ __align__(16) FpsRanks<OWN ? 2 : 1> ranks;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -1401,6 +1485,34 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
     return;
   const int64_t first_piece = fps_first_piece(start_idx, b);
   const float4 *rows = p.rows + first_piece * kWave;
+  // Examples whose rows fit the registers after all (a bound of 16,385: 8 x 16,384
+  // rows, 1,000 samples 727 -> 589 us, 8,300 666 -> 521).  Not in calls of larger
+  // ones: the registers make those 1 % slower.
+  if (OWN && count >= kFpsOwnLeast && count <= 16 * kFpsThreads) {
+    float at[DIM];
+    const int64_t first = start_idx + (start ? start[b] : 0);
+    if (tid == 0)
+      out[o_begin] = first;
+#pragma unroll
+    for (int c = 0; c < DIM; ++c)
+      at[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
+    auto run = [&](auto rows_of_lane) {
+      fps_own_rows<DIM, decltype(rows_of_lane)::value>(
+          [&](int i, float (&x)[DIM]) {
+            const float4 row = rows[i];
+            x[0] = row.x;
+            x[1] = row.y;
+            x[2] = row.z;
+            return __float_as_uint(row.w);
+          },
+          count, ranks, at, (int)(o_end - o_begin), start_idx, out + o_begin);
+    };
+    if (count > 8 * kFpsThreads)
+      run(std::integral_constant<int, 16>{});
+    else
+      run(std::integral_constant<int, 8>{});
+    return;
+  }
   float *minima = p.minima + first_piece * kWave;
   const int pieces = (count + kWave - 1) / kWave;
   const int chunks =
@@ -1722,6 +1834,11 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
   }
 }
 
+// Up to 1,024 rows the kernels that look at every row take less of a compute unit:
+// for more examples than this.  Every row / stretches, us: 400 rows, 200 samples, 256
+// examples 102 / 84, 300 105 / 133; 1,024 rows, 60 samples 56 / 56, 63 / 89.
+constexpr int kFpsOwnMost = 256;
+
 template <int DIM>
 hipError_t launch_fps_on_chip(const float *src, const int64_t *ptr,
                               const int64_t *out_ptr, const int64_t *start,
@@ -1732,16 +1849,21 @@ hipError_t launch_fps_on_chip(const float *src, const int64_t *ptr,
                      src, ptr, out_ptr, start, d, out)
   // (shapes by measurement: 16 examples of each size on one device; the
   // kernels' comments give the times on both sides of a limit)
+  const bool many = num_segments > kFpsOwnMost;
   if (max_rows <= 256)
     PCA_FPS_LAUNCH((fps_reg_kernel<DIM, 4, 64>), 64);
-  else if (max_rows <= 512)
+  else if (max_rows <= 512 && many)
     PCA_FPS_LAUNCH((fps_reg_kernel<DIM, 8, 64>), 64);
-  else if (max_rows <= 1024)
+  else if (max_rows <= 1024 && many)
     PCA_FPS_LAUNCH((fps_reg_kernel<DIM, 2, 512>), 512);
+  else if (max_rows <= 1024)
+    PCA_FPS_LAUNCH((fps_own_kernel<DIM, 1024>), 1024);
+  else if (max_rows <= 2048)
+    PCA_FPS_LAUNCH((fps_own_kernel<DIM, 2048>), 1024);
   else if (max_rows <= 4096)
     PCA_FPS_LAUNCH((fps_own_kernel<DIM, 4096>), 1024);
-  else if (DIM <= 3 && max_rows <= 8192)
-    PCA_FPS_LAUNCH((fps_own_kernel<DIM <= 3 ? DIM : 3, 8192>), 1024);
+  else if (max_rows <= 8192)
+    PCA_FPS_LAUNCH((fps_own_kernel<DIM, 8192>), 1024);
   else
     PCA_FPS_LAUNCH((fps_bucket_kernel<DIM, 16, 16>), 1024);
 #undef PCA_FPS_LAUNCH
@@ -1823,18 +1945,20 @@ hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
   // (half as many rows to a bucket where the lanes suffice: 8 x 60,000 rows, 600
   // samples each, R = 1 / 2 910 / 840 us, 8 x 20,000 1,160 / 1,240; the scans, at
   // most 200,000 rows, R = 4 2.8 ms, 2 x 4 2.9)
-#define PCA_FPS_STREAM(S_, MANY_)                                              \
-  hipLaunchKernelGGL((fps_stream_kernel<kFpsWaves, S_, MANY_>),                \
+#define PCA_FPS_STREAM(S_, MANY_, OWN_)                                        \
+  hipLaunchKernelGGL((fps_stream_kernel<kFpsWaves, S_, MANY_, OWN_>),          \
                      dim3(num_segments), dim3(kFpsThreads), 0, stream, src,    \
                      ptr, out_ptr, start, d, p, out)
-  if (rows <= kWave * kFpsThreads / 2)
-    PCA_FPS_STREAM(1, false);
+  if (rows <= 16 * kFpsThreads + 1)
+    PCA_FPS_STREAM(1, false, true);
+  else if (rows <= kWave * kFpsThreads / 2)
+    PCA_FPS_STREAM(1, false, false);
   else if (rows <= kWave * kFpsThreads)
-    PCA_FPS_STREAM(2, false);
+    PCA_FPS_STREAM(2, false, false);
   else if (rows <= 4 * kWave * kFpsThreads)
-    PCA_FPS_STREAM(4, false);
+    PCA_FPS_STREAM(4, false, false);
   else
-    PCA_FPS_STREAM(4, true);
+    PCA_FPS_STREAM(4, true, false);
 #undef PCA_FPS_STREAM
   return hipGetLastError();
 }

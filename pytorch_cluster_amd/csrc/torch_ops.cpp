@@ -994,13 +994,13 @@ at::Tensor fps_host(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
 // at in every step, 0.6 us per 1,000 rows.  All rows / sorted, us: 4 x 17,000 rows, 4
 // samples each 35 / 69, 8 79 / 89, 16 167 / 108; 2 x 60,000, 2 samples 38 / 75, 4 107 /
 // 97.  Between 8,192 and 16,384 rows of up to 3 dimensions examples of many samples
-// are better off sorted as well, several samples to a step: on the chip / sorted
-// 16 x 8,300 rows, 200 samples 263 / 276, 300 390 / 327, 500 512 / 424; 8 x 16,384,
-// 200 262 / 309, 300 389 / 371; 200 x 9,000, 300 413 / 431.
+// are better off sorted as well: every row on the chip / sorted, stretches in
+// registers, 16 x 8,300 rows, 200 samples 283 / 258, 320 435 / 310; 8 x 16,384, 200 283
+// / 285, 320 436 / 340; 64 x 12,000, 240 337 / 338, 320 440 / 368.
 int64_t fps_bound(int64_t longest, int64_t samples, int64_t d) {
   if (longest > 16384)
     return (samples - 1) * longest <= 130000 ? 0 : longest;
-  return longest > 8192 && samples >= 340 && d <= 3 ? 16385 : longest;
+  return longest > 8192 && samples >= 240 && d <= 3 ? 16385 : longest;
 }
 
 at::Tensor fps(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
