@@ -9,7 +9,8 @@ Outputs (next to this file, git-ignored):
   _torch_ops.so         TorchScript operator binding (links the above)
   libpca_probe.so       csrc/probes/: measurement and checking aids
                         (`bench.py --probe`, the bf16 rounding check of
-                        tests/test_gpu_dtypes.py), no part of the searches
+                        tests/test_gpu_dtypes.py, the impatient fps of
+                        tests/test_gpu_fps.py), no part of the searches
 """
 import argparse
 import concurrent.futures
@@ -84,7 +85,9 @@ def build_capi(jobs):
 
 def build_probes():
     sources = sorted(glob.glob(os.path.join(CSRC, "probes", "*.hip")))
-    _run([HIPCC] + HIP_FLAGS + ["-shared"] + sources + ["-o", PROBE_LIB])
+    _run([HIPCC] + HIP_FLAGS + ["-shared"] + sources +
+         ["-o", PROBE_LIB, "-L", HERE, "-lpca_neighbors",
+          "-Wl,-rpath,$ORIGIN"])
     return PROBE_LIB
 
 

@@ -18,17 +18,19 @@
 //     -1 (every distance NaN) the sample is row 0.
 //
 // The sampling is a chain of dependent steps, each an arg-max over the
-// example's rows, so the time per sample is what counts, and an example is one
-// workgroup's (a step that several workgroups share costs two trips through
-// the L2).  fps_own_kernel and fps_stream_kernel have several samples per step
-// ("a wave's own stretch of the curve", "several samples per step").  Up to 256
+// example's rows, so the time per sample is what counts, and an example of up to
+// 8,192 rows is one workgroup's (what several workgroups tell each other takes 1.3 us
+// of a step).  fps_own_kernel, fps_shared_kernel and fps_stream_kernel have several
+// samples per step ("a wave's own stretch of the curve", "the same, an example by
+// several workgroups", "several samples per step").  Up to 256
 // rows of up to 4 dimensions, and up to 1,024 in calls of more examples than there
 // are compute units, fps_reg_kernel looks at
 // every row in every step, from registers.  Beyond that most rows are left
 // alone (see "rows in buckets" below) where more than a hundred or so samples
 // repay the sort: fps_own_kernel up to 8,192 rows and fps_bucket_kernel up to
-// 16,384, from registers, fps_stream_kernel any number in memory (up to 3
-// dimensions).  fps_any_kernel (any size, dimension
+// 16,384, from registers, fps_shared_kernel up to 524,288 of few examples, from the
+// registers of several workgroups, and fps_stream_kernel any number in memory (both
+// up to 3 dimensions).  fps_any_kernel (any size, dimension
 // and element type) streams the rows and a `dist` array from memory.
 #include "device_utils.hpp"
 #include "launchers.hpp"
@@ -93,6 +95,16 @@ __device__ __forceinline__ uint32_t row16_umax_all(uint32_t v) {
   PCA_DPP_UMAX(v, 0x124, 0xf); // row_ror:4
   PCA_DPP_UMAX(v, 0x122, 0xf); // row_ror:2
   PCA_DPP_UMAX(v, 0x121, 0xf); // row_ror:1
+  return v;
+}
+// Every lane gets the sum of its eight.
+__device__ __forceinline__ uint32_t row8_sum(uint32_t v) {
+#define PCA_DPP_ADD(ctrl)                                                      \
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xf, 0xf, false)
+  PCA_DPP_ADD(0xb1);  // quad_perm 1,0,3,2
+  PCA_DPP_ADD(0x4e);  // quad_perm 2,3,0,1
+  PCA_DPP_ADD(0x141); // row_half_mirror
+#undef PCA_DPP_ADD
   return v;
 }
 // U waves' worth of values at once: their steps fill each other's wait states.
@@ -868,7 +880,8 @@ __device__ __forceinline__ void fps_few_samples(
 }
 
 // ---- fp32, up to 8,192 rows: a wave's own stretch of the curve ------------------
-// (up to 16,384 of sorted rows of up to 3 dimensions, by fps_stream_kernel)
+// (up to 16,384 of sorted rows of up to 3 dimensions, by fps_stream_kernel, in calls of
+// many examples)
 //
 // The rows of an example in curve order are dealt to the 16 waves of a workgroup,
 // a stretch each, and stay in registers: row r of a lane is the lane's of the r-th
@@ -916,14 +929,17 @@ template <int D> struct FpsRanks {
 };
 
 // The low word of a key: the complement of the tie rule's number of a row of up to
-// 16,384 (15 bits of it: never 0, which is no row), then the piece that it is in.
+// 2^BITS (BITS + 1 bits of it: never 0, which is no row), then the piece that it is
+// in.
+template <int BITS>
 __device__ __forceinline__ uint32_t fps_code(uint32_t rel, int piece) {
-  const uint32_t tie = (rel & 255u) << 6 | rel >> 8;
-  return (~tie & 0x7fffu) << 4 | (uint32_t)piece;
+  const uint32_t tie = (rel & 255u) << (BITS - 8) | rel >> 8;
+  return (~tie & ((2u << BITS) - 1)) << 4 | (uint32_t)piece;
 }
+template <int BITS>
 __device__ __forceinline__ uint32_t fps_row_of(uint32_t code) {
-  const uint32_t tie = ~(code >> 4) & 0x3fffu;
-  return (tie & 63u) << 8 | tie >> 6;
+  const uint32_t tie = ~(code >> 4) & ((1u << BITS) - 1);
+  return (tie & ((1u << (BITS - 8)) - 1)) << 8 | tie >> (BITS - 8);
 }
 template <int N, typename F> __device__ __forceinline__ void for_each_of(F f) {
   if constexpr (N > 0) {
@@ -932,79 +948,93 @@ template <int N, typename F> __device__ __forceinline__ void for_each_of(F f) {
   }
 }
 
-// `row_at`(i, x): number and coordinates of the i-th row along the curve.
-template <int DIM, int R, int D, typename Rows>
-__device__ __forceinline__ void
-fps_own_rows(const Rows &row_at, int count, FpsRanks<D> &t,
-             const float (&begin_at)[DIM], int steps, int64_t start_idx,
-             int64_t *__restrict__ out) {
-  constexpr int W = kFpsWaves;
-  constexpr int CHUNKS = (R + 3) / 4; // of four boxes
-  static_assert(D * W <= kWave, "a lane per entry");
+// The rows of a wave, R of a lane, with the boxes of its pieces and its D entries.
+// S: samples of a step at most; BITS: row numbers.
+template <int DIM, int R, int D, int S, int BITS> struct FpsHeld {
+  static constexpr int BOXES = kWave / S; // a lane per box and sample
+  static constexpr int CHUNKS = (R + BOXES - 1) / BOXES;
+  static constexpr bool KEEP = R <= 8; // (16 rows: not the registers; formed again)
+  // boxes (16 pieces and 32 samples a step: in LDS, as registers they are spilled)
+  static constexpr bool IN_REGS = R <= 8 || S <= 16;
   static_assert(R <= 16, "pieces of 4 bits in a code");
-  const int tid = threadIdx.x;
-  const int lane = tid & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int from = wave * count / W, to = (wave + 1) * count / W;
-
+  float x[R][DIM];
   // a row's key: running minimum above, code below (minima are in [0, 5e4]: read
   // as doubles the keys order as they should, and none is a NaN); `left`: with the
   // entries found so far sampled
-  float x[R][DIM];
-  constexpr bool KEEP = R <= 8; // (16 rows: not the registers; formed again)
   double low[R], left[KEEP ? R : 1];
-  float blo[CHUNKS][DIM], bhi[CHUNKS][DIM]; // box 4 i + lane / 16
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int at = from + r * kWave + lane;
-    const bool ok = at < to;
-    // (where there is none, the last one again)
-    const uint32_t rel = row_at(min(at, to - 1), x[r]);
-    low[r] = __hiloint2double(__float_as_int(ok ? 5e4f : 0.0f),
-                              (int)(ok ? fps_code(rel, r) : 0u));
-    if (KEEP)
-      left[KEEP ? r : 0] = low[r];
+  // box BOXES i + lane / S
+  float blo[IN_REGS ? CHUNKS : 1][DIM], bhi[IN_REGS ? CHUNKS : 1][DIM];
+  // the wave's entries (uniform), and what is left after them
+  uint32_t value[D], value_code[D], rest, rest_code;
+  float q[D][DIM];
+
+  static __device__ __forceinline__ float minimum(double key) {
+    return __int_as_float(__double2hiint(key));
   }
+  static __device__ __forceinline__ double with_minimum(double key, float m) {
+    return __hiloint2double(__float_as_int(m), __double2loint(key));
+  }
+
+  // lower corner, upper corner of a piece's box
+  static __device__ __forceinline__ float4 *box_of(int piece) {
+    __shared__ float4 boxes[kFpsWaves][R][2];
+    return boxes[threadIdx.x / kWave][piece];
+  }
+
+  // `row_at`(i, x): number and coordinates of the i-th row along the curve; piece r
+  // is the rows from `place`(r) on that are before `to`.
+  template <typename Rows, typename Place>
+  __device__ __forceinline__ void load(const Rows &row_at, const Place &place,
+                                       int to, const float (&begin_at)[DIM]) {
+    const int lane = threadIdx.x & (kWave - 1);
 #pragma unroll
-  for (int i = 0; i < CHUNKS; ++i)
-#pragma unroll
-    for (int c = 0; c < DIM; ++c) {
-      blo[i][c] = __builtin_inff();
-      bhi[i][c] = -__builtin_inff();
+    for (int r = 0; r < R; ++r) {
+      const int at = place(r) + lane;
+      const bool ok = at < to;
+      // (where there is none, the last one again)
+      const uint32_t rel = row_at(min(at, to - 1), x[r]);
+      low[r] = __hiloint2double(__float_as_int(ok ? 5e4f : 0.0f),
+                                (int)(ok ? fps_code<BITS>(rel, r) : 0u));
+      if (KEEP)
+        left[KEEP ? r : 0] = low[r];
     }
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const bool ok = __double2loint(low[r]) != 0;
+    for (int i = 0; IN_REGS && i < CHUNKS; ++i)
 #pragma unroll
-    for (int c = 0; c < DIM; ++c) {
-      // (a NaN is left out: such a row's minimum never changes)
-      const float v = x[r][c];
-      const bool in = ok && v == v;
-      const float hi = wave_fmax(in ? v : -__builtin_inff());
-      const float lo = -wave_fmax(in ? -v : -__builtin_inff());
-      if (lane / 16 == (r & 3)) {
-        blo[r / 4][c] = lo;
-        bhi[r / 4][c] = hi;
+      for (int c = 0; c < DIM; ++c) {
+        blo[IN_REGS ? i : 0][c] = __builtin_inff();
+        bhi[IN_REGS ? i : 0][c] = -__builtin_inff();
+      }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const bool ok = __double2loint(low[r]) != 0;
+      float lo[4] = {}, hi[4] = {};
+#pragma unroll
+      for (int c = 0; c < DIM; ++c) {
+        // (a NaN is left out: such a row's minimum never changes)
+        const float v = x[r][c];
+        const bool in = ok && v == v;
+        hi[c] = wave_fmax(in ? v : -__builtin_inff());
+        lo[c] = -wave_fmax(in ? -v : -__builtin_inff());
+        if (IN_REGS && lane / S == r % BOXES) {
+          blo[IN_REGS ? r / BOXES : 0][c] = lo[c];
+          bhi[IN_REGS ? r / BOXES : 0][c] = hi[c];
+        }
+      }
+      if (!IN_REGS && lane == 0) {
+        box_of(r)[0] = make_float4(lo[0], lo[1], lo[2], lo[3]);
+        box_of(r)[1] = make_float4(hi[0], hi[1], hi[2], hi[3]);
       }
     }
-  }
-  auto minimum = [](double key) {
-    return __int_as_float(__double2hiint(key));
-  };
-  auto with_minimum = [](double key, float m) {
-    return __hiloint2double(__float_as_int(m), __double2loint(key));
-  };
 #pragma unroll
-  for (int r = 0; r < R; ++r)
-    low[r] = with_minimum(low[r],
-                          fps_lower<DIM>(begin_at, x[r], minimum(low[r])));
+    for (int r = 0; r < R; ++r)
+      low[r] = with_minimum(low[r],
+                            fps_lower<DIM>(begin_at, x[r], minimum(low[r])));
+  }
 
-  // the wave's entries (uniform), and what is left after them
-  uint32_t value[D], value_code[D], rest = 0u, rest_code = 0u;
-  float q[D][DIM];
-  // the first of the rows with the entries found before sampled
-  auto best_of = [&](auto found, uint32_t &most, uint32_t &its_code) {
-    constexpr int l = decltype(found)::value;
+  // the first of the rows with the l entries found before sampled
+  template <int l>
+  __device__ __forceinline__ int best_of(uint32_t &most, uint32_t &its_code) {
     double key = 0.0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -1036,11 +1066,11 @@ fps_own_rows(const Rows &row_at, int count, FpsRanks<D> &t,
     }
     its_code = lane_value(word, at);
     return at;
-  };
-  auto find_entries = [&]() {
+  }
+  __device__ __forceinline__ void find_entries() {
     for_each_of<D>([&](auto which) {
       constexpr int l = decltype(which)::value;
-      const int at = best_of(which, value[l], value_code[l]);
+      const int at = this->template best_of<l>(value[l], value_code[l]);
       const int piece = (int)(value_code[l] & 15u);
 #pragma unroll
       for (int r = 0; r < R; ++r)
@@ -1050,8 +1080,83 @@ fps_own_rows(const Rows &row_at, int count, FpsRanks<D> &t,
             q[l][c] = lane_value(x[r][c], at);
         }
     });
-    best_of(std::integral_constant<int, D>{}, rest, rest_code);
-  };
+    best_of<D>(rest, rest_code);
+  }
+  // entry l is the one before it (a row that would be sampled again)
+  __device__ __forceinline__ bool again(int l) const {
+    return l > 0 && value[l] == value[l > 0 ? l - 1 : 0] &&
+           value_code[l] == value_code[l > 0 ? l - 1 : 0];
+  }
+
+  // the pieces that a sample is near to, by samples (lane i % S: sample i)
+  __device__ __forceinline__ void find_near(const float (&s)[DIM],
+                                            uint64_t (&near)[CHUNKS]) const {
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i) {
+      float dd;
+      if constexpr (IN_REGS) {
+        dd = fps_box_distance<DIM>(s, blo[i], bhi[i]);
+      } else {
+        const float4 *box =
+            box_of(i * BOXES + (int)(threadIdx.x & (kWave - 1)) / S);
+        const float4 at[2] = {box[0], box[1]};
+        const float lo[4] = {at[0].x, at[0].y, at[0].z, at[0].w};
+        const float hi[4] = {at[1].x, at[1].y, at[1].z, at[1].w};
+        float l[DIM], u[DIM];
+#pragma unroll
+        for (int c = 0; c < DIM; ++c) {
+          l[c] = lo[c];
+          u[c] = hi[c];
+        }
+        dd = fps_box_distance<DIM>(s, l, u);
+      }
+      near[i] = __ballot(!(dd >= __uint_as_float(value[0])));
+    }
+  }
+  // the first `got` samples; whether a minimum of the wave is another now
+  __device__ __forceinline__ bool sample(const float (&s)[DIM],
+                                         const uint64_t (&near)[CHUNKS],
+                                         int got) {
+    bool lower = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      uint32_t some = (uint32_t)(near[r / BOXES] >> (r % BOXES) * S) &
+                      (S < 32 ? (1u << got) - 1 : 0xffffffffu >> (32 - got));
+      if (some != 0) {
+        const float was = minimum(low[r]);
+        float now = was;
+        do {
+          float at[DIM];
+#pragma unroll
+          for (int c = 0; c < DIM; ++c)
+            at[c] = lane_value(s[c], __builtin_ctz(some));
+          some &= some - 1;
+          now = fps_lower<DIM>(at, x[r], now);
+        } while (some != 0);
+        lower |= now < was;
+        low[r] = with_minimum(low[r], now);
+      }
+    }
+    return __ballot(lower) != 0;
+  }
+};
+
+template <int DIM, int R, int D, typename Rows>
+__device__ __forceinline__ void
+fps_own_rows(const Rows &row_at, int count, FpsRanks<D> &t,
+             const float (&begin_at)[DIM], int steps, int64_t start_idx,
+             int64_t *__restrict__ out) {
+  constexpr int W = kFpsWaves;
+  constexpr int BITS = 14;
+  static_assert(D * W <= kWave, "a lane per entry");
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int from = wave * count / W, to = (wave + 1) * count / W;
+
+  typedef FpsHeld<DIM, R, D, kFpsBatch, BITS> Held;
+  Held h;
+  h.load(row_at, [&](int r) { return from + r * kWave; }, to, begin_at);
   if (tid < 2)
     t.end[tid] = kFpsBatch;
 
@@ -1059,11 +1164,11 @@ fps_own_rows(const Rows &row_at, int count, FpsRanks<D> &t,
   bool changed = true;
   while (true) {
     if (changed) {
-      find_entries();
+      h.find_entries();
       if (lane == 0) {
 #pragma unroll
         for (int l = 0; l < D; ++l)
-          t.key[l * W + wave] = (uint64_t)value[l] << 32 | value_code[l];
+          t.key[l * W + wave] = (uint64_t)h.value[l] << 32 | h.value_code[l];
       }
     }
     fps_meet();
@@ -1072,18 +1177,17 @@ fps_own_rows(const Rows &row_at, int count, FpsRanks<D> &t,
     int rank = 0;
 #pragma unroll
     for (int l = 0; l < D; ++l) {
-      const uint64_t mine = (uint64_t)value[l] << 32 | value_code[l];
-      // (a row that would be sampled again)
-      const bool again = l > 0 && value[l] == value[l > 0 ? l - 1 : 0] &&
-                         value_code[l] == value_code[l > 0 ? l - 1 : 0];
-      rank = again ? rank + 1 : __builtin_popcountll(__ballot(key > mine));
+      const uint64_t mine = (uint64_t)h.value[l] << 32 | h.value_code[l];
+      rank = h.again(l) ? rank + 1
+                        : __builtin_popcountll(__ballot(key > mine));
       if (rank < kFpsBatch && lane == 0) {
-        t.place[rank] = make_float4(q[l][0], DIM > 1 ? q[l][DIM > 1 ? 1 : 0] : 0.0f,
-                                    DIM > 2 ? q[l][DIM > 2 ? 2 : 0] : 0.0f,
-                                    DIM > 3 ? q[l][DIM > 3 ? 3 : 0] : 0.0f);
-        t.what[rank] = make_uint4(value[l], value_code[l],
-                                  l == D - 1 ? rest : 0u,
-                                  l == D - 1 ? rest_code : 0u);
+        t.place[rank] =
+            make_float4(h.q[l][0], DIM > 1 ? h.q[l][DIM > 1 ? 1 : 0] : 0.0f,
+                        DIM > 2 ? h.q[l][DIM > 2 ? 2 : 0] : 0.0f,
+                        DIM > 3 ? h.q[l][DIM > 3 ? 3 : 0] : 0.0f);
+        t.what[rank] = make_uint4(h.value[l], h.value_code[l],
+                                  l == D - 1 ? h.rest : 0u,
+                                  l == D - 1 ? h.rest_code : 0u);
       }
     }
     fps_meet();
@@ -1117,46 +1221,22 @@ fps_own_rows(const Rows &row_at, int count, FpsRanks<D> &t,
       if (ends != 0 && lane == 0)
         atomicMin(&t.end[par], (int)__builtin_ctzll(ends) / 16 * 4 + wave);
     }
-    // the pieces that a sample is near to, by samples
-    uint64_t near[CHUNKS];
-#pragma unroll
-    for (int i = 0; i < CHUNKS; ++i)
-      near[i] = __ballot(!(fps_box_distance<DIM>(sx, blo[i], bhi[i]) >=
-                           __uint_as_float(value[0])));
+    uint64_t near[Held::CHUNKS];
+    h.find_near(sx, near);
     fps_meet();
     const int end = t.end[par];
     const int got = min(__builtin_amdgcn_readfirstlane(end), steps - m);
     par ^= 1;
     if (wave == W - 1 && lane < got) {
       // (nobody waits for the stores)
-      out[m + lane] = start_idx + fps_row_of(of.y);
+      out[m + lane] = start_idx + fps_row_of<BITS>(of.y);
       if (lane == 0)
         t.end[par] = kFpsBatch;
     }
     m += got;
     if (m >= steps)
       break;
-    bool lower = false;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      uint32_t some = (uint32_t)(near[r / 4] >> (r & 3) * 16) &
-                      ((1u << got) - 1);
-      if (some != 0) {
-        const float was = minimum(low[r]);
-        float now = was;
-        do {
-          float s[DIM];
-#pragma unroll
-          for (int c = 0; c < DIM; ++c)
-            s[c] = lane_value(sx[c], __builtin_ctz(some));
-          some &= some - 1;
-          now = fps_lower<DIM>(s, x[r], now);
-        } while (some != 0);
-        lower |= now < was;
-        low[r] = with_minimum(low[r], now);
-      }
-    }
-    changed = __ballot(lower) != 0;
+    changed = h.sample(sx, near, got);
   }
 }
 
@@ -1391,14 +1471,31 @@ struct FpsPieces {
 };
 constexpr int kFpsPieces = 4;
 static_assert(kFpsPieces == kBlock / kWave, "a block of the kernel below");
+// What the workgroups of an example tell each other (see fps_shared_kernel): by
+// turns two sets of kFpsShareWords, and whether one of them gave up.
+constexpr int kFpsShareMost = 32; // workgroups of an example at most
+constexpr int kFpsShareRows = 1;  // rows of a lane that a workgroup is worth
+constexpr int kFpsTold = 128;     // entries that they tell each other, of all
+constexpr int kFpsShareWords = kFpsTold * 4;
+struct FpsShare {
+  uint64_t *words;  // [examples][2][kFpsShareWords]; NULL: not shared
+  uint32_t *failed; // [examples]
+};
 __host__ __device__ constexpr int64_t fps_first_piece(int64_t begin, int b) {
   return begin / kWave + (int64_t)kFpsPieces * b;
 }
 __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
     const float *__restrict__ src, const int64_t *__restrict__ ptr, int d,
-    int first_segment, const uint32_t *__restrict__ perm, FpsPieces out) {
+    int first_segment, const uint32_t *__restrict__ perm, FpsPieces out,
+    FpsShare share) {
   const int b = first_segment + blockIdx.y;
   const int lane = threadIdx.x & (kWave - 1);
+  if (share.words != nullptr && blockIdx.x == 0) {
+    for (int i = threadIdx.x; i < 2 * kFpsShareWords; i += kBlock)
+      share.words[(size_t)b * (2 * kFpsShareWords) + i] = 0u;
+    if (threadIdx.x == 0)
+      share.failed[b] = 0u;
+  }
   const int64_t begin = ptr[b], end = ptr[b + 1];
   if (begin + (int64_t)blockIdx.x * kBlock >= end)
     return;
@@ -1432,6 +1529,307 @@ __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
   }
 }
 
+// ---- the same, an example by several workgroups -----------------------------------
+//
+// The pieces of an example are dealt in turn to up to 32 workgroups of 16 waves,
+// which hold their rows in registers as in fps_own_kernel: along the curve the next
+// piece is another workgroup's, so that the places where samples are found (the thin
+// outer parts of a scan) are everybody's.  A workgroup ranks the entries and the
+// `rest` of its waves and tells the others the first seven and, as a bound, the
+// eighth; no row after a `rest` is told but after it.  All read what all
+// told and go on alike: the entries that are before every bound are ranked, up to 32
+// of them, and the samples of the step are the longest run of first ones that are
+// pairwise apart.  (Three or seven entries of a workgroup are enough: of the scans
+// below 18.5 samples per step with seven entries, 17.5 with three, simulated.)
+//
+// What is told are words of 8 bytes, half of each the step's number, so that a
+// reader knows by the word itself that it has arrived: one trip through the
+// memory that the XCDs share, no fence, no flag.  A workgroup writes a set again two
+// steps later, when all have told the step between, that is, have read the set.
+//
+// All workgroups of an example have to run at the same time.  The launch asks for no
+// more than the device has compute units, but work on other streams may hold some:
+// every wait ends after `patience` looks (about a millisecond), the workgroup then
+// marks the example and ends, and so do the others, which hear nothing more from it.
+// fps_stream_kernel, launched behind, samples the marked examples from the start.
+//
+// Bound by the chain of a step, about 12,000 cycles for 16 samples of a scan of
+// 200,000 rows by 32 workgroups: rows and entries 2,900 (of the slowest wave), what
+// is told 5,200 (3,000 of 8 workgroups), ranks 1,300, pairs and boxes 900, four
+// meetings.  Calls, us, one workgroup each -> shared: eight scans of 60,000 - 200,000
+// rows, 2 % sampled, 2,795 -> 1,121; one of them 1,198 -> 522; uniform rows, 8 x
+// 16,384, 1,000 samples 601 -> 485; 16 x 16,384, a quarter 1,588 -> 886; 64 x 20,000,
+// a tenth 1,783 -> 1,079; 1 x 500,000, 5,000 samples 9,952 -> 2,535; 128 x 20,000, two
+// workgroups each, 1,276 -> 1,350: not below four.  What else was tried, eight scans /
+// one scan: the words of an entry in four lines that all workgroups write to 2,073 /
+// 1,063 (before ranks and layout as they are 1,558 / 763); ranks by a wave of each
+// SIMD, an entry after the other, 4,600 cycles; 16 workgroups of an example 1,866 /
+// 633; a pause between two looks no change; a workgroup for 2,048 rows at least 1 x
+// 16,000, 1,600 samples 581, for 4,096 706, for 1,024 526.
+struct FpsTold {
+  uint64_t key[3 * kFpsWaves]; // of this workgroup: entries, then rests
+  // of all: value and code (0: none); coordinates; the bounds
+  uint64_t first[kFpsTold];
+  float at[kFpsTold][3];
+  uint64_t bound[kFpsShareMost];
+  // of rank i: coordinates and value; code, step that it is of
+  float4 place[32];
+  uint2 what[32];
+  int end[2]; // the first rank that is no sample of the step (by turns)
+  int late;
+};
+template <int R, int S>
+__device__ __forceinline__ bool
+fps_shared_rows(const float4 *__restrict__ rows, int count, int part, int parts,
+                FpsTold &t, uint64_t *words, int patience,
+                const float (&begin_at)[3], int steps, int64_t start_idx,
+                int64_t *__restrict__ out) {
+  constexpr int W = kFpsWaves;
+  constexpr int D = 2;
+  constexpr int BITS = 19;
+  constexpr uint32_t STEP = (1u << 12) - 1; // below a code's 20 bits
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+
+  typedef FpsHeld<3, R, D, S, BITS> Held;
+  Held h;
+  h.load(
+      [&](int i, float (&x)[3]) {
+        const float4 row = rows[i];
+        x[0] = row.x;
+        x[1] = row.y;
+        x[2] = row.z;
+        return __float_as_uint(row.w);
+      },
+      [&](int r) { return ((r * W + wave) * parts + part) * kWave; }, count,
+      begin_at);
+  if (tid < 2)
+    t.end[tid] = S;
+  if (tid == 0)
+    t.late = 0;
+  if (tid < kFpsTold)
+    t.first[tid] = 0u;
+  if (tid < kFpsShareMost)
+    t.bound[tid] = 0u;
+  if (tid < 32)
+    t.what[tid] = make_uint2(0u, 0u);
+
+  // (entries of a workgroup)
+  const int tells = parts > 16 ? 4 : parts > 8 ? 8 : 16;
+  const int slots = parts * tells;
+  int m = 1, step = 0;
+  bool changed = true;
+  while (m < steps) {
+    ++step;
+    uint64_t *const set = words + (step & 1) * kFpsShareWords;
+    if (changed) {
+      h.find_entries();
+      if (lane == 0) {
+#pragma unroll
+        for (int l = 0; l < D; ++l)
+          t.key[l * W + wave] = (uint64_t)h.value[l] << 32 | h.value_code[l];
+        t.key[D * W + wave] = (uint64_t)h.rest << 32 | h.rest_code;
+      }
+    }
+    fps_meet();
+    {
+      const uint64_t key = lane < (D + 1) * W ? t.key[lane] : 0u;
+      int rank = 0;
+#pragma unroll
+      for (int l = 0; l <= D; ++l) {
+        const uint32_t value = l < D ? h.value[l < D ? l : 0] : h.rest;
+        const uint32_t code = l < D ? h.value_code[l < D ? l : 0] : h.rest_code;
+        const bool again =
+            l < D ? h.again(l)
+                  : value == h.value[D - 1] && code == h.value_code[D - 1];
+        const uint64_t mine = (uint64_t)value << 32 | code;
+        const uint64_t more = __ballot(key > mine);
+        rank = again ? rank + 1 : __builtin_popcountll(more);
+        if (rank < tells && lane < 4) {
+          // the first rest, or what there is no room for, is the bound (told in the
+          // first place); nothing is told after it
+          const bool over = (more >> D * W) != 0;
+          const bool bound = !over && (l == D || rank == tells - 1);
+          const bool none = over || bound;
+          const int n = l < D ? l : 0;
+          const uint32_t low = code >> 4 << 12;
+          // (by bits: a choice among members would put them in memory)
+          uint32_t high = none ? 0u : value;
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            const uint32_t at = __float_as_uint(h.q[n][c]);
+            high = lane == 1 + c ? at : high;
+          }
+          const uint32_t tag = (uint32_t)step & STEP;
+          uint64_t *const to = set + part * tells * 4 + lane;
+          if (rank < tells - 1)
+            __hip_atomic_store(to + (1 + rank) * 4,
+                               (uint64_t)high << 32 |
+                                   (lane == 0 ? (none ? 0u : low) | tag
+                                              : (uint32_t)step),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (bound)
+            __hip_atomic_store(to, (uint64_t)value << 32 | low | tag,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+    }
+    if (tid < slots * 4) {
+      const int slot = tid / 4, c = tid & 3;
+      const uint32_t mask = (slot & (tells - 1)) == 0 || c == 0 ? STEP : ~0u;
+      uint64_t word;
+      bool here;
+      int looks = 0;
+      do {
+        word = __hip_atomic_load(set + tid, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+        here = (((uint32_t)word ^ (uint32_t)step) & mask) == 0;
+      } while (!here && ++looks < patience);
+      if (!here)
+        t.late = 1;
+      if (c != 0)
+        t.at[slot][c - 1] = __uint_as_float((uint32_t)(word >> 32));
+      else if ((slot & (tells - 1)) == 0)
+        t.bound[slot / tells] = word & ~(uint64_t)STEP;
+      else
+        t.first[slot] = word & ~(uint64_t)STEP;
+    }
+    fps_meet();
+    if (t.late != 0)
+      return false;
+    // eight lanes count what comes before an entry; those before every bound have a
+    // rank
+    {
+      static_assert(kFpsThreads == 8 * kFpsTold, "eight lanes for an entry");
+      const int e = tid / 8, j = tid & 7;
+      const uint64_t mine = t.first[e];
+      if (__ballot(mine != 0u) != 0) {
+        uint32_t rank = 0u;
+        // (all at once takes registers that the rows need: eight scans 1,255 us)
+#pragma unroll 4
+        for (int i = 0; i < kFpsTold / 16; ++i) {
+          rank += t.first[i * 16 + j * 2] > mine;
+          rank += t.first[i * 16 + j * 2 + 1] > mine;
+        }
+        bool over = false;
+#pragma unroll
+        for (int i = 0; i < kFpsShareMost / 16; ++i) {
+          over |= t.bound[i * 16 + j * 2] > mine;
+          over |= t.bound[i * 16 + j * 2 + 1] > mine;
+        }
+        rank += over ? 256u : 0u;
+        rank = row8_sum(rank);
+        if (j == 0 && mine != 0u && rank < (uint32_t)S) {
+          t.place[rank] = make_float4(t.at[e][0], t.at[e][1], t.at[e][2],
+                                      __uint_as_float((uint32_t)(mine >> 32)));
+          t.what[rank] = make_uint2((uint32_t)mine >> 12 << 4, (uint32_t)step);
+        }
+      }
+    }
+    fps_meet();
+    // lane i % S: the entry of rank i
+    const int a = lane & (S - 1);
+    const float4 at = t.place[a];
+    const uint2 of = t.what[a];
+    const float sx[3] = {at.x, at.y, at.z};
+    {
+      // against those that may follow them, 64 / S of a wave
+      constexpr int OF = kWave / S;
+      const int b = wave * OF + lane / S;
+      const float4 at_b = t.place[b & (S - 1)];
+      const bool is = t.what[b & (S - 1)].y == (uint32_t)step;
+      const float xb[3] = {at_b.x, at_b.y, at_b.z};
+      float dd = 0.0f;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const float df = sx[c] - xb[c];
+        dd = c == 0 ? df * df : __builtin_fmaf(df, df, dd);
+      }
+      // (a distance that is NaN ends the run)
+      const uint64_t ends =
+          __ballot((a < b) & (b < S) & !(is & (dd >= at_b.w)));
+      if (ends != 0 && lane == 0)
+        atomicMin(&t.end[step & 1],
+                  wave * OF + (int)__builtin_ctzll(ends) / S);
+    }
+    uint64_t near[Held::CHUNKS];
+    h.find_near(sx, near);
+    fps_meet();
+    const int end = __builtin_amdgcn_readfirstlane(t.end[step & 1]);
+    const int got = min(end, steps - m);
+    if (wave == W - 1) {
+      if (part == 0 && lane < got)
+        out[m + lane] = start_idx + fps_row_of<BITS>(of.x);
+      if (lane == 0)
+        t.end[(step & 1) ^ 1] = S;
+    }
+    m += got;
+    changed = h.sample(sx, near, got);
+  }
+  return true;
+}
+
+// `most` workgroups for every example, in a row, so that they are spread over the
+// XCDs (all of an example on one XCD: the scans 1,355 us, spread 1,259).
+constexpr int kFpsShareGrid = 256; // all of a launch at most: a compute unit each
+template <int R, int S>
+__global__ __launch_bounds__(kFpsThreads) void fps_shared_kernel(
+    const float *__restrict__ src, const int64_t *__restrict__ ptr,
+    const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
+    int d, int most, FpsPieces p, FpsShare share,
+    int patience, int64_t *__restrict__ out) {
+  __shared__ __align__(16) FpsTold told;
+  const int b = blockIdx.x / most, part = blockIdx.x % most;
+  const int64_t start_idx = ptr[b];
+  const int64_t rows = ptr[b + 1] - start_idx;
+  const int64_t o_begin = out_ptr[b];
+  const int64_t o_end = out_ptr[b + 1];
+  if (o_begin >= o_end || rows <= 0)
+    return;
+  // (every wave has a row, and every row a wave)
+  const int64_t parts64 =
+      min((int64_t)most, rows / (kFpsWaves * kWave * kFpsShareRows));
+  const bool fits = parts64 >= 1 && rows <= parts64 * R * kFpsThreads;
+  if (!fits) {
+    if (part == 0 && threadIdx.x == 0)
+      share.failed[b] = 1u;
+    return;
+  }
+  const int parts = (int)parts64;
+  if (part >= parts)
+    return;
+  const int64_t first = start_idx + (start ? start[b] : 0);
+  if (part == 0 && threadIdx.x == 0)
+    out[o_begin] = first;
+  float at[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    at[c] = c < d ? src[(size_t)first * d + c] : 0.0f;
+  const int need = (int)((rows + parts * kFpsThreads - 1) / (parts * kFpsThreads));
+  auto run = [&](auto rows_of_lane) {
+    return fps_shared_rows<decltype(rows_of_lane)::value, S>(
+        p.rows + fps_first_piece(start_idx, b) * kWave, (int)rows, part, parts,
+        told, share.words + (size_t)b * (2 * kFpsShareWords), patience, at,
+        (int)(o_end - o_begin), start_idx, out + o_begin);
+  };
+  bool done;
+  if (R > 8 && need > 8)
+    done = run(std::integral_constant<int, R>{});
+  else if (need > 4)
+    done = run(std::integral_constant<int, 8>{});
+  else if (need > 2)
+    done = run(std::integral_constant<int, 4>{});
+  else
+    done = run(std::integral_constant<int, 2>{});
+  if (!done && threadIdx.x == 0)
+    __hip_atomic_store(share.failed + b, 1u, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// For calls that fps_shared_kernel does not take, and the examples that it marks
+// (`only`; NULL: all).
+//
 // A bucket has R pieces of 64 rows (MANY: a multiple of that) and belongs to a
 // lane of the workgroup: its box and its best row are in that lane's registers; the
 // rows and their running minima stay in memory, that is in the L2 of the
@@ -1460,7 +1858,8 @@ template <int W, int R, bool MANY, bool OWN>
 __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
     const float *__restrict__ src, const int64_t *__restrict__ ptr,
     const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
-    int d, FpsPieces p, int64_t *__restrict__ out) {
+    int d, FpsPieces p, const uint32_t *__restrict__ only,
+    int64_t *__restrict__ out) {
   constexpr int DIM = 3;
   static_assert(W * 4 == kWave, "a group per row of 16 lanes");
   static_assert(kFpsPieces % R == 0, "whole buckets");
@@ -1481,13 +1880,14 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
   const int count = (int)(ptr[b + 1] - start_idx);
   const int64_t o_begin = out_ptr[b];
   const int64_t o_end = out_ptr[b + 1];
-  if (o_begin >= o_end || count <= 0)
+  if (o_begin >= o_end || count <= 0 || (only != nullptr && only[b] == 0u))
     return;
   const int64_t first_piece = fps_first_piece(start_idx, b);
   const float4 *rows = p.rows + first_piece * kWave;
   // Examples whose rows fit the registers after all (a bound of 16,385: 8 x 16,384
-  // rows, 1,000 samples 727 -> 589 us, 8,300 666 -> 521).  Not in calls of larger
-  // ones: the registers make those 1 % slower.
+  // rows, 1,000 samples 727 -> 589 us, 8,300 666 -> 521; 200 x 9,000, 450 samples, with
+  // 16 rows of a lane 468, with 12 425).  Not in calls of larger ones: the registers
+  // make those 1 % slower.
   if (OWN && count >= kFpsOwnLeast && count <= 16 * kFpsThreads) {
     float at[DIM];
     const int64_t first = start_idx + (start ? start[b] : 0);
@@ -1507,8 +1907,10 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
           },
           count, ranks, at, (int)(o_end - o_begin), start_idx, out + o_begin);
     };
-    if (count > 8 * kFpsThreads)
+    if (count > 12 * kFpsThreads)
       run(std::integral_constant<int, 16>{});
+    else if (count > 8 * kFpsThreads)
+      run(std::integral_constant<int, 12>{});
     else
       run(std::integral_constant<int, 8>{});
     return;
@@ -1898,6 +2300,19 @@ static bool fps_streams(int dtype, int d, int64_t max_rows) {
 
 static size_t fps_align(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// Workgroups of an example, for calls of few enough examples (else 0).
+static int fps_share_most(int num_segments) {
+  const int most = std::min(kFpsShareMost, kFpsShareGrid / num_segments);
+  return most >= 4 ? most : 0;
+}
+static size_t fps_share_bytes(int num_segments) {
+  if (fps_share_most(num_segments) == 0)
+    return 0;
+  return fps_align(sizeof(uint64_t) * 2 * kFpsShareWords *
+                   (size_t)num_segments) +
+         fps_align(sizeof(uint32_t) * (size_t)num_segments);
+}
+
 size_t fps_scratch_bytes(int dtype, int n, int d, int num_segments,
                          int64_t max_rows) {
   if (fps_on_chip(dtype, d, max_rows))
@@ -1910,6 +2325,7 @@ size_t fps_scratch_bytes(int dtype, int n, int d, int num_segments,
   return std::max(dist, fps_align(sizeof(float4) * kWave * pieces) +
                             fps_align(sizeof(float) * kWave * pieces) +
                             fps_align(sizeof(float) * 8 * pieces) +
+                            fps_share_bytes(num_segments) +
                             curve_order_bytes(n, num_segments));
 }
 
@@ -1917,7 +2333,8 @@ namespace {
 hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
                              const int64_t *out_ptr, const int64_t *start,
                              int n, int d, int num_segments, int64_t max_rows,
-                             void *scratch, int64_t *out, hipStream_t stream) {
+                             void *scratch, int patience, int64_t *out,
+                             hipStream_t stream) {
   char *cursor = static_cast<char *>(scratch);
   auto take = [&cursor](size_t bytes) {
     char *piece = cursor;
@@ -1929,18 +2346,43 @@ hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
   p.rows = static_cast<float4 *>(take(sizeof(float4) * kWave * pieces));
   p.minima = static_cast<float *>(take(sizeof(float) * kWave * pieces));
   p.boxes = static_cast<float *>(take(sizeof(float) * 8 * pieces));
+  const int64_t rows = std::min(max_rows, (int64_t)n);
+  const int most = fps_share_most(num_segments);
+  FpsShare share = {nullptr, nullptr};
+  if (most > 0) {
+    void *words = take(sizeof(uint64_t) * 2 * kFpsShareWords *
+                       (size_t)num_segments);
+    void *failed = take(sizeof(uint32_t) * (size_t)num_segments);
+    int device = 0, units = 0;
+    if (rows <= (int64_t)most * 16 * kFpsThreads &&
+        hipGetDevice(&device) == hipSuccess &&
+        hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount,
+                              device) == hipSuccess &&
+        units >= kFpsShareGrid)
+      share = {static_cast<uint64_t *>(words), static_cast<uint32_t *>(failed)};
+  }
   const uint32_t *perm = nullptr;
   hipError_t err = launch_curve_order(src, ptr, n, d, num_segments, cursor,
                                       &perm, stream);
   if (err != hipSuccess)
     return err;
-  const int64_t rows = std::min(max_rows, (int64_t)n);
   for (int b0 = 0; b0 < num_segments; b0 += 65535) {
     const int some = std::min(65535, num_segments - b0);
     hipLaunchKernelGGL(fps_gather_kernel,
                        dim3((unsigned)((rows + kBlock - 1) / kBlock), some),
                        dim3(kBlock), 0, stream, src, ptr, d, b0, perm,
-                       p);
+                       p, share);
+  }
+  if (share.words != nullptr) {
+#define PCA_FPS_SHARED(R_, S_)                                                 \
+  hipLaunchKernelGGL((fps_shared_kernel<R_, S_>), dim3(num_segments *most),    \
+                     dim3(kFpsThreads), 0, stream, src, ptr, out_ptr, start,   \
+                     d, most, p, share, patience, out)
+    if (rows <= (int64_t)most * 8 * kFpsThreads)
+      PCA_FPS_SHARED(8, 32);
+    else
+      PCA_FPS_SHARED(16, 32);
+#undef PCA_FPS_SHARED
   }
   // (half as many rows to a bucket where the lanes suffice: 8 x 60,000 rows, 600
   // samples each, R = 1 / 2 910 / 840 us, 8 x 20,000 1,160 / 1,240; the scans, at
@@ -1948,7 +2390,7 @@ hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
 #define PCA_FPS_STREAM(S_, MANY_, OWN_)                                        \
   hipLaunchKernelGGL((fps_stream_kernel<kFpsWaves, S_, MANY_, OWN_>),          \
                      dim3(num_segments), dim3(kFpsThreads), 0, stream, src,    \
-                     ptr, out_ptr, start, d, p, out)
+                     ptr, out_ptr, start, d, p, share.failed, out)
   if (rows <= 16 * kFpsThreads + 1)
     PCA_FPS_STREAM(1, false, true);
   else if (rows <= kWave * kFpsThreads / 2)
@@ -1967,7 +2409,8 @@ hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
 hipError_t launch_fps(int dtype, const void *src, const int64_t *ptr,
                       const int64_t *out_ptr, const int64_t *start, int n,
                       int d, int num_segments, int64_t max_rows, void *scratch,
-                      bool captured, int64_t *out, hipStream_t stream) {
+                      bool captured, int64_t *out, hipStream_t stream,
+                      int patience) {
   if (fps_on_chip(dtype, d, max_rows)) {
     const float *s = static_cast<const float *>(src);
     if (d <= 2)
@@ -1981,8 +2424,8 @@ hipError_t launch_fps(int dtype, const void *src, const int64_t *ptr,
   }
   if (fps_streams(dtype, d, max_rows) && !captured)
     return launch_fps_stream(static_cast<const float *>(src), ptr, out_ptr,
-                             start, n, d, num_segments, max_rows, scratch, out,
-                             stream);
+                             start, n, d, num_segments, max_rows, scratch,
+                             patience, out, stream);
   switch (dtype) {
   case 0:
     return launch_fps_any<FpsF32>(src, ptr, out_ptr, start, d, num_segments,

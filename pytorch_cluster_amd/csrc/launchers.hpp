@@ -361,12 +361,16 @@ hipError_t launch_curve_order(const float *x, const int64_t *ptr, int n, int d,
 // unknown bound, max_rows = 0).
 size_t fps_scratch_bytes(int dtype, int n, int d, int num_segments,
                          int64_t max_rows);
-// One workgroup per example.  start: NULL = first row of every example.
+// An example by one or several workgroups.  start: NULL = first row of every example.
 // captured: the stream is being captured into a graph (no sort then).
+// patience: how often a workgroup looks for what another one of its example tells
+// before it gives up (a look takes about a microsecond; see fps_shared_kernel).
+constexpr int kFpsPatience = 2048;
 hipError_t launch_fps(int dtype, const void *src, const int64_t *ptr,
                       const int64_t *out_ptr, const int64_t *start, int n,
                       int d, int num_segments, int64_t max_rows, void *scratch,
-                      bool captured, int64_t *out, hipStream_t stream);
+                      bool captured, int64_t *out, hipStream_t stream,
+                      int patience = kFpsPatience);
 
 // --- radius_mc.hip ---------------------------------------------------------
 

@@ -989,18 +989,26 @@ at::Tensor fps_host(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
 }
 
 // The bound on the rows of an example that pca_fps is given: it selects the kernel,
-// by the longest example and the most samples of one.  Beyond 16,384 rows the rows are
-// sorted, 60 us and more, for steps of 2 - 12 us; with the bound 0 every row is looked
-// at in every step, 0.6 us per 1,000 rows.  All rows / sorted, us: 4 x 17,000 rows, 4
-// samples each 35 / 69, 8 79 / 89, 16 167 / 108; 2 x 60,000, 2 samples 38 / 75, 4 107 /
-// 97.  Between 8,192 and 16,384 rows of up to 3 dimensions examples of many samples
-// are better off sorted as well: every row on the chip / sorted, stretches in
-// registers, 16 x 8,300 rows, 200 samples 283 / 258, 320 435 / 310; 8 x 16,384, 200 283
-// / 285, 320 436 / 340; 64 x 12,000, 240 337 / 338, 320 440 / 368.
-int64_t fps_bound(int64_t longest, int64_t samples, int64_t d) {
+// by the longest example, the most samples of one and the number of examples.  Beyond
+// 16,384 rows the rows are sorted, 60 us and more, for steps of 3 - 12 us; with the
+// bound 0 every row is looked at in every step, 0.6 us per 1,000 rows.  All rows /
+// sorted, us: 4 x 17,000 rows, 4 samples each 38 / 66, 8 82 / 79, 10 104 / 85; 2 x
+// 60,000, 2 samples 41 / 62, 4 109 / 69.
+// Smaller examples of up to 3 dimensions are sorted as well, in memory, and shared by
+// several workgroups, where many samples repay the sort.  On the chip / sorted, 8 or 16
+// examples: 16,384 rows, 180 samples 236 / 252, 240 313 / 274; 8,192, 1,000 358 / 421,
+// 2,000 583 / 557, 4,000 1,001 / 809; 5,000, 2,000 530 / 523; 64 examples: 12,000 rows,
+// 180 237 / 317, 240 312 / 339; 8,192, 2,000 584 / 624, 4,000 1,004 / 894.
+int64_t fps_bound(int64_t longest, int64_t samples, int64_t d,
+                  int64_t examples) {
   if (longest > 16384)
     return (samples - 1) * longest <= 130000 ? 0 : longest;
-  return longest > 8192 && samples >= 240 && d <= 3 ? 16385 : longest;
+  const int64_t enough = longest > 8192    ? (examples <= 16 ? 210 : 270)
+                         : longest <= 4096 ? INT64_MAX
+                         : examples <= 16  ? 2100
+                         : examples <= 64  ? 2800
+                                           : INT64_MAX;
+  return samples >= enough && d <= 3 ? 16385 : longest;
 }
 
 at::Tensor fps(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
@@ -1041,7 +1049,8 @@ at::Tensor fps(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
     return out;
   const int64_t d = src.size(1);
   const int64_t max_rows =
-      fps_bound(sizes[2].item<int64_t>(), sizes[1].item<int64_t>(), d);
+      fps_bound(sizes[2].item<int64_t>(), sizes[1].item<int64_t>(), d,
+                batch_size);
   const int dtype = dtype_code(src);
   TORCH_CHECK(dtype != PCA_BF16, "fps is not implemented for 'BFloat16'");
   const size_t ws_bytes =
@@ -1131,7 +1140,7 @@ at::Tensor fps_batched(at::Tensor src, std::optional<at::Tensor> batch,
   if (samples == 0)
     return out;
   const int64_t most = (int64_t)std::ceil((float)longest * (float)ratio);
-  longest = fps_bound(longest, most, d);
+  longest = fps_bound(longest, most, d, examples);
   const size_t ws_bytes =
       pca_fps_workspace_bytes(n, d, examples, longest, PCA_F32);
   TORCH_CHECK(ws_bytes > 0, "problem size not supported");

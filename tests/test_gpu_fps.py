@@ -164,6 +164,86 @@ def test_stretches_of_every_length(oracle, sizes, d, kind):
     assert (got == oracle.fps_op(x, ptr, share, start)).all()
 
 
+# An example by several workgroups, one for 1,024 rows up to 32 of them, up to 256 of
+# all examples; 2, 4, 8, 16 rows of a lane; 4, 8, 16 entries told (17, 9, fewer
+# workgroups).  Examples of fewer than 1,024 rows, and those beyond 16,384 rows of a
+# workgroup, are one workgroup's.
+SHARED = [([16384, 1023, 1024, 2047, 2048, 40], 3),
+          ([9215, 9216, 16385, 17407, 17408], 2), ([65536, 65537, 33000], 3),
+          ([131073, 1100], 1), ([262144, 262145], 3), ([524288], 3),
+          ([524289], 3), ([40] * 63 + [32769], 3), ([1500] * 63 + [65537], 3),
+          ([1025] * 24 + [16500], 2)]
+
+
+@pytest.mark.parametrize("kind", ["uniform", "grid", "odd"])
+@pytest.mark.parametrize("sizes,d", SHARED)
+def test_examples_of_several_workgroups(oracle, sizes, d, kind):
+    rng = np.random.default_rng(sum(sizes) + d)
+    ptr = np.cumsum([0] + sizes).astype(np.int64)
+    n = ptr[-1]
+    x = rng.integers(0, 17, (n, d)) if kind == "grid" else rng.random((n, d))
+    x = x.astype(np.float32)
+    if kind == "odd":
+        x[rng.random(n) < 0.1] *= 400.0  # minima clipped at first
+        x[rng.random(n) < 0.01, 0] = np.nan
+        x[rng.random(n) < 0.001] = np.inf
+    samples = 120 if n > 300000 else 500
+    share = np.array([min(samples, 2 * s) / s for s in sizes])
+    start = np.array([s // 2 for s in sizes], dtype=np.int64)
+    got = gpu_fps(oracle, x, ptr, share, start, max(max(sizes), 16385))
+    assert (got == oracle.fps_op(x, ptr, share, start)).all()
+
+
+# 4,096 rows, 2,100 and 2,800 samples, 16 and 64 examples: where rows that fit one
+# workgroup are shared all the same
+@pytest.mark.parametrize("rows,examples,samples", [
+    (4096, 2, 2110), (4097, 2, 2110), (8192, 2, 2090), (5000, 17, 2790),
+    (5000, 17, 2810), (9000, 16, 220), (9000, 17, 220)])
+def test_entry_points_where_examples_are_shared(oracle, rows, examples, samples):
+    rng = np.random.default_rng(rows + samples)
+    sizes = [rows] + [300] * (examples - 2) + [rows // 3]
+    ptr = np.cumsum([0] + sizes).astype(np.int64)
+    x = rng.random((ptr[-1], 3)).astype(np.float32)
+    batch = np.repeat(np.arange(examples), sizes)
+    ratio = samples / rows
+    want = oracle.fps_op(x, ptr, np.float32(ratio))
+    got = pca.fps(dev(x), dev(batch, torch.long), ratio, random_start=False)
+    assert (got.cpu().numpy() == want).all()
+    got = torch.ops.torch_cluster.fps(
+        dev(x), dev(ptr, torch.long),
+        torch.tensor(ratio, dtype=torch.float32, device=DEV), False)
+    assert (got.cpu().numpy() == want).all()
+
+
+@pytest.mark.parametrize("patience", [0, 1, 3])
+def test_workgroups_that_do_not_wait(oracle, patience):
+    """A workgroup that does not hear from the others in time marks its example
+    and ends; another kernel samples that one from the start."""
+    import ctypes
+    import os
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(pca.__file__),
+                                   "libpca_probe.so"))
+    rng = np.random.default_rng(5)
+    ptr = np.array([0, 20000, 21500, 61500], dtype=np.int64)
+    x = rng.random((ptr[-1], 3)).astype(np.float32)
+    ratio = 0.02
+    out_ptr = oracle.fps_out_ptr(ptr, ratio, np.float32)
+    bytes_ = capi.capi.pca_fps_workspace_bytes(len(x), 3, 3, 40000, 0)
+    held = [dev(x), dev(ptr, torch.long), dev(out_ptr, torch.long),
+            torch.full((int(out_ptr[-1]),), -1, dtype=torch.long, device=DEV),
+            torch.empty(bytes_, dtype=torch.uint8, device=DEV)]
+    src, ptr_, out_ptr_, out, work = [ctypes.c_void_p(t.data_ptr())
+                                      for t in held]
+    torch.cuda.synchronize()
+    assert lib.pca_probe_fps(src, ptr_, out_ptr_, ctypes.c_int64(len(x)),
+                             ctypes.c_int64(3), ctypes.c_int64(3),
+                             ctypes.c_int64(40000), ctypes.c_int(patience),
+                             out, work, ctypes.c_size_t(bytes_)) == 0
+    torch.cuda.synchronize()
+    want = oracle.fps_op(x, ptr, np.float32(ratio))
+    assert (held[3].cpu().numpy() == want).all()
+
+
 # 8,192 / 16,384 rows, 340 samples: where the entry points change between the
 # kernels on the chip and rows in curve order
 @pytest.mark.parametrize("rows,samples", [(8192, 400), (8193, 330), (8193, 345),
