@@ -994,19 +994,22 @@ at::Tensor fps_host(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
 // bound 0 every row is looked at in every step, 0.6 us per 1,000 rows.  All rows /
 // sorted, us: 4 x 17,000 rows, 4 samples each 38 / 66, 8 82 / 79, 10 104 / 85; 2 x
 // 60,000, 2 samples 41 / 62, 4 109 / 69.
-// Smaller examples of up to 3 dimensions are sorted as well, in memory, and shared by
-// several workgroups, where many samples repay the sort.  On the chip / sorted, 8 or 16
-// examples: 16,384 rows, 180 samples 236 / 252, 240 313 / 274; 8,192, 1,000 358 / 421,
-// 2,000 583 / 557, 4,000 1,001 / 809; 5,000, 2,000 530 / 523; 64 examples: 12,000 rows,
-// 180 237 / 317, 240 312 / 339; 8,192, 2,000 584 / 624, 4,000 1,004 / 894.
+// Smaller examples of up to 3 dimensions go through memory as well, in curve order,
+// and are shared by several workgroups, where many samples repay it.  One workgroup
+// each / shared: 8 x 16,384 rows, 180 samples 238 / 248, 240 314 / 269; 16 x 8,300,
+// 180 238 / 235; 64 x 12,000, 180 240 / 286, 240 313 / 312; 100 x 12,000 (too many to
+// be shared), 140 190 / 206, 240 316 / 248; 16 x 8,192, 1,000 359 / 400, 1,500 474 /
+// 470, 2,000 584 / 541, 4,000 1,013 / 795; 8 x 5,000, 1,000 323 / 349, 2,000 532 /
+// 499; 64 x 8,192, 1,000 360 / 430, 2,000 586 / 589, 4,000 1,010 / 869; 100 x 8,192,
+// 4,000 1,014 / 1,044.
 int64_t fps_bound(int64_t longest, int64_t samples, int64_t d,
                   int64_t examples) {
   if (longest > 16384)
     return (samples - 1) * longest <= 130000 ? 0 : longest;
-  const int64_t enough = longest > 8192    ? (examples <= 16 ? 210 : 270)
+  const int64_t enough = longest > 8192    ? (examples <= 16 ? 190 : 240)
                          : longest <= 4096 ? INT64_MAX
-                         : examples <= 16  ? 2100
-                         : examples <= 64  ? 2800
+                         : examples <= 16  ? 1600
+                         : examples <= 64  ? 2300
                                            : INT64_MAX;
   return samples >= enough && d <= 3 ? 16385 : longest;
 }

@@ -194,11 +194,12 @@ def test_examples_of_several_workgroups(oracle, sizes, d, kind):
     assert (got == oracle.fps_op(x, ptr, share, start)).all()
 
 
-# 4,096 rows, 2,100 and 2,800 samples, 16 and 64 examples: where rows that fit one
-# workgroup are shared all the same
+# 4,096 rows, 1,600 and 2,300 samples, 16 and 64 examples: where rows that fit one
+# workgroup are shared all the same; 16,384 / 16,385: rows that are ordered in LDS
 @pytest.mark.parametrize("rows,examples,samples", [
-    (4096, 2, 2110), (4097, 2, 2110), (8192, 2, 2090), (5000, 17, 2790),
-    (5000, 17, 2810), (9000, 16, 220), (9000, 17, 220)])
+    (4096, 2, 1610), (4097, 2, 1610), (8192, 2, 1590), (5000, 17, 2290),
+    (5000, 17, 2310), (9000, 16, 200), (9000, 17, 200), (8193, 65, 300),
+    (12288, 3, 250), (12289, 3, 250), (16384, 3, 250), (16385, 3, 250)])
 def test_entry_points_where_examples_are_shared(oracle, rows, examples, samples):
     rng = np.random.default_rng(rows + samples)
     sizes = [rows] + [300] * (examples - 2) + [rows // 3]
@@ -242,6 +243,25 @@ def test_workgroups_that_do_not_wait(oracle, patience):
     torch.cuda.synchronize()
     want = oracle.fps_op(x, ptr, np.float32(ratio))
     assert (held[3].cpu().numpy() == want).all()
+
+
+def test_shared_examples_on_several_streams():
+    """Calls that each ask for every compute unit, side by side: the workgroups
+    of one wait for units that the other holds."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    ids = torch.arange(8, device=DEV).repeat_interleave(40000)
+    xs = [torch.rand(320000, 3, generator=g, device=DEV) for _ in range(3)]
+    want = [pca.fps(x, ids, 0.01, random_start=False) for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in xs]
+    got = []
+    for _ in range(3):
+        for x, stream in zip(xs, streams):
+            with torch.cuda.stream(stream):
+                got.append(pca.fps(x, ids, 0.01, random_start=False))
+    torch.cuda.synchronize()
+    for i, rows in enumerate(got):
+        assert torch.equal(rows, want[i % 3])
 
 
 # 8,192 / 16,384 rows, 340 samples: where the entry points change between the
