@@ -420,15 +420,17 @@ class Cases:
             ms, out = _median_ms(
                 t, lambda: t.ops.torch_cluster.fps(pts, ptr, ratio, False),
                 reps or 5)
-            # A step depends on the one before it, and a cloud is one
-            # workgroup's, so the floor is latency, not bandwidth or rows
-            # (most rows are left alone in a step): about 100 vector
-            # instructions that wait for each other, 4 cycles each, and
-            # three trips to the LDS of 64 cycles, at 2.4 GHz.  A step finds
-            # at most sixteen samples (about nine in these clouds), so no
-            # sample takes less than a sixteenth of that.
+            # A step depends on the one before it, so the floor is latency,
+            # not bandwidth or rows (most rows are left alone in a step):
+            # about 100 vector instructions that wait for each other, 4
+            # cycles each, and three trips to the LDS of 64 cycles, at 2.4
+            # GHz.  A step finds at most sixteen samples (about nine in
+            # these clouds), thirty-two where several workgroups share a
+            # cloud, so no sample takes less than that part of it.
+            most = 16 if points <= 8192 else 32
+            units = clouds * (1 if points <= 8192 else min(32, points // 1024))
             sample_us = ms * 1e3 / (points // 4)
-            floor_us = (100 * 4 + 3 * 64) / 2400.0 / 16
+            floor_us = (100 * 4 + 3 * 64) / 2400.0 / most
             report["fps %dx%d ratio 0.25" % (clouds, points)] = {
                 "ms": ms, "samples": int(out.numel()),
                 "us_per_sample": sample_us,
@@ -438,9 +440,9 @@ class Cases:
                     "frac": floor_us / sample_us,
                     "note": "dependent instructions and LDS trips of a step "
                             "that looks at one piece of rows and finds the "
-                            "most samples it can, sixteen; "
+                            "most samples it can, %d; "
                             "clouds run side by side, %d of the chip's "
-                            "256 units busy" % clouds}}
+                            "256 units busy" % (most, units)}}
         return report
 
     # "auto" against the clock: whole calls of knn / radius / nearest on
