@@ -1581,18 +1581,18 @@ __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
 // All workgroups of an example have to run at the same time.  The launch asks for no
 // more than the device has compute units, but work on other streams may hold some.
 // (Workgroups start in order, example by example: of two such calls side by side the
-// first examples run and make room.)  Every wait ends after `patience` looks (about a
-// millisecond); the workgroup then marks the example and ends, and so do the others,
+// first examples run and make room.)  Every wait ends after `patience` looks (1.3 ms);
+// the workgroup then marks the example and ends, and so do the others,
 // which hear nothing more from it.
 // fps_stream_kernel, launched behind, samples the marked examples from the start.
 //
-// Bound by the chain of a step, about 12,000 cycles for 16 samples of a scan of
+// Bound by the chain of a step, about 10,000 cycles for 16 samples of a scan of
 // 200,000 rows by 32 workgroups: rows and entries 2,900 (of the slowest wave), what
-// is told 5,200 (3,000 of 8 workgroups), ranks 1,300, pairs and boxes 900, four
+// is told 4,000 (2,500 of 8 workgroups), ranks 1,300, pairs and boxes 900, four
 // meetings.  Calls, us, one workgroup each -> shared: eight scans of 60,000 - 200,000
-// rows, 2 % sampled, 2,795 -> 1,121; one of them 1,198 -> 522; uniform rows, 8 x
-// 16,384, 1,000 samples 601 -> 485; 16 x 16,384, a quarter 1,588 -> 886; 64 x 20,000,
-// a tenth 1,783 -> 1,079; 1 x 500,000, 5,000 samples 9,952 -> 2,535; 128 x 20,000, two
+// rows, 2 % sampled, 2,795 -> 1,028; one of them 1,198 -> 477; uniform rows, 8 x
+// 16,384, 1,000 samples 601 -> 425; 16 x 16,384, a quarter 1,588 -> 770; 64 x 20,000,
+// a tenth 1,783 -> 1,034; 1 x 500,000, 5,000 samples 9,952 -> 2,407; 128 x 20,000, two
 // workgroups each, 1,276 -> 1,350: not below four.  What else was tried, eight scans /
 // one scan: the words of an entry in four lines that all workgroups write to 2,073 /
 // 1,063 (before ranks and layout as they are 1,558 / 763); ranks by a wave of each
@@ -1600,6 +1600,7 @@ __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
 // 633; a pause between two looks no change; a workgroup for 2,048 rows at least 1 x
 // 16,000, 1,600 samples 581, for 4,096 706, for 1,024 526.
 struct FpsTold {
+  uint64_t tell[64];           // what this workgroup tells
   uint64_t key[3 * kFpsWaves]; // of this workgroup: entries, then rests
   // of all: value and code (0: none); coordinates; the bounds
   uint64_t first[kFpsTold];
@@ -1695,19 +1696,22 @@ fps_shared_rows(const float4 *__restrict__ rows, int count, int part, int parts,
             high = lane == 1 + c ? at : high;
           }
           const uint32_t tag = (uint32_t)step & STEP;
-          uint64_t *const to = set + part * tells * 4 + lane;
+          uint64_t *const to = t.tell + lane;
           if (rank < tells - 1)
-            __hip_atomic_store(to + (1 + rank) * 4,
-                               (uint64_t)high << 32 |
-                                   (lane == 0 ? (none ? 0u : low) | tag
-                                              : (uint32_t)step),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            to[(1 + rank) * 4] = (uint64_t)high << 32 |
+                                 (lane == 0 ? (none ? 0u : low) | tag
+                                            : (uint32_t)step);
           if (bound)
-            __hip_atomic_store(to, (uint64_t)value << 32 | low | tag,
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            to[0] = (uint64_t)value << 32 | low | tag;
         }
       }
     }
+    fps_meet();
+    // (whole lines: written entry by entry, by their waves, the scans took 1,119 us
+    // instead of 1,028, 16 x 16,384 rows 865 instead of 770)
+    if (tid < tells * 4)
+      __hip_atomic_store(set + part * tells * 4 + tid, t.tell[tid],
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (tid < slots * 4) {
       const int slot = tid / 4, c = tid & 3;
       const uint32_t mask = (slot & (tells - 1)) == 0 || c == 0 ? STEP : ~0u;

@@ -364,8 +364,9 @@ size_t fps_scratch_bytes(int dtype, int n, int d, int num_segments,
 // An example by one or several workgroups.  start: NULL = first row of every example.
 // captured: the stream is being captured into a graph (no sort then).
 // patience: how often a workgroup looks for what another one of its example tells
-// before it gives up (a look takes about a microsecond; see fps_shared_kernel).
-constexpr int kFpsPatience = 2048;
+// before it gives up (a look takes 0.16 us: 1.3 ms, about a call of eight scans, which
+// may be what the others wait for; see fps_shared_kernel).
+constexpr int kFpsPatience = 8192;
 hipError_t launch_fps(int dtype, const void *src, const int64_t *ptr,
                       const int64_t *out_ptr, const int64_t *start, int n,
                       int d, int num_segments, int64_t max_rows, void *scratch,

@@ -996,20 +996,19 @@ at::Tensor fps_host(at::Tensor src, at::Tensor ptr, at::Tensor ratio,
 // 60,000, 2 samples 41 / 62, 4 109 / 69.
 // Smaller examples of up to 3 dimensions go through memory as well, in curve order,
 // and are shared by several workgroups, where many samples repay it.  One workgroup
-// each / shared: 8 x 16,384 rows, 180 samples 238 / 248, 240 314 / 269; 16 x 8,300,
-// 180 238 / 235; 64 x 12,000, 180 240 / 286, 240 313 / 312; 100 x 12,000 (too many to
-// be shared), 140 190 / 206, 240 316 / 248; 16 x 8,192, 1,000 359 / 400, 1,500 474 /
-// 470, 2,000 584 / 541, 4,000 1,013 / 795; 8 x 5,000, 1,000 323 / 349, 2,000 532 /
-// 499; 64 x 8,192, 1,000 360 / 430, 2,000 586 / 589, 4,000 1,010 / 869; 100 x 8,192,
-// 4,000 1,014 / 1,044.
+// each / shared: 8 x 16,384 rows, 140 samples 186 / 207, 180 237 / 224; 16 x 8,300,
+// 140 186 / 201, 180 237 / 221; 64 x 12,000, 180 238 / 266, 240 313 / 296; 100 x 12,000
+// (too many to be shared), 140 192 / 206, 240 317 / 248; 16 x 8,192, 1,000 358 / 368,
+// 1,500 475 / 430, 4,000 1,002 / 706; 8 x 5,000, 1,000 321 / 321, 2,000 529 / 463; 64 x
+// 8,192, 1,000 360 / 393, 2,000 586 / 535; 100 x 8,192, 4,000 1,011 / 1,043.
 int64_t fps_bound(int64_t longest, int64_t samples, int64_t d,
                   int64_t examples) {
   if (longest > 16384)
     return (samples - 1) * longest <= 130000 ? 0 : longest;
-  const int64_t enough = longest > 8192    ? (examples <= 16 ? 190 : 240)
+  const int64_t enough = longest > 8192    ? (examples <= 16 ? 170 : 220)
                          : longest <= 4096 ? INT64_MAX
-                         : examples <= 16  ? 1600
-                         : examples <= 64  ? 2300
+                         : examples <= 16  ? 1100
+                         : examples <= 64  ? 1600
                                            : INT64_MAX;
   return samples >= enough && d <= 3 ? 16385 : longest;
 }

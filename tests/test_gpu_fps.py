@@ -194,11 +194,11 @@ def test_examples_of_several_workgroups(oracle, sizes, d, kind):
     assert (got == oracle.fps_op(x, ptr, share, start)).all()
 
 
-# 4,096 rows, 1,600 and 2,300 samples, 16 and 64 examples: where rows that fit one
+# 4,096 rows, 1,100 and 1,600 samples, 16 and 64 examples: where rows that fit one
 # workgroup are shared all the same; 16,384 / 16,385: rows that are ordered in LDS
 @pytest.mark.parametrize("rows,examples,samples", [
-    (4096, 2, 1610), (4097, 2, 1610), (8192, 2, 1590), (5000, 17, 2290),
-    (5000, 17, 2310), (9000, 16, 200), (9000, 17, 200), (8193, 65, 300),
+    (4096, 2, 1110), (4097, 2, 1110), (8192, 2, 1090), (5000, 17, 1590),
+    (5000, 17, 1610), (9000, 16, 200), (9000, 17, 200), (8193, 65, 300),
     (12288, 3, 250), (12289, 3, 250), (16384, 3, 250), (16385, 3, 250)])
 def test_entry_points_where_examples_are_shared(oracle, rows, examples, samples):
     rng = np.random.default_rng(rows + samples)
