@@ -1590,9 +1590,9 @@ __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
 // 200,000 rows by 32 workgroups: rows and entries 2,900 (of the slowest wave), what
 // is told 4,000 (2,500 of 8 workgroups), ranks 1,300, pairs and boxes 900, four
 // meetings.  Calls, us, one workgroup each -> shared: eight scans of 60,000 - 200,000
-// rows, 2 % sampled, 2,795 -> 1,028; one of them 1,198 -> 477; uniform rows, 8 x
-// 16,384, 1,000 samples 601 -> 425; 16 x 16,384, a quarter 1,588 -> 770; 64 x 20,000,
-// a tenth 1,783 -> 1,034; 1 x 500,000, 5,000 samples 9,952 -> 2,407; 128 x 20,000, two
+// rows, 2 % sampled, 2,795 -> 1,001; one of them 1,198 -> 475; uniform rows, 8 x
+// 16,384, 1,000 samples 601 -> 409; 16 x 16,384, a quarter 1,588 -> 741; 64 x 20,000,
+// a tenth 1,783 -> 999; 1 x 500,000, 5,000 samples 9,952 -> 2,407; 128 x 20,000, two
 // workgroups each, 1,276 -> 1,350: not below four.  What else was tried, eight scans /
 // one scan: the words of an entry in four lines that all workgroups write to 2,073 /
 // 1,063 (before ranks and layout as they are 1,558 / 763); ranks by a wave of each
@@ -1807,8 +1807,9 @@ fps_shared_rows(const float4 *__restrict__ rows, int count, int part, int parts,
   return true;
 }
 
-// `most` workgroups for every example, in a row, so that they are spread over the
-// XCDs (all of an example on one XCD: the scans 1,355 us, spread 1,259).
+// `most` workgroups for every example, those of an example on one XCD where every XCD
+// gets as many examples (16 x 16,384 rows, a quarter 742 us, spread over the XCDs 784;
+// 64 x 20,000, a tenth 992, 1,056; eight scans 994, 1,032), else in a row.
 constexpr int kFpsShareGrid = 256; // all of a launch at most: a compute unit each
 template <int R, int S>
 __global__ __launch_bounds__(kFpsThreads) void fps_shared_kernel(
@@ -1817,7 +1818,13 @@ __global__ __launch_bounds__(kFpsThreads) void fps_shared_kernel(
     int d, int most, FpsPieces p, FpsShare share,
     int patience, int64_t *__restrict__ out) {
   __shared__ __align__(16) FpsTold told;
-  const int b = blockIdx.x / most, part = blockIdx.x % most;
+  int b = blockIdx.x / most, part = blockIdx.x % most;
+  if (gridDim.x / most % 8 == 0) {
+    // (workgroup i is on XCD i % 8)
+    const int at_xcd = blockIdx.x / 8;
+    b = (int)(blockIdx.x % 8) + 8 * (at_xcd / most);
+    part = at_xcd % most;
+  }
   const int64_t start_idx = ptr[b];
   const int64_t rows = ptr[b + 1] - start_idx;
   const int64_t o_begin = out_ptr[b];
