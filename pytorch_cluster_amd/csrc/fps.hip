@@ -1503,15 +1503,19 @@ struct FpsPieces {
 constexpr int kFpsPieces = 4;
 static_assert(kFpsPieces == kBlock / kWave, "a block of the kernel below");
 // What the workgroups of an example tell each other (see fps_shared_kernel): by
-// turns two sets of kFpsShareWords, and whether one of them gave up.
+// turns two sets of kFpsShareWords, and who they are (fps_crew).
 constexpr int kFpsShareMost = 32; // workgroups of an example at most
 constexpr int kFpsShareRows = 1;  // rows of a lane that a workgroup is worth
 constexpr int kFpsTold = 128;     // entries that they tell each other, of all
 constexpr int kFpsShareWords = kFpsTold * 4;
 struct FpsShare {
-  uint64_t *words;  // [examples][2][kFpsShareWords]; NULL: not shared
-  uint32_t *failed; // [examples]
+  uint64_t *words; // [examples][2][kFpsShareWords]; NULL: not shared
+  uint32_t *state; // [examples]
 };
+// A state: the workgroups that came, from bit 16 on the number of them that go to work
+// where it was closed before all were there, and whether the example is left to
+// fps_stream_kernel.
+constexpr uint32_t kFpsClosed = 1u << 31, kFpsMarked = 1u << 30;
 __host__ __device__ constexpr int64_t fps_first_piece(int64_t begin, int b) {
   return begin / kWave + (int64_t)kFpsPieces * b;
 }
@@ -1525,7 +1529,7 @@ __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
     for (int i = threadIdx.x; i < 2 * kFpsShareWords; i += kBlock)
       share.words[(size_t)b * (2 * kFpsShareWords) + i] = 0u;
     if (threadIdx.x == 0)
-      share.failed[b] = 0u;
+      share.state[b] = 0u;
   }
   const int64_t begin = ptr[b], end = ptr[b + 1];
   if (begin + (int64_t)blockIdx.x * kBlock >= end)
@@ -1579,12 +1583,12 @@ __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
 // steps later, when all have told the step between, that is, have read the set.
 //
 // All workgroups of an example have to run at the same time.  The launch asks for no
-// more than the device has compute units, but work on other streams may hold some.
-// (Workgroups start in order, example by example: of two such calls side by side the
-// first examples run and make room.)  Every wait ends after `patience` looks (1.3 ms);
-// the workgroup then marks the example and ends, and so do the others,
-// which hear nothing more from it.
-// fps_stream_kernel, launched behind, samples the marked examples from the start.
+// more than the device has compute units, but each of them takes a whole one, and
+// work on other streams may hold some.  So the workgroups of an example meet first
+// (fps_crew), and those that came in time deal the pieces among themselves; one that
+// comes later ends at once.  Where too few came to hold the rows, or one waits in vain
+// for what another tells (`patience` looks, 1.3 ms, while both run), the example is
+// marked, and fps_stream_kernel, launched behind, samples it from the start.
 //
 // Bound by the chain of a step, about 10,000 cycles for 16 samples of a scan of
 // 200,000 rows by 32 workgroups: rows and entries 2,900 (of the slowest wave), what
@@ -1807,6 +1811,45 @@ fps_shared_rows(const float4 *__restrict__ rows, int count, int part, int parts,
   return true;
 }
 
+// The workgroups of an example agree on who they are; one thread of each calls this.
+// Returns which one it is, of how many (y); -1: it is not needed.  `most`: at most so
+// many, `least`: as many as hold the rows.  They wait for each other, `patience` looks
+// of 0.12 us (30 us), and 16 times as long (0.5 ms) for the least, which a call of many
+// examples has once its first ones are done.  So units that are held by other work cost
+// a call that wait and their part of the speed, not the sharing.  One word decides, so
+// all see the same.
+// Calls, us, alone / beside a wave that sleeps on another stream, without this meeting
+// (a held unit cost its example 1.3 ms and the sharing) / now, and beside three: eight
+// scans 1,015 / 3,670 / 996, 1,025; 16 x 16,384 rows, a quarter 740 / 1,450 / 749, 787;
+// 64 x 20,000, a tenth 798 / 1,380 / 814, 1,385.
+__device__ __forceinline__ int2 fps_crew(uint32_t *state, int most, int least,
+                                         int patience) {
+  constexpr uint32_t CAME = 0xffffu;
+  const uint32_t before = __hip_atomic_fetch_add(
+      state, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int part = (int)(before & CAME);
+  if ((before & kFpsClosed) != 0 || part >= most)
+    return make_int2(-1, 0);
+  for (int looks = 0;; ++looks) {
+    uint32_t now = __hip_atomic_load(state, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+    const int here = (int)(now & CAME);
+    if ((now & kFpsClosed) != 0) {
+      const int parts = (int)(now >> 16 & 0xffu);
+      return make_int2(parts >= least ? part : -1, parts);
+    }
+    if (here >= most)
+      return make_int2(part, most);
+    // (tried again only if one more came, at most `most` times)
+    if (looks >= (here >= least ? patience : 16 * patience))
+      __hip_atomic_compare_exchange_strong(
+          state, &now,
+          now | kFpsClosed | (here < least ? kFpsMarked : 0u) |
+              (uint32_t)here << 16,
+          __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
 // `most` workgroups for every example, those of an example on one XCD where every XCD
 // gets as many examples (16 x 16,384 rows, a quarter 742 us, spread over the XCDs 784;
 // 64 x 20,000, a tenth 992, 1,056; eight scans 994, 1,032), else in a row.
@@ -1815,16 +1858,14 @@ template <int R, int S>
 __global__ __launch_bounds__(kFpsThreads) void fps_shared_kernel(
     const float *__restrict__ src, const int64_t *__restrict__ ptr,
     const int64_t *__restrict__ out_ptr, const int64_t *__restrict__ start,
-    int d, int most, FpsPieces p, FpsShare share,
-    int patience, int64_t *__restrict__ out) {
+    int d, int most, FpsPieces p, FpsShare share, int patience, int meeting,
+    int64_t *__restrict__ out) {
   __shared__ __align__(16) FpsTold told;
-  int b = blockIdx.x / most, part = blockIdx.x % most;
-  if (gridDim.x / most % 8 == 0) {
+  __shared__ int2 s_crew;
+  int b = blockIdx.x / most;
+  if (gridDim.x / most % 8 == 0)
     // (workgroup i is on XCD i % 8)
-    const int at_xcd = blockIdx.x / 8;
-    b = (int)(blockIdx.x % 8) + 8 * (at_xcd / most);
-    part = at_xcd % most;
-  }
+    b = (int)(blockIdx.x % 8) + 8 * ((int)(blockIdx.x / 8) / most);
   const int64_t start_idx = ptr[b];
   const int64_t rows = ptr[b + 1] - start_idx;
   const int64_t o_begin = out_ptr[b];
@@ -1834,14 +1875,20 @@ __global__ __launch_bounds__(kFpsThreads) void fps_shared_kernel(
   // (every wave has a row, and every row a wave)
   const int64_t parts64 =
       min((int64_t)most, rows / (kFpsWaves * kWave * kFpsShareRows));
-  const bool fits = parts64 >= 1 && rows <= parts64 * R * kFpsThreads;
-  if (!fits) {
-    if (part == 0 && threadIdx.x == 0)
-      share.failed[b] = 1u;
+  if (parts64 < 1 || rows > parts64 * R * kFpsThreads) {
+    if (threadIdx.x == 0)
+      __hip_atomic_store(share.state + b, kFpsMarked, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
     return;
   }
-  const int parts = (int)parts64;
-  if (part >= parts)
+  if (threadIdx.x == 0)
+    s_crew = fps_crew(share.state + b, (int)parts64,
+                      (int)((rows + R * kFpsThreads - 1) / (R * kFpsThreads)),
+                      meeting);
+  __syncthreads();
+  const int part = __builtin_amdgcn_readfirstlane(s_crew.x);
+  const int parts = __builtin_amdgcn_readfirstlane(s_crew.y);
+  if (part < 0)
     return;
   const int64_t first = start_idx + (start ? start[b] : 0);
   if (part == 0 && threadIdx.x == 0)
@@ -1867,8 +1914,8 @@ __global__ __launch_bounds__(kFpsThreads) void fps_shared_kernel(
   else
     done = run(std::integral_constant<int, 2>{});
   if (!done && threadIdx.x == 0)
-    __hip_atomic_store(share.failed + b, 1u, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_fetch_or(share.state + b, kFpsMarked, __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // For calls that fps_shared_kernel does not take, and the examples that it marks
@@ -1924,7 +1971,8 @@ __global__ __launch_bounds__(W *kWave) void fps_stream_kernel(
   const int count = (int)(ptr[b + 1] - start_idx);
   const int64_t o_begin = out_ptr[b];
   const int64_t o_end = out_ptr[b + 1];
-  if (o_begin >= o_end || count <= 0 || (only != nullptr && only[b] == 0u))
+  if (o_begin >= o_end || count <= 0 ||
+      (only != nullptr && (only[b] & kFpsMarked) == 0u))
     return;
   const int64_t first_piece = fps_first_piece(start_idx, b);
   const float4 *rows = p.rows + first_piece * kWave;
@@ -2357,6 +2405,17 @@ static size_t fps_share_bytes(int num_segments) {
          fps_align(sizeof(uint32_t) * (size_t)num_segments);
 }
 
+static size_t fps_pieces_bytes(size_t pieces) {
+  return fps_align(sizeof(float4) * kWave * pieces) +
+         fps_align(sizeof(float) * kWave * pieces) +
+         fps_align(sizeof(float) * 8 * pieces);
+}
+size_t fps_states_at(int n, int num_segments) {
+  return fps_pieces_bytes((size_t)fps_first_piece(n, num_segments)) +
+         fps_align(sizeof(uint64_t) * 2 * kFpsShareWords *
+                   (size_t)num_segments);
+}
+
 size_t fps_scratch_bytes(int dtype, int n, int d, int num_segments,
                          int64_t max_rows) {
   if (fps_on_chip(dtype, d, max_rows))
@@ -2366,9 +2425,7 @@ size_t fps_scratch_bytes(int dtype, int n, int d, int num_segments,
     return dist;
   const size_t pieces = (size_t)fps_first_piece(n, num_segments);
   // (a stream that is being captured takes fps_any_kernel and its `dist`)
-  return std::max(dist, fps_align(sizeof(float4) * kWave * pieces) +
-                            fps_align(sizeof(float) * kWave * pieces) +
-                            fps_align(sizeof(float) * 8 * pieces) +
+  return std::max(dist, fps_pieces_bytes(pieces) +
                             fps_share_bytes(num_segments) +
                             std::max(curve_order_bytes(n, num_segments),
                                      fps_align(sizeof(uint32_t) * (size_t)n)));
@@ -2378,7 +2435,7 @@ namespace {
 hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
                              const int64_t *out_ptr, const int64_t *start,
                              int n, int d, int num_segments, int64_t max_rows,
-                             void *scratch, int patience, int64_t *out,
+                             void *scratch, FpsPatience patience, int64_t *out,
                              hipStream_t stream) {
   char *cursor = static_cast<char *>(scratch);
   auto take = [&cursor](size_t bytes) {
@@ -2397,14 +2454,14 @@ hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
   if (most > 0) {
     void *words = take(sizeof(uint64_t) * 2 * kFpsShareWords *
                        (size_t)num_segments);
-    void *failed = take(sizeof(uint32_t) * (size_t)num_segments);
+    void *state = take(sizeof(uint32_t) * (size_t)num_segments);
     int device = 0, units = 0;
     if (rows <= (int64_t)most * 16 * kFpsThreads &&
         hipGetDevice(&device) == hipSuccess &&
         hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount,
                               device) == hipSuccess &&
         units >= kFpsShareGrid)
-      share = {static_cast<uint64_t *>(words), static_cast<uint32_t *>(failed)};
+      share = {static_cast<uint64_t *>(words), static_cast<uint32_t *>(state)};
   }
   const uint32_t *perm = nullptr;
   if (rows <= 16 * kFpsThreads + 1) {
@@ -2429,11 +2486,8 @@ hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
 #define PCA_FPS_SHARED(R_, S_)                                                 \
   hipLaunchKernelGGL((fps_shared_kernel<R_, S_>), dim3(num_segments *most),    \
                      dim3(kFpsThreads), 0, stream, src, ptr, out_ptr, start,   \
-                     d, most, p, share, patience, out)
-    if (rows <= (int64_t)most * 8 * kFpsThreads)
-      PCA_FPS_SHARED(8, 32);
-    else
-      PCA_FPS_SHARED(16, 32);
+                     d, most, p, share, patience.told, patience.came, out)
+    PCA_FPS_SHARED(16, 32);
 #undef PCA_FPS_SHARED
   }
   // (half as many rows to a bucket where the lanes suffice: 8 x 60,000 rows, 600
@@ -2442,7 +2496,7 @@ hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
 #define PCA_FPS_STREAM(S_, MANY_, OWN_)                                        \
   hipLaunchKernelGGL((fps_stream_kernel<kFpsWaves, S_, MANY_, OWN_>),          \
                      dim3(num_segments), dim3(kFpsThreads), 0, stream, src,    \
-                     ptr, out_ptr, start, d, p, share.failed, out)
+                     ptr, out_ptr, start, d, p, share.state, out)
   if (rows <= 16 * kFpsThreads + 1)
     PCA_FPS_STREAM(1, false, true);
   else if (rows <= kWave * kFpsThreads / 2)
@@ -2462,7 +2516,7 @@ hipError_t launch_fps(int dtype, const void *src, const int64_t *ptr,
                       const int64_t *out_ptr, const int64_t *start, int n,
                       int d, int num_segments, int64_t max_rows, void *scratch,
                       bool captured, int64_t *out, hipStream_t stream,
-                      int patience) {
+                      FpsPatience patience) {
   if (fps_on_chip(dtype, d, max_rows)) {
     const float *s = static_cast<const float *>(src);
     if (d <= 2)

@@ -363,15 +363,21 @@ size_t fps_scratch_bytes(int dtype, int n, int d, int num_segments,
                          int64_t max_rows);
 // An example by one or several workgroups.  start: NULL = first row of every example.
 // captured: the stream is being captured into a graph (no sort then).
-// patience: how often a workgroup looks for what another one of its example tells
-// before it gives up (a look takes 0.16 us: 1.3 ms, about a call of eight scans, which
-// may be what the others wait for; see fps_shared_kernel).
-constexpr int kFpsPatience = 8192;
+// patience: where an example is several workgroups', how often one looks for what
+// another one tells, and before that for the others to come, until it goes on without
+// (see fps_shared_kernel).
+struct FpsPatience {
+  int told = 8192;
+  int came = 256;
+};
 hipError_t launch_fps(int dtype, const void *src, const int64_t *ptr,
                       const int64_t *out_ptr, const int64_t *start, int n,
                       int d, int num_segments, int64_t max_rows, void *scratch,
                       bool captured, int64_t *out, hipStream_t stream,
-                      int patience = kFpsPatience);
+                      FpsPatience patience = FpsPatience());
+// Where in the scratch the states of the examples are after a call that shared them
+// (for tests): bit 30 of a word is set if fps_stream_kernel sampled the example.
+size_t fps_states_at(int n, int num_segments);
 
 // --- radius_mc.hip ---------------------------------------------------------
 

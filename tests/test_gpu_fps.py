@@ -216,33 +216,68 @@ def test_entry_points_where_examples_are_shared(oracle, rows, examples, samples)
     assert (got.cpu().numpy() == want).all()
 
 
-@pytest.mark.parametrize("patience", [0, 1, 3])
-def test_workgroups_that_do_not_wait(oracle, patience):
-    """A workgroup that does not hear from the others in time marks its example
-    and ends; another kernel samples that one from the start."""
+def probe_fps(oracle, x, ptr, ratio, max_rows, told=-1, came=-1):
+    """launch_fps with a patience (-1: its own); samples, and which examples
+    one workgroup sampled after all."""
     import ctypes
     import os
     lib = ctypes.CDLL(os.path.join(os.path.dirname(pca.__file__),
                                    "libpca_probe.so"))
+    count = len(ptr) - 1
+    out_ptr = oracle.fps_out_ptr(ptr, ratio, np.float32)
+    bytes_ = capi.capi.pca_fps_workspace_bytes(len(x), x.shape[1], count,
+                                               max_rows, 0)
+    held = [dev(x), dev(ptr, torch.long), dev(out_ptr, torch.long),
+            torch.full((int(out_ptr[-1]),), -1, dtype=torch.long, device=DEV),
+            torch.empty(bytes_, dtype=torch.uint8, device=DEV),
+            torch.zeros(count, dtype=torch.int32, device=DEV)]
+    src, ptr_, out_ptr_, out, work, states = [ctypes.c_void_p(t.data_ptr())
+                                              for t in held]
+    torch.cuda.current_stream().synchronize()
+    assert lib.pca_probe_fps(src, ptr_, out_ptr_, ctypes.c_int64(len(x)),
+                             ctypes.c_int64(x.shape[1]), ctypes.c_int64(count),
+                             ctypes.c_int64(max_rows), ctypes.c_int(told),
+                             ctypes.c_int(came), out, work,
+                             ctypes.c_size_t(bytes_), states) == 0
+    return held[3].cpu().numpy(), (held[5].cpu().numpy() >> 30 & 1).tolist()
+
+
+@pytest.mark.parametrize("told,came", [(0, -1), (1, -1), (3, -1), (-1, 0),
+                                       (-1, 1), (-1, -1)])
+def test_workgroups_that_do_not_wait(oracle, told, came):
+    """A workgroup that does not hear from the others in time marks its example
+    and ends; another kernel samples that one from the start.  One that does not
+    see the others come goes to work with those that did, if they are enough."""
     rng = np.random.default_rng(5)
     ptr = np.array([0, 20000, 21500, 61500], dtype=np.int64)
     x = rng.random((ptr[-1], 3)).astype(np.float32)
     ratio = 0.02
-    out_ptr = oracle.fps_out_ptr(ptr, ratio, np.float32)
-    bytes_ = capi.capi.pca_fps_workspace_bytes(len(x), 3, 3, 40000, 0)
-    held = [dev(x), dev(ptr, torch.long), dev(out_ptr, torch.long),
-            torch.full((int(out_ptr[-1]),), -1, dtype=torch.long, device=DEV),
-            torch.empty(bytes_, dtype=torch.uint8, device=DEV)]
-    src, ptr_, out_ptr_, out, work = [ctypes.c_void_p(t.data_ptr())
-                                      for t in held]
-    torch.cuda.synchronize()
-    assert lib.pca_probe_fps(src, ptr_, out_ptr_, ctypes.c_int64(len(x)),
-                             ctypes.c_int64(3), ctypes.c_int64(3),
-                             ctypes.c_int64(40000), ctypes.c_int(patience),
-                             out, work, ctypes.c_size_t(bytes_)) == 0
-    torch.cuda.synchronize()
-    want = oracle.fps_op(x, ptr, np.float32(ratio))
-    assert (held[3].cpu().numpy() == want).all()
+    got, marked = probe_fps(oracle, x, ptr, ratio, 40000, told, came)
+    assert (got == oracle.fps_op(x, ptr, np.float32(ratio))).all()
+    if told == 0:  # (nobody hears 31 others at the first look, 50 times over)
+        assert marked[2] == 1
+    if told == came == -1:
+        assert marked == [0, 0, 0]
+
+
+def test_units_that_are_held_cost_workgroups_not_the_sharing(oracle):
+    """A wave of another stream's kernel leaves no room on its compute unit: the
+    example goes to the workgroups that came."""
+    rng = np.random.default_rng(6)
+    ptr = np.arange(9, dtype=np.int64) * 33000
+    x = rng.random((ptr[-1], 3)).astype(np.float32)
+    want = oracle.fps_op(x, ptr, np.float32(0.01))
+    probe_fps(oracle, x, ptr, 0.01, 33000)
+    side = [torch.cuda.Stream() for _ in range(3)]
+    for streams in (1, 3):
+        for stream in side[:streams]:
+            with torch.cuda.stream(stream):
+                torch.cuda._sleep(24000000)  # (10 ms)
+        got, marked = probe_fps(oracle, x, ptr, 0.01, 33000)
+        asleep = not side[0].query()
+        torch.cuda.synchronize()
+        assert (got == want).all()
+        assert asleep and marked == [0] * 8
 
 
 def test_shared_examples_on_several_streams():
