@@ -929,8 +929,8 @@ template <int D> struct FpsRanks {
 };
 
 // The low word of a key: the complement of the tie rule's number of a row of up to
-// 2^BITS (BITS + 1 bits of it: never 0, which is no row), then the piece that it is
-// in.
+// 2^BITS (BITS + 1 bits of it: never 0, which is no row), then, in 4 bits, the piece
+// that it is in.
 template <int BITS>
 __device__ __forceinline__ uint32_t fps_code(uint32_t rel, int piece) {
   const uint32_t tie = (rel & 255u) << (BITS - 8) | rel >> 8;
@@ -954,7 +954,9 @@ template <int DIM, int R, int D, int S, int BITS> struct FpsHeld {
   static constexpr int BOXES = kWave / S; // a lane per box and sample
   static constexpr int CHUNKS = (R + BOXES - 1) / BOXES;
   static constexpr bool KEEP = R <= 8; // (16 rows: not the registers; formed again)
-  // boxes (16 pieces and 32 samples a step: in LDS, as registers they are spilled)
+  // boxes (16 pieces and 32 samples a step: in LDS, as registers they are spilled; with
+  // 16 samples a few are, which costs less: 100 x 16,000 rows, 480 samples 441 us, from
+  // LDS 448, and with 12 pieces 100 x 12,000, 600 397, 413)
   static constexpr bool IN_REGS = R <= 8 || S <= 16;
   static_assert(R <= 16, "pieces of 4 bits in a code");
   float x[R][DIM];
@@ -982,7 +984,9 @@ template <int DIM, int R, int D, int S, int BITS> struct FpsHeld {
   }
 
   // `row_at`(i, x): number and coordinates of the i-th row along the curve; piece r
-  // is the rows from `place`(r) on that are before `to`.
+  // is the rows from `place`(r) on that are before `to`.  (Lanes without a row: minimum
+  // 0 and a code below those of rows, another one in every wave, so that waves without
+  // any row have ranks of their own behind all others.)
   template <typename Rows, typename Place>
   __device__ __forceinline__ void load(const Rows &row_at, const Place &place,
                                        int to, const float (&begin_at)[DIM]) {
@@ -993,8 +997,9 @@ template <int DIM, int R, int D, int S, int BITS> struct FpsHeld {
       const bool ok = at < to;
       // (where there is none, the last one again)
       const uint32_t rel = row_at(min(at, to - 1), x[r]);
-      low[r] = __hiloint2double(__float_as_int(ok ? 5e4f : 0.0f),
-                                (int)(ok ? fps_code<BITS>(rel, r) : 0u));
+      low[r] = __hiloint2double(
+          __float_as_int(ok ? 5e4f : 0.0f),
+          (int)(ok ? fps_code<BITS>(rel, r) : threadIdx.x / kWave));
       if (KEEP)
         left[KEEP ? r : 0] = low[r];
     }
@@ -1007,7 +1012,7 @@ template <int DIM, int R, int D, int S, int BITS> struct FpsHeld {
       }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const bool ok = __double2loint(low[r]) != 0;
+      const bool ok = place(r) + lane < to;
       float lo[4] = {}, hi[4] = {};
 #pragma unroll
       for (int c = 0; c < DIM; ++c) {
@@ -1872,10 +1877,13 @@ __global__ __launch_bounds__(kFpsThreads) void fps_shared_kernel(
   const int64_t o_end = out_ptr[b + 1];
   if (o_begin >= o_end || rows <= 0)
     return;
-  // (every wave has a row, and every row a wave)
+  // (Of fewer than 1,024 rows some waves have none.  Such examples were left to
+  // fps_stream_kernel, behind the others: 4 x 20,000 rows, a tenth sampled, and 12 x
+  // 1,000, all sampled, 1,227 -> 629 us; 8 x 9,000 and 8 x 1,023, a fifth, 567 -> 476.)
   const int64_t parts64 =
-      min((int64_t)most, rows / (kFpsWaves * kWave * kFpsShareRows));
-  if (parts64 < 1 || rows > parts64 * R * kFpsThreads) {
+      max((int64_t)1, min((int64_t)most,
+                          rows / (kFpsWaves * kWave * kFpsShareRows)));
+  if (rows > parts64 * R * kFpsThreads) {
     if (threadIdx.x == 0)
       __hip_atomic_store(share.state + b, kFpsMarked, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);

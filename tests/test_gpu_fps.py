@@ -280,6 +280,22 @@ def test_units_that_are_held_cost_workgroups_not_the_sharing(oracle):
         assert asleep and marked == [0] * 8
 
 
+@pytest.mark.parametrize("kind", ["uniform", "grid"])
+def test_short_examples_among_shared_ones_do_not_wait_for_them(oracle, kind):
+    """Examples of fewer rows than two workgroups share are sampled beside the
+    others, by the same kernel."""
+    rng = np.random.default_rng(7)
+    sizes = [20000, 1, 255, 256, 257, 0, 1023, 1024, 2047, 2048]
+    ptr = np.cumsum([0] + sizes).astype(np.int64)
+    x = rng.random((ptr[-1], 3)) if kind == "uniform" else \
+        rng.integers(0, 9, (ptr[-1], 3))
+    x = x.astype(np.float32)
+    share = np.array([0.02] + [0.7] * 9).astype(np.float32)
+    got, marked = probe_fps(oracle, x, ptr, share, 20000)
+    assert (got == oracle.fps_op(x, ptr, share)).all()
+    assert marked == [0] * 10
+
+
 def test_shared_examples_on_several_streams():
     """Calls that each ask for every compute unit, side by side: the workgroups
     of one wait for units that the other holds."""
