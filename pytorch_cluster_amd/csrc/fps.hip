@@ -1867,10 +1867,13 @@ __global__ __launch_bounds__(kFpsThreads) void fps_shared_kernel(
     int64_t *__restrict__ out) {
   __shared__ __align__(16) FpsTold told;
   __shared__ int2 s_crew;
-  int b = blockIdx.x / most;
-  if (gridDim.x / most % 8 == 0)
+  int b = blockIdx.x / most, index = blockIdx.x % most;
+  if (gridDim.x / most % 8 == 0) {
     // (workgroup i is on XCD i % 8)
-    b = (int)(blockIdx.x % 8) + 8 * ((int)(blockIdx.x / 8) / most);
+    const int at_xcd = blockIdx.x / 8;
+    b = (int)(blockIdx.x % 8) + 8 * (at_xcd / most);
+    index = at_xcd % most;
+  }
   const int64_t start_idx = ptr[b];
   const int64_t rows = ptr[b + 1] - start_idx;
   const int64_t o_begin = out_ptr[b];
@@ -1894,8 +1897,10 @@ __global__ __launch_bounds__(kFpsThreads) void fps_shared_kernel(
                       (int)((rows + R * kFpsThreads - 1) / (R * kFpsThreads)),
                       meeting);
   __syncthreads();
-  const int part = __builtin_amdgcn_readfirstlane(s_crew.x);
   const int parts = __builtin_amdgcn_readfirstlane(s_crew.y);
+  // (in order if all came: one scan 420 us of this kernel as they came, 409 in order)
+  const int part = parts == most ? index
+                                 : __builtin_amdgcn_readfirstlane(s_crew.x);
   if (part < 0)
     return;
   const int64_t first = start_idx + (start ? start[b] : 0);
