@@ -194,6 +194,27 @@ def test_examples_of_several_workgroups(oracle, sizes, d, kind):
     assert (got == oracle.fps_op(x, ptr, share, start)).all()
 
 
+# More than 64 examples in curve order, not shared: stretches of 8, 12 and 16 rows of
+# a lane (8,192 and 12,288 rows), other examples beside them.
+@pytest.mark.parametrize("kind", ["uniform", "grid", "odd"])
+@pytest.mark.parametrize("d", [2, 3])
+def test_stretches_of_rows_in_memory(oracle, d, kind):
+    rng = np.random.default_rng(70 + d)
+    sizes = [16384, 12289, 16383, 12288, 8193, 8192, 256, 255] + [300] * 57
+    ptr = np.cumsum([0] + sizes).astype(np.int64)
+    n = ptr[-1]
+    x = rng.integers(0, 17, (n, d)) if kind == "grid" else rng.random((n, d))
+    x = x.astype(np.float32)
+    if kind == "odd":
+        x[rng.random(n) < 0.1] *= 400.0
+        x[rng.random(n) < 0.01, 0] = np.nan
+        x[rng.random(n) < 0.001] = np.inf
+    share = np.array([min(400, 2 * s) / s for s in sizes])
+    start = np.array([s // 2 for s in sizes], dtype=np.int64)
+    got = gpu_fps(oracle, x, ptr, share, start, 16385)
+    assert (got == oracle.fps_op(x, ptr, share, start)).all()
+
+
 # 4,096 rows, 1,100 and 1,600 samples, 16 and 64 examples: where rows that fit one
 # workgroup are shared all the same; 8,192 rows, 170 and 220 samples: where larger
 # ones go through memory; 16,384 / 16,385: rows that are ordered in LDS
@@ -260,6 +281,22 @@ def test_workgroups_that_do_not_wait(oracle, told, came):
         assert marked[2] == 1
     if told == came == -1:
         assert marked == [0, 0, 0]
+
+
+@pytest.mark.parametrize("kind", ["uniform", "grid"])
+@pytest.mark.parametrize("told,came", [(0, -1), (-1, -1)])
+def test_examples_given_up_are_sampled_in_stretches(oracle, told, came, kind):
+    """The same where the other kernel holds the rows in registers (a bound of
+    16,385): 16, 12 and 8 rows of a lane."""
+    rng = np.random.default_rng(8)
+    ptr = np.cumsum([0, 16384, 12289, 12288, 8192, 700]).astype(np.int64)
+    x = rng.random((ptr[-1], 3)) if kind == "uniform" else \
+        rng.integers(0, 17, (ptr[-1], 3))
+    x = x.astype(np.float32)
+    got, marked = probe_fps(oracle, x, ptr, 0.03, 16385, told, came)
+    assert (got == oracle.fps_op(x, ptr, np.float32(0.03))).all()
+    assert marked[:4] == [int(told == 0)] * 4
+    assert told == 0 or marked[4] == 0
 
 
 def test_units_that_are_held_cost_workgroups_not_the_sharing(oracle):
