@@ -434,11 +434,17 @@ int pca_nearest_host(const void *x, const void *y, const int64_t *ptr_x,
  *            segments of up to 16,384 rows are sampled on chip, larger ones
  *            of up to 3 dimensions from rows in curve order, everything else
  *            row by row), or 0 = unknown (row by row; also the faster choice
- *            for a handful of samples from larger segments; more than 16,384
- *            is the faster one for hundreds of samples from segments of
- *            more than 8,192 rows).
- * A stream that is being captured into a graph may be used: segments beyond
- * 16,384 rows (by max_segment_rows) are then sampled row by row.
+ *            for a handful of samples from larger segments).  A bound of
+ *            16,385 for smaller segments of up to 3 dimensions is the faster
+ *            choice from 170 samples of a segment of more than 8,192 rows on
+ *            (more than 16 segments: 220), and of more than 4,096 rows from
+ *            1,100 (17 - 64 segments: 1,600; not of more).
+ * With a bound above 16,384 up to 64 segments are shared by several workgroups
+ * each, 256 in all of 1,024 threads that take a compute unit each for the whole
+ * search.  Those that find one within 30 us (0.5 ms where too few have) share it, so work on
+ * other streams costs the search time, and the other way round; waits are bounded.
+ * A stream that is being captured into a graph may be used: with a bound above
+ * 16,384 segments are then sampled row by row.
  *
  * Stands under the reference operator
  *   torch_cluster::fps(src, ptr, ratio, random_start)

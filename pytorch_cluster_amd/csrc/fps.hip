@@ -1,6 +1,6 @@
 // Farthest point sampling: the `fps` operator of the reference
-// (csrc/cuda/fps_cuda.cu:10-66, fps_kernel), one workgroup of 1,024 threads
-// per example.
+// (csrc/cuda/fps_cuda.cu:10-66, fps_kernel), an example by one workgroup of up to
+// 1,024 threads or by several of 1,024.
 //
 // What the reference computes, and what is reproduced bit for bit: the first
 // sample of an example is its start row; every further sample is the row with
@@ -17,21 +17,27 @@
 //   * `best` starts at -1 and `best_idx` at 0: when no row has a value above
 //     -1 (every distance NaN) the sample is row 0.
 //
-// The sampling is a chain of dependent steps, each an arg-max over the
-// example's rows, so the time per sample is what counts, and an example of up to
-// 8,192 rows is one workgroup's (what several workgroups tell each other takes 1.3 us
-// of a step).  fps_own_kernel, fps_shared_kernel and fps_stream_kernel have several
-// samples per step ("a wave's own stretch of the curve", "the same, an example by
-// several workgroups", "several samples per step").  Up to 256
-// rows of up to 4 dimensions, and up to 1,024 in calls of more examples than there
-// are compute units, fps_reg_kernel looks at
-// every row in every step, from registers.  Beyond that most rows are left
-// alone (see "rows in buckets" below) where more than a hundred or so samples
-// repay the sort: fps_own_kernel up to 8,192 rows and fps_bucket_kernel up to
-// 16,384, from registers, fps_shared_kernel up to 524,288 of few examples, from the
-// registers of several workgroups, and fps_stream_kernel any number in memory (both
-// up to 3 dimensions).  fps_any_kernel (any size, dimension
-// and element type) streams the rows and a `dist` array from memory.
+// The sampling is a chain of dependent steps, each an arg-max over the example's
+// rows, so the time per sample is what counts.  Who samples (fp32; the caller's bound
+// on the rows of an example decides, which for the operators is that of
+// torch_ops.cpp::fps_bound):
+//   * fps_reg_kernel, up to 256 rows of up to 4 dimensions and up to 1,024 in calls of
+//     more than 256 examples: every row in every step, from registers.  So do all
+//     others where few samples are wanted (fps_few, fps_bound).
+//   * Beyond that most rows are left alone (see "rows in buckets" below).
+//     fps_own_kernel, up to 8,192 rows of up to 4 dimensions: one workgroup, several
+//     samples per step ("a wave's own stretch of the curve").
+//   * fps_bucket_kernel, up to 16,384 rows of up to 4 dimensions by such a bound: one
+//     workgroup, one sample per step.
+//   * fps_shared_kernel, up to 524,288 rows of up to 3 dimensions in calls of up to 64
+//     examples: several workgroups, several samples per step ("the same, an example by
+//     several workgroups").  What they tell each other takes 1.3 us of a step.  Any
+//     bound above 16,384 leads here, for the operators also examples of 8,193 - 16,384
+//     rows from 170 (220) samples on and of 4,097 - 8,192 from 1,100 (1,600) on.
+//   * fps_stream_kernel, any number of rows of up to 3 dimensions: one workgroup,
+//     several samples per step ("several samples per step").
+//   * fps_any_kernel, any size, dimension and element type: rows and a `dist` array
+//     stream from memory.
 #include "device_utils.hpp"
 #include "launchers.hpp"
 
