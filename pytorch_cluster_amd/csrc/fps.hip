@@ -911,11 +911,12 @@ __device__ __forceinline__ void fps_few_samples(
 // A wave then tests the boxes of its pieces against all samples at once (16 samples
 // x 4 boxes are its lanes) and goes through the pieces that a sample is near to.
 //
-// Bound by the chain of a step, about 5,000 cycles for nine samples of 4,096 rows:
-// three meetings with an LDS trip each, and the
-// instructions between them, of which the four waves of a SIMD execute their own
-// (1,500 for the entries of a wave whose rows changed, ten of sixteen do, 750 for the
-// rows themselves, 500 for ranks, 400 for pairs and boxes).
+// Bound by the chain of a step, about 5,250 cycles for nine samples of 4,096 rows (by
+// the cycle counter, read after every meeting): 1,100 for the rows of the samples,
+// 2,600 from there to the first meeting (1,400 for the entries of a wave whose rows
+// changed, ten of sixteen do, the rest waits for the slowest), 850 to the second, 700
+// to the third, 400 of them pairs and boxes.  The four waves of a SIMD issue vector
+// instructions, some 150 each, in 53 % of it.
 // 16 uniform clouds, calls, before (64 buckets in LDS, one entry each, the waves
 // sharing the buckets of a step; up to 1,024 rows every row in every step) and now:
 // 1,024 rows, 300 samples 180 -> 100 us; 2,048, 512 258 -> 158;
@@ -1601,10 +1602,11 @@ __global__ __launch_bounds__(kBlock) void fps_gather_kernel(
 // for what another tells (`patience` looks, 1.3 ms, while both run), the example is
 // marked, and fps_stream_kernel, launched behind, samples it from the start.
 //
-// Bound by the chain of a step, about 10,000 cycles for 16 samples of a scan of
-// 200,000 rows by 32 workgroups: rows and entries 2,900 (of the slowest wave), what
-// is told 4,000 (2,500 of 8 workgroups), ranks 1,300, pairs and boxes 900, four
-// meetings.  Calls, us, one workgroup each -> shared: eight scans of 60,000 - 200,000
+// Bound by the chain of a step, about 9,000 cycles for 16 samples of a scan of
+// 200,000 rows by 32 workgroups (by the cycle counter, read after every meeting): rows
+// of the samples and entries 2,500, of the slowest wave, a workgroup's own ranks 1,000,
+// what is told 2,700 (of 16 workgroups 2,050), ranks of all 1,700, pairs and boxes
+// 1,100.  Calls, us, one workgroup each -> shared: eight scans of 60,000 - 200,000
 // rows, 2 % sampled, 2,795 -> 1,001; one of them 1,198 -> 475; uniform rows, 8 x
 // 16,384, 1,000 samples 601 -> 409; 16 x 16,384, a quarter 1,588 -> 741; 64 x 20,000,
 // a tenth 1,783 -> 999; 1 x 500,000, 5,000 samples 9,952 -> 2,407; 128 x 20,000, two
