@@ -420,17 +420,20 @@ class Cases:
             ms, out = _median_ms(
                 t, lambda: t.ops.torch_cluster.fps(pts, ptr, ratio, False),
                 reps or 5)
-            # A step depends on the one before it, so the floor is latency,
-            # not bandwidth or rows (most rows are left alone in a step):
-            # about 100 vector instructions that wait for each other, 4
-            # cycles each, and three trips to the LDS of 64 cycles, at 2.4
-            # GHz.  A step finds at most sixteen samples (about nine in
-            # these clouds), thirty-two where several workgroups share a
-            # cloud, so no sample takes less than that part of it.
-            most = 16 if points <= 8192 else 32
-            units = clouds * (1 if points <= 8192 else min(32, points // 1024))
+            # A step depends on the one before it, so what it takes bounds a
+            # call, not bandwidth or rows (most rows are left alone in a
+            # step).  Counted in these clouds: a wave has 150 vector
+            # instructions per step (116 where several workgroups share a
+            # cloud), the four waves of a SIMD issue them in 4 cycles each,
+            # and results go through the LDS, 64 cycles, three (five) times,
+            # at 2.4 GHz; a step finds nine (eighteen) samples.  What shared
+            # clouds' workgroups tell each other and the waits for the slowest
+            # wave are not in it.
+            shared = points > 8192
+            instructions, trips, found = (116, 5, 18) if shared else (150, 3, 9)
+            units = clouds * (points // 1024 if shared else 1)
             sample_us = ms * 1e3 / (points // 4)
-            floor_us = (100 * 4 + 3 * 64) / 2400.0 / most
+            floor_us = (instructions * 4 * 4 + trips * 64) / 2400.0 / found
             report["fps %dx%d ratio 0.25" % (clouds, points)] = {
                 "ms": ms, "samples": int(out.numel()),
                 "us_per_sample": sample_us,
@@ -438,11 +441,11 @@ class Cases:
                     "bound": "latency", "unit": "us/sample",
                     "floor": floor_us, "achieved": sample_us,
                     "frac": floor_us / sample_us,
-                    "note": "dependent instructions and LDS trips of a step "
-                            "that looks at one piece of rows and finds the "
-                            "most samples it can, %d; "
-                            "clouds run side by side, %d of the chip's "
-                            "256 units busy" % (most, units)}}
+                    "note": "vector issue of a step of the kernel, four "
+                            "waves per SIMD, and its LDS trips, over the %d "
+                            "samples that a step finds; clouds run side by "
+                            "side, %d of the chip's 256 units busy" %
+                            (found, units)}}
         return report
 
     # "auto" against the clock: whole calls of knn / radius / nearest on
