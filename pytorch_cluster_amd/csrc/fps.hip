@@ -31,7 +31,7 @@
 //     workgroup, one sample per step.
 //   * fps_shared_kernel, up to 524,288 rows of up to 3 dimensions in calls of up to 64
 //     examples: several workgroups, several samples per step ("the same, an example by
-//     several workgroups").  What they tell each other takes 1.3 us of a step.  Any
+//     several workgroups").  What they tell each other takes 1.1 us of a step.  Any
 //     bound above 16,384 leads here, for the operators also examples of 8,193 - 16,384
 //     rows from 170 (220) samples on and of 4,097 - 8,192 from 1,100 (1,600) on.
 //   * fps_stream_kernel, any number of rows of up to 3 dimensions: one workgroup,
