@@ -441,9 +441,10 @@ int pca_nearest_host(const void *x, const void *y, const int64_t *ptr_x,
  *            1,100 (17 - 64 segments: 1,600; not of more).
  * With a bound above 16,384 up to 64 segments are shared by several workgroups
  * each, 256 in all of 1,024 threads that take a compute unit each for the whole
- * search.  Those that find a unit within 30 us (0.5 ms where too few have) share the
- * segment, so work on other streams costs the search time, and the other way
- * round; all waits are bounded.
+ * search.  Those that find a unit in time share the segment (30 us; 0.5 ms, or 0.5
+ * us per sample, while fewer than half have or too few for the rows), so work on
+ * other streams costs the search time, and the other way round; all waits are
+ * bounded.
  * A stream that is being captured into a graph may be used: with a bound above
  * 16,384 segments are then sampled row by row.
  *

@@ -9,8 +9,8 @@ Outputs (next to this file, git-ignored):
   _torch_ops.so         TorchScript operator binding (links the above)
   libpca_probe.so       csrc/probes/: measurement and checking aids
                         (`bench.py --probe`, the bf16 rounding check of
-                        tests/test_gpu_dtypes.py, the impatient fps of
-                        tests/test_gpu_fps.py), no part of the searches
+                        tests/test_gpu_dtypes.py, the impatient fps and the held
+                        units of tests/test_gpu_fps.py), no part of the searches
 """
 import argparse
 import concurrent.futures

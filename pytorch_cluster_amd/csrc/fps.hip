@@ -1826,23 +1826,32 @@ fps_shared_rows(const float4 *__restrict__ rows, int count, int part, int parts,
 
 // The workgroups of an example agree on who they are; one thread of each calls this.
 // Returns which one it is, of how many (y); -1: it is not needed.  `most`: at most so
-// many, `least`: as many as hold the rows.  They wait for each other, `patience` looks
-// of 0.12 us (30 us), and 16 times as long (0.5 ms) for the least, which a call of many
-// examples has once its first ones are done.  So units that are held by other work cost
-// a call that wait and their part of the speed, not the sharing.  One word decides, so
+// many, `least`: as many as hold the rows.  They wait for each other: `patience`
+// looks of 0.12 us (30 us) once half of them are there and hold the rows, and while not
+// 16 times as long (0.5 ms) or, if that is more, a patience for every 64 of the `steps`
+// samples, since examples that run make room when they are done and one workgroup
+// takes about twice that for the samples.  So units that are held by other work cost a
+// call that wait and their part of the speed, not the sharing.  One word decides, so
 // all see the same.
 // Calls, us, alone / beside a wave that sleeps on another stream, without this meeting
 // (a held unit cost its example 1.3 ms and the sharing) / now, and beside three: eight
 // scans 1,015 / 3,670 / 996, 1,025; 16 x 16,384 rows, a quarter 740 / 1,450 / 749, 787;
-// 64 x 20,000, a tenth 798 / 1,380 / 814, 1,385.
+// 64 x 20,000, a tenth 798 / 1,380 / 814, 1,385.  Three calls at once, without this
+// meeting / with 30 us for all numbers that hold the rows and 0.5 ms for fewer / now:
+// 5 x 100,000 rows, 2 % 1,580 / 1,571 - 2,820 / 1,583 - 1,659; 8 x 130,000, 2 % 7,200 /
+// 2,079 - 5,268 / 2,084 - 2,881; 16 x 16,384, a quarter 5,300 / 2,130 / 2,160.
+constexpr int kFpsCrewWait = 64; // samples that a patience more is waited for
 __device__ __forceinline__ int2 fps_crew(uint32_t *state, int most, int least,
-                                         int patience) {
+                                         int patience, int steps) {
   constexpr uint32_t CAME = 0xffffu;
   const uint32_t before = __hip_atomic_fetch_add(
       state, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const int part = (int)(before & CAME);
   if ((before & kFpsClosed) != 0 || part >= most)
     return make_int2(-1, 0);
+  const int enough = max(least, most / 2);
+  const int64_t for_enough =
+      (int64_t)patience * max(16, (steps + kFpsCrewWait - 1) / kFpsCrewWait);
   for (int looks = 0;; ++looks) {
     uint32_t now = __hip_atomic_load(state, __ATOMIC_RELAXED,
                                      __HIP_MEMORY_SCOPE_AGENT);
@@ -1854,7 +1863,7 @@ __device__ __forceinline__ int2 fps_crew(uint32_t *state, int most, int least,
     if (here >= most)
       return make_int2(part, most);
     // (tried again only if one more came, at most `most` times)
-    if (looks >= (here >= least ? patience : 16 * patience))
+    if (looks >= (here >= enough ? (int64_t)patience : for_enough))
       __hip_atomic_compare_exchange_strong(
           state, &now,
           now | kFpsClosed | (here < least ? kFpsMarked : 0u) |
@@ -1903,7 +1912,7 @@ __global__ __launch_bounds__(kFpsThreads) void fps_shared_kernel(
   if (threadIdx.x == 0)
     s_crew = fps_crew(share.state + b, (int)parts64,
                       (int)((rows + R * kFpsThreads - 1) / (R * kFpsThreads)),
-                      meeting);
+                      meeting, (int)(o_end - o_begin));
   __syncthreads();
   const int parts = __builtin_amdgcn_readfirstlane(s_crew.y);
   // (in order if all came: one scan 420 us of this kernel as they came, 409 in order)

@@ -239,13 +239,19 @@ def test_entry_points_where_examples_are_shared(oracle, rows, examples, samples)
     assert (got.cpu().numpy() == want).all()
 
 
-def probe_fps(oracle, x, ptr, ratio, max_rows, told=-1, came=-1):
-    """launch_fps with a patience (-1: its own); samples, and which examples
-    one workgroup sampled after all."""
+def probe_library():
     import ctypes
     import os
-    lib = ctypes.CDLL(os.path.join(os.path.dirname(pca.__file__),
-                                   "libpca_probe.so"))
+    return ctypes.CDLL(os.path.join(os.path.dirname(pca.__file__),
+                                    "libpca_probe.so"))
+
+
+def probe_fps(oracle, x, ptr, ratio, max_rows, told=-1, came=-1,
+              before=lambda: None):
+    """launch_fps with a patience (-1: its own); samples, and which examples
+    one workgroup sampled after all.  `before` is called right before it."""
+    import ctypes
+    lib = probe_library()
     count = len(ptr) - 1
     out_ptr = oracle.fps_out_ptr(ptr, ratio, np.float32)
     bytes_ = capi.capi.pca_fps_workspace_bytes(len(x), x.shape[1], count,
@@ -257,6 +263,7 @@ def probe_fps(oracle, x, ptr, ratio, max_rows, told=-1, came=-1):
     src, ptr_, out_ptr_, out, work, states = [ctypes.c_void_p(t.data_ptr())
                                               for t in held]
     torch.cuda.current_stream().synchronize()
+    before()
     assert lib.pca_probe_fps(src, ptr_, out_ptr_, ctypes.c_int64(len(x)),
                              ctypes.c_int64(x.shape[1]), ctypes.c_int64(count),
                              ctypes.c_int64(max_rows), ctypes.c_int(told),
@@ -299,6 +306,25 @@ def test_examples_given_up_are_sampled_in_stretches(oracle, told, came, kind):
     assert told == 0 or marked[4] == 0
 
 
+def streams_beside(count):
+    """Streams whose work does not hold up the current one (streams share a few
+    queues of the hardware)."""
+    found = []
+    for _ in range(32):
+        stream = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            torch.cuda._sleep(2400000)  # (1 ms)
+        torch.zeros(1, device=DEV)
+        torch.cuda.current_stream().synchronize()
+        if not stream.query():
+            found.append(stream)
+        if len(found) == count:
+            torch.cuda.synchronize()
+            return found
+    pytest.skip("no %d streams beside the current one" % count)
+
+
 def test_units_that_are_held_cost_workgroups_not_the_sharing(oracle):
     """A wave of another stream's kernel leaves no room on its compute unit: the
     example goes to the workgroups that came."""
@@ -307,7 +333,7 @@ def test_units_that_are_held_cost_workgroups_not_the_sharing(oracle):
     x = rng.random((ptr[-1], 3)).astype(np.float32)
     want = oracle.fps_op(x, ptr, np.float32(0.01))
     probe_fps(oracle, x, ptr, 0.01, 33000)
-    side = [torch.cuda.Stream() for _ in range(3)]
+    side = streams_beside(3)
     for streams in (1, 3):
         for stream in side[:streams]:
             with torch.cuda.stream(stream):
@@ -317,6 +343,32 @@ def test_units_that_are_held_cost_workgroups_not_the_sharing(oracle):
         torch.cuda.synchronize()
         assert (got == want).all()
         assert asleep and marked == [0] * 8
+
+
+@pytest.mark.parametrize("came", [0, -1])
+def test_workgroups_wait_for_as_many_as_hold_the_rows(oracle, came):
+    """32 units are free, a workgroup's each: 28 take the first example, the four
+    that begin the second wait for a fifth until the first one is done."""
+    import ctypes
+    rng = np.random.default_rng(9)
+    ptr = np.cumsum([0, 70000, 70000] + [40] * 7).astype(np.int64)
+    x = rng.random((ptr[-1], 3)).astype(np.float32)
+    ratio = np.float32(1999.5 / 70000)
+    want = oracle.fps_op(x, ptr, ratio)
+    side, = streams_beside(1)
+
+    def hold(us):
+        assert probe_library().pca_probe_hold(
+            224, us, ctypes.c_void_p(side.cuda_stream)) == 0
+
+    hold(1)
+    assert probe_fps(oracle, x, ptr, ratio, 70000)[1] == [0] * 9
+    got, marked = probe_fps(oracle, x, ptr, ratio, 70000, -1, came,
+                            lambda: hold(4000))
+    held = not side.query()
+    torch.cuda.synchronize()
+    assert held and (got == want).all()
+    assert marked == [0, int(came == 0)] + [0] * 7
 
 
 @pytest.mark.parametrize("kind", ["uniform", "grid"])
