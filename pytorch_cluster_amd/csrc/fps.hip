@@ -2517,7 +2517,14 @@ hipError_t launch_fps_stream(const float *src, const int64_t *ptr,
   hipLaunchKernelGGL((fps_shared_kernel<R_, S_>), dim3(num_segments *most),    \
                      dim3(kFpsThreads), 0, stream, src, ptr, out_ptr, start,   \
                      d, most, p, share, patience.told, patience.came, out)
-    PCA_FPS_SHARED(16, 32);
+    // (rows of a lane at most: with 16 a quarter of the workgroups can do what all do
+    // with four; where two rows are enough for all, eight are that many.  The kernel
+    // without 16 is the faster one there, calls, us, with / without: 16 x 16,384 rows, a
+    // quarter 740 / 730; 16 x 8,000, 1,200 samples 372 / 365)
+    if (rows <= (int64_t)most * 2 * kFpsThreads)
+      PCA_FPS_SHARED(8, 32);
+    else
+      PCA_FPS_SHARED(16, 32);
 #undef PCA_FPS_SHARED
   }
   // (half as many rows to a bucket where the lanes suffice: 8 x 60,000 rows, 600
